@@ -487,8 +487,7 @@ int kr_cast_f32_to_fp8(const void* src, int64_t n, void* dst, void* stream);
  *   out_kind: 0 = bf16, 1 = fp32, 2 = fp8 (e4m3fn; fp32 sums rounded once, nearest even, magnitudes
  *   from 448 on give +-448, NaN stays NaN -- the conversion of kr_cast_f32_to_fp8); out is [M, N]
  *   contiguous.
- * M % 256 == 0, N % 256 == 0, K % 128 == 0 (other shapes: convert with kr_cast_fp8_to_bf16 and use the
- * bf16 entry points); lda, ldb >= K and multiples of 16; pointers 16-byte aligned.
+ * M % 256 == 0, N % 256 == 0, K % 128 == 0 (other shapes: kr_gemm_fp8_ws); lda, ldb >= K and multiples of 16; pointers 16-byte aligned.
  */
 int kr_gemm_fp8(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
                 void* out, int out_kind, void* stream);
@@ -507,6 +506,21 @@ int kr_all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, in
                              void* stream);
 
 /*
+ * The same two products for any number of rows, N and K multiples of 16, K >= 128 (edge tiles and a last
+ * k-step that is not full are handled by the kernel).  kr_gemm_fp8_ws: with a workspace of
+ * kr_gemm_fp8_workspace_bytes bytes (0: none needed), shapes with few tiles share each tile's K loop
+ * between workgroups, whose fp32 parts meet there and are summed in a fixed order; contents are scratch,
+ * and calls that may overlap need one each.
+ */
+int64_t kr_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int kr_gemm_fp8_ws(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                   void* out, int out_kind, void* workspace, int64_t workspace_bytes, void* stream);
+int kr_all_gather_matmul_fp8_ragged(const void* A, int64_t lda, const void* A_local, int64_t lda_local, const void* Bt,
+                                    int64_t ldb, int64_t M, int64_t N, int64_t K, int W, int rank, int splits_per_rank,
+                                    const uint32_t* progress, int64_t wait_limit_us, int32_t* status, void* out,
+                                    int out_kind, void* stream);
+
+/*
  * Which kernel kr_gemm_reduce_*_bf16 would run for a shape (contiguous operands), decided by the
  * same code that launches it; for benchmarks and logs that want to name the kernel they timed.
  * No counterpart in the reference (its tile sizes are keyword arguments of the wrappers,
@@ -519,7 +533,7 @@ int kr_all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, in
  *   plan[3] 256 tile: tiles of the last partial round that are split, plan[4] parts of each
  *   plan[5] column panels per scheduling group
  *   plan[6] 1: tiles that lie wholly in the reduce band add the peers on the matrix cores
- *   plan[7] bit 0: M or N is not a multiple of the tile (bounds-checked edge tiles); bit 1: the
+ *   plan[7] bit 0: M or N is not a multiple of the tile or K of 64 (bounds-checked edges); bit 1: the
  *           tile is 256 x 224 (a plain product with transposed-contiguous B that fills whole rounds
  *           of the compute units with 224-column tiles and not with 256-column ones)
  */

@@ -456,6 +456,28 @@ static int64_t gemm_dtl_tail_workspace_bytes(int tail_tiles, int splits) {
     return (int64_t)tail_tiles * splits * (256 * 256 * 4);
 }
 
+// fp8 operands: which tiles share their K loop, and how many workgroups each gets.  With at most 128 tiles
+// the whole launch is a partial round (half the compute units or more would idle) and every tile may be
+// split; otherwise the rule of the bf16 kernel, on the same number of k-steps (one is 128 long here).
+// A k-step takes 0.9 us, a part that is written and summed 0.09 us, the finishing launch 3 us; the split
+// with the least sum is taken if it saves a tenth of the k loop.  Measured (one pass / split, us):
+// 64 x 6656 x 8192 66 / 29 in 5 parts (34 in 8), 512 x 6656 x 8192 66 / 45 in 4, 1024 x 6656 x 16384 142 / 107
+// in 2, but 1024 x 6656 x 4096 38 / 48 and 512 x 6656 x 2048 23 / 32, which stay in one pass.
+static void fp8_split_plan(int64_t M, int64_t N, int64_t K, int* tail_out, int* splits_out) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), steps = (K + 127) / 128;
+    *tail_out = 0;
+    *splits_out = 1;
+    if (tiles > 128) return tail_split_plan(tiles, K / 2, tail_out, splits_out);
+    int64_t best = 81 * steps;   // nine tenths of the one-pass k loop, in 0.01 us
+    for (int64_t s = 2; s <= kMaxTailSplits && s * tiles <= 256 && s <= steps / 4; ++s) {
+        const int64_t cost = 90 * steps / s + 9 * tiles * s + 300;
+        if (cost >= best) continue;
+        best = cost;
+        *tail_out = (int)tiles;
+        *splits_out = (int)s;
+    }
+}
+
 // Few rows, long K: whether the 256x256 kernel with every tile's K loop split (the whole launch
 // treated as a partial round) beats the 128x128 kernel with its split.  Measured on N = 6656,
 // M = 256 / 512 / 1024 (26 / 52 / 104 tiles), caches flushed: row-major B wins from K = 4096 on
@@ -517,8 +539,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
                           bool dtl_ok) {
     GemmPlan p{};
     // Tile choice: the 256x256 tile of the LDS-DMA kernel (4 waves x 128x128) has the highest
-    // MFMA work per LDS/HBM byte; it needs K % 64 == 0 and a K loop long enough to amortise
-    // its epilogue.  Otherwise 128x128 tiles, two of which share a CU so that one
+    // MFMA work per LDS/HBM byte; it needs a K loop long enough to amortise its epilogue.  Otherwise 128x128 tiles, two of which share a CU so that one
     // tile's epilogue overlaps the other's MFMAs; they also win while all of them fit on the
     // 256 CUs at once (512 tiles = 128 of the large ones): measured, the large tile is 15-30 %
     // faster from 144 tiles on and 5-10 % slower at 128, for K from 1024 to 8192.
@@ -564,7 +585,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     // 256x256 kernel: the last partial round of tiles, split over the idle CUs (workspace given)
     p.tail_tiles = 0;
     p.tail_splits = 1;
-    if (dtl && has_workspace && !has_progress && M % 256 == 0 && N % 256 == 0) {
+    if (dtl && has_workspace && !has_progress && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
         int tail, ts;
         tail_split_plan(tiles_m * tiles_n, K, &tail, &ts);
         if (tail > 0 && gemm_dtl_tail_workspace_bytes(tail, ts) <= workspace_bytes) {
@@ -581,7 +602,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     // (An A that arrives while the kernel runs is fine: the tile waits for its rows' flags before its
     // first load, whatever its width.)
     p.n224 = 0;
-    if (dtl && p.mi16 && b_nt && plain && plain_bf16_all_rows && M % 256 == 0 && N % 224 == 0) {
+    if (dtl && p.mi16 && b_nt && plain && plain_bf16_all_rows && M % 256 == 0 && N % 224 == 0 && K % 64 == 0) {
         const int64_t t8 = tiles_m * tiles_n, t7 = (M / 256) * (N / 224);
         const double cost8 = (double)((t8 + 255) / 256) * 256.0, cost7 = (double)((t7 + 255) / 256) * 224.0 * 1.03;
         bool use = cost7 < cost8;
@@ -835,12 +856,15 @@ extern "C" int kr_gemm_producer_bf16(const void* A, int64_t lda_m, int64_t lda_k
 // Product of fp8 (e4m3fn) operands on the fp8 matrix-core instruction (all_gather_matmul.py:53,121,213: fp8 shards and
 // weight, fp8 result).  The kernel is the 256x256 LDS-DMA kernel with its k-step on 16x16x128 blocks; it reads the operands
 // as matrices of two-byte units, hence the halved K and row strides below.  `gather`: rows of A that arrive while the
-// kernel runs (flags, local shard), as for the bf16 all-gather matmul.
+// kernel runs (flags, local shard), as for the bf16 all-gather matmul.  whole_tiles: the entry points
+// that take whole tiles only.
 static int gemm_fp8(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
-                    void* out, int out_kind, void* stream, const GatherSpec* gather) {
+                    void* out, int out_kind, void* stream, const GatherSpec* gather, bool whole_tiles,
+                    void* workspace = nullptr, int64_t workspace_bytes = 0) {
     if (M < 0 || N < 0 || K < 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return KR_ERR_BAD_DIM;
     if (out_kind < 0 || out_kind > 2) return KR_ERR_BAD_DIM;
-    if (M % 256 != 0 || N % 256 != 0 || K % 128 != 0) return KR_ERR_BAD_DIM;
+    if (whole_tiles ? (M % 256 != 0 || N % 256 != 0 || K % 128 != 0) : (N % 16 != 0 || K % 16 != 0 || (K > 0 && K < 128)))
+        return KR_ERR_BAD_DIM;
     if (M == 0 || N == 0) return KR_OK;
     if (K == 0) return KR_ERR_BAD_DIM;
     if (A == nullptr || Bt == nullptr || out == nullptr) return KR_ERR_NULL_POINTER;
@@ -873,24 +897,45 @@ static int gemm_fp8(const void* A, int64_t lda, const void* Bt, int64_t ldb, int
     g.out = out;
     g.out_is_fp32 = out_kind == 1;
     g.out_fp8 = out_kind == 2;
-    g.tiles_m = (int)(M / 256);
-    g.tiles_n = (int)(N / 256);
+    g.tiles_m = (int)((M + 255) / 256);
+    g.tiles_n = (int)((N + 255) / 256);
     g.pivot_tiles = (int)((pivot_row / 256) % g.tiles_m);
     g.group_n = env_switches().gemm_group > 0 ? env_switches().gemm_group : 4;
     g.k_splits = 1;
     g.mi16 = 1;
-    return (int)launch_gemm_dtl8(g, (hipStream_t)stream);
+    if (workspace != nullptr && g.progress == nullptr) {
+        if (!aligned16(workspace)) return KR_ERR_ALIGNMENT;
+        int tail, ts;
+        fp8_split_plan(M, N, K, &tail, &ts);
+        if (tail > 0 && gemm_dtl_tail_workspace_bytes(tail, ts) <= workspace_bytes) {
+            g.tail_tiles = tail;
+            g.k_splits = ts;
+        }
+    }
+    return (int)launch_gemm_dtl8(g, (hipStream_t)stream, workspace);
 }
 
 extern "C" int kr_gemm_fp8(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
                            void* out, int out_kind, void* stream) {
-    return gemm_fp8(A, lda, Bt, ldb, M, N, K, out, out_kind, stream, nullptr);
+    return gemm_fp8(A, lda, Bt, ldb, M, N, K, out, out_kind, stream, nullptr, true);
 }
 
-extern "C" int kr_all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, int64_t lda_local, const void* Bt,
-                                        int64_t ldb, int64_t M, int64_t N, int64_t K, int W, int rank, int splits_per_rank,
-                                        const uint32_t* progress, int64_t wait_limit_us, int32_t* status, void* out,
-                                        int out_kind, void* stream) {
+extern "C" int64_t kr_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K < 128) return 0;
+    int tail, ts;
+    fp8_split_plan(M, N, K, &tail, &ts);
+    return tail > 0 ? gemm_dtl_tail_workspace_bytes(tail, ts) : 0;
+}
+
+extern "C" int kr_gemm_fp8_ws(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                              void* out, int out_kind, void* workspace, int64_t workspace_bytes, void* stream) {
+    return gemm_fp8(A, lda, Bt, ldb, M, N, K, out, out_kind, stream, nullptr, false, workspace, workspace_bytes);
+}
+
+static int all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, int64_t lda_local, const void* Bt,
+                                 int64_t ldb, int64_t M, int64_t N, int64_t K, int W, int rank, int splits_per_rank,
+                                 const uint32_t* progress, int64_t wait_limit_us, int32_t* status, void* out,
+                                 int out_kind, void* stream, bool whole_tiles) {
     if (W < 1 || W > KR_MAX_WORLD) return KR_ERR_WORLD_SIZE;
     if (rank < 0 || rank >= W || splits_per_rank < 1) return KR_ERR_STRIPE;
     if (M < 0 || M % ((int64_t)W * splits_per_rank) != 0) return KR_ERR_BAND;
@@ -907,7 +952,23 @@ extern "C" int kr_all_gather_matmul_fp8(const void* A, int64_t lda, const void* 
     gs.comm_rows = M > 0 ? M / ((int64_t)W * splits_per_rank) : 1;
     gs.wait_limit_us = wait_limit_us > 0 ? wait_limit_us : 5000000;   // 5 s
     gs.status = status;
-    return gemm_fp8(A, lda, Bt, ldb, M, N, K, out, out_kind, stream, &gs);
+    return gemm_fp8(A, lda, Bt, ldb, M, N, K, out, out_kind, stream, &gs, whole_tiles);
+}
+
+extern "C" int kr_all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, int64_t lda_local, const void* Bt,
+                                        int64_t ldb, int64_t M, int64_t N, int64_t K, int W, int rank, int splits_per_rank,
+                                        const uint32_t* progress, int64_t wait_limit_us, int32_t* status, void* out,
+                                        int out_kind, void* stream) {
+    return all_gather_matmul_fp8(A, lda, A_local, lda_local, Bt, ldb, M, N, K, W, rank, splits_per_rank, progress,
+                                 wait_limit_us, status, out, out_kind, stream, true);
+}
+
+extern "C" int kr_all_gather_matmul_fp8_ragged(const void* A, int64_t lda, const void* A_local, int64_t lda_local, const void* Bt,
+                                        int64_t ldb, int64_t M, int64_t N, int64_t K, int W, int rank, int splits_per_rank,
+                                        const uint32_t* progress, int64_t wait_limit_us, int32_t* status, void* out,
+                                        int out_kind, void* stream) {
+    return all_gather_matmul_fp8(A, lda, A_local, lda_local, Bt, ldb, M, N, K, W, rank, splits_per_rank, progress,
+                                 wait_limit_us, status, out, out_kind, stream, false);
 }
 
 extern "C" int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, int n_peers, int64_t band_rows,
@@ -932,7 +993,7 @@ extern "C" int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, i
     plan[4] = p.tail_splits;
     plan[5] = p.group_n;
     plan[6] = whole_band_peers ? 1 : 0;
-    plan[7] = (M % p.tile != 0 || N % p.tile != 0) ? 1 : 0;
+    plan[7] = (M % p.tile != 0 || N % p.tile != 0 || K % 64 != 0) ? 1 : 0;
     if (p.n224) plan[7] |= 2;   // bit 1: 256 x 224 tiles
     return KR_OK;
 }
@@ -944,8 +1005,8 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     bool big = ((M + 255) / 256) * ((N + 255) / 256) > 128 && K >= 256;
     if (force_tile == 128) big = false;
     if (force_tile == 256) big = true;
-    if (big && K % 64 == 0 && K >= 64) {
-        if (M % 256 != 0 || N % 256 != 0) return 0;
+    if (big && K >= 64) {
+        if (M % 256 != 0 || N % 256 != 0 || K % 64 != 0) return 0;
         int tail, ts;
         tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
         return tail > 0 ? gemm_dtl_tail_workspace_bytes(tail, ts) : 0;

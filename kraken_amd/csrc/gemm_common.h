@@ -64,10 +64,10 @@ inline hipError_t lds_opt_in(const void* fn, int bytes, std::atomic<uint64_t>& d
     return hipSuccess;
 }
 
-// LDS-DMA kernel for shapes the 256x256 tile divides (gemm_dtl.hip)
+// LDS-DMA kernel with 256x256 tiles (gemm_dtl.hip)
 bool gemm_dtl_supported(const GemmArgs& g);
 hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* workspace);
-hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st);   // fp8 operands (gemm_dtl.hip)
+hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace);   // fp8 operands (gemm_dtl.hip)
 
 constexpr int kXcds = 8;
 

@@ -1,5 +1,5 @@
-// bf16 GEMM main loop with direct global->LDS loads ("LDS DMA"), 256x256 tiles, for K % 64 == 0
-// (M and N may be ragged: the tiles at the lower and right edge are handled below).
+// GEMM main loop with direct global->LDS loads ("LDS DMA"), 256x256 tiles (M, N and K may be ragged:
+// the tiles at the lower and right edge and a last k-step that is not full are handled below).
 //
 // Workgroup tile 256 x 256, four wavefronts (2 x 2), each owning 128 x 128 of C as 4 x 4
 // v_mfma_f32_32x32x16_bf16 accumulators (256 AGPRs).  The k loop advances 64 at a time through a
@@ -107,9 +107,10 @@ __device__ __forceinline__ uint32_t pack2_e4m3(float a, float b, uint32_t old) {
 // row l%16, columns 4(l/16) .. +3 of a block): per 16-row slab a lane's four values of a block become
 // one word of a per-wave LDS patch [16][128 + 16] bytes (the pad keeps the 64 word stores of a block on
 // 64 banks), and the slab leaves as 16-byte chunks of whole 128-byte rows.  `dst`: the wave's first
-// row and column; ld in bytes.
+// row and column; ld in bytes.  MASKED: only the first `rows` rows and `cols` columns (a multiple of 16) exist.
+template <bool MASKED>
 __device__ __forceinline__ void store_tile_fp8_blocks(const f32x4 (&acc16)[2 * TM][2 * TN], unsigned char* smem, uint8_t* dst, int64_t ld,
-                                                      int lane, int wave) {
+                                                      int lane, int wave, int rows, int cols) {
     constexpr int COLS = 2 * TN * 16, LD = COLS + 16, CPR = COLS / 16;
     static_assert(16 * CPR == 128, "two chunks per lane and slab");
     unsigned char* patch = smem + wave * 4096;
@@ -129,7 +130,7 @@ __device__ __forceinline__ void store_tile_fp8_blocks(const f32x4 (&acc16)[2 * T
         for (int it = 0; it < 2; ++it) {
             const int idx = it * 64 + lane, r = idx / CPR, c = idx % CPR;
             const u32x4 v = *(const u32x4*)(patch + r * LD + c * 16);
-            st_stream((u32x4*)(dst + (int64_t)(16 * i + r) * ld + c * 16), v);
+            if (!MASKED || (16 * i + r < rows && c * 16 < cols)) st_stream((u32x4*)(dst + (int64_t)(16 * i + r) * ld + c * 16), v);
         }
         asm volatile("" ::: "memory");   // the next slab's stores stay behind these reads
     }
@@ -139,7 +140,8 @@ __device__ __forceinline__ void store_tile_fp8_blocks(const f32x4 (&acc16)[2 * T
 // partial sums, k loop) for tiles whose peers are added on the matrix cores.
 // SPLIT: the workgroup is one of g.k_splits that share a tile of the last partial round: it
 // runs its share of the k-steps and leaves its accumulators in the workspace (no epilogue).
-// RAGGED: M or N is not a multiple of 256 (edge tiles get the bounds-checked epilogue).
+// RAGGED: M or N is not a multiple of 256 (edge tiles get the bounds-checked epilogue) or K not of 64
+// (the pieces past K of the last k-step are requested out of range, which puts zeros into the LDS stage).
 // MI16: the k loop uses v_mfma_f32_16x16x32_bf16 (8 x 8 blocks of 16 x 16 per wave) instead of
 // 32x32x16 (4 x 4 blocks of 32 x 32): same operand traffic, but the matrix cores draw less power
 // per flop with it (under the power limit, matrix-core-only loops on random operands sustain
@@ -155,7 +157,7 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     // F8: the operands are fp8 (e4m3fn) and g describes them as bf16 matrices of half the width (g.K, g.lda, g.ldb in
     // two-byte units), so a stage still holds 128-byte rows -- 128 k now -- and every load and LDS address below is unchanged;
     // only the k-step differs (k_step8: 16x16x128 MFMAs on the same 16 x 16 accumulator blocks).
-    static_assert(!F8 || (MI16 && B_NT && !SPLIT && !RAGGED && !PEERS_FIRST && NB == 2 * TN), "fp8: plain NT products on whole tiles");
+    static_assert(!F8 || (MI16 && B_NT && !PEERS_FIRST && NB == 2 * TN), "fp8: plain NT products");
     constexpr int BNX = WN * NB * 16;                            // columns of the workgroup tile
     constexpr int WTNX = NB * 16;                                // columns of a wave
     constexpr int LOADS_B = BNX * BKD * 2 / 1024 / (WM * WN);    // LDS-DMA loads of B per wave per k-step: 8 or 7
@@ -178,7 +180,7 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
                   tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BNX;
     // k-steps of this workgroup: all of them, or the split's share
-    const int kt_all = g.K / BKD;
+    const int kt_all = RAGGED ? (g.K + BKD - 1) / BKD : g.K / BKD;
     const int kt_begin = SPLIT ? (int)((int64_t)kt_all * split / g.k_splits) : 0;
     const int kt_total = SPLIT ? (int)((int64_t)kt_all * (split + 1) / g.k_splits) - kt_begin : kt_all;
     const int k_begin = kt_begin * BKD;
@@ -199,8 +201,17 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     const int dma_sw = (4 * (wave & 1) + (lane >> 4)) & 7;
     const uint32_t a_voff_lane = (uint32_t)(((int64_t)(lane >> 3) * lda + (((lane & 7) ^ dma_sw) << 3)) * 2);
     uint32_t b_voff_lane, b_voff_odd = 0;
+    // RAGGED: the lane offsets of the last k-step of the matrix.  A piece at or past K gets an offset past
+    // every descriptor's end (it would otherwise be the start of the next row): such a load fetches
+    // nothing and writes zeros to its LDS slot (measured), so the k-step multiplies zeros there.
+    // (Row-major B needs no such offsets: its k-rows past K lie past the matrix' end.)
+    constexpr uint32_t kOob = 0x80000000u;
+    const int t_tail = RAGGED ? kt_all - 1 - kt_begin : 0;
+    uint32_t a_voff_tail = 0, b_voff_tail = 0;
+    if (RAGGED) a_voff_tail = (((lane & 7) ^ dma_sw) << 3) < g.K - (kt_all - 1) * BKD ? a_voff_lane : kOob;
     if (B_NT) {
         b_voff_lane = (uint32_t)(((int64_t)(lane >> 3) * g.ldb + (((lane & 7) ^ dma_sw) << 3)) * 2);
+        if (RAGGED) b_voff_tail = a_voff_tail == kOob ? kOob : b_voff_lane;
     } else {
         // row-major B: chunk = 2 k-rows of 512 B; lane l -> k-row l/32, piece slot l%32 holds piece
         // slot ^ 4*(k & 3); k & 3 = 2*(chunk & 1) + l/32 and chunk & 1 == wave & 1
@@ -254,8 +265,9 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
         const bool live = t < kt_total;
         const int tt = min(t, kt_total - 1);
         const int k0 = tt * BKD;
-        const uint32_t a_voff = live ? a_voff_lane : 0u;
-        const uint32_t b_voff = !live ? 0u : (MI16 && !B_NT && ((q % LOADS_A) & 1)) ? b_voff_odd : b_voff_lane;
+        const bool tail = RAGGED && t == t_tail;
+        const uint32_t a_voff = !live ? 0u : tail ? a_voff_tail : a_voff_lane;
+        const uint32_t b_voff = !live ? 0u : (MI16 && !B_NT && ((q % LOADS_A) & 1)) ? b_voff_odd : B_NT && tail ? b_voff_tail : b_voff_lane;
         const int ch = wave + 4 * (q % LOADS_A);
         if (q < LOADS_A) {
             lds_dma_b128(a_rsrc, stage * A_ST + ch * 1024, a_voff, (int)(((int64_t)8 * ch * lda + k0) * 2));
@@ -926,8 +938,11 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     pin_accumulators();
     // peers and bias that are already in the accumulators are not added again
     if (F8 && g.out_fp8) {
-        if constexpr (F8)
-            store_tile_fp8_blocks(acc16, smem, (uint8_t*)g.out + (int64_t)(m0 + wm * WTM) * g.N + n0 + wn * WTN, g.N, lane, wave);
+        if constexpr (F8) {
+            uint8_t* dst = (uint8_t*)g.out + (int64_t)(m0 + wm * WTM) * g.N + n0 + wn * WTN;
+            if (full_tile) store_tile_fp8_blocks<false>(acc16, smem, dst, g.N, lane, wave, 0, 0);
+            else if constexpr (RAGGED) store_tile_fp8_blocks<true>(acc16, smem, dst, g.N, lane, wave, g.M - m0 - wm * WTM, g.N - n0 - wn * WTN);
+        }
     } else if constexpr (NB != 2 * TN) {
         // 224-column tile of a plain product: every row goes to `out`
         store_tile_bf16_blocks<NB>(acc16, smem, (uint16_t*)g.out + (int64_t)(m0 + wm * WTM) * g.N + n0 + wn * WTNX, g.N, lane, wave);
@@ -971,28 +986,21 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl16n7_kernel(const GemmArg
     gemm_dtl_tile<true, false, false, false, true, 7>(g, smem);
 }
 
-// fp8 (e4m3fn) operands, transposed-contiguous B, whole 256 x 256 tiles; the result is fp8, bf16 or fp32.
+// fp8 (e4m3fn) operands, transposed-contiguous B; the result is fp8, bf16 or fp32.
+template <bool RAGGED>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl8_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gemm_dtl_tile<true, false, false, false, true, 2 * TN, true>(g, smem);
+    gemm_dtl_tile<true, false, false, RAGGED, true, 2 * TN, true>(g, smem);
 }
 
 }  // namespace
 
-// g as for the bf16 kernel with the fp8 operands described in two-byte units (K, lda, ldb halved).
-hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st) {
-    static std::atomic<uint64_t> opted;
-    if (hipError_t e = lds_opt_in((const void*)gemm_dtl8_kernel, LDS_BYTES, opted); e != hipSuccess) return e;
-    hipLaunchKernelGGL(gemm_dtl8_kernel, dim3((unsigned)(g.tiles_m * g.tiles_n)), dim3(WM * WN * 64), LDS_BYTES, st, g);
-    return hipGetLastError();
-}
-
 // Second launch of a call with a split tail: g.k_splits workgroups per tile of the last partial
 // round (g.out = workspace).
-template <bool B_NT, bool MI16>
+template <bool B_NT, bool MI16, bool RAGGED = false, bool F8 = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_split_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gemm_dtl_tile<B_NT, false, true, false, MI16>(g, smem);
+    gemm_dtl_tile<B_NT, false, true, RAGGED, MI16, 2 * TN, F8>(g, smem);
 }
 
 // Third launch: sums the parts of every tail tile in the order 0..S-1 and applies the epilogue
@@ -1024,6 +1032,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
         n = tile_n * BN + (wave % WN) * WTN + j * 32 + 8 * v4 + 4 * (lane >> 5);
     }
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    if (m >= g.M || n >= g.N) return;   // an edge tile's missing rows and columns (N is a multiple of 8)
+    if (g.out_fp8) {
+        *(uint32_t*)((uint8_t*)g.out + (int64_t)m * g.N + n) = pack2_e4m3<true>(sum.z, sum.w, pack2_e4m3<false>(sum.x, sum.y, 0u));
+        return;
+    }
     const int mb = m - g.band_row0;
     if (mb < 0 || mb >= g.band_rows) {
         if (g.c_full != nullptr)
@@ -1061,13 +1074,13 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
 }
 
 bool gemm_dtl_supported(const GemmArgs& g) {
-    return g.K % BKD == 0 && g.K >= BKD &&
+    return g.K % 8 == 0 && g.K >= BKD &&
            (int64_t)BM * g.lda * 2 < 0x7fffffffLL && (int64_t)(BN > 64 ? BN : 64) * g.ldb * 2 < 0x7fffffffLL;
 }
 
 hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* workspace) {
     const dim3 grid((unsigned)(g.tiles_m * g.tiles_n - g.tail_tiles)), block(WM * WN * 64);
-    const bool ragged = g.M % BM != 0 || g.N % BN != 0;
+    const bool ragged = g.M % BM != 0 || g.N % BN != 0 || g.K % BKD != 0;
     const void* kfn = b_nt ? (ragged ? (const void*)gemm_dtl_kernel<true, true> : (const void*)gemm_dtl_kernel<true, false>)
                            : (ragged ? (const void*)gemm_dtl_kernel<false, true> : (const void*)gemm_dtl_kernel<false, false>);
     if (g.mi16)
@@ -1120,6 +1133,34 @@ hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* w
         }
         e = hipGetLastError();
         if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(gemm_dtl_tail_finish_kernel, dim3((unsigned)(g.tail_tiles * TM * TN * 4)), block, 0, st, g,
+                           (const f32x4*)workspace);
+    }
+    return hipGetLastError();
+}
+
+// g as for the bf16 kernel with the fp8 operands described in two-byte units (K, lda, ldb halved);
+// g.tail_tiles tiles are split over g.k_splits workgroups each, as for the bf16 kernel.
+hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace) {
+    const bool ragged = g.M % BM != 0 || g.N % BN != 0 || g.K % BKD != 0;
+    const dim3 grid((unsigned)(g.tiles_m * g.tiles_n - g.tail_tiles)), block(WM * WN * 64);
+    static std::atomic<uint64_t> opted[4];
+    if (grid.x > 0) {
+        const void* kfn = ragged ? (const void*)gemm_dtl8_kernel<true> : (const void*)gemm_dtl8_kernel<false>;
+        if (hipError_t e = lds_opt_in(kfn, LDS_BYTES, opted[ragged]); e != hipSuccess) return e;
+        if (ragged) hipLaunchKernelGGL(gemm_dtl8_kernel<true>, grid, block, LDS_BYTES, st, g);
+        else hipLaunchKernelGGL(gemm_dtl8_kernel<false>, grid, block, LDS_BYTES, st, g);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    if (g.tail_tiles > 0) {
+        GemmArgs gs = g;
+        gs.out = workspace;
+        const dim3 sgrid((unsigned)(g.tail_tiles * g.k_splits));
+        const void* sfn = ragged ? (const void*)gemm_dtl_split_kernel<true, true, true, true> : (const void*)gemm_dtl_split_kernel<true, true, false, true>;
+        if (hipError_t e = lds_opt_in(sfn, LDS_BYTES, opted[2 + ragged]); e != hipSuccess) return e;
+        if (ragged) hipLaunchKernelGGL((gemm_dtl_split_kernel<true, true, true, true>), sgrid, block, LDS_BYTES, st, gs);
+        else hipLaunchKernelGGL((gemm_dtl_split_kernel<true, true, false, true>), sgrid, block, LDS_BYTES, st, gs);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         hipLaunchKernelGGL(gemm_dtl_tail_finish_kernel, dim3((unsigned)(g.tail_tiles * TM * TN * 4)), block, 0, st, g,
                            (const f32x4*)workspace);
     }

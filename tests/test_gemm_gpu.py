@@ -1086,3 +1086,52 @@ def test_split_tiles_round_like_unsplit_tiles(dev, monkeypatch, peers_mode, mfma
     once = (prod + peers.float().sum(0) + bias.float()).to(BF16)
     twice = (prod.to(BF16).float() + peers.float().sum(0) + bias.float()).to(BF16)
     assert not torch.equal(once, twice)
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 128), (255, 272, 144), (257, 240, 1040), (300, 528, 2064), (2049, 4112, 272), (4096, 272, 1136)])
+def test_fp8_kernel_ragged_shapes(dev, M, N, K, split):
+    """kr_gemm_fp8_ws on sizes no tile divides: one row, one column block, a row or column more or less than a
+    tile, every kind of last k-step (16, 32, 96, 112 of 128 k), one tile up to more than a round of them, with and
+    without the split of the K loop.  Small integers and halves: every fp32 sum is exact, so all result types
+    equal the exact product bit for bit; what lies between the rows (stride > K) must not be read."""
+    fp8 = torch.float8_e4m3fn
+    g = torch.Generator().manual_seed(M + N + K)
+    lda, ldb = K + 16, K + 32
+    a, b = torch.full((M, lda), 3.0).to(fp8), torch.full((N, ldb), 3.0).to(fp8)
+    a[:, :K] = torch.randint(-2, 3, (M, K), generator=g).float().to(fp8)
+    b[:, :K] = (torch.randint(-3, 4, (N, K), generator=g).float() * 0.5).to(fp8)
+    ad, bd = a.to(dev), b.to(dev)
+    exact = (ad[:, :K].float() @ bd[:, :K].float().T)          # small integers and halves: exact in fp32
+    lib = _lib.load()
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    need = lib.kr_gemm_fp8_workspace_bytes(M, N, K) if split else 0
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    for kind, dtype in ((0, BF16), (1, torch.float32), (2, fp8)):
+        out = torch.zeros(M + 1, N, dtype=torch.float32, device=dev).to(dtype)
+        rc = lib.kr_gemm_fp8_ws(ad.data_ptr(), lda, bd.data_ptr(), ldb, M, N, K, out.data_ptr(), kind,
+                                ws.data_ptr() if need else None, need, stream)
+        assert rc == 0, _lib.strerror(rc)
+        want = exact.clamp(-448.0, 448.0).to(fp8) if kind == 2 else exact.to(dtype)
+        assert torch.equal(out[:M].float(), want.float()), (M, N, K, kind)
+        assert (out[M].float() == 0).all()                     # nothing past the last row
+
+
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 72), (512, 264, 120), (264, 512, 328), (511, 520, 1016)])
+def test_large_tile_kernel_last_k_step_not_full(dev, monkeypatch, M, N, K, b_t):
+    """The 256 x 256 kernel with K no multiple of its k-step: the pieces past K of the last step are zeros whatever
+    follows them in memory (here NaN: strides larger than the rows, and the next row otherwise)."""
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_TILE", "256")
+    g = torch.Generator().manual_seed(K)
+    a = torch.full((M, K + 64), float("nan"))
+    b = torch.full((N, K + 64) if b_t else (K + 64, N), float("nan"))
+    a[:, :K] = torch.randn(M, K, generator=g)
+    if b_t:
+        b[:, :K] = torch.randn(N, K, generator=g) * 0.05
+    else:
+        b[:K] = torch.randn(K, N, generator=g) * 0.05
+    ad, bd = a.to(BF16).to(dev)[:, :K], b.to(BF16).to(dev)
+    bd = bd[:, :K].T if b_t else bd[:K]
+    out = fused.gemm_one_shot_all_reduce_fused(ad, bd)
+    torch.testing.assert_close(out.cpu(), ad.float().cpu() @ bd.float().cpu(), rtol=1e-3, atol=1e-3)
