@@ -132,6 +132,7 @@ struct EnvSwitches {
     int gemm_splitk;     // KRAKEN_AMD_GEMM_SPLITK=<n>
     int gemm_tailsplit;  // KRAKEN_AMD_GEMM_TAILSPLIT=<n>
     int gemm_n224;       // KRAKEN_AMD_GEMM_N224=0|1
+    int gemm_ks;         // KRAKEN_AMD_GEMM_KS=0|1
 };
 const EnvSwitches& env_switches();   // status.hip
 

@@ -410,25 +410,8 @@ static hipError_t launch_gemm(const GemmArgs& g, bool b_nt, bool even, hipStream
 
 using namespace kr;
 
-// ---- split K loop: how many workgroups share a tile ------------------------------------------
-// A tile's K loop is split when the tiles alone leave CUs empty: into as many parts as fill the
-// 256 CUs once (measured on M = 128..1024, N = 6656, K = 4096 and 16384: 52 tiles -> 4 parts,
-// 104 -> 2, 208 and more -> 1 were the fastest or within a few percent of it; more parts only
-// add partial products to write and read), each with at least kMinSplitSteps k-steps of 64.
 constexpr int kMaxSplits = 16;
 constexpr int kMinSplitSteps = 8;
-static int split_k_factor(int64_t tiles, int64_t K) {
-    if (const int v = env_switches().gemm_splitk; v >= 1 && v <= kMaxSplits)   // testing and tuning
-        return (int)std::min<int64_t>(v, std::max<int64_t>(1, (K + BK - 1) / BK));
-    // (up to 256 tiles a second workgroup per tile still finds a place next to the first; it pays
-    // once the K loop is long: 208 tiles at K = 16384 measured 197 -> 178 us, at K = 4096 54 -> 62 us)
-    if (tiles > 128 && tiles <= 256 && K >= 12288) return 2;
-    if (tiles <= 0 || tiles * 2 > 256) return 1;
-    int64_t s = 256 / tiles;
-    s = std::min<int64_t>(s, ((K + BK - 1) / BK) / kMinSplitSteps);
-    s = std::min<int64_t>(s, kMaxSplits);
-    return (int)std::max<int64_t>(s, 1);
-}
 // ---- 256x256 kernel: split of the last partial round ------------------------------------------
 // 256 tiles run at a time (one per CU).  When the tile count leaves a last round that is at most
 // 3/8 full and K is long enough, its tiles get S = 256 / tail workgroups each (at least kMinSplitSteps k-steps per
@@ -478,25 +461,57 @@ static void fp8_split_plan(int64_t M, int64_t N, int64_t K, int* tail_out, int* 
     }
 }
 
-// Few rows, long K: whether the 256x256 kernel with every tile's K loop split (the whole launch
-// treated as a partial round) beats the 128x128 kernel with its split.  Measured on N = 6656,
-// M = 256 / 512 / 1024 (26 / 52 / 104 tiles), caches flushed: row-major B wins from K = 4096 on
-// (M = 512, K = 16384: 200 -> 146 us; M = 1024, K = 32768: 622 -> 434 us) except 104 tiles at
-// K = 4096; transposed-contiguous B only with much work per tile (52 tiles at K = 32768
-// 308 -> 279 us, 104 tiles at K = 16384 287 -> 281 us; below that up to 15 % slower).
-// (plain: a product without peers, band or second output.  There the finishing pass only sums and
-// stores, and with the 16x16x32 kernels transposed B pays from 48 tiles and K = 8192 on: 52 tiles
-// 99 -> 94 us, 104 tiles 144 -> 139 us; with a reduce-scatter epilogue the same shapes lose 5-10 %.)
-static bool whole_launch_split_pays(int64_t M, int64_t N, int64_t K, bool b_nt, bool plain) {
-    if (M <= 0 || N <= 0 || M % 256 != 0 || N % 256 != 0 || K % 64 != 0) return false;
-    const int64_t tiles = (M / 256) * (N / 256);
-    if (tiles < 24 || tiles > 128) return false;
-    if (b_nt) return tiles * K >= (int64_t)52 * 32768 || (plain && tiles >= 48 && K >= 8192);
-    return K >= 8192 || (K >= 4096 && tiles <= 64);
-}
-
 // workspace of the two-pass form: S fp32 partial products of the whole [M, N] result
 static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (int64_t)S * M * N * 4; }
+
+// ---- at most 128 tiles of 256x256: which kernel, and how many workgroups share a tile -----------------
+// Three candidates, by what they cost in 0.01 us (measured with operands that are in no cache, M = 128 .. 2000,
+// N = 1024 .. 6656, K = 512 .. 16384; the model is within 15 % of the measurements where it matters):
+//   gemm_ks_kernel, S workgroups per 128x128 tile: 6.5 us to start and finish, 0.56 us (row-major B 0.60) per
+//     k-step of 64 and round of 256 workgroups -- a compute unit takes in about 57 GB/s of operands that other
+//     units are waiting for too, whatever its pipeline; S > 1 adds a launch and S fp32 parts written and read;
+//   the 256x256 kernel with every tile's K loop split: 1.2 us per k-step, twice the work per operand byte, but
+//     parts of whole 256 KiB tiles (512 x 6656 x 16384: 122 us against 150 with gemm_ks_kernel; 512 x 4096 x 8192:
+//     51 against 43);
+//   gemm_reduce_kernel, two workgroups per compute unit: where more than 256 tiles have short K loops, one
+//     tile's epilogue beside another's k loop is worth more (1000 x 6656 x 1024, transposed B: 21 against 25 us;
+//     row-major B 28 against 27, x 4096 83 against 68).
+struct SmallPlan {
+    int big;      // 256x256 kernel, every tile split
+    int ks;       // gemm_ks_kernel, else gemm_reduce_kernel
+    int splits;   // workgroups per tile of the 128x128 kernels
+};
+static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool dtl_ok, bool may_split, bool may_big) {
+    SmallPlan p{0, 0, 1};
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
+    p.ks = dtl_ok && (tiles <= 256 || K >= (b_nt ? 4096 : 1024));
+    if (env_switches().gemm_ks >= 0) p.ks = dtl_ok && env_switches().gemm_ks != 0;
+    if (!may_split) return p;
+    if (const int v = env_switches().gemm_splitk; v >= 1 && v <= kMaxSplits) {   // testing and tuning
+        p.splits = (int)std::min<int64_t>(v, steps);
+        return p;
+    }
+    const int64_t step = b_nt ? 56 : 60;
+    auto cost = [&](int64_t s) {
+        return 650 + (tiles * s + 255) / 256 * step * ((steps + s - 1) / s) + (s > 1 ? 600 + s * M * N * 16 / 100000 : 0);
+    };
+    int64_t best = cost(1);
+    for (int64_t s = 2; s <= kMaxSplits && 2 * s <= steps && s * tiles <= 512; ++s)
+        if (const int64_t c = cost(s); c < best) {
+            best = c;
+            p.splits = (int)s;
+        }
+    if (may_big && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
+        int tail, ts;
+        const int64_t big_tiles = (M / 256) * (N / 256);
+        tail_split_plan(big_tiles, K, &tail, &ts);
+        if (tail == big_tiles && 800 + 120 * ((steps + ts - 1) / ts) + 600 + ts * big_tiles * 262144 * 2 / 50000 < best) {
+            p.big = 1;
+            p.splits = 1;
+        }
+    }
+    return p;
+}
 
 // ---- the workspace form for callers that cannot allocate ------------------------------------------
 // The split-K workspace lives in a device array of the library instead of caller memory.  Host code
@@ -532,6 +547,7 @@ struct GemmPlan {
     int tail_tiles;      // 256x256 kernel: tiles of the last partial round that are split ...
     int tail_splits;     // ... into this many parts each
     int splits;          // 128x128 kernel: workgroups per tile (split K loop), 1 = one pass
+    int ks;              // 128x128 tiles: k divided among the waves (gemm_ks.hip), else among 64-wide fragments of each wave
     int n224;            // 256x224 tiles instead of 256x256 (whole rounds of compute units where those leave a partial one)
 };
 static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peers, int64_t band_rows, bool plain,
@@ -539,16 +555,21 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
                           bool dtl_ok) {
     GemmPlan p{};
     // Tile choice: the 256x256 tile of the LDS-DMA kernel (4 waves x 128x128) has the highest
-    // MFMA work per LDS/HBM byte; it needs a K loop long enough to amortise its epilogue.  Otherwise 128x128 tiles, two of which share a CU so that one
-    // tile's epilogue overlaps the other's MFMAs; they also win while all of them fit on the
+    // MFMA work per LDS/HBM byte; it needs a K loop long enough to amortise its epilogue.
+    // Otherwise 128x128 tiles; they also win while all of them fit on the
     // 256 CUs at once (512 tiles = 128 of the large ones): measured, the large tile is 15-30 %
     // faster from 144 tiles on and 5-10 % slower at 128, for K from 1024 to 8192.
     bool big = ((M + 255) / 256) * ((N + 255) / 256) > 128 && K >= 256;
-    // (few rows and a long K loop: the large tile again, with every tile's K loop split)
-    if (!big && has_workspace && !has_gather && whole_launch_split_pays(M, N, K, b_nt, plain)) {
-        int tail, ts;
-        tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
-        big = tail > 0 && gemm_dtl_tail_workspace_bytes(tail, ts) <= workspace_bytes;
+    // (few tiles: the large tile again with every tile's K loop split, where that is cheaper)
+    SmallPlan small{0, 0, 1};
+    if (!big || !dtl_ok || env_switches().gemm_tile == 128) {
+        small = plan_small(M, N, K, b_nt, dtl_ok, has_workspace, has_workspace && !has_gather && env_switches().gemm_tile != 128);
+        if (small.big) {
+            int tail, ts;
+            tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
+            if (gemm_dtl_tail_workspace_bytes(tail, ts) > workspace_bytes) small = plan_small(M, N, K, b_nt, dtl_ok, has_workspace, false);
+        }
+        big = small.big != 0;
     }
     // KRAKEN_AMD_GEMM_TILE=128|256 overrides the choice (testing and tuning)
     if (env_switches().gemm_tile == 128) big = false;
@@ -613,11 +634,11 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
             p.tail_splits = 1;
         }
     }
-    // Split K loop (128x128 kernel, workspace given): with few tiles most CUs would idle, so S
-    // workgroups share a tile's K loop and meet in the workspace.
+    // Split K loop (128x128 kernels, workspace given): S workgroups share a tile's K loop and meet in the workspace.
     p.splits = 1;
-    if (!dtl && has_workspace) {
-        p.splits = split_k_factor(tiles_m * tiles_n, K);
+    if (!dtl) {
+        p.ks = small.ks;
+        p.splits = small.splits;
         if (p.splits > 1 && split_k_workspace_bytes(M, N, p.splits) > workspace_bytes) p.splits = 1;
     }
     return p;
@@ -627,6 +648,8 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
 // the library's code for the current device (a lazily loaded code object is what allocates the
 // device memory of the scratch array) and looks the array up.
 extern "C" int kr_init(void) {
+    if (hipError_t e = load_gemm_dtl(); e != hipSuccess) return (int)e;
+    if (hipError_t e = load_gemm_ks(); e != hipSuccess) return (int)e;
     void* p = nullptr;
     return static_scratch(&p);
 }
@@ -776,7 +799,7 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
         g1.band_row0 = 0;
         g1.band_rows = (int)M;
         g1.c_full = nullptr;
-        hipError_t e = launch_gemm<128, 128, 2, 2>(g1, b_nt, even, (hipStream_t)stream);
+        hipError_t e = plan.ks ? launch_gemm_ks(g1, b_nt, (hipStream_t)stream) : launch_gemm<128, 128, 2, 2>(g1, b_nt, even, (hipStream_t)stream);
         if (e != hipSuccess) return (int)e;
         const int64_t vecs = M * (N / 8);
         hipLaunchKernelGGL(splitk_finish_kernel, dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0,
@@ -784,6 +807,7 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
         return (int)hipGetLastError();
     }
     hipError_t e = dtl ? launch_gemm_dtl(g, b_nt, (hipStream_t)stream, workspace)
+                       : plan.ks ? launch_gemm_ks(g, b_nt, (hipStream_t)stream)
                        : launch_gemm<128, 128, 2, 2>(g, b_nt, even, (hipStream_t)stream);
     return (int)e;
 }
@@ -1011,14 +1035,17 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
         tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
         return tail > 0 ? gemm_dtl_tail_workspace_bytes(tail, ts) : 0;
     }
-    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    const int S = split_k_factor(tiles, K);
-    int64_t bytes = S > 1 ? split_k_workspace_bytes(M, N, S) : 0;
-    // the layout of B is not known here: enough for either kernel
-    if (force_tile < 0 && (whole_launch_split_pays(M, N, K, true, true) || whole_launch_split_pays(M, N, K, false, true))) {
-        int tail, ts;
-        tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
-        if (tail > 0) bytes = std::max(bytes, gemm_dtl_tail_workspace_bytes(tail, ts));
+    // the layout of B is not known here: enough for either
+    int64_t bytes = 0;
+    for (const bool b_nt : {false, true}) {
+        const SmallPlan p = plan_small(M, N, K, b_nt, K % 8 == 0 && K >= 64, true, force_tile != 128);
+        if (p.big) {
+            int tail, ts;
+            tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
+            bytes = std::max(bytes, gemm_dtl_tail_workspace_bytes(tail, ts));
+        } else if (p.splits > 1) {
+            bytes = std::max(bytes, split_k_workspace_bytes(M, N, p.splits));
+        }
     }
     return bytes;
 }

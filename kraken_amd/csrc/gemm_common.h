@@ -69,6 +69,27 @@ bool gemm_dtl_supported(const GemmArgs& g);
 hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* workspace);
 hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace);   // fp8 operands (gemm_dtl.hip)
 
+hipError_t launch_gemm_ks(const GemmArgs& g, bool b_nt, hipStream_t st);           // 128x128 tiles, k divided between waves (gemm_ks.hip)
+hipError_t load_gemm_dtl();
+hipError_t load_gemm_ks();
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+// raw buffer descriptor: 48-bit base, stride 0, num_records bytes, 32-bit data format
+__device__ __forceinline__ i32x4 raw_rsrc(const void* base, int64_t bytes) {
+    const uint64_t b = (uint64_t)base;
+    return i32x4{(int)(uint32_t)b, (int)((b >> 32) & 0xffff), (int)(bytes < 0x7fffffff ? (bytes > 0 ? bytes : 0) : 0x7fffffff), 0x00020000};
+}
+// One wave-wide LDS-DMA load: lane l's 16 bytes at (descriptor base + voff + soff) go to lds_addr + 16 l; past the
+// descriptor's end zeros are written.  Inline assembly on purpose: the compiler then does not know that LDS is written
+// behind its back and leaves the ordering to explicit s_waitcnt vmcnt / s_barrier pairs.
+__device__ __forceinline__ void lds_dma_b128(i32x4 rsrc, uint32_t lds_addr, uint32_t voff, int soff) {
+    // (one wait state between the scalar write of M0 and the instruction that reads it)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
+}
+
 constexpr int kXcds = 8;
 
 // A operand of the tile that starts at row m0 (bm rows), for the all-gather matmul: rows arrive
@@ -118,9 +139,14 @@ __device__ __forceinline__ int64_t wave_uniform(int64_t v) {
 // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2), so workgroup ids are
 // re-numbered to give every XCD a contiguous range of the order: XCD x owns positions
 // [x * ntiles/8, (x+1) * ntiles/8) and a launch over fewer tiles takes the first count/8 of each
-// range (`first` skips positions an earlier launch has taken).
+// range (`first` skips positions an earlier launch has taken).  Where 8 does not divide the count, the
+// first ntiles % 8 XCDs own one position more (launches over all tiles only).
 __device__ __forceinline__ int schedule_position(const GemmArgs& g, int wg, int first = 0) {
     const int ntiles = g.tiles_m * g.tiles_n;
+    if (ntiles % kXcds != 0 && (g.tail_tiles == 0 || g.tail_tiles == ntiles)) {
+        const int x = wg % kXcds;
+        return x * (ntiles / kXcds) + min(x, ntiles % kXcds) + wg / kXcds;
+    }
     if (ntiles % kXcds != 0 || first % kXcds != 0) return first + wg;
     return (wg % kXcds) * (ntiles / kXcds) + first / kXcds + wg / kXcds;
 }

@@ -1078,6 +1078,12 @@ bool gemm_dtl_supported(const GemmArgs& g) {
            (int64_t)BM * g.lda * 2 < 0x7fffffffLL && (int64_t)(BN > 64 ? BN : 64) * g.ldb * 2 < 0x7fffffffLL;
 }
 
+// Loads the file's device code for the current device.
+hipError_t load_gemm_dtl() {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, (const void*)gemm_dtl16_kernel<true, false>);
+}
+
 hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* workspace) {
     const dim3 grid((unsigned)(g.tiles_m * g.tiles_n - g.tail_tiles)), block(WM * WN * 64);
     const bool ragged = g.M % BM != 0 || g.N % BN != 0 || g.K % BKD != 0;

@@ -1135,3 +1135,29 @@ def test_large_tile_kernel_last_k_step_not_full(dev, monkeypatch, M, N, K, b_t):
     bd = bd[:, :K].T if b_t else bd[:K]
     out = fused.gemm_one_shot_all_reduce_fused(ad, bd)
     torch.testing.assert_close(out.cpu(), ad.float().cpu() @ bd.float().cpu(), rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (1, 8, 72), (130, 136, 128), (129, 264, 320), (256, 128, 392), (131, 1032, 1000)])
+def test_deep_ring_kernel_edges(dev, monkeypatch, M, N, K, b_t):
+    """The 128 x 128 kernel with a five-stage ring (KRAKEN_AMD_GEMM_KS=1): one k-step, fewer steps than stages, one
+    more, many; a last step that is not full; ragged rows and columns; a number of tiles 8 does not divide; one
+    part and three.  Small integers: every fp32 sum is exact, so all of them equal the product bit for bit; what
+    lies between the rows (NaN) is not read."""
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_TILE", "128")
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_KS", "1")
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.full((M, K + 8), float("nan"))
+    b = torch.full((N, K + 8) if b_t else (K, N + 8), float("nan"))
+    a[:, :K] = torch.randint(-4, 5, (M, K), generator=g).float()
+    bk = torch.randint(-4, 5, (K, N), generator=g).float()
+    if b_t:
+        b[:, :K] = bk.T
+    else:
+        b[:, :N] = bk
+    ad, bd = a.to(BF16).to(dev)[:, :K], b.to(BF16).to(dev)
+    bd = bd[:, :K].T if b_t else bd[:, :N]
+    want = a[:, :K] @ bk
+    for splits in ("1", "3"):
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_SPLITK", splits)
+        assert torch.equal(fused.gemm_one_shot_all_reduce_fused(ad, bd).cpu(), want), splits
