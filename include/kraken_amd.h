@@ -521,6 +521,21 @@ int kr_all_gather_matmul_fp8_ragged(const void* A, int64_t lda, const void* A_lo
                                     int out_kind, void* stream);
 
 /*
+ * kr_gemm_reduce_ptrs_ws_bf16 for fp32 operands (the operands of test/test_gemm_allreduce.py:57-58, which the
+ * reference runs through TF32 tl.dot, kraken/fused/gemm_one_shot_all_reduce_fused.py:56-64): every element is split
+ * into two bf16 parts on its way to the matrix cores and three of the four partial products are accumulated in
+ * fp32 (about 16 mantissa bits, the arithmetic of kr_split_fp32 followed by a product of 3K).
+ *   A, B: fp32, strides in elements, rows 16-byte aligned (strides multiples of 4); peers and bias bf16; K, N
+ *   multiples of 8; workspace of kr_gemm_f32_workspace_bytes bytes (0: none needed).
+ */
+int64_t kr_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int kr_gemm_reduce_f32_ws(const void* A, int64_t lda_m, int64_t lda_k, const void* B, int64_t ldb_k,
+                          int64_t ldb_n, int64_t M, int64_t N, int64_t K, const void* const* peers,
+                          int n_peers, const void* bias, int64_t band_row0, int64_t band_rows, void* c_full,
+                          void* out, int out_is_fp32, int64_t tile_pivot, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
+/*
  * Which kernel kr_gemm_reduce_*_bf16 would run for a shape (contiguous operands), decided by the
  * same code that launches it; for benchmarks and logs that want to name the kernel they timed.
  * No counterpart in the reference (its tile sizes are keyword arguments of the wrappers,

@@ -114,6 +114,13 @@ _SIGNATURES = {
     "kr_gemm_fp8": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p]),
     "kr_all_gather_matmul_fp8": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,
                                          c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_void_p]),
+    "kr_gemm_f32_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
+    "kr_gemm_reduce_f32_ws": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64,
+         c_void_p, c_int, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64,
+         c_void_p, c_int64, c_void_p],
+    ),
     "kr_gemm_fp8_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "kr_gemm_fp8_ws": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p, c_int64,
                                c_void_p]),

@@ -644,6 +644,30 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     return p;
 }
 
+// fp32 operands split in registers (gemm_f32.hip): 128x128 tiles, S workgroups per tile by the same kind of model
+// as plan_small: 7 us to start and finish, 0.9 us per step of 64 k and round of 256 workgroups.
+static int split_f32(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
+    if (const int v = env_switches().gemm_splitk; v >= 1 && v <= kMaxSplits) return (int)std::min<int64_t>(v, steps);   // testing and tuning
+    auto cost = [&](int64_t s) {
+        return 700 + (tiles * s + 255) / 256 * 90 * ((steps + s - 1) / s) + (s > 1 ? 600 + s * M * N * 16 / 100000 : 0);
+    };
+    int best = 1;
+    for (int s = 2; s <= kMaxSplits && 2 * s <= steps && s * tiles <= 512; ++s)
+        if (cost(s) < cost(best)) best = s;
+    return best;
+}
+static GemmPlan plan_gemm_f32(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peers, int64_t band_rows, int64_t workspace_bytes) {
+    GemmPlan p{};
+    p.tile = 128;
+    p.group_n = (n_peers > 0 && band_rows * 2 >= M) ? 16 : (b_nt ? 4 : 8);
+    if (const int v = env_switches().gemm_group; v >= 1 && v <= 64) p.group_n = v;
+    p.tail_splits = 1;
+    p.splits = split_f32(M, N, K);
+    if (p.splits > 1 && split_k_workspace_bytes(M, N, p.splits) > workspace_bytes) p.splits = 1;
+    return p;
+}
+
 // Everything kr_gemm_reduce_noalloc_bf16 would otherwise do on its first call on a device: loads
 // the library's code for the current device (a lazily loaded code object is what allocates the
 // device memory of the scratch array) and looks the array up.
@@ -677,7 +701,7 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
                        const void* const* peer_ptrs, int64_t peers_stride, const void* bias,
                        int64_t band_row0, int64_t band_rows, void* c_full, void* out, int out_is_fp32,
                        int64_t tile_pivot, void* stream, const GatherSpec* gather = nullptr,
-                       void* workspace = nullptr, int64_t workspace_bytes = 0, bool static_ws = false) {
+                       void* workspace = nullptr, int64_t workspace_bytes = 0, bool static_ws = false, bool f32 = false) {
     if (M < 0 || N < 0 || K < 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL)
         return KR_ERR_BAD_DIM;
     if (n_peers < 0 || n_peers >= KR_MAX_WORLD) return KR_ERR_WORLD_SIZE;
@@ -693,7 +717,7 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
     if (!b_nt && ldb_n != 1) return KR_ERR_LAYOUT;
     const int64_t ldb = b_nt ? ldb_n : ldb_k;
     if (lda_m < K || (b_nt ? ldb < K : ldb < N)) return KR_ERR_LAYOUT;
-    if (lda_m % 8 != 0 || ldb % 8 != 0) return KR_ERR_ALIGNMENT;
+    if (lda_m % (f32 ? 4 : 8) != 0 || ldb % (f32 ? 4 : 8) != 0) return KR_ERR_ALIGNMENT;
     if (!aligned16(A) || !aligned16(B) || !aligned16(bias) || !aligned16(c_full) || !aligned16(out))
         return KR_ERR_ALIGNMENT;
     // (arguments are checked; a shape that is split now gets the library's own workspace)
@@ -754,7 +778,8 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
     g.out_is_fp32 = out_is_fp32;
     g.out_fp8 = 0;
 
-    const GemmPlan plan = plan_gemm(M, N, K, b_nt, n_peers, band_rows, n_peers == 0 && c_full == nullptr && bias == nullptr,
+    const GemmPlan plan = f32 ? plan_gemm_f32(M, N, K, b_nt, n_peers, band_rows, workspace != nullptr ? workspace_bytes : 0)
+                              : plan_gemm(M, N, K, b_nt, n_peers, band_rows, n_peers == 0 && c_full == nullptr && bias == nullptr,
                                     !out_is_fp32 && band_row0 == 0 && band_rows == M, workspace != nullptr, workspace_bytes, gather != nullptr, g.progress != nullptr,
                                     g.progress != nullptr || g.band_counter != nullptr,
                                     gemm_dtl_supported(g) && (g.a_local == nullptr || (int64_t)256 * g.lda_local * 2 < 0x7fffffffLL));
@@ -764,7 +789,7 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
     // refused rather than read as zeros.
     if (!dtl) {
         const int64_t reach = std::max<int64_t>(std::max(lda_m, ldb), g.a_local != nullptr ? g.lda_local : 0);
-        if ((128 * reach + std::max(K, N)) * 2 >= 0x7fffffffLL) return KR_ERR_LAYOUT;
+        if ((128 * reach + std::max(K, N)) * (f32 ? 4 : 2) >= 0x7fffffffLL) return KR_ERR_LAYOUT;
     }
     g.peers_on_mfma = plan.peers_on_mfma;
     g.mi16 = plan.mi16;
@@ -799,14 +824,16 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
         g1.band_row0 = 0;
         g1.band_rows = (int)M;
         g1.c_full = nullptr;
-        hipError_t e = plan.ks ? launch_gemm_ks(g1, b_nt, (hipStream_t)stream) : launch_gemm<128, 128, 2, 2>(g1, b_nt, even, (hipStream_t)stream);
+        hipError_t e = f32 ? launch_gemm_f32(g1, b_nt, (hipStream_t)stream)
+                       : plan.ks ? launch_gemm_ks(g1, b_nt, (hipStream_t)stream) : launch_gemm<128, 128, 2, 2>(g1, b_nt, even, (hipStream_t)stream);
         if (e != hipSuccess) return (int)e;
         const int64_t vecs = M * (N / 8);
         hipLaunchKernelGGL(splitk_finish_kernel, dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0,
                            (hipStream_t)stream, g, (const float*)workspace, splits);
         return (int)hipGetLastError();
     }
-    hipError_t e = dtl ? launch_gemm_dtl(g, b_nt, (hipStream_t)stream, workspace)
+    hipError_t e = f32 ? launch_gemm_f32(g, b_nt, (hipStream_t)stream)
+                       : dtl ? launch_gemm_dtl(g, b_nt, (hipStream_t)stream, workspace)
                        : plan.ks ? launch_gemm_ks(g, b_nt, (hipStream_t)stream)
                        : launch_gemm<128, 128, 2, 2>(g, b_nt, even, (hipStream_t)stream);
     return (int)e;
@@ -1071,6 +1098,23 @@ extern "C" int kr_gemm_reduce_ptrs_ws_bf16(const void* A, int64_t lda_m, int64_t
     return gemm_reduce(A, lda_m, lda_k, B, ldb_k, ldb_n, M, N, K, peers, n_peers,
                        peers != nullptr ? peers : kNoPeers, 0, bias, band_row0, band_rows, c_full, out,
                        out_is_fp32, tile_pivot, stream, nullptr, workspace, workspace_bytes);
+}
+
+extern "C" int64_t kr_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const int S = split_f32(M, N, K);
+    return S > 1 ? split_k_workspace_bytes(M, N, S) : 0;
+}
+
+extern "C" int kr_gemm_reduce_f32_ws(const void* A, int64_t lda_m, int64_t lda_k, const void* B, int64_t ldb_k,
+                                     int64_t ldb_n, int64_t M, int64_t N, int64_t K, const void* const* peers,
+                                     int n_peers, const void* bias, int64_t band_row0, int64_t band_rows,
+                                     void* c_full, void* out, int out_is_fp32, int64_t tile_pivot, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+    static const void* const kNoPeers[1] = {nullptr};
+    return gemm_reduce(A, lda_m, lda_k, B, ldb_k, ldb_n, M, N, K, peers, n_peers,
+                       peers != nullptr ? peers : kNoPeers, 0, bias, band_row0, band_rows, c_full, out,
+                       out_is_fp32, tile_pivot, stream, nullptr, workspace, workspace_bytes, false, /*f32=*/true);
 }
 
 extern "C" int kr_gemm_reduce_noalloc_bf16(const void* A, int64_t lda_m, int64_t lda_k, const void* B,

@@ -70,6 +70,7 @@ hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* w
 hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace);   // fp8 operands (gemm_dtl.hip)
 
 hipError_t launch_gemm_ks(const GemmArgs& g, bool b_nt, hipStream_t st);           // 128x128 tiles, k divided between waves (gemm_ks.hip)
+hipError_t launch_gemm_f32(const GemmArgs& g, bool b_nt, hipStream_t st);          // fp32 operands (gemm_f32.hip); A, B, lda, ldb in fp32 elements
 hipError_t load_gemm_dtl();
 hipError_t load_gemm_ks();
 

@@ -32,9 +32,7 @@ def split_fp32(a: torch.Tensor, b: torch.Tensor) -> tuple[torch.Tensor, torch.Te
     dev = _lib.require_device(a, b)
     stream = _lib.current_stream(dev)
 
-    def rows_ok(t):      # columns contiguous, rows 16-byte aligned
-        return t.stride(1) == 1 and t.stride(0) % 4 == 0 and t.stride(0) >= t.shape[1] and t.data_ptr() % 16 == 0
-
+    rows_ok = fp32_rows_ok
     if not rows_ok(a):
         a = a.contiguous()
     a3 = torch.empty((M, 3 * K), dtype=torch.bfloat16, device=dev)
@@ -52,15 +50,33 @@ def split_fp32(a: torch.Tensor, b: torch.Tensor) -> tuple[torch.Tensor, torch.Te
     return a3, b3
 
 
+def fp32_rows_ok(t: torch.Tensor) -> bool:
+    """Columns contiguous, rows 16-byte aligned."""
+    return t.stride(1) == 1 and t.stride(0) % 4 == 0 and t.stride(0) >= t.shape[1] and t.data_ptr() % 16 == 0
+
+
+def fp32_direct(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether fp32 operands go to the kernel that splits them in registers (``kr_gemm_reduce_f32_ws``).
+
+    Up to two rounds of its 128 x 128 tiles on the 256 compute units: 2000 x 4096 x 2048 takes 117 us there and 166 us
+    as a split pass and a bf16 product; with more tiles the 256 x 256 bf16 kernel wins the pass back
+    (4096 x 4096 x 1024: 135 against 104 us).
+    """
+    if not (a.is_cuda and b.is_cuda) or a.shape[1] % 8 != 0 or b.shape[1] % 8 != 0:
+        return False
+    return -(-a.shape[0] // 128) * -(-b.shape[1] // 128) <= 512
+
+
 def prepare_operands(a: torch.Tensor, b: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    """Return bf16 operands in a layout the kernel reads directly.
+    """Return operands in a type and layout the kernel reads directly.
 
     A must be k-contiguous; B either row-major or transposed-contiguous; any row
     stride that is a multiple of 8 elements is read in place (the kernels address
     operands through buffer descriptors built from the caller's strides).  Other
     stridings (the reference accepts any 2-D strides,
-    ``gemm_one_shot_all_reduce_fused.py:163-166``) take one copy.  fp32 operands are
-    split into bf16 parts by one kernel pass each (``split_fp32``).
+    ``gemm_one_shot_all_reduce_fused.py:163-166``) take one copy.  fp32 operands stay fp32
+    where the product splits them itself (``fp32_direct``), else they are split into bf16
+    parts by one kernel pass each (``split_fp32``).
     K is padded to a multiple of 8 with zeros when necessary.
     """
     assert a.dim() == 2 and b.dim() == 2
@@ -68,6 +84,8 @@ def prepare_operands(a: torch.Tensor, b: torch.Tensor) -> tuple[torch.Tensor, to
     assert a.dtype == b.dtype, "Input tensors must have the same dtype"
     assert a.dtype in (torch.bfloat16, torch.float32), "bfloat16 (or float32) operands expected"
     if a.dtype == torch.float32:
+        if fp32_direct(a, b):
+            return (a if fp32_rows_ok(a) else a.contiguous()), (b if fp32_rows_ok(b) or fp32_rows_ok(b.T) else b.contiguous())
         a, b = split_fp32(a, b)
     K = a.shape[1]
     if K % 8 != 0:
@@ -105,6 +123,19 @@ def launch(name, a, b, M, N, peers, n_peers, peers_stride, bias, band_row0, band
     output tiles get a workspace and go through the ``_ws`` entry points (split K loop)."""
     lib = _lib.load()
     out_fp32 = int(out is not None and out.dtype == torch.float32)
+    if a.dtype == torch.float32:
+        K = a.shape[1]
+        plist = peers if isinstance(peers, (list, tuple)) else [] if peers is None else list(peers)
+        dev = _lib.require_device(a, b, *plist, bias, c_full, out)
+        ws = workspace(dev, lib.kr_gemm_f32_workspace_bytes(M, N, K))
+        table = (ctypes.c_void_p * max(n_peers, 1))(*[t.data_ptr() for t in plist])
+        rc = lib.kr_gemm_reduce_f32_ws(
+            a.data_ptr(), a.stride(0), a.stride(1), b.data_ptr(), b.stride(0), b.stride(1), M, N, K,
+            table, n_peers, _lib.ptr(bias), band_row0, band_rows, _lib.ptr(c_full), _lib.ptr(out), out_fp32, pivot,
+            _lib.ptr(ws), ws.numel() if ws is not None else 0, _lib.current_stream(dev),
+        )
+        _lib.check(rc, name)
+        return
     ws = workspace(a.device, lib.kr_gemm_workspace_bytes(M, N, a.shape[1])) if a.is_cuda else None
     if ws is not None:
         if isinstance(peers, (list, tuple)):

@@ -1161,3 +1161,41 @@ def test_deep_ring_kernel_edges(dev, monkeypatch, M, N, K, b_t):
     for splits in ("1", "3"):
         monkeypatch.setenv("KRAKEN_AMD_GEMM_SPLITK", splits)
         assert torch.equal(fused.gemm_one_shot_all_reduce_fused(ad, bd).cpu(), want), splits
+
+
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (1, 8, 8), (130, 136, 40), (129, 264, 96), (256, 128, 328), (131, 1032, 1000)])
+def test_fp32_operands_split_in_registers(dev, monkeypatch, M, N, K, b_t):
+    """kr_gemm_reduce_f32_ws: one k-step down to 8 k, last steps of every kind (a stage missing, half a stage), fewer
+    steps than the ring has stages, ragged rows and columns, one part and three, with peers and bias.  Exact part:
+    integers up to 2^11 times integers up to 8 -- hi and lo parts are exact, every partial sum is below 2^24 --
+    equal the product bit for bit.  Random part: within 2^-15 of sum |a||b| of the double-precision product (the
+    dropped a_lo b_lo is below 2^-18, the rounding of lo below 2^-18 twice, fp32 sums of K terms below K 2^-24)."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.full((M, K + 4), float("nan"))
+    b = torch.full((N, K + 4) if b_t else (K, N + 4), float("nan"))
+
+    def operands(av, bv):
+        a[:, :K] = av
+        if b_t:
+            b[:, :K] = bv.T
+        else:
+            b[:, :N] = bv
+        bd = b.to(dev)
+        return a.to(dev)[:, :K], bd[:, :K].T if b_t else bd[:, :N]
+
+    peers = torch.randint(-8, 9, (3, M, N), generator=g).to(BF16)
+    bias = torch.randint(-8, 9, (N,), generator=g).to(BF16)
+    av = torch.randint(-2047, 2048, (M, K), generator=g).float()
+    bv = torch.randint(-8, 9, (K, N), generator=g).float()
+    exact = av.double() @ bv.double() + peers.double().sum(0) + bias.double()
+    assert K * 2047 * 8 < 1 << 24
+    ar, br = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
+    for splits in ("1", "3"):
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_SPLITK", splits)
+        ad, bd = operands(av, bv)
+        out = fused.gemm_one_shot_all_reduce_fused(ad, bd, peers=peers.to(dev), bias=bias.to(dev))
+        assert torch.equal(out.cpu().double(), exact), splits
+        ad, bd = operands(ar, br)
+        out = fused.gemm_one_shot_all_reduce_fused(ad, bd).cpu().double()
+        assert ((out - ar.double() @ br.double()).abs() <= 2.0 ** -15 * (ar.abs().double() @ br.abs().double())).all(), splits
