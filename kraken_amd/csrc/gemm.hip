@@ -536,6 +536,48 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool dtl
     return p;
 }
 
+// ---- at most 64 rows (gemm_skinny.hip): columns per workgroup and workgroups that share a K loop -------------
+// By a model of what the forms cost, in 0.01 us, fitted to measurements with B in no cache (M = 2 .. 64, N = 1024 ..
+// 8192, K = 576 .. 16384; within 15 %): 6 us to start and finish, 5 us for every further round of 256 workgroups; a
+// compute unit takes in 64 GB/s of 128-byte rows, and a k-row of a row-major B costs it 2.3 / 3.0 / 3.4 ns for 32 / 64 /
+// 128 bytes; HBM 6 TB/s; parts of K a second launch and their bytes.  Against the 128x128 kernel and its parts, us:
+// 16 x 8192 x 3584 with seven peers 20.9 -> 14.1 (row-major B 21.9 -> 18.8), 4 x 3360 x 976 14.1 -> 6.3, 4 x 2816 x 576
+// row-major 15.0 -> 6.1, 16 x 1024 x 16384 22.6 -> 15.5, fp32 2 x 1216 x 1280 17.1 -> 7.8, 16 x 4096 x 4096 28.7 -> 17.6;
+// 64 x 8192 x 3584 24.4 -> 19.2, row-major level (24.4 / 24.7).  From 65 rows on the rows of A, which every workgroup
+// reads, outweigh B.
+constexpr int64_t kMaxPartsBytes = KR_STATIC_SCRATCH_BYTES;   // (the form that allocates nothing takes every split)
+struct SkinnyPlan {
+    int cb;       // columns of a workgroup / 16; 0: not for this call
+    int splits;   // parts of K, summed by a second launch
+};
+static SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool b_nt, bool f32, int64_t parts_bytes) {
+    SkinnyPlan p{0, 1};
+    const EnvSwitches& env = env_switches();
+    if (M > 64 || N < 16 || env.gemm_tile > 0 || env.gemm_ks >= 0 || env.gemm_splitk >= 1 || env.gemm_skinny == 0) return p;
+    const int64_t e = f32 ? 4 : 2, units = (K * e + 127) / 128, rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+    parts_bytes = std::min(parts_bytes, kMaxPartsBytes);
+    if (const int cb = env.gemm_skinny / 100, s = env.gemm_skinny % 100; cb > 0) {   // testing and tuning
+        if (cb != 1 && cb != 2 && (cb != 4 || f32)) return p;
+        p.cb = cb;
+        if (s >= 1 && s <= units && s * M * N * 4 <= parts_bytes) p.splits = s;
+        return p;
+    }
+    int64_t best = 0;
+    for (int cb = 1; cb <= (f32 || M > 32 ? 2 : 4); cb *= 2) {
+        for (int64_t s = 1; s <= kMaxSplits && (s == 1 || (4 * s <= units && s * M * N * 4 <= parts_bytes)); s *= 2) {
+            const int64_t rounds = ((N + 16 * cb - 1) / (16 * cb) * s + 255) / 256, k = (K + s - 1) / s, line = 16 * cb * e;
+            const int64_t b_time = b_nt ? line * k / 640 : (line <= 32 ? 23 : line <= 64 ? 30 : 34) * k / 100;
+            const int64_t c = 600 + 500 * (rounds - 1) + std::max(rounds * (rows * e * k / 640 + b_time), N * K * e / 60000) +
+                              (s > 1 ? 400 + 50 * s + s * M * N * 8 / 50000 : 0);
+            if (p.cb != 0 && c >= best) continue;
+            best = c;
+            p.cb = cb;
+            p.splits = (int)s;
+        }
+    }
+    return p;
+}
+
 // ---- the workspace form for callers that cannot allocate ------------------------------------------
 // The split-K workspace lives in a device array of the library instead of caller memory.  Host code
 // never uses the array's name as an address: each device's copy is looked up once, with that device
@@ -571,12 +613,27 @@ struct GemmPlan {
     int tail_splits;     // ... into this many parts each
     int splits;          // 128x128 kernel: workgroups per tile (split K loop), 1 = one pass
     int ks;              // 128x128 tiles: k divided among the waves (gemm_ks.hip), else among 64-wide fragments of each wave
+    int skinny;          // at most 64 rows: columns of a workgroup / 16 (gemm_skinny.hip), 0: another kernel
     int n224;            // 256x224 tiles instead of 256x256 (whole rounds of compute units where those leave a partial one)
 };
+static GemmPlan plan_of_skinny(const SkinnyPlan& sk) {
+    GemmPlan p{};
+    p.tile = 128;   // (the tile order of the 128x128 kernels; not used)
+    p.mi16 = 1;
+    p.group_n = 1;
+    p.tail_splits = 1;
+    p.splits = sk.splits;
+    p.skinny = sk.cb;
+    return p;
+}
 static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peers, int64_t band_rows, bool plain,
                           bool plain_bf16_all_rows, bool has_workspace, int64_t workspace_bytes, bool has_gather, bool has_progress, bool flagged,
-                          bool dtl_ok) {
+                          bool dtl_ok, bool skinny_ok) {
     GemmPlan p{};
+    if (skinny_ok && !flagged) {
+        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, false, has_workspace ? workspace_bytes : 0);
+        if (sk.cb != 0) return plan_of_skinny(sk);
+    }
     // Tile choice: the 256x256 tile of the LDS-DMA kernel (4 waves x 128x128) has the highest
     // MFMA work per LDS/HBM byte; it needs a K loop long enough to amortise its epilogue.
     // Otherwise 128x128 tiles; they also win while all of them fit on the
@@ -680,8 +737,13 @@ static int split_f32(int64_t M, int64_t N, int64_t K) {
         if (cost(s) < cost(best)) best = s;
     return best;
 }
-static GemmPlan plan_gemm_f32(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peers, int64_t band_rows, int64_t workspace_bytes) {
+static GemmPlan plan_gemm_f32(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peers, int64_t band_rows, int64_t workspace_bytes,
+                              bool skinny_ok) {
     GemmPlan p{};
+    if (skinny_ok) {
+        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, true, workspace_bytes);
+        if (sk.cb != 0) return plan_of_skinny(sk);
+    }
     p.tile = 128;
     p.group_n = (n_peers > 0 && band_rows * 2 >= M) ? 16 : (b_nt ? 4 : 8);
     if (const int v = env_switches().gemm_group; v >= 1 && v <= 64) p.group_n = v;
@@ -697,6 +759,7 @@ static GemmPlan plan_gemm_f32(int64_t M, int64_t N, int64_t K, bool b_nt, int n_
 extern "C" int kr_init(void) {
     if (hipError_t e = load_gemm_dtl(); e != hipSuccess) return (int)e;
     if (hipError_t e = load_gemm_ks(); e != hipSuccess) return (int)e;
+    if (hipError_t e = load_gemm_skinny(); e != hipSuccess) return (int)e;
     void* p = nullptr;
     return static_scratch(&p);
 }
@@ -801,16 +864,20 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
     g.out_is_fp32 = out_is_fp32;
     g.out_fp8 = 0;
 
-    const GemmPlan plan = f32 ? plan_gemm_f32(M, N, K, b_nt, n_peers, band_rows, workspace != nullptr ? workspace_bytes : 0)
+    // gemm_skinny_kernel addresses both operands and the band with 32-bit byte offsets
+    const int64_t esize = f32 ? 4 : 2;
+    const bool skinny_ok = M <= 64 && (M * lda_m + K + 64) * esize < 0x7fffffffLL && M * N * 2 < 0x7fffffffLL &&
+                           (b_nt ? 64 * ldb + K + 64 : (K + 64) * ldb + N) * esize < 0x7fffffffLL;
+    const GemmPlan plan = f32 ? plan_gemm_f32(M, N, K, b_nt, n_peers, band_rows, workspace != nullptr ? workspace_bytes : 0, skinny_ok)
                               : plan_gemm(M, N, K, b_nt, n_peers, band_rows, n_peers == 0 && c_full == nullptr && bias == nullptr,
                                     !out_is_fp32 && band_row0 == 0 && band_rows == M, workspace != nullptr, workspace_bytes, gather != nullptr, g.progress != nullptr,
                                     g.progress != nullptr || g.band_counter != nullptr,
-                                    gemm_dtl_supported(g) && (g.a_local == nullptr || (int64_t)256 * g.lda_local * 2 < 0x7fffffffLL));
+                                    gemm_dtl_supported(g) && (g.a_local == nullptr || (int64_t)256 * g.lda_local * 2 < 0x7fffffffLL), skinny_ok);
     const bool dtl = plan.tile == 256;
     // The 128x128 kernel addresses a tile's operand panels with 32-bit byte offsets from the
     // panel's first row (through a 2 GiB buffer descriptor): row strides beyond that reach are
     // refused rather than read as zeros.
-    if (!dtl) {
+    if (!dtl && plan.skinny == 0) {
         const int64_t reach = std::max<int64_t>(std::max(lda_m, ldb), g.a_local != nullptr ? g.lda_local : 0);
         if ((128 * reach + std::max(K, N)) * (f32 ? 4 : 2) >= 0x7fffffffLL) return KR_ERR_LAYOUT;
     }
@@ -847,7 +914,8 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
         g1.band_row0 = 0;
         g1.band_rows = (int)M;
         g1.c_full = nullptr;
-        hipError_t e = f32 ? launch_gemm_f32(g1, b_nt, (hipStream_t)stream)
+        hipError_t e = plan.skinny ? launch_gemm_skinny(g1, b_nt, f32, plan.skinny, (hipStream_t)stream)
+                       : f32 ? launch_gemm_f32(g1, b_nt, (hipStream_t)stream)
                        : plan.ks ? launch_gemm_ks(g1, b_nt, (hipStream_t)stream) : launch_gemm<128, 128, 2, 2>(g1, b_nt, even, (hipStream_t)stream);
         if (e != hipSuccess) return (int)e;
         const int64_t vecs = M * (N / 8);
@@ -856,7 +924,8 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
                            (hipStream_t)stream, g, (const float*)workspace, splits);
         return (int)hipGetLastError();
     }
-    hipError_t e = f32 ? launch_gemm_f32(g, b_nt, (hipStream_t)stream)
+    hipError_t e = plan.skinny ? launch_gemm_skinny(g, b_nt, f32, plan.skinny, (hipStream_t)stream)
+                       : f32 ? launch_gemm_f32(g, b_nt, (hipStream_t)stream)
                        : dtl ? launch_gemm_dtl(g, b_nt, (hipStream_t)stream, workspace)
                        : plan.ks ? launch_gemm_ks(g, b_nt, (hipStream_t)stream)
                        : launch_gemm<128, 128, 2, 2>(g, b_nt, even, (hipStream_t)stream);
@@ -1059,7 +1128,7 @@ extern "C" int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, i
     g.lda = K;
     g.ldb = b_transposed ? K : N;
     const GemmPlan p = plan_gemm(M, N, K, b_transposed != 0, n_peers, band_rows, n_peers == 0 && !has_c_full && !has_bias,
-                                 band_rows == M, workspace_bytes > 0, workspace_bytes, false, false, false, gemm_dtl_supported(g));
+                                 band_rows == M, workspace_bytes > 0, workspace_bytes, false, false, false, gemm_dtl_supported(g), true);
     const bool whole_band_peers = p.tile == 256 && n_peers > 0 && p.peers_on_mfma != 0;
     plan[0] = p.tile;
     plan[1] = p.tile == 256 ? (p.mi16 ? 16 : 32) : 32;   // MFMA block rows: 16x16x32 or 32x32x16
@@ -1070,6 +1139,7 @@ extern "C" int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, i
     plan[6] = whole_band_peers ? 1 : 0;
     plan[7] = (M % p.tile != 0 || N % p.tile != 0 || K % 64 != 0) ? 1 : 0;
     if (p.n224) plan[7] |= 2;   // bit 1: 256 x 224 tiles
+    if (p.skinny) plan[7] |= 4;   // bit 2: gemm_skinny_kernel
     return KR_OK;
 }
 
@@ -1089,6 +1159,10 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     // the layout of B is not known here: enough for either
     int64_t bytes = 0;
     for (const bool b_nt : {false, true}) {
+        if (const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, false, kMaxPartsBytes); sk.cb != 0) {
+            if (sk.splits > 1) bytes = std::max(bytes, split_k_workspace_bytes(M, N, sk.splits));
+            continue;
+        }
         const SmallPlan p = plan_small(M, N, K, b_nt, K % 8 == 0 && K >= 64, true, force_tile != 128);
         if (p.big) {
             int tail, ts;
@@ -1126,6 +1200,14 @@ extern "C" int kr_gemm_reduce_ptrs_ws_bf16(const void* A, int64_t lda_m, int64_t
 
 extern "C" int64_t kr_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
+    int64_t skinny_bytes = 0;
+    bool skinny = false;
+    for (const bool b_nt : {false, true}) {
+        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, true, kMaxPartsBytes);
+        skinny = sk.cb != 0;
+        if (skinny && sk.splits > 1) skinny_bytes = std::max(skinny_bytes, split_k_workspace_bytes(M, N, sk.splits));
+    }
+    if (skinny) return skinny_bytes;
     const int S = split_f32(M, N, K);
     return S > 1 ? split_k_workspace_bytes(M, N, S) : 0;
 }

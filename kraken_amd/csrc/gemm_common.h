@@ -71,8 +71,10 @@ hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace);
 
 hipError_t launch_gemm_ks(const GemmArgs& g, bool b_nt, hipStream_t st);           // 128x128 tiles, k divided between waves (gemm_ks.hip)
 hipError_t launch_gemm_f32(const GemmArgs& g, bool b_nt, hipStream_t st);          // fp32 operands (gemm_f32.hip); A, B, lda, ldb in fp32 elements
+hipError_t launch_gemm_skinny(const GemmArgs& g, bool b_nt, bool f32, int cb, hipStream_t st);   // at most 64 rows, 16 cb columns per workgroup (gemm_skinny.hip)
 hipError_t load_gemm_dtl();
 hipError_t load_gemm_ks();
+hipError_t load_gemm_skinny();
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 // raw buffer descriptor: 48-bit base, stride 0, num_records bytes, 32-bit data format

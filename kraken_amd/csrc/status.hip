@@ -23,6 +23,7 @@ static EnvSwitches read_env() {
     e.gemm_tailsplit = num("KRAKEN_AMD_GEMM_TAILSPLIT");
     e.gemm_n224 = num("KRAKEN_AMD_GEMM_N224");
     e.gemm_ks = num("KRAKEN_AMD_GEMM_KS");
+    e.gemm_skinny = num("KRAKEN_AMD_GEMM_SKINNY");
     return e;
 }
 static EnvSwitches& env_storage() {

@@ -1199,3 +1199,49 @@ def test_fp32_operands_split_in_registers(dev, monkeypatch, M, N, K, b_t):
         ad, bd = operands(ar, br)
         out = fused.gemm_one_shot_all_reduce_fused(ad, bd).cpu().double()
         assert ((out - ar.double() @ br.double()).abs() <= 2.0 ** -15 * (ar.abs().double() @ br.abs().double())).all(), splits
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (16, 32, 64), (17, 40, 72), (32, 264, 520), (33, 136, 1000), (64, 1032, 1096)])
+def test_few_rows_kernel(dev, monkeypatch, M, N, K, b_t, fp32):
+    """gemm_skinny_kernel: every number of columns per workgroup, one part and three, one row up to 64, fewer units of
+    64 k than wavefronts and more than they keep in flight, a last unit that is not full, columns no width divides,
+    eight or more peers than are requested early, a bias, a band that is part of the rows.  Small integers (fp32
+    operands: up to 2^11, hi and lo parts exact): every fp32 sum is exact, results equal the product bit for bit; what
+    lies between the rows (NaN) is not read."""
+    g = torch.Generator().manual_seed(M + N + K)
+    dt = torch.float32 if fp32 else BF16
+    a = torch.full((M, K + 8), float("nan"))
+    b = torch.full((N, K + 8) if b_t else (K, N + 8), float("nan"))
+    big = 2047 if fp32 else 4
+    a[:, :K] = torch.randint(-big, big + 1, (M, K), generator=g).float()
+    bk = torch.randint(-4, 5, (K, N), generator=g).float()
+    if b_t:
+        b[:, :K] = bk.T
+    else:
+        b[:, :N] = bk
+    ad, bd = a.to(dt).to(dev)[:, :K], b.to(dt).to(dev)
+    bd = bd[:, :K].T if b_t else bd[:, :N]
+    product = a[:, :K] @ bk
+    peers = torch.randint(-8, 9, (9, M, N), generator=g).to(BF16)
+    bias = torch.randint(-8, 9, (N,), generator=g).to(BF16)
+    lib = _lib.load()
+    for cb in (1, 2) if fp32 else (1, 2, 4):
+        for splits in (1, 5):
+            monkeypatch.setenv("KRAKEN_AMD_GEMM_SKINNY", str(100 * cb + splits))
+            _lib.reload_env()
+            out = fused.gemm_one_shot_all_reduce_fused(ad, bd, peers=peers.to(dev), bias=bias.to(dev))
+            assert torch.equal(out.cpu(), product + peers.float().sum(0) + bias.float()), (cb, splits)
+            if not fp32 and M % 2 == 0:
+                c = torch.zeros(M, N, dtype=BF16, device=dev)
+                half = M // 2
+                out = fused.gemm_reduce_scatter(ad, bd, peers=peers[:1, :half].contiguous().to(dev), rank=1, c_scratch=c)
+                want = product.to(BF16)
+                assert torch.equal(out.cpu(), (want[half:].float() + peers[0, :half].float()).to(BF16)), (cb, splits)
+                assert torch.equal(c.cpu()[:half], want[:half]), (cb, splits)
+    plan = _lib.gemm_plan(M, N, K, b_t)
+    assert fp32 or plan["kernel"] == "gemm_skinny_kernel"
+    monkeypatch.delenv("KRAKEN_AMD_GEMM_SKINNY")
+    _lib.reload_env()
+    assert lib.kr_gemm_workspace_bytes(M, N, K) >= 0
