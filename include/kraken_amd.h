@@ -423,6 +423,18 @@ int kr_flag_arrive_wait(uint32_t* flags, int producers, int consumers, int64_t w
                         int32_t* status, void* stream);
 
 /*
+ * All chunks of an all-gather and their flags in one launch: source r's buffer srcs[r] (a host array of W device
+ * pointers) holds splits_per_rank chunks of chunk_bytes; chunk c = r * splits_per_rank + s is copied to
+ * dst + c * chunk_bytes, and progress[c] is 1 once it has arrived (visible to kernels that read the flag).  Chunks are
+ * taken in the order of the source ranks rank+1, rank+2, ..., rank.  progress[] must be zero when the kernel starts; a
+ * chunk that is still arriving may show any even count there.  chunk_bytes a multiple of 16, pointers 16-byte aligned.
+ * Replaces the loop of copies and flag writes of the reference's chunked all-gather
+ * (kraken/comm/copy_engine_all_gather.py:38-53).
+ */
+int kr_gather_chunks(const void* const* srcs, int W, int splits_per_rank, int rank, int64_t chunk_bytes, void* dst,
+                     uint32_t* progress, void* stream);
+
+/*
  * Stream-ordered device-to-device copy of `bytes` bytes that runs on the GPU's copy engines
  * (SDMA) and not as a copy kernel, so it takes no compute units from a GEMM running beside it.
  * Source and destination must not overlap.  bytes == 0: nothing is done.

@@ -22,6 +22,7 @@ KR_ERR_BAND = -8
 KR_ERR_LAYOUT = -9
 KR_ERR_STRIPE = -10
 KR_ERR_SCRATCH = -11
+KR_MAX_WORLD = 16
 
 _SIGNATURES = {
     "kr_version": (c_int, []),
@@ -105,6 +106,7 @@ _SIGNATURES = {
          c_int, c_int, c_void_p, c_void_p, c_void_p],
     ),
     "kr_stream_wait_value32": (c_int, [c_void_p, ctypes.c_uint32, c_int64, c_void_p, c_void_p]),
+    "kr_gather_chunks": (c_int, [c_void_p, c_int, c_int, c_int, c_int64, c_void_p, c_void_p, c_void_p]),
     "kr_copy_engine_memcpy": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
     "kr_flag_arrive_wait": (c_int, [c_void_p, c_int, c_int, c_int64, c_void_p, c_void_p]),
     "kr_reduce_rotated_bf16": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int, c_int, c_void_p, c_void_p]),

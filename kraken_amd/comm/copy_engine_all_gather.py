@@ -1,10 +1,17 @@
 """Chunked all-gather with arrival flags (``kraken/comm/copy_engine_all_gather.py``)."""
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib
 from ._common import PeerBuffers
+
+# Up to here the sixteen launches of eight copies and flags bound the call (all_gather_matmul, K = 8192, N = 3584: eight
+# shards of 4 .. 128 rows 212 us, in one launch 114; 256 rows, 32 MiB gathered, 225 / 180; 512 rows 233 / 235).  Above,
+# the product does, and copies that come one behind the other leave it more of the memory (1024 rows 405 / 438).
+ONE_LAUNCH_BYTES = 48 << 20
 
 _backend_streams: dict[int, torch.cuda.Stream] = {}
 
@@ -43,8 +50,10 @@ def _copy_engine_all_gather_w_progress(
     ``output`` and then ``progress[chunk]`` is set to 1 by a stream-ordered
     flag write (``:47-53``).  The side stream first waits for the current
     stream (``:35``); the caller makes the current stream wait for the returned
-    stream when it needs the gathered tensor (``:118``).  The copies are ordinary
-    device-to-device copy kernels; ``copy_engine=True`` hands them to the GPU's
+    stream when it needs the gathered tensor (``:118``).  All chunks and flags
+    of a gather of up to ``ONE_LAUNCH_BYTES`` are one launch (``kr_gather_chunks``); larger ones, and
+    chunks that are no multiple of 16 bytes, are copied one by one by ordinary device-to-device copy
+    kernels with a flag write behind each; ``copy_engine=True`` hands them to the GPU's
     copy engines (``kr_copy_engine_memcpy``), which take no compute units but
     are slower within one GPU.  ``progress`` must have been zeroed on the current
     stream beforehand.
@@ -66,6 +75,14 @@ def _copy_engine_all_gather_w_progress(
     chunk = peers.cap // splits_per_rank
     flat_out = output.view(-1)
     backend_stream.wait_stream(torch.cuda.current_stream(dev))
+    chunk_bytes = chunk * output.element_size()
+    sources = [peers.slice(r).data_ptr() for r in range(W)]
+    if (not copy_engine and chunk_bytes * n_chunks <= ONE_LAUNCH_BYTES and W <= _lib.KR_MAX_WORLD and chunk_bytes % 16 == 0 and output.data_ptr() % 16 == 0
+            and all(p % 16 == 0 for p in sources)):
+        rc = lib.kr_gather_chunks((ctypes.c_void_p * W)(*sources), W, splits_per_rank, rank, chunk_bytes,
+                                  output.data_ptr(), progress.data_ptr(), backend_stream.cuda_stream)
+        _lib.check(rc, "gather_chunks")
+        return backend_stream
     with torch.cuda.stream(backend_stream):
         for step in range(W):
             src_rank = (rank + step + 1) % W

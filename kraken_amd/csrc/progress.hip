@@ -1,5 +1,7 @@
 // Stream-ordered flag write and flag wait, and the copy-engine copy they bracket: the pieces of
 // the overlap of copies with a running GEMM (all-gather matmul, copy-engine reduce-scatter).
+#include <algorithm>
+
 #include "common.h"
 
 namespace kr {
@@ -31,6 +33,54 @@ __global__ __launch_bounds__(kWave) void wait_value32_kernel(const uint32_t* add
         __builtin_amdgcn_s_sleep(32);
     }
     __atomic_thread_fence(__ATOMIC_ACQUIRE);
+}
+
+// All chunks of a gather in one launch, each flagged as it completes.  Workgroups walk runs of 16 KiB pieces in the
+// order of the chunks; the pieces are stored through to memory (system scope), the workgroup waits for its stores,
+// and one lane counts the run into the chunk's flag word: 2 per run, so that no count reads as 1, and the workgroup
+// whose count is the last one stores the 1 that readers wait for.  No cache write-back is needed for that order, where a
+// release would also flush what a product running beside this kernel has written.  Nothing here waits for
+// anything but its own loads and stores.  At most kGatherGroups workgroups of few registers: they fit beside a GEMM
+// workgroup on its compute unit.
+//
+// What it replaces: a copy kernel and a flag kernel per chunk, sixteen launches for eight shards.  Bound by HBM, or
+// by the counts: all flags share a line that takes one count in 12.5 ns, more while tiles poll it, hence runs of up
+// to 16 pieces (8 x 16 MiB: 104 us with a count per piece, 43 us with one per 16; eight copies 51; 8 x 1 MiB: 10.8 /
+// 7.4 (one per 4) / 42).
+constexpr int kPieceVecs = 4;                                // 16-byte vectors per thread and piece
+constexpr int kGatherThreads = 256;
+constexpr uint32_t kPieceBytes = kGatherThreads * kPieceVecs * 16;
+constexpr int kGatherGroups = 1024;
+
+__global__ __launch_bounds__(kGatherThreads) void gather_chunks_kernel(const PeerTab src, int W, int splits, int rank, int64_t chunk_bytes, int run_pieces,
+                                                                      uint32_t runs_per_chunk, uint32_t runs, unsigned char* dst, uint32_t* flags) {
+    for (uint32_t run = blockIdx.x; run < runs; run += gridDim.x) {
+        const uint32_t o = run / runs_per_chunk, in_chunk = run - o * runs_per_chunk;
+        const uint32_t step = o / (uint32_t)splits, split = o - step * (uint32_t)splits;
+        const uint32_t from = ((uint32_t)rank + 1u + step) % (uint32_t)W;
+        const uint32_t chunk = from * (uint32_t)splits + split;
+        const char* in0 = (const char*)src.at((int)from) + (int64_t)split * chunk_bytes;
+        unsigned char* out0 = dst + (int64_t)chunk * chunk_bytes;
+        for (int p = 0; p < run_pieces; ++p) {
+            const int64_t off = ((int64_t)in_chunk * run_pieces + p) * kPieceBytes, left = chunk_bytes - off;
+            if (left <= 0) break;
+            const uint32_t bytes = left < (int64_t)kPieceBytes ? (uint32_t)left : kPieceBytes;
+            // (accesses past the piece's end read zeros and store nothing)
+            const __amdgpu_buffer_rsrc_t in = stream_rsrc(in0 + off, bytes), out = stream_rsrc(out0 + off, bytes);
+            u32x4 v[kPieceVecs];
+#pragma unroll
+            for (int j = 0; j < kPieceVecs; ++j) v[j] = ld_stream(in, (threadIdx.x + j * kGatherThreads) * 16);
+#pragma unroll
+            for (int j = 0; j < kPieceVecs; ++j)
+                __builtin_amdgcn_raw_buffer_store_b128(v[j], out, (int)((threadIdx.x + j * kGatherThreads) * 16), 0, 1 | 16 /* sc0 sc1: system scope */);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wavefront's stores have reached memory
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint32_t before = __hip_atomic_fetch_add(flags + chunk, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (before == 2u * (runs_per_chunk - 1u)) __hip_atomic_store(flags + chunk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
 }
 
 // The two flag primitives the kernels of the all-gather matmul and of the producer GEMM use, in
@@ -89,6 +139,26 @@ extern "C" int kr_stream_wait_value32(const uint32_t* addr, uint32_t value, int6
     const uint64_t ticks = (uint64_t)(wait_limit_us > 0 ? wait_limit_us : 5000000) * 100u;   // default 5 s
     hipLaunchKernelGGL(kr::wait_value32_kernel, dim3(1), dim3(kr::kWave), 0, (hipStream_t)stream, addr, value, ticks,
                        status);
+    return (int)hipGetLastError();
+}
+
+extern "C" int kr_gather_chunks(const void* const* srcs, int W, int splits_per_rank, int rank, int64_t chunk_bytes, void* dst,
+                                uint32_t* progress, void* stream) {
+    if (W < 1 || W > KR_MAX_WORLD) return KR_ERR_WORLD_SIZE;
+    if (rank < 0 || rank >= W || splits_per_rank < 1) return KR_ERR_STRIPE;
+    if (chunk_bytes < 0 || chunk_bytes % 16 != 0) return KR_ERR_BAD_DIM;
+    if (chunk_bytes == 0) return KR_OK;
+    if (dst == nullptr || progress == nullptr) return KR_ERR_NULL_POINTER;
+    if (!kr::aligned16(dst) || (reinterpret_cast<uintptr_t>(progress) & 3u) != 0) return KR_ERR_ALIGNMENT;
+    kr::PeerTab tab;
+    if (const int rc = kr::peer_tab_from_ptrs(tab, srcs, W); rc != KR_OK) return rc;
+    const int64_t chunks = (int64_t)W * splits_per_rank, per_chunk = (chunk_bytes + kr::kPieceBytes - 1) / kr::kPieceBytes;
+    if (chunks > 0x7fffffff || per_chunk > 0x3fffffff / chunks) return KR_ERR_BAD_DIM;
+    const int64_t run_pieces = std::min<int64_t>(std::max<int64_t>(per_chunk * chunks / 128, 1), 16);
+    const int64_t runs_per_chunk = (per_chunk + run_pieces - 1) / run_pieces, runs = runs_per_chunk * chunks;
+    hipLaunchKernelGGL(kr::gather_chunks_kernel, dim3((unsigned)std::min<int64_t>(runs, kr::kGatherGroups)), dim3(kr::kGatherThreads), 0,
+                       (hipStream_t)stream, tab, W, splits_per_rank, rank, chunk_bytes, (int)run_pieces, (uint32_t)runs_per_chunk, (uint32_t)runs,
+                       (unsigned char*)dst, progress);
     return (int)hipGetLastError();
 }
 

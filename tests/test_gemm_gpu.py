@@ -1,5 +1,6 @@
 """GPU parity of the bf16 MFMA GEMM with fused reduce(+bias) epilogue against the CPU oracle.
 Gate: rtol = atol = 2e-2 for bf16 outputs vs the fp32-accumulated oracle."""
+import ctypes
 import os
 
 import pytest
@@ -1245,3 +1246,20 @@ def test_few_rows_kernel(dev, monkeypatch, M, N, K, b_t, fp32):
     monkeypatch.delenv("KRAKEN_AMD_GEMM_SKINNY")
     _lib.reload_env()
     assert lib.kr_gemm_workspace_bytes(M, N, K) >= 0
+
+
+@pytest.mark.parametrize("W,splits,rank,nbytes", [(1, 1, 0, 16), (2, 1, 1, 16384), (3, 2, 0, 16400), (8, 3, 5, 49136), (16, 1, 15, 1 << 20)])
+def test_gather_chunks(dev, W, splits, rank, nbytes):
+    """kr_gather_chunks: one vector, a piece exactly, a piece and one vector, a piece short of one, more pieces than
+    workgroups; all bytes arrive, nothing behind them is written, and every flag reads 1."""
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(nbytes)
+    src = [torch.randint(0, 256, (splits * nbytes + 64,), generator=g, dtype=torch.uint8).to(dev) for _ in range(W)]
+    dst = torch.full((W * splits * nbytes + 64,), 7, dtype=torch.uint8, device=dev)
+    flags = torch.zeros(W * splits + 1, dtype=torch.int32, device=dev)
+    table = (ctypes.c_void_p * W)(*[t.data_ptr() for t in src])
+    rc = lib.kr_gather_chunks(table, W, splits, rank, nbytes, dst.data_ptr(), flags.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+    assert rc == 0, _lib.strerror(rc)
+    assert flags.tolist() == [1] * (W * splits) + [0]
+    assert torch.equal(dst[:W * splits * nbytes], torch.cat([t[:splits * nbytes] for t in src]))
+    assert (dst[W * splits * nbytes:] == 7).all()
