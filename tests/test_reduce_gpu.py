@@ -129,6 +129,25 @@ def test_separate_buffers_match_the_stacked_form(dev, W):
     assert same_bits(out, orc.reduce(staged, full_bias, bias_first=True))
 
 
+@pytest.mark.parametrize("numel", [8, 2040, 2056, 256 * 4 * 8 * 256 + 8, 256 * 4 * 8 * 1024 + 2048 + 8])
+@pytest.mark.parametrize("W", [1, 5, 6, 7, 8, 9, 15, 16])
+def test_groups_of_buffers_and_the_last_block(dev, W, numel):
+    """Every size of the last group of buffers, with the last block cut at either side of a workgroup's vectors, for
+    one and four vectors per thread and for a second trip of the grid: exact."""
+    if W * numel > 9 * (1 << 23):
+        W = 5 if W % 2 else 6
+    stack = orc.make_stack(W, (numel,), seed0=21)
+    stack[:, ::3] = -0.0
+    bias = orc.randn_bf16((numel,), 4)
+    bias[:3] = -0.0
+    want, want_bias = orc.reduce(stack), orc.reduce(stack, bias, bias_first=True)
+    for src in (stack.to(dev), scattered(stack, dev)):
+        assert same_bits(comm.one_shot_all_reduce(src), want)
+        out = torch.empty(numel, dtype=BF16, device=dev)
+        fused.one_shot_all_reduce_bias(src, None, bias.to(dev), out)
+        assert same_bits(out, want_bias)
+
+
 def test_separate_buffers_two_shot_shares(dev):
     W, numel, block = 8, 2048 * 8 * 3 + 8 * 100, 2048
     stack = orc.make_stack(W, (numel,), seed0=5)
