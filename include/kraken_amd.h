@@ -456,6 +456,11 @@ int kr_copy_engine_memcpy(void* dst, const void* src, int64_t bytes, void* strea
 int kr_reduce_rotated_bf16(const void* in, int W, int64_t rows, int64_t N, int rank,
                            int acc_bf16, void* out, void* stream);
 
+/* The same with the W bands in buffers of their own: `bands` is a host array of W device pointers, 16-byte aligned,
+ * entry r = band r as [rows, N] contiguous bf16. */
+int kr_reduce_rotated_ptrs_bf16(const void* const* bands, int W, int64_t rows, int64_t N, int rank,
+                                int acc_bf16, void* out, void* stream);
+
 /*
  * fp32 operands for the bf16 GEMM entry points: x = hi + lo with hi = bf16(x), lo = bf16(x - hi),
  * written in one pass as the three bf16 blocks of a product that is three times as long:

@@ -146,20 +146,36 @@ __global__ __launch_bounds__(kThreads) void reduce_striped_kernel(
 }
 
 // Rotated-order tile reduce of the copy-engine reduce-scatter variant:
-// out[v] = sum_i in[((i + rank + 1) % W) * band_v + v], optionally rounding
-// the running sum to bf16 after every add.
-template <bool ACC_BF16>
+// out[v] = sum_i band_{(i + rank + 1) % W}[v], optionally rounding
+// the running sum to bf16 after every add.  Up to eight bands are requested together.  The bands are
+// the slices of one tensor or buffers of their own (SRC, common.h), so what the other ranks sent is read where it is.
+template <class SRC, bool ACC_BF16>
 __global__ __launch_bounds__(kThreads) void reduce_rotated_kernel(
-    const u32x4* __restrict__ in, int W, int64_t band_v, int rank, u32x4* __restrict__ out) {
+    const SRC src, int W, int64_t band_v, int rank, u32x4* __restrict__ out) {
+    constexpr int G = 8;
     const int64_t v = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (v >= band_v) return;
     float acc[8];
-    int cur = (rank + 1) % W;
-    unpack8(ld_stream(in + cur * band_v + v), acc);
-    for (int i = 1; i < W; ++i) {
-        cur = cur + 1 == W ? 0 : cur + 1;
-        add8(ld_stream(in + cur * band_v + v), acc);
-        if (ACC_BF16) unpack8(pack8(acc), acc);
+    const int first = (rank + 1) % W;
+    for (int i0 = 0; i0 < W; i0 += G) {
+        u32x4 x[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            if (i0 + g < W) {
+                const int cur = first + i0 + g;
+                x[g] = ld_stream(src.at(cur >= W ? cur - W : cur) + v);
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            if (i0 + g >= W) break;
+            if (i0 + g == 0) {
+                unpack8(x[g], acc);
+            } else {
+                add8(x[g], acc);
+                if (ACC_BF16) unpack8(pack8(acc), acc);
+            }
+        }
     }
     st_stream(out + v, pack8(acc));
 }
@@ -343,24 +359,46 @@ extern "C" int kr_reduce_striped_ptrs_bf16(const void* const* bufs, int W, int64
     return launch_striped(tab, W, share, bias, stripe_block, rank, out, stream);
 }
 
-extern "C" int kr_reduce_rotated_bf16(const void* in, int W, int64_t rows, int64_t N, int rank, int acc_bf16,
-                                      void* out, void* stream) {
+template <class SRC>
+static int launch_rotated(const SRC& src, int W, int64_t band_v, int rank, int acc_bf16, void* out, void* stream) {
+    const int64_t blocks = (band_v + kThreads - 1) / kThreads;
+    if (blocks > 0x7fffffffLL) return KR_ERR_BAD_DIM;
+    if (acc_bf16)
+        hipLaunchKernelGGL((reduce_rotated_kernel<SRC, true>), dim3((unsigned)blocks), dim3(kThreads), 0,
+                           (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);
+    else
+        hipLaunchKernelGGL((reduce_rotated_kernel<SRC, false>), dim3((unsigned)blocks), dim3(kThreads), 0,
+                           (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);
+    return (int)hipGetLastError();
+}
+
+// Argument checks of the rotated reduce; `first` is the stacked tensor or the table.  Returns the vectors of a band
+// (0: nothing to do), or a negative argument error.
+static int64_t check_rotated(const void* first, int W, int64_t rows, int64_t N, int rank, const void* out) {
     if (W < 1 || W > KR_MAX_WORLD) return KR_ERR_WORLD_SIZE;
     if (rows < 0 || N < 0) return KR_ERR_BAD_DIM;
     if (rank < 0 || rank >= W) return KR_ERR_STRIPE;
     const int64_t band = rows * N;
     if (band % 8 != 0) return KR_ERR_NUMEL_MOD8;
-    if (band == 0) return KR_OK;
-    if (in == nullptr || out == nullptr) return KR_ERR_NULL_POINTER;
-    if (!aligned16(in) || !aligned16(out)) return KR_ERR_ALIGNMENT;
-    const int64_t band_v = band / 8;
-    const int64_t blocks = (band_v + kThreads - 1) / kThreads;
-    if (blocks > 0x7fffffffLL) return KR_ERR_BAD_DIM;
-    if (acc_bf16)
-        hipLaunchKernelGGL((reduce_rotated_kernel<true>), dim3((unsigned)blocks), dim3(kThreads), 0,
-                           (hipStream_t)stream, (const u32x4*)in, W, band_v, rank, (u32x4*)out);
-    else
-        hipLaunchKernelGGL((reduce_rotated_kernel<false>), dim3((unsigned)blocks), dim3(kThreads), 0,
-                           (hipStream_t)stream, (const u32x4*)in, W, band_v, rank, (u32x4*)out);
-    return (int)hipGetLastError();
+    if (band == 0) return 0;
+    if (first == nullptr || out == nullptr) return KR_ERR_NULL_POINTER;
+    if (!aligned16(out)) return KR_ERR_ALIGNMENT;
+    return band / 8;
+}
+
+extern "C" int kr_reduce_rotated_bf16(const void* in, int W, int64_t rows, int64_t N, int rank, int acc_bf16,
+                                      void* out, void* stream) {
+    const int64_t band_v = check_rotated(in, W, rows, N, rank, out);
+    if (band_v <= 0) return (int)band_v;
+    if (!aligned16(in)) return KR_ERR_ALIGNMENT;
+    return launch_rotated(StackedPeers{(const u32x4*)in, band_v}, W, band_v, rank, acc_bf16, out, stream);
+}
+
+extern "C" int kr_reduce_rotated_ptrs_bf16(const void* const* bands, int W, int64_t rows, int64_t N, int rank,
+                                           int acc_bf16, void* out, void* stream) {
+    const int64_t band_v = check_rotated(bands, W, rows, N, rank, out);
+    if (band_v <= 0) return (int)band_v;
+    PeerTab tab;
+    if (const int rc = peer_tab_from_ptrs(tab, bands, W); rc != KR_OK) return rc;
+    return launch_rotated(tab, W, band_v, rank, acc_bf16, out, stream);
 }

@@ -1,6 +1,8 @@
 """GEMM + copy-engine reduce-scatter, local arithmetic (``kraken/fused/gemm_reduce_scatter_ce_persistent.py``)."""
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib, _waits
@@ -65,8 +67,7 @@ def gemm_producer_w_progress(
     dev = _lib.require_device(a2, b2, gemm_out, progress, signal_pad)
     lib = _lib.load()
     pivot = ((rank + 1) % W) * (M // W)
-    one_round = -(-M // 256) * -(-N // 256) <= torch.cuda.get_device_properties(dev).multi_processor_count
-    if one_round and lib.kr_gemm_workspace_bytes(M, N, a2.shape[1]) > 0:
+    if _one_round(dev, M, N) and lib.kr_gemm_workspace_bytes(M, N, a2.shape[1]) > 0:
         _gemm.launch("gemm_producer_w_progress", a2, b2, M, N, None, 0, 0, None, 0, 0, gemm_out, None, pivot)
         signal_pad.fill_(1)
         return
@@ -76,6 +77,38 @@ def gemm_producer_w_progress(
         _lib.current_stream(dev),
     )
     _lib.check(rc, "gemm_producer_w_progress")
+
+
+def _one_round(dev: torch.device, M: int, N: int) -> bool:
+    """Whether all output tiles run at once, so that all bands finish together."""
+    return -(-M // 256) * -(-N // 256) <= torch.cuda.get_device_properties(dev).multi_processor_count
+
+
+def _byte_range(t: torch.Tensor) -> tuple[int, int]:
+    """First and past-the-last byte a tensor's elements lie in."""
+    if t.numel() == 0:
+        return t.data_ptr(), t.data_ptr()
+    last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+    return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
+
+
+def _readable_in_place(bands: list[torch.Tensor], written: list[torch.Tensor]) -> bool:
+    """Whether the reduce may read the bands where they are while ``written`` is being written."""
+    if any(t.data_ptr() % 16 != 0 or t.device != bands[0].device for t in bands):
+        return False
+    reads = [_byte_range(t) for t in bands]
+    return all(hi <= r_lo or r_hi <= lo for lo, hi in map(_byte_range, written) for r_lo, r_hi in reads)
+
+
+def _reduce_bands(bands: list[torch.Tensor], rows: int, N: int, output: torch.Tensor, configs: dict) -> torch.Tensor:
+    """``reduce`` of W bands in buffers of their own."""
+    dev = _lib.require_device(output, *bands)
+    rc = _lib.load().kr_reduce_rotated_ptrs_bf16(
+        (ctypes.c_void_p * len(bands))(*[t.data_ptr() for t in bands]), len(bands), rows, N, configs["RANK"],
+        int(not configs["fp32_acc"]), output.data_ptr(), _lib.current_stream(dev),
+    )
+    _lib.check(rc, "gemm_reduce_scatter_ce_persistent")
+    return output
 
 
 def copy_engine_scatter(
@@ -147,18 +180,16 @@ def gemm_reduce_scatter_ce_persistent(
     Counterpart of ``kraken.fused.gemm_reduce_scatter_ce_persistent``
     (``kraken/fused/gemm_reduce_scatter_ce_persistent.py:324-375``).  The producer
     GEMM writes the full bf16 ``C = a @ b`` on the current stream and flags every
-    band as it completes; a side stream, which first waits for the current stream
-    (``:345-346``), copies each flagged band to its destination (``:367-368``).  On
-    one GPU the destinations are: this rank's own band -> slot ``rank`` of the
-    scatter buffer ``[W, M/W, N]``; the bands of the other ranks -> ``sent[r]`` when
-    the kwarg ``sent`` (``[W, M/W, N]`` tensor or sequence) is given, else nowhere
-    (the own band, the last to finish, is then copied in stream order behind the
-    GEMM and no flag is waited for).
-    What the other ranks would push arrives from the pre-staged ``peers`` (kwarg,
-    ``[W-1, M/W, N]``, the other ranks in ascending order), copied on the side
-    stream while the GEMM runs.  The current stream then waits for the side stream
-    (``:370``) and the reduce sums the W bands starting at ``rank + 1``
-    (``:258-279``).  kwargs ``rank`` (default 0), ``world_size``, ``fp32_acc``,
+    band as it completes; with the kwarg ``sent`` (``[W, M/W, N]`` tensor or sequence) a side
+    stream, which first waits for the current stream (``:345-346``), copies the flagged band of
+    every other rank r to ``sent[r]`` (``:367-368``).  What the other ranks would push is in the
+    pre-staged ``peers`` (kwarg, ``[W-1, M/W, N]`` or a sequence, the other ranks in ascending
+    order).  The reduce (``:258-279``) sums the W bands starting at ``rank + 1`` and reads them where
+    they are, the peers in their own buffers and the own band in ``C``, instead of through a
+    scatter buffer they are first copied to; peers that overlap ``sent`` or are not 16-byte
+    aligned are copied in front of the GEMM.  Where all bands finish together (one round of
+    output tiles or less) the copies follow the GEMM on the current stream.  It otherwise
+    waits for the side stream (``:370``).  kwargs ``rank`` (default 0), ``world_size``, ``fp32_acc``,
     ``wait_limit_us``, ``status``, ``copy_engine``.
     """
     assert reduce_op == "sum", "only support sum for now"
@@ -174,37 +205,55 @@ def gemm_reduce_scatter_ce_persistent(
     dev = _lib.require_device(a, b)
     _waits.check()      # an earlier call's failed wait is reported before anything of this call is enqueued
     gemm_out = torch.empty((M, N), dtype=a.dtype, device=dev)
-    scatter_out = torch.empty((world_size, m_per_rank, N), dtype=a.dtype, device=dev)
     output = torch.empty((m_per_rank, N), dtype=a.dtype, device=dev)
     configs = {"RANK": rank, "WORLD_SIZE": world_size, "fp32_acc": kwargs.get("fp32_acc", False)}
     if M == 0 or N == 0:
         return output
+    sent = kwargs.get("sent")
+    dests = [None if sent is None or r == rank else sent[r] for r in range(world_size)]
+    bands = list(peers) if peers is not None else []
+    bands.insert(rank, gemm_out[rank * m_per_rank:(rank + 1) * m_per_rank])
+    written = [t for t in dests if t is not None]
+
+    if not _readable_in_place(bands, written):
+        scatter_out = torch.empty((world_size, m_per_rank, N), dtype=a.dtype, device=dev)
+        for r, t in enumerate(bands):
+            if r != rank:
+                scatter_out[r].copy_(t)
+                bands[r] = scatter_out[r]
+    # One round of tiles or less: all bands finish together, so they leave behind the GEMM in stream order, without
+    # flags, and the GEMM may be any (W = 8, 2048 x 4096 x 4096 with all bands sent: 219 us with a wait and a copy per
+    # band on a side stream, 74 us with two copies).
+    if _one_round(dev, M, N) and not (written and kwargs.get("copy_engine", False)):
+        for t in written:
+            assert tuple(t.shape) == (m_per_rank, N) and t.dtype == a.dtype
+        _lib.require_device(a, *written)
+        _gemm.launch("gemm_reduce_scatter_ce_persistent", *_gemm.prepare_operands(a, b), M, N, None, 0, 0, None, 0, 0,
+                     gemm_out, None, ((rank + 1) % world_size) * m_per_rank)
+        by_rank = gemm_out.view(world_size, m_per_rank, N)
+        if isinstance(sent, torch.Tensor) and sent.shape[0] == world_size:
+            for run in (slice(0, rank), slice(rank + 1, world_size)):
+                if run.start < run.stop:
+                    sent[run].copy_(by_rank[run])
+        else:
+            for r, t in enumerate(dests):
+                if t is not None:
+                    t.copy_(by_rank[r])
+        return _reduce_bands(bands, m_per_rank, N, output, configs)
     progress = torch.zeros(world_size, dtype=torch.int32, device=dev)
     signal_pad = torch.zeros(world_size, dtype=torch.int32, device=dev)
-    sent = kwargs.get("sent")
-    dests = [None if sent is None else sent[r] for r in range(world_size)]
-    dests[rank] = scatter_out[rank]
-
     current = torch.cuda.current_stream(dev)
-    backend_stream = _get_backend_stream(dev)
-    backend_stream.wait_stream(current)
+    if written:
+        backend_stream = _get_backend_stream(dev)
+        backend_stream.wait_stream(current)
     gemm_producer_w_progress(a, b, gemm_out, progress, signal_pad, configs)
-    with torch.cuda.stream(backend_stream):
-        if isinstance(peers, torch.Tensor):
-            # the other ranks in ascending order: two runs, below and above the own slot
-            scatter_out[:rank].copy_(peers[:rank])
-            scatter_out[rank + 1:].copy_(peers[rank:])
-        else:
-            others = [r for r in range(world_size) if r != rank]
-            for j, r in enumerate(others):
-                scatter_out[r].copy_(peers[j])
-        if sent is not None:
+    if written:
+        with torch.cuda.stream(backend_stream):
             copy_engine_scatter(gemm_out, dests, signal_pad, rank=rank,
                                 wait_limit_us=kwargs.get("wait_limit_us", 0), status=kwargs.get("status"),
                                 copy_engine=kwargs.get("copy_engine", False))
-    if sent is None:
-        # only the own band has a destination on this GPU, and it is the last one the GEMM
-        # finishes: its copy gains nothing from a flag and goes behind the GEMM in stream order
-        scatter_out[rank].copy_(gemm_out[rank * m_per_rank:(rank + 1) * m_per_rank])
-    current.wait_stream(backend_stream)
-    return reduce(scatter_out.view(M, N), output, configs)
+    # the own band is complete behind the GEMM in stream order: the reduce runs while the last bands leave
+    _reduce_bands(bands, m_per_rank, N, output, configs)
+    if written:
+        current.wait_stream(backend_stream)
+    return output

@@ -867,6 +867,49 @@ def test_separate_peer_buffers_match_the_stacked_form(dev, tile, P):
     assert torch.equal(o3, o4)
 
 
+@pytest.mark.parametrize("M,N,K", [(8, 512, 256), (512, 1024, 4096), (2048, 8192, 256)])   # bands together; one by one
+@pytest.mark.parametrize("form", ["stack", "list", "strided", "overlap", "misaligned", "host"])
+def test_ce_reduce_reads_the_bands_in_place(dev, M, N, K, form):
+    """Where the peers and the destinations lie does not change a bit of the result, also where the reduce may not
+    read them in place: peers that are overwritten by what is sent, that are not aligned, or in host memory."""
+    W, rank, m = 4, 2, M // 4
+    a, b, _ = mk(M, N, K, 0, True, seed=5)
+    a, b = a.to(dev), b.to(dev)
+    peers = torch.stack([orc.randn_bf16((m, N), 100 + j) for j in range(W - 1)])
+    sent = torch.full((W, m, N), 7.0, dtype=BF16, device=dev)
+    plain = torch.zeros_like(sent)
+    c = torch.empty(M, N, dtype=BF16, device=dev)
+    from kraken_amd.fused.gemm_reduce_scatter_ce_persistent import gemm_producer_w_progress
+    gemm_producer_w_progress(a, b, c, *(torch.zeros(W, dtype=torch.int32, device=dev) for _ in range(2)),
+                             {"RANK": rank, "WORLD_SIZE": W})
+    bands = list(peers)
+    bands.insert(rank, c[rank * m:(rank + 1) * m].cpu())
+    want = orc.reduce_rotated(torch.cat(bands, 0), W, rank, acc_bf16=True)
+    if form == "stack":
+        arg = peers.to(dev)
+    elif form == "list":
+        arg = [p.to(dev) for p in peers]
+    elif form == "strided":
+        arg = torch.zeros(W - 1, 2, m, N, dtype=BF16, device=dev)[:, 1]
+        arg.copy_(peers)
+        sent = torch.full((W, m, 2 * N), 7.0, dtype=BF16, device=dev)[:, :, :N]
+    elif form == "overlap":
+        arg = sent[:W - 1]
+        arg.copy_(peers)
+        sent[rank].copy_(peers[rank])
+    elif form == "misaligned":
+        arg = torch.empty((W - 1) * m * N + 1, dtype=BF16, device=dev)[1:].view(W - 1, m, N)
+        arg.copy_(peers)
+    else:
+        arg = peers
+    own = sent[rank].clone()
+    out = fused.gemm_reduce_scatter_ce_persistent(a, b, peers=arg, rank=rank, sent=sent)
+    for r in range(W):
+        assert torch.equal(sent[r], own if r == rank else c[r * m:(r + 1) * m])
+    assert torch.equal(out.cpu(), want)
+    assert torch.equal(out, fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers.to(dev), rank=rank, sent=list(plain)))
+
+
 @pytest.mark.parametrize("splits", [2, 3, 5, 16])
 @pytest.mark.parametrize("b_t", [False, True])
 def test_split_k_loop(dev, monkeypatch, splits, b_t):
