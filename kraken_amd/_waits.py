@@ -39,12 +39,13 @@ def on_failure(hook) -> None:
     _failure_hooks.append(hook)
 
 
-def new_status(dev: torch.device) -> torch.Tensor:
-    """The status word of the current stream of ``dev`` (zero unless an earlier wait on this stream
+def new_status(dev: torch.device, stream_handle: int | None = None) -> torch.Tensor:
+    """The status word of the current stream of ``dev`` (``stream_handle``, if the caller has it at hand; zero unless an earlier wait on this stream
     has run out and has not been reported yet).  Every wait of one call shares it: the first wait
     that runs out makes the later ones give up at once instead of each running to the limit."""
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(dev).cuda_stream)
+    if stream_handle is None:
+        stream_handle = torch.cuda.current_stream(dev).cuda_stream
+    key = (dev.index if dev.index is not None else torch.cuda.current_device(), stream_handle)
     with _lock:
         word = _words.get(key)
         if word is None:
