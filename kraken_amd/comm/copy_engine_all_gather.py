@@ -10,7 +10,8 @@ from ._common import PeerBuffers
 
 # Up to here the sixteen launches of eight copies and flags bound the call (all_gather_matmul, K = 8192, N = 3584: eight
 # shards of 4 .. 128 rows 212 us, in one launch 114; 256 rows, 32 MiB gathered, 225 / 180; 512 rows 233 / 235).  Above,
-# the product does, and copies that come one behind the other leave it more of the memory (1024 rows 405 / 438).
+# the product does, and copies that come one behind the other leave it more of the memory (1024 rows 405 / 438;
+# the same kernel once per chunk 424).
 ONE_LAUNCH_BYTES = 48 << 20
 
 _backend_streams: dict[int, torch.cuda.Stream] = {}
