@@ -495,10 +495,13 @@ int kr_cast_fp8_to_bf16(const void* src, int64_t n, void* dst, void* stream);
 int kr_cast_f32_to_fp8(const void* src, int64_t n, void* dst, void* stream);
 
 /*
- * out[M, N] = A[M, K] @ Bt[N, K]^T on fp8 (e4m3fn) operands with fp32 accumulation, on the fp8
+ * out[M, N] = A[M, K] @ Bt[N, K]^T on fp8 (e4m3fn) operands, on the fp8
  * matrix-core instruction (v_mfma_f32_16x16x128_f8f6f4): the product of the fp8 branch of
  * kraken/fused/all_gather_matmul.py:53,121,213 (tl.dot of float8e4nv tiles, fp32 accumulator,
  * result cast to the operands' type) at twice the bf16 rate, without widening the operands.
+ * Precision: the accumulators are fp32, but the instruction keeps about 16 bits of a sum: 1.1e-5 to
+ * 1.5e-5 in the 2-norm against 64 bits for K = 128 .. 16384, where widened operands on the bf16
+ * instruction show 2e-9 (K = 4096).  An fp8 result is then one step off in 5e-4 of its elements.
  *   A: row-major, lda bytes between rows; Bt: the right operand transposed (k contiguous), ldb
  *   bytes between its rows -- the layout the reference's benchmark passes (`b.T` of an [N, K] tensor).
  *   out_kind: 0 = bf16, 1 = fp32, 2 = fp8 (e4m3fn; fp32 sums rounded once, nearest even, magnitudes
@@ -524,7 +527,8 @@ int kr_all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, in
 
 /*
  * The same two products for any number of rows, N and K multiples of 16, K >= 128 (edge tiles and a last
- * k-step that is not full are handled by the kernel).  kr_gemm_fp8_ws: with a workspace of
+ * k-step that is not full are handled by the kernel).  The Python layer calls them for whole tiles only,
+ * because of the precision stated above; other shapes are widened there.  kr_gemm_fp8_ws: with a workspace of
  * kr_gemm_fp8_workspace_bytes bytes (0: none needed), shapes with few tiles share each tile's K loop
  * between workgroups, whose fp32 parts meet there and are summed in a fixed order; contents are scratch,
  * and calls that may overlap need one each.

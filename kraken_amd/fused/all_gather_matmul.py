@@ -39,13 +39,17 @@ def _matmul_w_progress(a, a_local, b, progress, configs, status=None) -> torch.T
 
 
 def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **kwargs):
-    """The fp8 branch of ``all_gather_matmul`` (``all_gather_matmul.py:53,121,213``): fp8 product with fp32
-    accumulation, rounded to fp8 once.  From K = 128 on the product runs on the fp8 matrix-core instruction
-    (``kr_gemm_fp8_ws``, or ``kr_all_gather_matmul_fp8_ragged`` for ``gather=True``: the shards are copied chunk
-    by chunk on a side stream while the tiles wait for their chunk's flag, as in the bf16 form); shorter K is
-    widened to bf16 (exact), multiplied by the bf16 kernels with an fp32 result, and rounded by
-    ``kr_cast_f32_to_fp8`` -- the same sums up to fp32 summation order -- after the gather has finished.
-    ``fp8_kernel=False`` forces the widening path."""
+    """The fp8 branch of ``all_gather_matmul`` (``all_gather_matmul.py:53,121,213``): fp8 product, rounded to
+    fp8 once.  Shapes of whole tiles (M, N multiples of 256, K of 128) run on
+    the fp8 matrix-core instruction (``kr_gemm_fp8_ws``, or ``kr_all_gather_matmul_fp8`` for ``gather=True``: the
+    shards are copied chunk by chunk on a side stream while the tiles wait for their chunk's flag, as in the
+    bf16 form); others are widened to bf16 (exact), multiplied by the bf16 kernels with an fp32 result, and
+    rounded by ``kr_cast_f32_to_fp8`` after the gather has finished.  ``fp8_kernel=False`` forces the widening path.
+
+    The two differ in the precision of the sums: the fp8 instruction keeps about 16 bits of them (1.2e-5 in the
+    2-norm against 64 bits, K = 128 .. 16384; both the 16x16x32 and the 16x16x128 form, to the same bits), the bf16
+    instruction all 24 (2e-9 at K = 4096), so ragged shapes are not sent to the fp8 kernel although its C entry points
+    take them: 4000 x 6656 x 4096 takes 83 us there and 250 us here, with 5e-4 of the results one fp8 step off."""
     fp8 = torch.float8_e4m3fn
     W = peers.W
     m, K = peers.slice(0).shape
@@ -63,7 +67,7 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
     dev = _lib.require_device(*peers.tensors, b, a_out, progress)
     lib = _lib.load()
     stream = _lib.current_stream(dev)
-    native = kwargs.get("fp8_kernel", True) and K >= 128
+    native = kwargs.get("fp8_kernel", True) and M % 256 == 0 and N % 256 == 0 and K % 128 == 0
     if gather:
         assert m % splits == 0, "splits_per_rank must divide the rows of a shard"
         _waits.check()      # an earlier call's failed wait is reported before anything of this call is enqueued
@@ -85,7 +89,7 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
             a_local = peers.slice(rank)
             assert a_local.stride(1) == 1
             c = torch.empty((M, N), dtype=fp8, device=dev)
-            rc = lib.kr_all_gather_matmul_fp8_ragged(
+            rc = lib.kr_all_gather_matmul_fp8(
                 a_out.data_ptr(), K, a_local.data_ptr(), a_local.stride(0), b.T.data_ptr(), K, M, N, K, W, rank, splits,
                 progress.data_ptr(), int(kwargs.get("wait_limit_us", 0)), _lib.ptr(status), c.data_ptr(), 2, stream)
             _lib.check(rc, "all_gather_matmul(fp8)")
@@ -164,8 +168,9 @@ def all_gather_matmul(
     fp8 operands (``torch.float8_e4m3fn`` for the shards and ``b``) give an fp8 ``c``
     like in the reference (``:53,121,213``): fp32 accumulate, one rounding to fp8
     (nearest even, magnitudes of 448 and more saturate to 448), in both modes.
-    From K = 128 on the product runs on the fp8 matrix-core instruction; a shorter K
-    (and ``fp8_kernel=False``) is widened to bf16 by one conversion pass per operand
+    With M and N multiples of 256 and K of 128 the product runs on the fp8
+    matrix-core instruction, whose sums keep about 16 bits; other sizes (multiples of 16,
+    and ``fp8_kernel=False``) are widened to bf16 by one conversion pass per operand
     (exact: every e4m3 value is a bf16 value), multiplied by the bf16 kernels with an
     fp32 result and rounded to fp8 by a third pass, after the gather has finished.
     ``a_gathered`` stays fp8.

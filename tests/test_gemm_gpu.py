@@ -1161,6 +1161,26 @@ def test_fp8_kernel_ragged_shapes(dev, M, N, K, split):
         assert (out[M].float() == 0).all()                     # nothing past the last row
 
 
+@pytest.mark.parametrize("gather", [False, True])
+@pytest.mark.parametrize("m,K,N", [(250, 144, 528), (33, 208, 4112), (256, 144, 512), (250, 128, 512)])
+def test_all_gather_matmul_fp8_ragged_sums_keep_their_bits(dev, m, K, N, gather):
+    """fp8 shapes that are no whole 256 x 256 x 128 tiles: the fp32 sums are exact, so the fp8 result is the rounded
+    64-bit product in every element.  Operands N(0, 1) and N(0, 0.25) in e4m3 are multiples of 2^-9, their products
+    of 2^-18, and with sum |a||b| below 2^6 every partial sum has at most 24 bits, whatever the order."""
+    fp8 = torch.float8_e4m3fn
+    W = 8
+    g = torch.Generator().manual_seed(m + K + N)
+    a = torch.randn(W, m, K, generator=g).to(fp8)
+    bT = (torch.randn(N, K, generator=g) * 0.25).to(fp8)
+    a2, b2 = a.reshape(W * m, K).double(), bT.double().T
+    assert (a2.abs() @ b2.abs()).max() < 64.0
+    want = (a2 @ b2).float().to(fp8)
+    shards = [t.to(dev) for t in a] if gather else a.to(dev)
+    a_out, c = fused.all_gather_matmul(shards, bT.to(dev).T, rank=2, gather=gather)
+    assert torch.equal(a_out.cpu().view(torch.uint8), a.reshape(W * m, K).view(torch.uint8))
+    assert torch.equal(c.cpu().float(), want.float()), int((c.cpu().float() != want.float()).sum())
+
+
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("M,N,K", [(256, 256, 72), (512, 264, 120), (264, 512, 328), (511, 520, 1016)])
 def test_large_tile_kernel_last_k_step_not_full(dev, monkeypatch, M, N, K, b_t):
