@@ -67,16 +67,16 @@ def fp32_direct(a: torch.Tensor, b: torch.Tensor) -> bool:
     return -(-a.shape[0] // 128) * -(-b.shape[1] // 128) <= 512
 
 
-def prepare_operands(a: torch.Tensor, b: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+def prepare_operands(a: torch.Tensor, b: torch.Tensor, keep_fp32: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """Return operands in a type and layout the kernel reads directly.
 
     A must be k-contiguous; B either row-major or transposed-contiguous; any row
     stride that is a multiple of 8 elements is read in place (the kernels address
     operands through buffer descriptors built from the caller's strides).  Other
     stridings (the reference accepts any 2-D strides,
-    ``gemm_one_shot_all_reduce_fused.py:163-166``) take one copy.  fp32 operands stay fp32
-    where the product splits them itself (``fp32_direct``), else they are split into bf16
-    parts by one kernel pass each (``split_fp32``).
+    ``gemm_one_shot_all_reduce_fused.py:163-166``) take one copy.  fp32 operands are split into
+    bf16 parts by one kernel pass each (``split_fp32``); with ``keep_fp32``, for callers whose
+    product goes through ``launch``, they stay fp32 where it splits them itself (``fp32_direct``).
     K is padded to a multiple of 8 with zeros when necessary.
     """
     assert a.dim() == 2 and b.dim() == 2
@@ -84,7 +84,7 @@ def prepare_operands(a: torch.Tensor, b: torch.Tensor) -> tuple[torch.Tensor, to
     assert a.dtype == b.dtype, "Input tensors must have the same dtype"
     assert a.dtype in (torch.bfloat16, torch.float32), "bfloat16 (or float32) operands expected"
     if a.dtype == torch.float32:
-        if fp32_direct(a, b):
+        if keep_fp32 and fp32_direct(a, b):
             return (a if fp32_rows_ok(a) else a.contiguous()), (b if fp32_rows_ok(b) or fp32_rows_ok(b.T) else b.contiguous())
         a, b = split_fp32(a, b)
     K = a.shape[1]

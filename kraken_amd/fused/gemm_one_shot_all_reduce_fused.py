@@ -25,7 +25,7 @@ def gemm_one_shot_all_reduce(a: torch.Tensor, b: torch.Tensor, **kwargs) -> torc
     ``group``, ``BLOCK_SIZE_M/N/K``, ``GROUP_SIZE_M``, ``num_warps`` and
     ``num_stages`` are accepted and ignored.
     """
-    a, b = _gemm.prepare_operands(a, b)
+    a, b = _gemm.prepare_operands(a, b, keep_fp32=True)
     M, N = a.shape[0], b.shape[1]
     assert N % 8 == 0, "N must be a multiple of 8"
     peers = kwargs.get("peers")

@@ -28,7 +28,7 @@ def gemm_reduce_scatter(a: torch.Tensor, b: torch.Tensor, **kwargs) -> torch.Ten
     Returns ``[M/W, N]`` in ``a.dtype``.  Tile-size kwargs are ignored.
     """
     in_dtype = a.dtype
-    a, b = _gemm.prepare_operands(a, b)
+    a, b = _gemm.prepare_operands(a, b, keep_fp32=True)
     M, N = a.shape[0], b.shape[1]
     assert N % 8 == 0, "N must be a multiple of 8"
     peers = kwargs.get("peers")

@@ -910,6 +910,25 @@ def test_ce_reduce_reads_the_bands_in_place(dev, M, N, K, form):
     assert torch.equal(out, fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers.to(dev), rank=rank, sent=list(plain)))
 
 
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 256), (512, 1024, 4096), (2304, 8192, 256)])   # one pass, split K loop, more than a round
+def test_producer_takes_fp32_operands(dev, M, N, K, b_t):
+    """gemm_producer_w_progress with fp32 operands, at shapes with and without a workspace: integers up to 2^8 times
+    integers up to 8 are one bf16 value each, so every fp32 sum is exact and gemm_out the product rounded once."""
+    from kraken_amd.fused.gemm_reduce_scatter_ce_persistent import gemm_producer_w_progress
+    g = torch.Generator().manual_seed(K)
+    a = torch.randint(-256, 257, (M, K), generator=g).float()
+    b = torch.randint(-8, 9, (K, N), generator=g).float()
+    assert K * 256 * 8 < 1 << 24
+    ad, bd = a.to(dev), b.T.contiguous().to(dev).T if b_t else b.to(dev)
+    W = 4
+    c = torch.empty(M, N, dtype=BF16, device=dev)
+    progress, signal_pad = (torch.zeros(W, dtype=torch.int32, device=dev) for _ in range(2))
+    gemm_producer_w_progress(ad, bd, c, progress, signal_pad, {"RANK": 1, "WORLD_SIZE": W})
+    assert torch.equal(c, (ad @ bd).to(BF16)), (c.float() - ad @ bd).abs().max()
+    assert (signal_pad == 1).all()
+
+
 @pytest.mark.parametrize("splits", [2, 3, 5, 16])
 @pytest.mark.parametrize("b_t", [False, True])
 def test_split_k_loop(dev, monkeypatch, splits, b_t):
