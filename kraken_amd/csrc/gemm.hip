@@ -658,8 +658,10 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     p.tile = dtl ? 256 : 128;
     // KRAKEN_AMD_GEMM_PEERS=epilogue keeps the peers' partial sums out of the matrix cores
     // (they are then added in the epilogue, where a non-finite value stays in its element)
-    p.peers_on_mfma = 1;
-    if (env_switches().gemm_peers >= 0) p.peers_on_mfma = env_switches().gemm_peers;
+    // K no multiple of the k-step: always in the epilogue, which is where every kernel that takes such shapes
+    // adds them (the matrix cores would turn the 16 columns around an Inf into NaN)
+    p.peers_on_mfma = K % 64 == 0;
+    if (env_switches().gemm_peers >= 0 && K % 64 == 0) p.peers_on_mfma = env_switches().gemm_peers;
     // MFMA block shape of the 256x256 kernel: 16x16x32 draws less power per flop than 32x32x16 and
     // the chip is power-limited (k loop 5-10 % faster with warm operands; results agree to fp32
     // rounding), and its peer phase takes two peers per MFMA.  KRAKEN_AMD_GEMM_MFMA=16|32 overrides.

@@ -331,6 +331,19 @@ def test_gemm_plan_reports_the_dispatch(lib, monkeypatch):
         _lib.reload_env()
 
 
+@pytest.mark.parametrize("mode", [None, "mfma", "first", "last", "epilogue"])
+def test_gemm_plan_peers_of_a_ragged_k_stay_in_the_epilogue(lib, monkeypatch, mode):
+    """Peers are added on the matrix cores only where K is a multiple of 64, which is the condition the header gives
+    for a non-finite partial sum spreading over its 16 columns."""
+    if mode is not None:
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_PEERS", mode)
+    for b_t in (False, True):
+        for K in (4112, 4104, 264):
+            p = _lib.gemm_plan(4096, 4096, K, b_t, 7, 4096)
+            assert p["tile"] == 256 and not p["peers_on_mfma"]
+        assert _lib.gemm_plan(4096, 4096, 4096, b_t, 7, 4096)["peers_on_mfma"] == (mode != "epilogue")
+
+
 def test_split_fp32_argument_errors(lib):
     f = lib.kr_split_fp32
     assert f(FAKE, 16, 12, 12, 1, 0, FAKE, 36, None) == _lib.KR_ERR_NUMEL_MOD8

@@ -815,6 +815,30 @@ def test_non_finite_partial_sum_stays_local(dev, monkeypatch, mode):
     torch.testing.assert_close(out[~group], want[~group], **TOL)
 
 
+@pytest.mark.parametrize("M,N,K", [(3072, 3072, 264), (3000, 3080, 328)])    # 144 tiles of 256 x 256, whole and ragged
+@pytest.mark.parametrize("b_t", [False, True])
+def test_non_finite_partial_sum_stays_in_its_element_with_a_ragged_k(dev, M, N, K, b_t):
+    """K no multiple of 64: an Inf and a NaN in one peer each stay in their own element, and a bf16 result is the
+    product rounded to bf16, then the sum with the peers rounded once more (small integers: all sums exact)."""
+    g = torch.Generator().manual_seed(K)
+    a = torch.randint(-4, 5, (M, K), generator=g).float()
+    b = torch.randint(-4, 5, (K, N), generator=g).float()
+    peers = torch.randint(-8, 9, (3, M, N), generator=g).float()
+    product = a @ b
+    once = product + peers.sum(0)
+    twice = product.to(BF16).float() + peers.sum(0)
+    assert not torch.equal(once.to(BF16), twice.to(BF16))
+    peers[1, 300, 77], peers[2, 700, 1030] = float("inf"), float("nan")
+    once[300, 77] = twice[300, 77] = float("inf")
+    once[700, 1030] = twice[700, 1030] = float("nan")
+    ad, pd = a.to(BF16).to(dev), peers.to(BF16).to(dev)
+    bd = b.T.contiguous().to(BF16).to(dev).T if b_t else b.to(BF16).to(dev)
+    for dtype, want in ((torch.float32, once), (BF16, twice.to(BF16))):
+        out = fused.gemm_one_shot_all_reduce_fused(ad, bd, peers=pd, out_dtype=dtype).cpu()
+        assert torch.equal(torch.isnan(out), torch.isnan(want))
+        assert torch.equal(torch.nan_to_num(out.float(), nan=0.5), torch.nan_to_num(want.float(), nan=0.5))
+
+
 @pytest.mark.parametrize("P", [1, 2, 7, 8, 15])
 def test_gemm_all_reduce_world_sizes(dev, tile, P):
     """Every world size the C ABI accepts (W = P + 1 up to 16), on a shape with whole-band
