@@ -60,11 +60,25 @@ def fp32_direct(a: torch.Tensor, b: torch.Tensor) -> bool:
 
     Up to two rounds of its 128 x 128 tiles on the 256 compute units: 2000 x 4096 x 2048 takes 117 us there and 166 us
     as a split pass and a bf16 product; with more tiles the 256 x 256 bf16 kernel wins the pass back
-    (4096 x 4096 x 1024: 135 against 104 us).
+    (4096 x 4096 x 1024: 135 against 104 us).  The kernel addresses 128 rows of an operand with 32-bit byte offsets: row
+    strides beyond that reach (from about 4.19 million elements on) take the split pass, which reads any stride.
     """
     if not (a.is_cuda and b.is_cuda) or a.shape[1] % 8 != 0 or b.shape[1] % 8 != 0:
         return False
-    return -(-a.shape[0] // 128) * -(-b.shape[1] // 128) <= 512
+    return -(-a.shape[0] // 128) * -(-b.shape[1] // 128) <= 512 and _fp32_in_reach(a, b)
+
+
+def _fp32_in_reach(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether ``kr_gemm_reduce_f32_ws`` takes the row strides of ``fp32_layout(a, b)``, whatever the other sizes."""
+    K, N = b.shape
+    lda = a.stride(0) if fp32_rows_ok(a) else K
+    ldb = b.stride(0) if fp32_rows_ok(b) else b.stride(1) if fp32_rows_ok(b.T) else N
+    return (128 * max(lda, ldb) + max(K, N)) * 4 < 0x7fffffff
+
+
+def fp32_layout(a: torch.Tensor, b: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """fp32 operands in a layout ``kr_gemm_reduce_f32_ws`` reads."""
+    return (a if fp32_rows_ok(a) else a.contiguous()), (b if fp32_rows_ok(b) or fp32_rows_ok(b.T) else b.contiguous())
 
 
 def prepare_operands(a: torch.Tensor, b: torch.Tensor, keep_fp32: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
@@ -85,7 +99,7 @@ def prepare_operands(a: torch.Tensor, b: torch.Tensor, keep_fp32: bool = False) 
     assert a.dtype in (torch.bfloat16, torch.float32), "bfloat16 (or float32) operands expected"
     if a.dtype == torch.float32:
         if keep_fp32 and fp32_direct(a, b):
-            return (a if fp32_rows_ok(a) else a.contiguous()), (b if fp32_rows_ok(b) or fp32_rows_ok(b.T) else b.contiguous())
+            return fp32_layout(a, b)
         a, b = split_fp32(a, b)
     K = a.shape[1]
     if K % 8 != 0:

@@ -1308,6 +1308,26 @@ def test_fp32_operands_split_in_registers(dev, monkeypatch, M, N, K, b_t):
         assert ((out - ar.double() @ br.double()).abs() <= 2.0 ** -15 * (ar.abs().double() @ br.abs().double())).all(), splits
 
 
+@pytest.mark.parametrize("wide", ["a", "b", "b_t"])
+def test_fp32_operands_with_very_wide_rows(dev, wide):
+    """fp32 operands that are slices of matrices with rows of 4.2 million elements: 128 such rows reach past the 2 GiB that
+    the kernel which splits in registers can address, so they take the split pass.  Small integers: the product is exact."""
+    M, N, K, ld = 72, 136, 64, 4_200_000
+    rows = {"a": M, "b": K, "b_t": N}[wide]
+    big = torch.zeros(rows, ld, dtype=torch.float32, device=dev)     # 1.1 to 2.3 GB
+    g = torch.Generator().manual_seed(ld)
+    a = torch.randint(-8, 9, (M, K), generator=g).float().to(dev)
+    b = torch.randint(-8, 9, (K, N), generator=g).float().to(dev)
+    want = a @ b
+    part = big[:, 16:16 + {"a": K, "b": N, "b_t": K}[wide]]
+    part.copy_({"a": a, "b": b, "b_t": b.T}[wide])
+    if wide == "a":
+        a = part
+    else:
+        b = part if wide == "b" else part.T
+    assert torch.equal(fused.gemm_one_shot_all_reduce_fused(a, b), want)
+
+
 @pytest.mark.parametrize("fp32", [False, True])
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (16, 32, 64), (17, 40, 72), (32, 264, 520), (33, 136, 1000), (64, 1032, 1096)])
