@@ -147,12 +147,12 @@ extern "C" int kr_gather_chunks(const void* const* srcs, int W, int splits_per_r
     if (W < 1 || W > KR_MAX_WORLD) return KR_ERR_WORLD_SIZE;
     if (rank < 0 || rank >= W || splits_per_rank < 1) return KR_ERR_STRIPE;
     if (chunk_bytes < 0 || chunk_bytes % 16 != 0) return KR_ERR_BAD_DIM;
-    if (chunk_bytes == 0) return KR_OK;
-    if (dst == nullptr || progress == nullptr) return KR_ERR_NULL_POINTER;
+    if ((chunk_bytes > 0 && dst == nullptr) || progress == nullptr) return KR_ERR_NULL_POINTER;
     if (!kr::aligned16(dst) || (reinterpret_cast<uintptr_t>(progress) & 3u) != 0) return KR_ERR_ALIGNMENT;
-    kr::PeerTab tab;
-    if (const int rc = kr::peer_tab_from_ptrs(tab, srcs, W); rc != KR_OK) return rc;
-    const int64_t chunks = (int64_t)W * splits_per_rank, per_chunk = (chunk_bytes + kr::kPieceBytes - 1) / kr::kPieceBytes;
+    kr::PeerTab tab{};   // (of empty chunks only the flags are written: one run each that copies nothing)
+    if (chunk_bytes > 0)
+        if (const int rc = kr::peer_tab_from_ptrs(tab, srcs, W); rc != KR_OK) return rc;
+    const int64_t chunks = (int64_t)W * splits_per_rank, per_chunk = std::max<int64_t>((chunk_bytes + kr::kPieceBytes - 1) / kr::kPieceBytes, 1);
     if (chunks > 0x7fffffff || per_chunk > 0x3fffffff / chunks) return KR_ERR_BAD_DIM;
     const int64_t run_pieces = std::min<int64_t>(std::max<int64_t>(per_chunk * chunks / 128, 1), 16);
     const int64_t runs_per_chunk = (per_chunk + run_pieces - 1) / run_pieces, runs = runs_per_chunk * chunks;

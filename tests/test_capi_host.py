@@ -399,6 +399,18 @@ def test_gemm_fp8_argument_errors(lib):
     assert gcall(M=1024, N=384) == _lib.KR_ERR_BAD_DIM   # the product's own shape rule
 
 
+def test_gather_chunks_argument_errors(lib):
+    f = lib.kr_gather_chunks
+    table = (ctypes.c_void_p * 2)(FAKE, FAKE)
+    assert f(table, 0, 1, 0, 16, FAKE, FAKE, None) == _lib.KR_ERR_WORLD_SIZE
+    assert f(table, 2, 1, 2, 16, FAKE, FAKE, None) == _lib.KR_ERR_STRIPE
+    assert f(table, 2, 1, 0, 24, FAKE, FAKE, None) == _lib.KR_ERR_BAD_DIM
+    assert f(table, 2, 1, 0, 16, None, FAKE, None) == _lib.KR_ERR_NULL_POINTER
+    assert f(table, 2, 1, 0, 16, FAKE + 8, FAKE, None) == _lib.KR_ERR_ALIGNMENT
+    assert f(table, 2, 1, 0, 16, FAKE, FAKE + 2, None) == _lib.KR_ERR_ALIGNMENT
+    assert f(None, 2, 1, 0, 0, None, None, None) == _lib.KR_ERR_NULL_POINTER     # empty chunks still have flags
+
+
 def test_probe_argument_errors(lib):
     assert lib.kr_probe_read(FAKE, 24, None, None) == _lib.KR_ERR_NUMEL_MOD8
     assert lib.kr_probe_read(None, 32, None, None) == _lib.KR_ERR_NULL_POINTER

@@ -1389,3 +1389,15 @@ def test_gather_chunks(dev, W, splits, rank, nbytes):
     assert flags.tolist() == [1] * (W * splits) + [0]
     assert torch.equal(dst[:W * splits * nbytes], torch.cat([t[:splits * nbytes] for t in src]))
     assert (dst[W * splits * nbytes:] == 7).all()
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("shape", [(0, 64), (6, 0)])
+def test_gather_of_empty_shards_sets_its_flags(dev, shape, splits):
+    """Chunks without bytes have arrived as soon as the gather runs: every flag reads 1, the others stay."""
+    W = 4
+    for shards in (torch.empty(W, *shape, dtype=BF16, device=dev), [torch.empty(shape, dtype=BF16, device=dev) for _ in range(W)]):
+        progress = torch.zeros(W * splits + 1, dtype=torch.int32, device=dev)
+        out = torch.empty(W * shape[0], shape[1], dtype=BF16, device=dev)
+        assert comm.all_gather_w_progress(shards, out, progress, splits_per_rank=splits, rank=1) is out
+        assert progress.tolist() == [1] * (W * splits) + [0]
