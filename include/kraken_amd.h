@@ -426,8 +426,9 @@ int kr_flag_arrive_wait(uint32_t* flags, int producers, int consumers, int64_t w
  * All chunks of an all-gather and their flags in one launch: source r's buffer srcs[r] (a host array of W device
  * pointers) holds splits_per_rank chunks of chunk_bytes; chunk c = r * splits_per_rank + s is copied to
  * dst + c * chunk_bytes, and progress[c] is 1 once it has arrived (visible to kernels that read the flag).  Chunks are
- * taken in the order of the source ranks rank+1, rank+2, ..., rank.  progress[] must be zero when the kernel starts; a
- * chunk that is still arriving may show any even count there.  chunk_bytes a multiple of 16, pointers 16-byte aligned; with
+ * taken in the order of the source ranks rank+1, rank+2, ..., rank.  For readers that wait, progress[] must be zero when
+ * the kernel starts (a flag of an earlier gather, 1, only ends at 1 again); a chunk that is still arriving may show any
+ * even count there.  chunk_bytes a multiple of 16, pointers 16-byte aligned; with
  * chunk_bytes == 0 the flags are set and srcs and dst are not looked at.
  * Replaces the loop of copies and flag writes of the reference's chunked all-gather
  * (kraken/comm/copy_engine_all_gather.py:38-53).

@@ -37,8 +37,9 @@ __global__ __launch_bounds__(kWave) void wait_value32_kernel(const uint32_t* add
 
 // All chunks of a gather in one launch, each flagged as it completes.  Workgroups walk runs of 16 KiB pieces in the
 // order of the chunks; the pieces are stored through to memory (system scope), the workgroup waits for its stores,
-// and one lane counts the run into the chunk's flag word: 2 per run, so that no count reads as 1, and the workgroup
-// whose count is the last one stores the 1 that readers wait for.  No cache write-back is needed for that order, where a
+// and one lane counts the run into the chunk's flag word: 2 per run, so that no count makes a 0 read as 1, and the
+// workgroup whose count is the last one stores the 1 that readers wait for.  The lowest bit is not part of the count: a
+// flag that an earlier gather has left at 1 ends at 1 again.  No cache write-back is needed for that order, where a
 // release would also flush what a product running beside this kernel has written.  Nothing here waits for
 // anything but its own loads and stores.  At most kGatherGroups workgroups of few registers: they fit beside a GEMM
 // workgroup on its compute unit.
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(kGatherThreads) void gather_chunks_kernel(const Pee
         __syncthreads();
         if (threadIdx.x == 0) {
             const uint32_t before = __hip_atomic_fetch_add(flags + chunk, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (before == 2u * (runs_per_chunk - 1u)) __hip_atomic_store(flags + chunk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (before >> 1 == runs_per_chunk - 1u) __hip_atomic_store(flags + chunk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 }

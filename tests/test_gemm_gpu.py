@@ -1401,3 +1401,17 @@ def test_gather_of_empty_shards_sets_its_flags(dev, shape, splits):
         out = torch.empty(W * shape[0], shape[1], dtype=BF16, device=dev)
         assert comm.all_gather_w_progress(shards, out, progress, splits_per_rank=splits, rank=1) is out
         assert progress.tolist() == [1] * (W * splits) + [0]
+
+
+@pytest.mark.parametrize("rows", [8, 520])      # a run of one piece per chunk, several runs
+def test_gather_over_the_flags_of_an_earlier_one(dev, rows):
+    """The chunked copy with flags that are still 1 from the gather before: the new shards arrive and the flags end at 1."""
+    from kraken_amd.comm.copy_engine_all_gather import _copy_engine_all_gather_w_progress
+    W, K = 4, 1024
+    progress = torch.zeros(W, dtype=torch.int32, device=dev)
+    out = torch.empty(W * rows, K, dtype=BF16, device=dev)
+    for seed in range(3):
+        shards = orc.randn_bf16((W, rows, K), seed).to(dev)
+        torch.cuda.current_stream(dev).wait_stream(_copy_engine_all_gather_w_progress(out, shards, progress, 1, rank=2))
+        assert torch.equal(out, shards.view(W * rows, K))
+        assert progress.tolist() == [1] * W
