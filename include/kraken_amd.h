@@ -574,7 +574,8 @@ int kr_gemm_reduce_f32_ws(const void* A, int64_t lda_m, int64_t lda_k, const voi
  *   plan[7] bit 0: M or N is not a multiple of the tile or K of 64 (bounds-checked edges); bit 1: the
  *           tile is 256 x 224 (a plain product with transposed-contiguous B that fills whole rounds
  *           of the compute units with 224-column tiles and not with 256-column ones); bit 2: at most 64
- *           rows, gemm_skinny_kernel (16 to 64 columns per workgroup instead of tiles)
+ *           rows, gemm_skinny_kernel (16 to 64 columns per workgroup instead of tiles); bit 3: 128x128
+ *           tiles in gemm_ks_kernel (no bit of 2 and 3: those of gemm_reduce_kernel)
  */
 int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, int n_peers, int64_t band_rows,
                  int has_bias, int has_c_full, int64_t workspace_bytes, int32_t plan[8]);

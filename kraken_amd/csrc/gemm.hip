@@ -1133,7 +1133,7 @@ extern "C" int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, i
                                  band_rows == M, workspace_bytes > 0, workspace_bytes, false, false, false, gemm_dtl_supported(g), true);
     const bool whole_band_peers = p.tile == 256 && n_peers > 0 && p.peers_on_mfma != 0;
     plan[0] = p.tile;
-    plan[1] = p.tile == 256 ? (p.mi16 ? 16 : 32) : 32;   // MFMA block rows: 16x16x32 or 32x32x16
+    plan[1] = (p.tile == 256 ? p.mi16 : p.ks || p.skinny) ? 16 : 32;   // MFMA block rows: 16x16x32 or 32x32x16
     plan[2] = p.splits;
     plan[3] = p.tail_tiles;
     plan[4] = p.tail_splits;
@@ -1142,6 +1142,7 @@ extern "C" int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, i
     plan[7] = (M % p.tile != 0 || N % p.tile != 0 || K % 64 != 0) ? 1 : 0;
     if (p.n224) plan[7] |= 2;   // bit 1: 256 x 224 tiles
     if (p.skinny) plan[7] |= 4;   // bit 2: gemm_skinny_kernel
+    if (p.ks) plan[7] |= 8;   // bit 3: gemm_ks_kernel
     return KR_OK;
 }
 

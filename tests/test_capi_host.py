@@ -309,7 +309,7 @@ def test_gemm_plan_reports_the_dispatch(lib, monkeypatch):
     assert _lib.gemm_plan(8192, 14336, 4096, True)["tile_n"] == 256          # 1792 tiles = 7 whole rounds already
     assert _lib.gemm_plan(8192, 4096, 8192, True)["tile_n"] == 256           # 224 does not divide N
     p = _lib.gemm_plan(256, 256, 100 * 8, False)                             # K not a multiple of 64
-    assert p["kernel"] == "gemm_reduce_kernel" and p["tile"] == 128 and p["k_splits"] == 1
+    assert p["kernel"] == "gemm_ks_kernel" and p["tile"] == 128 and p["k_splits"] == 1
     need = lib.kr_gemm_workspace_bytes(128, 6656, 4096)
     p = _lib.gemm_plan(128, 6656, 4096, False, workspace_bytes=need)         # few tiles: split K loop
     assert p["tile"] == 128 and p["k_splits"] > 1
@@ -342,6 +342,21 @@ def test_gemm_plan_peers_of_a_ragged_k_stay_in_the_epilogue(lib, monkeypatch, mo
             p = _lib.gemm_plan(4096, 4096, K, b_t, 7, 4096)
             assert p["tile"] == 256 and not p["peers_on_mfma"]
         assert _lib.gemm_plan(4096, 4096, 4096, b_t, 7, 4096)["peers_on_mfma"] == (mode != "epilogue")
+
+
+@pytest.mark.parametrize("M,N,K,b_t,kernel,mfma", [
+    (512, 4096, 1024, False, "gemm_ks_kernel", "16x16x32"),
+    (128, 6656, 4096, True, "gemm_ks_kernel", "16x16x32"),
+    (256, 256, 800, False, "gemm_ks_kernel", "16x16x32"),
+    (1000, 6656, 1024, True, "gemm_reduce_kernel", "32x32x16"),       # 416 tiles, K below 4096 (transposed B)
+    (2048, 4096, 512, False, "gemm_reduce_kernel", "32x32x16"),       # 512 tiles, K below 1024 (row-major B)
+    (256, 256, 56, False, "gemm_reduce_kernel", "32x32x16"),          # no whole k-step
+    (16, 8192, 3584, True, "gemm_skinny_kernel", "16x16x32"),
+    (4096, 4096, 4096, True, "gemm_dtl16_kernel", "16x16x32"),
+])
+def test_gemm_plan_names_every_kernel(lib, M, N, K, b_t, kernel, mfma):
+    p = _lib.gemm_plan(M, N, K, b_t, 7, M)
+    assert (p["kernel"], p["mfma"]) == (kernel, mfma)
 
 
 def test_split_fp32_argument_errors(lib):
