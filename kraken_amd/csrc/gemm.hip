@@ -876,10 +876,11 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
                                     g.progress != nullptr || g.band_counter != nullptr,
                                     gemm_dtl_supported(g) && (g.a_local == nullptr || (int64_t)256 * g.lda_local * 2 < 0x7fffffffLL), skinny_ok);
     const bool dtl = plan.tile == 256;
-    // The 128x128 kernel addresses a tile's operand panels with 32-bit byte offsets from the
+    // The 128x128 kernels address a tile's operand panels with 32-bit byte offsets from the
     // panel's first row (through a 2 GiB buffer descriptor): row strides beyond that reach are
-    // refused rather than read as zeros.
-    if (!dtl && plan.skinny == 0) {
+    // refused rather than read as zeros.  (gemm_skinny_kernel, which has fewer rows, would reach
+    // further; the rule does not depend on the number of rows.)
+    if (!dtl) {
         const int64_t reach = std::max<int64_t>(std::max(lda_m, ldb), g.a_local != nullptr ? g.lda_local : 0);
         if ((128 * reach + std::max(K, N)) * (f32 ? 4 : 2) >= 0x7fffffffLL) return KR_ERR_LAYOUT;
     }

@@ -217,6 +217,17 @@ def test_gemm_row_stride_beyond_the_kernels_reach(lib):
              None) == _lib.KR_ERR_LAYOUT
 
 
+@pytest.mark.parametrize("M", [1, 16, 64, 65, 128])
+def test_gemm_row_stride_rule_does_not_depend_on_the_rows(lib, M):
+    """128 rows of an operand must lie within 2 GiB, as the header says, also for a product of a few rows."""
+    f, N, K, wide = lib.kr_gemm_reduce_bf16, 256, 64, (1 << 23) + 8
+    for lda, lk, ln in ((wide, N, 1), (K, wide, 1), (K, 1, wide)):
+        assert f(FAKE, lda, 1, FAKE, lk, ln, M, N, K, None, 0, 0, None, 0, M, None, FAKE, 0, 0, None) == _lib.KR_ERR_LAYOUT
+    f32 = lib.kr_gemm_reduce_f32_ws
+    for lda, lk, ln in ((wide // 2, N, 1), (K, wide // 2, 1), (K, 1, wide // 2)):
+        assert f32(FAKE, lda, 1, FAKE, lk, ln, M, N, K, None, 0, None, 0, M, None, FAKE, 1, 0, None, 0, None) == _lib.KR_ERR_LAYOUT
+
+
 def test_gemm_producer_argument_errors(lib):
     f = lib.kr_gemm_producer_bf16
     def args(**kw):
