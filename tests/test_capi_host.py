@@ -370,6 +370,22 @@ def test_gemm_plan_names_every_kernel(lib, M, N, K, b_t, kernel, mfma):
     assert (p["kernel"], p["mfma"]) == (kernel, mfma)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (2, 1216, 16384), (16, 1024, 16384), (16, 1024, 8192), (32, 512, 8192), (64, 1032, 16384), (64, 8192, 3584)])
+def test_few_rows_workspace_covers_either_layout(lib, M, N, K):
+    """kr_gemm_workspace_bytes does not know the layout of B: it is enough for the parts the rule takes with either one,
+    so that the plan does not change when the workspace is larger, and no larger than the larger of the two."""
+    need = lib.kr_gemm_workspace_bytes(M, N, K)
+    largest = 0
+    for b_t in (False, True):
+        plan = _lib.gemm_plan(M, N, K, b_t, workspace_bytes=need)
+        assert plan["kernel"] == "gemm_skinny_kernel"
+        assert plan == _lib.gemm_plan(M, N, K, b_t, workspace_bytes=1 << 40)
+        if plan["k_splits"] > 1:
+            largest = max(largest, plan["k_splits"] * M * N * 4)
+    assert need == largest
+    assert (need > 0) == (K >= 8192)
+
+
 def test_split_fp32_argument_errors(lib):
     f = lib.kr_split_fp32
     assert f(FAKE, 16, 12, 12, 1, 0, FAKE, 36, None) == _lib.KR_ERR_NUMEL_MOD8

@@ -14,13 +14,16 @@ BF16 = torch.bfloat16
 TOL = dict(rtol=2e-2, atol=2e-2)
 
 
-@pytest.fixture(params=["128", "256", "256-epilogue"])
+@pytest.fixture(params=["128", "128-staged", "256", "256-epilogue"])
 def tile(request, monkeypatch):
-    """Force each GEMM kernel in turn: the register-staged kernel with 128x128 tiles; the
-    LDS-DMA kernel with 256x256 tiles (shapes it cannot take fall back to the other), with the
+    """Force each GEMM kernel in turn: with 128x128 tiles the deep-ring kernel (a K below 64 falls
+    back to the register-staged one) and the register-staged one; the
+    LDS-DMA kernel with 256x256 tiles (shapes it cannot take fall back to the others), with the
     peers' partial sums of whole-band tiles added on the matrix cores (default) or in the
     epilogue."""
     monkeypatch.setenv("KRAKEN_AMD_GEMM_TILE", request.param[:3])
+    if request.param[:3] == "128":
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_KS", "0" if request.param == "128-staged" else "1")
     monkeypatch.setenv("KRAKEN_AMD_GEMM_PEERS", "epilogue" if request.param.endswith("epilogue") else "mfma")
     return request.param
 
@@ -955,11 +958,13 @@ def test_producer_takes_fp32_operands(dev, M, N, K, b_t):
 
 @pytest.mark.parametrize("splits", [2, 3, 5, 16])
 @pytest.mark.parametrize("b_t", [False, True])
-def test_split_k_loop(dev, monkeypatch, splits, b_t):
+@pytest.mark.parametrize("ks", ["0", "1"])
+def test_split_k_loop(dev, monkeypatch, splits, b_t, ks):
     """Few output tiles: several workgroups share a tile's K loop, their partial products meet
     in the workspace.  Parity with the oracle for every epilogue form and the same bits run to
-    run (the parts are summed in a fixed order)."""
+    run (the parts are summed in a fixed order).  Both kernels with 128 x 128 tiles."""
     monkeypatch.setenv("KRAKEN_AMD_GEMM_TILE", "128")
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_KS", ks)
     monkeypatch.setenv("KRAKEN_AMD_GEMM_SPLITK", str(splits))
     for (M, N, K) in [(128, 384, 1024), (200, 136, 520), (256, 256, 64 * splits)]:
         a, b, peers = mk(M, N, K, 3, b_t, seed=splits)
@@ -986,6 +991,21 @@ def test_split_k_loop(dev, monkeypatch, splits, b_t):
     rows = torch.ones(M, dtype=torch.bool)
     rows[2 * M // W:3 * M // W] = False
     torch.testing.assert_close(c_scratch.cpu()[rows], c_want[rows], **TOL)
+
+
+@pytest.mark.parametrize("M,N,K,b_t", [(1000, 6656, 1024, True), (2048, 4096, 512, False), (1990, 4104, 200, True)])
+def test_register_staged_kernel_where_the_rule_takes_it(dev, M, N, K, b_t):
+    """More than 256 tiles of 128 x 128 and a short K loop, nothing forced: whole and ragged tiles, a last k-step that
+    is not full, seven peers and a bias.  Small integers: every fp32 sum is exact."""
+    assert _lib.gemm_plan(M, N, K, b_t, 7, M, True)["kernel"] == "gemm_reduce_kernel"
+    g = torch.Generator().manual_seed(K)
+    a = torch.randint(-4, 5, (M, K), generator=g).float().to(dev)
+    b = torch.randint(-4, 5, (K, N), generator=g).float().to(dev)
+    peers = torch.randint(-8, 9, (7, M, N), generator=g).to(BF16).to(dev)
+    bias = torch.randint(-8, 9, (N,), generator=g).to(BF16).to(dev)
+    b16 = b.T.contiguous().to(BF16).T if b_t else b.to(BF16)
+    out = fused.gemm_one_shot_all_reduce_fused(a.to(BF16), b16, peers=peers, bias=bias)
+    assert torch.equal(out, a @ b + peers.float().sum(0) + bias.float())
 
 
 @pytest.mark.parametrize("b_t", [False, True])
@@ -1224,6 +1244,72 @@ def test_all_gather_matmul_fp8_ragged_sums_keep_their_bits(dev, m, K, N, gather)
     assert torch.equal(c.cpu().float(), want.float()), int((c.cpu().float() != want.float()).sum())
 
 
+@pytest.mark.parametrize("m,K,N,kwargs", [(256, 1024, 768, {"fp8_kernel": False}), (32, 64, 272, {}), (256, 112, 512, {})])
+def test_all_gather_matmul_fp8_widened_behind_the_gather(dev, m, K, N, kwargs):
+    """gather=True where the product is widened to bf16: whole tiles with fp8_kernel=False, and a K below one k-step.
+    Small integers and halves: every fp32 sum is exact, the fp8 result is the rounded product."""
+    fp8 = torch.float8_e4m3fn
+    W = 8
+    g = torch.Generator().manual_seed(m + K)
+    a = torch.randint(-2, 3, (W, m, K), generator=g).float().to(fp8)
+    bT = (torch.randint(-3, 4, (N, K), generator=g).float() * 0.5).to(fp8)
+    want = (a.reshape(W * m, K).float() @ bT.float().T).clamp(-448.0, 448.0).to(fp8)
+    progress = torch.zeros(W, dtype=torch.int32, device=dev)
+    a_out, c = fused.all_gather_matmul(a.to(dev), bT.to(dev).T, None, progress, rank=3, gather=True, **kwargs)
+    assert torch.equal(a_out.cpu().view(torch.uint8), a.reshape(W * m, K).view(torch.uint8))
+    assert progress.tolist() == [1] * W
+    assert torch.equal(c.cpu().float(), want.float())
+
+
+@pytest.mark.parametrize("m,K,N", [(125, 144, 528), (64, 2064, 272), (256, 1136, 272)])
+def test_all_gather_matmul_fp8_ragged_entry(dev, m, K, N):
+    """kr_all_gather_matmul_fp8_ragged with chunks that have arrived (every flag is set before the launch) and the local
+    shard in a buffer of its own: the bits of the exact product of small integers and halves."""
+    fp8 = torch.float8_e4m3fn
+    W, rank = 4, 1
+    g = torch.Generator().manual_seed(K)
+    a = torch.randint(-2, 3, (W * m, K), generator=g).float().to(fp8)
+    bT = (torch.randint(-3, 4, (N, K), generator=g).float() * 0.5).to(fp8)
+    want = a.float() @ bT.float().T
+    ad, bd = a.to(dev), bT.to(dev)
+    local = ad[rank * m:(rank + 1) * m].clone()
+    if m % 256 == 0:
+        ad[rank * m:(rank + 1) * m].zero_()    # (tiles that lie in the local shard read their rows from it)
+    flags = torch.ones(W, dtype=torch.int32, device=dev)
+    status = torch.zeros(1, dtype=torch.int32, device=dev)
+    out = torch.empty(W * m, N, dtype=torch.float32, device=dev)
+    rc = _lib.load().kr_all_gather_matmul_fp8_ragged(
+        ad.data_ptr(), K, local.data_ptr(), K, bd.data_ptr(), K, W * m, N, K, W, rank, 1, flags.data_ptr(), 0,
+        status.data_ptr(), out.data_ptr(), 1, torch.cuda.current_stream(dev).cuda_stream)
+    assert rc == 0, _lib.strerror(rc)
+    assert torch.equal(out.cpu(), want) and status.item() == 0
+
+
+@pytest.mark.parametrize("K", [128, 2048, 16384])
+def test_fp8_kernel_precision_of_the_sums(dev, K):
+    """The fp8 instruction keeps about 16 bits of a sum: against 64 bits the fp32 result is off by 1.1e-5 to 1.5e-5 in
+    the 2-norm (measured, K = 128 .. 16384, N(0, 1) x N(0, 0.25)); the bound is twice that, 2^-15.  In one pass and
+    with the K loop split."""
+    fp8 = torch.float8_e4m3fn
+    M, N = 512, 768
+    g = torch.Generator().manual_seed(K)
+    a = torch.randn(M, K, generator=g).to(fp8)
+    bT = (torch.randn(N, K, generator=g) * 0.25).to(fp8)
+    exact = a.double() @ bT.double().T
+    ad, bd = a.to(dev), bT.to(dev)
+    lib = _lib.load()
+    need = lib.kr_gemm_fp8_workspace_bytes(M, N, K)
+    assert (need > 0) == (K > 128)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    for nbytes in {0, need}:
+        out = torch.empty(M, N, dtype=torch.float32, device=dev)
+        rc = lib.kr_gemm_fp8_ws(ad.data_ptr(), K, bd.data_ptr(), K, M, N, K, out.data_ptr(), 1, ws.data_ptr() if nbytes else None,
+                                nbytes, torch.cuda.current_stream(dev).cuda_stream)
+        assert rc == 0, _lib.strerror(rc)
+        err = ((out.cpu().double() - exact).norm() / exact.norm()).item()
+        assert err <= 2.0 ** -15, (nbytes, err)
+
+
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("M,N,K", [(256, 256, 72), (512, 264, 120), (264, 512, 328), (511, 520, 1016)])
 def test_large_tile_kernel_last_k_step_not_full(dev, monkeypatch, M, N, K, b_t):
@@ -1308,6 +1394,22 @@ def test_fp32_operands_split_in_registers(dev, monkeypatch, M, N, K, b_t):
         assert ((out - ar.double() @ br.double()).abs() <= 2.0 ** -15 * (ar.abs().double() @ br.abs().double())).all(), splits
 
 
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K", [(2304, 4096, 256), (2200, 4104, 72), (256, 4096, 260)])
+def test_fp32_operands_split_in_a_pass(dev, M, N, K, b_t):
+    """More than 512 tiles of 128 x 128, and a K that is no multiple of 8: the operands are split by a pass of their own
+    and multiplied as a bf16 product of 3K.  Integers up to 2^11 (hi and lo parts exact) times integers up to 8, every
+    sum below 2^24: exact."""
+    from kraken_amd.fused import _gemm
+    g = torch.Generator().manual_seed(K)
+    a = torch.randint(-2047, 2048, (M, K), generator=g).float().to(dev)
+    b = torch.randint(-8, 9, (K, N), generator=g).float().to(dev)
+    assert K * 2047 * 8 < 1 << 24
+    bd = b.T.contiguous().T if b_t else b
+    assert not _gemm.fp32_direct(a, bd)
+    assert torch.equal(fused.gemm_one_shot_all_reduce_fused(a, bd), a @ b)
+
+
 @pytest.mark.parametrize("wide", ["a", "b", "b_t"])
 def test_fp32_operands_with_very_wide_rows(dev, wide):
     """fp32 operands that are slices of matrices with rows of 4.2 million elements: 128 such rows reach past the 2 GiB that
@@ -1353,7 +1455,6 @@ def test_few_rows_kernel(dev, monkeypatch, M, N, K, b_t, fp32):
     product = a[:, :K] @ bk
     peers = torch.randint(-8, 9, (9, M, N), generator=g).to(BF16)
     bias = torch.randint(-8, 9, (N,), generator=g).to(BF16)
-    lib = _lib.load()
     for cb in (1, 2) if fp32 else (1, 2, 4):
         for splits in (1, 5):
             monkeypatch.setenv("KRAKEN_AMD_GEMM_SKINNY", str(100 * cb + splits))
@@ -1371,7 +1472,8 @@ def test_few_rows_kernel(dev, monkeypatch, M, N, K, b_t, fp32):
     assert fp32 or plan["kernel"] == "gemm_skinny_kernel"
     monkeypatch.delenv("KRAKEN_AMD_GEMM_SKINNY")
     _lib.reload_env()
-    assert lib.kr_gemm_workspace_bytes(M, N, K) >= 0
+    out = fused.gemm_one_shot_all_reduce_fused(ad, bd, peers=peers.to(dev), bias=bias.to(dev))
+    assert torch.equal(out.cpu(), product + peers.float().sum(0) + bias.float())
 
 
 @pytest.mark.parametrize("W,splits,rank,nbytes", [(1, 1, 0, 16), (2, 1, 1, 16384), (3, 2, 0, 16400), (8, 3, 5, 49136), (16, 1, 15, 1 << 20)])
