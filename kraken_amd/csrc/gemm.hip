@@ -497,8 +497,18 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     parts of whole 256 KiB tiles (512 x 6656 x 16384: 122 us against 150 with gemm_ks_kernel; 512 x 4096 x 8192:
 //     51 against 43);
 //   gemm_reduce_kernel, two workgroups per compute unit: where more than 256 tiles have short K loops, one
-//     tile's epilogue beside another's k loop is worth more (1000 x 6656 x 1024, transposed B: 21 against 25 us;
-//     row-major B 28 against 27, x 4096 83 against 68).
+//     tile's epilogue beside another's k loop is worth more.  With transposed B gemm_ks_kernel gains little and
+//     loses much where its five stages in flight ask the same memory channels for rows that lie a multiple of 4 KiB
+//     (and no power of two) apart.  gemm_ks_kernel / gemm_reduce_kernel, us, operands in no cache unless stated:
+//       above 256 tiles, transposed: 1000 x 6656 x 1024 27 / 23, x 4096 75 / 73, x 8192 136 / 132, x 12288 273 / 200;
+//         1100 x 4096 x 6144 124 / 94 (in the last-level cache 87 / 79), x 16384 248 / 228; 2048 x 4096 x 4096
+//         79 / 74, x 8192 122 / 122: never better by more than the noise, so it is not taken there;
+//       above 256 tiles, row-major: 1000 x 6656 x 512 20 / 18, x 1024 28.6 / 28.2 (cached 26.5 / 26.8), x 2048 45 / 47,
+//         x 4096 79 / 86, x 8192 144 / 165; 1536 x 4096 x 1024 25 / 24, x 2048 43 / 41, with seven peers 57 / 59;
+//       up to 256 tiles, transposed: 1024 x 4096 x 1024 14.0 / 14.7, x 5120 54 / 57, x 6144 70 / 65 (cached 52 / 60),
+//         x 8192 74 / 78 (cached 63 / 74); 1000 x 3328 x 10240 109 / 99, x 12288 144 / 119, x 14336 142 / 136, x 24576
+//         282 / 224: up to K = 8192;
+//       up to 256 tiles, row-major: 1024 x 4096 x 6144 64 / 93, 500 x 4096 x 12288 82 / 111: always.
 struct SmallPlan {
     int big;      // 256x256 kernel, every tile split
     int ks;       // gemm_ks_kernel, else gemm_reduce_kernel
@@ -507,7 +517,7 @@ struct SmallPlan {
 static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool dtl_ok, bool may_split, bool may_big) {
     SmallPlan p{0, 0, 1};
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
-    p.ks = dtl_ok && (tiles <= 256 || K >= (b_nt ? 4096 : 1024));
+    p.ks = dtl_ok && (b_nt ? tiles <= 256 && K <= 8192 : tiles <= 256 || K >= 1024);
     if (env_switches().gemm_ks >= 0) p.ks = dtl_ok && env_switches().gemm_ks != 0;
     if (!may_split) return p;
     if (const int v = env_switches().gemm_splitk; v >= 1 && v <= kMaxSplits) {   // testing and tuning

@@ -359,7 +359,12 @@ def test_gemm_plan_peers_of_a_ragged_k_stay_in_the_epilogue(lib, monkeypatch, mo
     (512, 4096, 1024, False, "gemm_ks_kernel", "16x16x32"),
     (128, 6656, 4096, True, "gemm_ks_kernel", "16x16x32"),
     (256, 256, 800, False, "gemm_ks_kernel", "16x16x32"),
-    (1000, 6656, 1024, True, "gemm_reduce_kernel", "32x32x16"),       # 416 tiles, K below 4096 (transposed B)
+    (1000, 6656, 1024, True, "gemm_reduce_kernel", "32x32x16"),       # 416 tiles (transposed B)
+    (1000, 6656, 12288, True, "gemm_reduce_kernel", "32x32x16"),
+    (1000, 6656, 4096, False, "gemm_ks_kernel", "16x16x32"),
+    (1000, 4096, 8192, True, "gemm_ks_kernel", "16x16x32"),
+    (1000, 4096, 12288, True, "gemm_reduce_kernel", "32x32x16"),      # 256 tiles, K above 8192 (transposed B)
+    (1000, 4096, 12288, False, "gemm_ks_kernel", "16x16x32"),
     (2048, 4096, 512, False, "gemm_reduce_kernel", "32x32x16"),       # 512 tiles, K below 1024 (row-major B)
     (256, 256, 56, False, "gemm_reduce_kernel", "32x32x16"),          # no whole k-step
     (16, 8192, 3584, True, "gemm_skinny_kernel", "16x16x32"),

@@ -993,11 +993,13 @@ def test_split_k_loop(dev, monkeypatch, splits, b_t, ks):
     torch.testing.assert_close(c_scratch.cpu()[rows], c_want[rows], **TOL)
 
 
-@pytest.mark.parametrize("M,N,K,b_t", [(1000, 6656, 1024, True), (2048, 4096, 512, False), (1990, 4104, 200, True)])
-def test_register_staged_kernel_where_the_rule_takes_it(dev, M, N, K, b_t):
-    """More than 256 tiles of 128 x 128 and a short K loop, nothing forced: whole and ragged tiles, a last k-step that
-    is not full, seven peers and a bias.  Small integers: every fp32 sum is exact."""
-    assert _lib.gemm_plan(M, N, K, b_t, 7, M, True)["kernel"] == "gemm_reduce_kernel"
+@pytest.mark.parametrize("M,N,K,b_t,splits", [(1000, 6656, 1024, True, 1), (2048, 4096, 512, False, 1), (1990, 4104, 200, True, 1),
+                                              (1100, 4096, 4168, True, 1), (300, 520, 8200, True, 15)])
+def test_register_staged_kernel_where_the_rule_takes_it(dev, M, N, K, b_t, splits):
+    """More than 256 tiles of 128 x 128, and few tiles with a long K loop in parts (transposed B), nothing forced: whole
+    and ragged tiles, a last k-step that is not full, seven peers and a bias.  Small integers: every fp32 sum is exact."""
+    plan = _lib.gemm_plan(M, N, K, b_t, 7, M, True, workspace_bytes=_lib.load().kr_gemm_workspace_bytes(M, N, K))
+    assert plan["kernel"] == "gemm_reduce_kernel" and plan["k_splits"] == splits
     g = torch.Generator().manual_seed(K)
     a = torch.randint(-4, 5, (M, K), generator=g).float().to(dev)
     b = torch.randint(-4, 5, (K, N), generator=g).float().to(dev)
