@@ -493,6 +493,9 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //   gemm_ks_kernel, S workgroups per 128x128 tile: 6.5 us to start and finish, 0.56 us (row-major B 0.60) per
 //     k-step of 64 and round of 256 workgroups -- a compute unit takes in about 57 GB/s of operands that other
 //     units are waiting for too, whatever its pipeline; S > 1 adds a launch and S fp32 parts written and read;
+//     S = 1 with peers and more than 16 k-steps 4 us more (fitted, the cause is not separated; one or three peers, in
+//     one pass / in three parts: 112 x 9216 x 1664 27.0 / 21.7, 256 x 4096 x 1536 25.0 / 20.8, 720 x 1280 x 1464 24.6 / 21.1,
+//     row-major 22.4 / 20.1; 360 x 768 x 1096 21.4 / 20.5; but 300 x 2048 x 1024 16.8 / 19.6, 128 x 4096 x 1024 16.5 / 19.1);
 //   the 256x256 kernel with every tile's K loop split: 1.2 us per k-step, twice the work per operand byte, but
 //     parts of whole 256 KiB tiles (512 x 6656 x 16384: 122 us against 150 with gemm_ks_kernel; 512 x 4096 x 8192:
 //     51 against 43);
@@ -514,7 +517,7 @@ struct SmallPlan {
     int ks;       // gemm_ks_kernel, else gemm_reduce_kernel
     int splits;   // workgroups per tile of the 128x128 kernels
 };
-static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool dtl_ok, bool may_split, bool may_big) {
+static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool peers, bool dtl_ok, bool may_split, bool may_big) {
     SmallPlan p{0, 0, 1};
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
     p.ks = dtl_ok && (b_nt ? tiles <= 256 && K <= 8192 : tiles <= 256 || K >= 1024);
@@ -526,7 +529,7 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool dtl
     }
     const int64_t step = b_nt ? 56 : 60;
     auto cost = [&](int64_t s) {
-        return 650 + (tiles * s + 255) / 256 * step * ((steps + s - 1) / s) + (s > 1 ? 600 + s * M * N * 16 / 100000 : 0);
+        return 650 + (tiles * s + 255) / 256 * step * ((steps + s - 1) / s) + (s > 1 ? 600 + s * M * N * 16 / 100000 : peers && steps > 16 ? 400 : 0);
     };
     int64_t best = cost(1);
     for (int64_t s = 2; s <= kMaxSplits && 2 * s <= steps && s * tiles <= 512; ++s)
@@ -653,11 +656,11 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     // (few tiles: the large tile again with every tile's K loop split, where that is cheaper)
     SmallPlan small{0, 0, 1};
     if (!big || !dtl_ok || env_switches().gemm_tile == 128) {
-        small = plan_small(M, N, K, b_nt, dtl_ok, has_workspace, has_workspace && !has_gather && env_switches().gemm_tile != 128);
+        small = plan_small(M, N, K, b_nt, n_peers > 0, dtl_ok, has_workspace, has_workspace && !has_gather && env_switches().gemm_tile != 128);
         if (small.big) {
             int tail, ts;
             tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
-            if (gemm_dtl_tail_workspace_bytes(tail, ts) > workspace_bytes) small = plan_small(M, N, K, b_nt, dtl_ok, has_workspace, false);
+            if (gemm_dtl_tail_workspace_bytes(tail, ts) > workspace_bytes) small = plan_small(M, N, K, b_nt, n_peers > 0, dtl_ok, has_workspace, false);
         }
         big = small.big != 0;
     }
@@ -1170,14 +1173,15 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
         tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
         return tail > 0 ? gemm_dtl_tail_workspace_bytes(tail, ts) : 0;
     }
-    // the layout of B is not known here: enough for either
+    // the layout of B and the number of peers are not known here: enough for any
     int64_t bytes = 0;
-    for (const bool b_nt : {false, true}) {
+    for (int form = 0; form < 4; ++form) {
+        const bool b_nt = form & 1, peers = form & 2;
         if (const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, false, kMaxPartsBytes); sk.cb != 0) {
             if (sk.splits > 1) bytes = std::max(bytes, split_k_workspace_bytes(M, N, sk.splits));
             continue;
         }
-        const SmallPlan p = plan_small(M, N, K, b_nt, K % 8 == 0 && K >= 64, true, force_tile != 128);
+        const SmallPlan p = plan_small(M, N, K, b_nt, peers, K % 8 == 0 && K >= 64, true, force_tile != 128);
         if (p.big) {
             int tail, ts;
             tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);

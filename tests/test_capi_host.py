@@ -391,6 +391,19 @@ def test_few_rows_workspace_covers_either_layout(lib, M, N, K):
     assert (need > 0) == (K >= 8192)
 
 
+@pytest.mark.parametrize("M,N,K,split", [(331, 2440, 1352, True), (382, 3536, 1848, True), (720, 1280, 1464, True), (300, 2048, 1024, False), (256, 8192, 1024, False)])
+def test_workspace_covers_the_plan_with_peers(lib, M, N, K, split):
+    """kr_gemm_workspace_bytes knows neither the layout of B nor the peers: it is enough for the parts of either plan.
+    With peers and more than 16 k-steps few tiles share their K loop where one pass is enough without peers."""
+    need = lib.kr_gemm_workspace_bytes(M, N, K)
+    for b_t in (False, True):
+        for P in (0, 1, 7):
+            plan = _lib.gemm_plan(M, N, K, b_t, P, M, workspace_bytes=need)
+            assert plan == _lib.gemm_plan(M, N, K, b_t, P, M, workspace_bytes=1 << 40)
+            assert plan["k_splits"] == 1 or plan["k_splits"] * M * N * 4 <= need
+            assert (plan["k_splits"] > 1) == (split and P > 0)
+
+
 def test_split_fp32_argument_errors(lib):
     f = lib.kr_split_fp32
     assert f(FAKE, 16, 12, 12, 1, 0, FAKE, 36, None) == _lib.KR_ERR_NUMEL_MOD8
