@@ -231,14 +231,16 @@ def gemm_reduce_scatter_ce_persistent(
         _gemm.launch("gemm_reduce_scatter_ce_persistent", *_gemm.prepare_operands(a, b), M, N, None, 0, 0, None, 0, 0,
                      gemm_out, None, ((rank + 1) % world_size) * m_per_rank)
         by_rank = gemm_out.view(world_size, m_per_rank, N)
-        if isinstance(sent, torch.Tensor) and sent.shape[0] == world_size:
+        if (written and isinstance(sent, torch.Tensor) and sent.shape[0] == world_size
+                and written[0].is_contiguous() and sent.stride(0) >= m_per_rank * N):
             for run in (slice(0, rank), slice(rank + 1, world_size)):
                 if run.start < run.stop:
                     sent[run].copy_(by_rank[run])
         else:
-            for r, t in enumerate(dests):
-                if t is not None:
-                    t.copy_(by_rank[r])
+            # (destinations may share memory, one scratch band for all: the order is that of copy_engine_scatter)
+            for r in (*range(rank + 1, world_size), *range(rank)):
+                if dests[r] is not None:
+                    dests[r].copy_(by_rank[r])
         return _reduce_bands(bands, m_per_rank, N, output, configs)
     progress = torch.zeros(world_size, dtype=torch.int32, device=dev)
     signal_pad = torch.zeros(world_size, dtype=torch.int32, device=dev)

@@ -937,6 +937,23 @@ def test_ce_reduce_reads_the_bands_in_place(dev, M, N, K, form):
     assert torch.equal(out, fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers.to(dev), rank=rank, sent=list(plain)))
 
 
+@pytest.mark.parametrize("M,N,K", [(512, 1024, 256), (2048, 8192, 256)])   # bands together; one by one
+@pytest.mark.parametrize("form", ["expanded", "list"])
+def test_ce_bands_sent_into_one_scratch_band(dev, M, N, K, form):
+    """Destinations that are one and the same memory, as a tensor expanded over the ranks or the same tensor W times:
+    the bands are copied there in the order rank + 1, rank + 2, ..., so that of rank - 1 remains."""
+    W, rank, m = 4, 2, M // 4
+    a, b, peers = mk(M, N, K, W - 1, True, seed=9)
+    a, b, peers = a.to(dev), b.to(dev), peers[:, :m].contiguous().to(dev)
+    apart = torch.zeros(W, m, N, dtype=BF16, device=dev)
+    want = fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers, rank=rank, sent=apart)
+    scratch = torch.zeros(m, N, dtype=BF16, device=dev)
+    sent = scratch.expand(W, m, N) if form == "expanded" else [scratch] * W
+    out = fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers, rank=rank, sent=sent)
+    assert torch.equal(scratch, apart[rank - 1])
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (512, 1024, 4096), (2304, 8192, 256)])   # one pass, split K loop, more than a round
 def test_producer_takes_fp32_operands(dev, M, N, K, b_t):
