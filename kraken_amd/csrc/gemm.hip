@@ -490,28 +490,28 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 // ---- at most 128 tiles of 256x256: which kernel, and how many workgroups share a tile -----------------
 // Three candidates, by what they cost in 0.01 us (measured with operands that are in no cache, M = 128 .. 2000,
 // N = 1024 .. 6656, K = 512 .. 16384; the model is within 15 % of the measurements where it matters):
-//   gemm_ks_kernel, S workgroups per 128x128 tile: 6.5 us to start and finish, 0.56 us (row-major B 0.60) per
+//   a 128x128 kernel, S workgroups per tile: 6.5 us to start and finish, 0.56 us (row-major B 0.60) per
 //     k-step of 64 and round of 256 workgroups -- a compute unit takes in about 57 GB/s of operands that other
-//     units are waiting for too, whatever its pipeline; S > 1 adds a launch and S fp32 parts written and read;
+//     units are waiting for too, whatever its pipeline; S > 1 adds a launch and S fp32 parts written and read (6 us and
+//     16 ns per million elements with row-major B, which runs gemm_ks_kernel; 2 us and 20 ns and parts of at least eight
+//     k-steps with transposed B, gemm_reduce_kernel: fitted to every split of 13 257 random shapes, 65 to 4096 rows, where
+//     this choice takes 1.009 (no peers) and 1.033 (peers) of the time of the best one);
 //     S = 1 with peers and more than 16 k-steps 4 us more (fitted, the cause is not separated; one or three peers, in
 //     one pass / in three parts: 112 x 9216 x 1664 27.0 / 21.7, 256 x 4096 x 1536 25.0 / 20.8, 720 x 1280 x 1464 24.6 / 21.1,
 //     row-major 22.4 / 20.1; 360 x 768 x 1096 21.4 / 20.5; but 300 x 2048 x 1024 16.8 / 19.6, 128 x 4096 x 1024 16.5 / 19.1);
 //   the 256x256 kernel with every tile's K loop split: 1.2 us per k-step, twice the work per operand byte, but
 //     parts of whole 256 KiB tiles (512 x 6656 x 16384: 122 us against 150 with gemm_ks_kernel; 512 x 4096 x 8192:
 //     51 against 43);
-//   gemm_reduce_kernel, two workgroups per compute unit: where more than 256 tiles have short K loops, one
-//     tile's epilogue beside another's k loop is worth more.  With transposed B gemm_ks_kernel gains little and
+// Which 128x128 kernel, by the time of gemm_ks_kernel over that of gemm_reduce_kernel (geometric means over 20 000 random
+// shapes, 1 to 8192 rows, operands in no cache):
+//   transposed B, in parts: 1.034 to 1.042 at every K: gemm_reduce_kernel.  In one pass, K a multiple of 64, no peers:
+//     1.05 below K = 362, 0.96 from 724 to 1448, 0.98 to 1.00 up to 8192; with peers 1.03 to 0.98, level on the whole; K no
+//     multiple of 64: 1.054.  Above 256 tiles 1000 x 6656 x 1024 27 / 23 us, x 4096 75 / 73, x 8192 136 / 132; above K = 8192 it
 //     loses much where its five stages in flight ask the same memory channels for rows that lie a multiple of 4 KiB
-//     (and no power of two) apart.  gemm_ks_kernel / gemm_reduce_kernel, us, operands in no cache unless stated:
-//       above 256 tiles, transposed: 1000 x 6656 x 1024 27 / 23, x 4096 75 / 73, x 8192 136 / 132, x 12288 273 / 200;
-//         1100 x 4096 x 6144 124 / 94 (in the last-level cache 87 / 79), x 16384 248 / 228; 2048 x 4096 x 4096
-//         79 / 74, x 8192 122 / 122: never better by more than the noise, so it is not taken there;
-//       above 256 tiles, row-major: 1000 x 6656 x 512 20 / 18, x 1024 28.6 / 28.2 (cached 26.5 / 26.8), x 2048 45 / 47,
-//         x 4096 79 / 86, x 8192 144 / 165; 1536 x 4096 x 1024 25 / 24, x 2048 43 / 41, with seven peers 57 / 59;
-//       up to 256 tiles, transposed: 1024 x 4096 x 1024 14.0 / 14.7, x 5120 54 / 57, x 6144 70 / 65 (cached 52 / 60),
-//         x 8192 74 / 78 (cached 63 / 74); 1000 x 3328 x 10240 109 / 99, x 12288 144 / 119, x 14336 142 / 136, x 24576
-//         282 / 224: up to K = 8192;
-//       up to 256 tiles, row-major: 1024 x 4096 x 6144 64 / 93, 500 x 4096 x 12288 82 / 111: always.
+//     (and no power of two) apart: 1000 x 3328 x 12288 144 / 119, x 24576 282 / 224, 1000 x 6656 x 12288 273 / 200.
+//   row-major B, up to 256 tiles: 0.88 at K = 256, 0.72 at 1024, 0.66 from 4096 on, in parts 0.88: gemm_ks_kernel.
+//     Above 256 tiles, where gemm_reduce_kernel has two workgroups per compute unit and one tile's epilogue runs beside
+//     another's k loop: 1000 x 6656 x 512 20 / 18, x 1024 28.6 / 28.2, x 2048 45 / 47, x 4096 79 / 86, x 8192 144 / 165.
 struct SmallPlan {
     int big;      // 256x256 kernel, every tile split
     int ks;       // gemm_ks_kernel, else gemm_reduce_kernel
@@ -520,19 +520,22 @@ struct SmallPlan {
 static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool peers, bool dtl_ok, bool may_split, bool may_big) {
     SmallPlan p{0, 0, 1};
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
-    p.ks = dtl_ok && (b_nt ? tiles <= 256 && K <= 8192 : tiles <= 256 || K >= 1024);
-    if (env_switches().gemm_ks >= 0) p.ks = dtl_ok && env_switches().gemm_ks != 0;
-    if (!may_split) return p;
+    auto choose_kernel = [&]() {
+        p.ks = dtl_ok && (b_nt ? p.splits == 1 && !peers && tiles <= 256 && K % 64 == 0 && K >= 640 && K <= 8192 : tiles <= 256 || K >= 1024);
+        if (env_switches().gemm_ks >= 0) p.ks = dtl_ok && env_switches().gemm_ks != 0;
+        return p;
+    };
+    if (!may_split) return choose_kernel();
     if (const int v = env_switches().gemm_splitk; v >= 1 && v <= kMaxSplits) {   // testing and tuning
         p.splits = (int)std::min<int64_t>(v, steps);
-        return p;
+        return choose_kernel();
     }
-    const int64_t step = b_nt ? 56 : 60;
+    const int64_t step = b_nt ? 56 : 60, launch = b_nt ? 200 : 600, part = b_nt ? 20 : 16, min_steps = b_nt ? kMinSplitSteps : 2;
     auto cost = [&](int64_t s) {
-        return 650 + (tiles * s + 255) / 256 * step * ((steps + s - 1) / s) + (s > 1 ? 600 + s * M * N * 16 / 100000 : peers && steps > 16 ? 400 : 0);
+        return 650 + (tiles * s + 255) / 256 * step * ((steps + s - 1) / s) + (s > 1 ? launch + s * M * N * part / 100000 : peers && steps > 16 ? 400 : 0);
     };
     int64_t best = cost(1);
-    for (int64_t s = 2; s <= kMaxSplits && 2 * s <= steps && s * tiles <= 512; ++s)
+    for (int64_t s = 2; s <= kMaxSplits && min_steps * s <= steps && s * tiles <= 512; ++s)
         if (const int64_t c = cost(s); c < best) {
             best = c;
             p.splits = (int)s;
@@ -546,7 +549,7 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool pee
             p.splits = 1;
         }
     }
-    return p;
+    return choose_kernel();
 }
 
 // ---- at most 64 rows (gemm_skinny.hip): columns per workgroup and workgroups that share a K loop -------------

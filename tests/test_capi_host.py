@@ -357,12 +357,13 @@ def test_gemm_plan_peers_of_a_ragged_k_stay_in_the_epilogue(lib, monkeypatch, mo
 
 @pytest.mark.parametrize("M,N,K,b_t,kernel,mfma", [
     (512, 4096, 1024, False, "gemm_ks_kernel", "16x16x32"),
-    (128, 6656, 4096, True, "gemm_ks_kernel", "16x16x32"),
+    (128, 6656, 4096, False, "gemm_ks_kernel", "16x16x32"),
+    (128, 6656, 4096, True, "gemm_reduce_kernel", "32x32x16"),        # transposed B and peers
     (256, 256, 800, False, "gemm_ks_kernel", "16x16x32"),
     (1000, 6656, 1024, True, "gemm_reduce_kernel", "32x32x16"),       # 416 tiles (transposed B)
     (1000, 6656, 12288, True, "gemm_reduce_kernel", "32x32x16"),
     (1000, 6656, 4096, False, "gemm_ks_kernel", "16x16x32"),
-    (1000, 4096, 8192, True, "gemm_ks_kernel", "16x16x32"),
+    (1000, 4096, 8192, True, "gemm_reduce_kernel", "32x32x16"),
     (1000, 4096, 12288, True, "gemm_reduce_kernel", "32x32x16"),      # 256 tiles, K above 8192 (transposed B)
     (1000, 4096, 12288, False, "gemm_ks_kernel", "16x16x32"),
     (2048, 4096, 512, False, "gemm_reduce_kernel", "32x32x16"),       # 512 tiles, K below 1024 (row-major B)
@@ -373,6 +374,25 @@ def test_gemm_plan_peers_of_a_ragged_k_stay_in_the_epilogue(lib, monkeypatch, mo
 def test_gemm_plan_names_every_kernel(lib, M, N, K, b_t, kernel, mfma):
     p = _lib.gemm_plan(M, N, K, b_t, 7, M)
     assert (p["kernel"], p["mfma"]) == (kernel, mfma)
+
+
+@pytest.mark.parametrize("M,N,K,P,kernel", [
+    (1000, 4096, 8192, 0, "gemm_ks_kernel"),         # one pass, no peers, whole k-steps
+    (256, 512, 640, 0, "gemm_ks_kernel"),
+    (256, 512, 576, 0, "gemm_reduce_kernel"),        # K below 640
+    (256, 512, 648, 0, "gemm_reduce_kernel"),        # K no multiple of 64
+    (1000, 4096, 8256, 0, "gemm_reduce_kernel"),     # K above 8192
+    (1000, 4224, 4096, 0, "gemm_reduce_kernel"),     # 264 tiles
+    (256, 512, 4096, 0, "gemm_reduce_kernel"),       # K loop in parts
+    (256, 512, 640, 1, "gemm_reduce_kernel"),        # peers
+])
+def test_gemm_plan_of_transposed_b_with_few_tiles(lib, M, N, K, P, kernel):
+    """With transposed B gemm_ks_kernel only where it is not slower than gemm_reduce_kernel, and parts of at least
+    eight k-steps."""
+    p = _lib.gemm_plan(M, N, K, True, P, M, workspace_bytes=lib.kr_gemm_workspace_bytes(M, N, K))
+    assert (p["kernel"], p["tile"]) == (kernel, 128)
+    assert p["k_splits"] == 1 or K // 64 >= 8 * p["k_splits"]
+    assert (p["k_splits"] > 1) == ((M, N, K) == (256, 512, 4096))
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (2, 1216, 16384), (16, 1024, 16384), (16, 1024, 8192), (32, 512, 8192), (64, 1032, 16384), (64, 8192, 3584)])
@@ -394,14 +414,14 @@ def test_few_rows_workspace_covers_either_layout(lib, M, N, K):
 @pytest.mark.parametrize("M,N,K,split", [(331, 2440, 1352, True), (382, 3536, 1848, True), (720, 1280, 1464, True), (300, 2048, 1024, False), (256, 8192, 1024, False)])
 def test_workspace_covers_the_plan_with_peers(lib, M, N, K, split):
     """kr_gemm_workspace_bytes knows neither the layout of B nor the peers: it is enough for the parts of either plan.
-    With peers and more than 16 k-steps few tiles share their K loop where one pass is enough without peers."""
+    With row-major B, peers and more than 16 k-steps few tiles share their K loop where one pass is enough without peers."""
     need = lib.kr_gemm_workspace_bytes(M, N, K)
     for b_t in (False, True):
         for P in (0, 1, 7):
             plan = _lib.gemm_plan(M, N, K, b_t, P, M, workspace_bytes=need)
             assert plan == _lib.gemm_plan(M, N, K, b_t, P, M, workspace_bytes=1 << 40)
             assert plan["k_splits"] == 1 or plan["k_splits"] * M * N * 4 <= need
-            assert (plan["k_splits"] > 1) == (split and P > 0)
+            assert b_t or (plan["k_splits"] > 1) == (split and P > 0)
 
 
 def test_split_fp32_argument_errors(lib):
