@@ -510,8 +510,9 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     loses much where its five stages in flight ask the same memory channels for rows that lie a multiple of 4 KiB
 //     (and no power of two) apart: 1000 x 3328 x 12288 144 / 119, x 24576 282 / 224, 1000 x 6656 x 12288 273 / 200.
 //   row-major B, up to 256 tiles: 0.88 at K = 256, 0.72 at 1024, 0.66 from 4096 on, in parts 0.88: gemm_ks_kernel.
-//     Above 256 tiles, where gemm_reduce_kernel has two workgroups per compute unit and one tile's epilogue runs beside
-//     another's k loop: 1000 x 6656 x 512 20 / 18, x 1024 28.6 / 28.2, x 2048 45 / 47, x 4096 79 / 86, x 8192 144 / 165.
+//     Above 256 tiles gemm_reduce_kernel has two workgroups per compute unit and one tile's epilogue runs beside
+//     another's k loop.  K a multiple of 64, without / with peers: 1.02 / 1.07 from 1024 to 2048, 0.94 / 0.97 above; no
+//     multiple: 1.08 / 1.08, 1.01 / 1.06.  1000 x 6656 x 1024 28.6 / 28.2 us, x 2048 45 / 47, x 4096 79 / 86, x 8192 144 / 165.
 struct SmallPlan {
     int big;      // 256x256 kernel, every tile split
     int ks;       // gemm_ks_kernel, else gemm_reduce_kernel
@@ -521,7 +522,7 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool pee
     SmallPlan p{0, 0, 1};
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
     auto choose_kernel = [&]() {
-        p.ks = dtl_ok && (b_nt ? p.splits == 1 && !peers && tiles <= 256 && K % 64 == 0 && K >= 640 && K <= 8192 : tiles <= 256 || K >= 1024);
+        p.ks = dtl_ok && (b_nt ? p.splits == 1 && !peers && tiles <= 256 && K % 64 == 0 && K >= 640 && K <= 8192 : tiles <= 256 || (K % 64 == 0 && K >= 2048));
         if (env_switches().gemm_ks >= 0) p.ks = dtl_ok && env_switches().gemm_ks != 0;
         return p;
     };

@@ -366,7 +366,11 @@ def test_gemm_plan_peers_of_a_ragged_k_stay_in_the_epilogue(lib, monkeypatch, mo
     (1000, 4096, 8192, True, "gemm_reduce_kernel", "32x32x16"),
     (1000, 4096, 12288, True, "gemm_reduce_kernel", "32x32x16"),      # 256 tiles, K above 8192 (transposed B)
     (1000, 4096, 12288, False, "gemm_ks_kernel", "16x16x32"),
-    (2048, 4096, 512, False, "gemm_reduce_kernel", "32x32x16"),       # 512 tiles, K below 1024 (row-major B)
+    (2048, 4096, 512, False, "gemm_reduce_kernel", "32x32x16"),       # 512 tiles, K below 2048 (row-major B)
+    (4352, 1496, 1984, False, "gemm_reduce_kernel", "32x32x16"),
+    (4352, 1496, 2048, False, "gemm_ks_kernel", "16x16x32"),
+    (4352, 1496, 4104, False, "gemm_reduce_kernel", "32x32x16"),      # 408 tiles, K no multiple of 64
+    (1000, 4096, 1032, False, "gemm_ks_kernel", "16x16x32"),          # 256 tiles: any K
     (256, 256, 56, False, "gemm_reduce_kernel", "32x32x16"),          # no whole k-step
     (16, 8192, 3584, True, "gemm_skinny_kernel", "16x16x32"),
     (4096, 4096, 4096, True, "gemm_dtl16_kernel", "16x16x32"),
