@@ -561,7 +561,10 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool pee
 // 16 x 8192 x 3584 with seven peers 20.9 -> 14.1 (row-major B 21.9 -> 18.8), 4 x 3360 x 976 14.1 -> 6.3, 4 x 2816 x 576
 // row-major 15.0 -> 6.1, 16 x 1024 x 16384 22.6 -> 15.5, fp32 2 x 1216 x 1280 17.1 -> 7.8, 16 x 4096 x 4096 28.7 -> 17.6;
 // 64 x 8192 x 3584 24.4 -> 19.2, row-major level (24.4 / 24.7).  From 65 rows on the rows of A, which every workgroup
-// reads, outweigh B.
+// reads, outweigh B; so they do below with wide outputs and a long K, where the model does not see it.  Time of this kernel
+// over that of the 128x128 kernels, bf16, N of 2048 and more (geometric means of random shapes): 33 to 64 rows, transposed
+// B 0.67 at K = 2048, 0.83 at 3500, 0.97 at 4900, 1.06 at 7000, 1.17 at 9700, 1.28 at 14000, row-major 0.86, 0.98, 1.08, 1.22,
+// 1.35, 1.48; 17 to 32 rows, transposed 0.87 at 7000, 0.97 at 9700, 1.07 at 14000.  Narrower ones stay below 1.
 constexpr int64_t kMaxPartsBytes = KR_STATIC_SCRATCH_BYTES;   // (the form that allocates nothing takes every split)
 struct SkinnyPlan {
     int cb;       // columns of a workgroup / 16; 0: not for this call
@@ -579,6 +582,7 @@ static SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool b_nt, bool f
         if (s >= 1 && s <= units && s * M * N * 4 <= parts_bytes) p.splits = s;
         return p;
     }
+    if (!f32 && M > 16 && N >= 2048 && K > (M > 32 ? (b_nt ? 4096 : 3584) : b_nt ? 11264 : INT64_MAX)) return p;
     int64_t best = 0;
     for (int cb = 1; cb <= (f32 || M > 32 ? 2 : 4); cb *= 2) {
         for (int64_t s = 1; s <= kMaxSplits && (s == 1 || (4 * s <= units && s * M * N * 4 <= parts_bytes)); s *= 2) {

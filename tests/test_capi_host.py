@@ -380,6 +380,21 @@ def test_gemm_plan_names_every_kernel(lib, M, N, K, b_t, kernel, mfma):
     assert (p["kernel"], p["mfma"]) == (kernel, mfma)
 
 
+@pytest.mark.parametrize("M,N,K,b_t,few", [
+    (64, 2048, 4096, True, True), (64, 2048, 4104, True, False), (64, 2040, 4104, True, True), (33, 2048, 4104, True, False),
+    (64, 2048, 3584, False, True), (64, 2048, 3592, False, False), (64, 2040, 3592, False, True),
+    (32, 2048, 11264, True, True), (32, 2048, 11272, True, False), (32, 2040, 11272, True, True), (17, 2048, 11272, True, False),
+    (32, 2048, 16384, False, True), (16, 8192, 16384, True, True), (16, 8192, 16384, False, True),
+])
+def test_gemm_plan_few_rows_up_to_a_k(lib, M, N, K, b_t, few):
+    """Wide outputs with a long K: from 17 rows on the few-rows kernel is left for one with 128 x 128 tiles."""
+    need = lib.kr_gemm_workspace_bytes(M, N, K)
+    p = _lib.gemm_plan(M, N, K, b_t, workspace_bytes=need)
+    assert (p["kernel"] == "gemm_skinny_kernel") == few
+    assert few or p["k_splits"] > 1
+    assert p == _lib.gemm_plan(M, N, K, b_t, workspace_bytes=1 << 40)
+
+
 @pytest.mark.parametrize("M,N,K,P,kernel", [
     (1000, 4096, 8192, 0, "gemm_ks_kernel"),         # one pass, no peers, whole k-steps
     (256, 512, 640, 0, "gemm_ks_kernel"),
