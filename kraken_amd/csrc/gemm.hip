@@ -496,7 +496,7 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     16 ns per million elements with row-major B, which runs gemm_ks_kernel; 2 us and 20 ns and parts of at least eight
 //     k-steps with transposed B, gemm_reduce_kernel: fitted to every split of 13 257 random shapes, 65 to 4096 rows, where
 //     this choice takes 1.009 (no peers) and 1.033 (peers) of the time of the best one);
-//     S = 1 with peers and more than 16 k-steps 4 us more (fitted, the cause is not separated; one or three peers, in
+//     S = 1 with peers and more than 16 k-steps (transposed B 15: 384 x 1712 x 1024 23.7 / 18.4) 4 us more (fitted, the cause is not separated; one or three peers, in
 //     one pass / in three parts: 112 x 9216 x 1664 27.0 / 21.7, 256 x 4096 x 1536 25.0 / 20.8, 720 x 1280 x 1464 24.6 / 21.1,
 //     row-major 22.4 / 20.1; 360 x 768 x 1096 21.4 / 20.5; but 300 x 2048 x 1024 16.8 / 19.6, 128 x 4096 x 1024 16.5 / 19.1);
 //   the 256x256 kernel with every tile's K loop split: 1.2 us per k-step, twice the work per operand byte, but
@@ -532,8 +532,9 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool pee
         return choose_kernel();
     }
     const int64_t step = b_nt ? 56 : 60, launch = b_nt ? 200 : 600, part = b_nt ? 20 : 16, min_steps = b_nt ? kMinSplitSteps : 2;
+    const bool long_peers = peers && steps > (b_nt ? 15 : 16);
     auto cost = [&](int64_t s) {
-        return 650 + (tiles * s + 255) / 256 * step * ((steps + s - 1) / s) + (s > 1 ? launch + s * M * N * part / 100000 : peers && steps > 16 ? 400 : 0);
+        return 650 + (tiles * s + 255) / 256 * step * ((steps + s - 1) / s) + (s > 1 ? launch + s * M * N * part / 100000 : long_peers ? 400 : 0);
     };
     int64_t best = cost(1);
     for (int64_t s = 2; s <= kMaxSplits && min_steps * s <= steps && s * tiles <= 512; ++s)

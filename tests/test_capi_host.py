@@ -404,6 +404,8 @@ def test_gemm_plan_few_rows_up_to_a_k(lib, M, N, K, b_t, few):
     (1000, 4224, 4096, 0, "gemm_reduce_kernel"),     # 264 tiles
     (256, 512, 4096, 0, "gemm_reduce_kernel"),       # K loop in parts
     (256, 512, 640, 1, "gemm_reduce_kernel"),        # peers
+    (384, 1712, 1024, 7, "gemm_reduce_kernel"),      # peers and sixteen k-steps: in parts
+    (384, 1712, 960, 7, "gemm_reduce_kernel"),
 ])
 def test_gemm_plan_of_transposed_b_with_few_tiles(lib, M, N, K, P, kernel):
     """With transposed B gemm_ks_kernel only where it is not slower than gemm_reduce_kernel, and parts of at least
@@ -411,7 +413,7 @@ def test_gemm_plan_of_transposed_b_with_few_tiles(lib, M, N, K, P, kernel):
     p = _lib.gemm_plan(M, N, K, True, P, M, workspace_bytes=lib.kr_gemm_workspace_bytes(M, N, K))
     assert (p["kernel"], p["tile"]) == (kernel, 128)
     assert p["k_splits"] == 1 or K // 64 >= 8 * p["k_splits"]
-    assert (p["k_splits"] > 1) == ((M, N, K) == (256, 512, 4096))
+    assert (p["k_splits"] > 1) == ((M, N, K) in ((256, 512, 4096), (384, 1712, 1024)))
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (2, 1216, 16384), (16, 1024, 16384), (16, 1024, 8192), (32, 512, 8192), (64, 1032, 16384), (64, 8192, 3584)])
