@@ -380,6 +380,14 @@ def test_gemm_plan_names_every_kernel(lib, M, N, K, b_t, kernel, mfma):
     assert (p["kernel"], p["mfma"]) == (kernel, mfma)
 
 
+@pytest.mark.parametrize("M,N,K", [(256, 7168, 12928), (512, 5376, 6400), (768, 3584, 13760)])
+def test_gemm_plan_few_tiles_stay_split_where_224_divides_n(lib, M, N, K):
+    """A plain product with transposed B whose few 256 x 256 tiles share their K loops keeps them where N is also a
+    multiple of 224."""
+    p = _lib.gemm_plan(M, N, K, True, workspace_bytes=lib.kr_gemm_workspace_bytes(M, N, K))
+    assert p["tile_n"] == 256 and p["tail_tiles"] == (M // 256) * (N // 256) and p["tail_splits"] > 1
+
+
 @pytest.mark.parametrize("M,N,K,b_t,few", [
     (64, 2048, 4096, True, True), (64, 2048, 4104, True, False), (64, 2040, 4104, True, True), (33, 2048, 4104, True, False),
     (64, 2048, 3584, False, True), (64, 2048, 3592, False, False), (64, 2040, 3592, False, True),
