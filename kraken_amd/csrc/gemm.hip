@@ -648,6 +648,15 @@ static GemmPlan plan_of_skinny(const SkinnyPlan& sk) {
     p.skinny = sk.cb;
     return p;
 }
+// Whether a shape has enough tiles of 256 x 256 for one-pass workgroups (see plan_gemm).  Not with transposed B, a short K
+// that is no multiple of the k-step and a last round that leaves the launch less than 5/8 full: by the time of the
+// 256x256 kernel over that of the 128x128 kernel (geometric means of random shapes) 1.08 below K = 448 and 0.99 from there
+// to 1024, with fuller rounds 0.99 and 0.92 or less (4096 x 4672 x 416, 304 tiles, 37.5 / 30.7 us); row-major B 0.93, 0.87.
+static bool many_big_tiles(int64_t M, int64_t N, int64_t K, bool b_nt) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    if (b_nt && K % 64 != 0 && K < 640 && (tiles + 255) / 256 * 256 * 5 >= tiles * 8) return false;
+    return tiles > 128 && K >= 256;
+}
 static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peers, int64_t band_rows, bool plain,
                           bool plain_bf16_all_rows, bool has_workspace, int64_t workspace_bytes, bool has_gather, bool has_progress, bool flagged,
                           bool dtl_ok, bool skinny_ok) {
@@ -661,7 +670,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     // Otherwise 128x128 tiles; they also win while all of them fit on the
     // 256 CUs at once (512 tiles = 128 of the large ones): measured, the large tile is 15-30 %
     // faster from 144 tiles on and 5-10 % slower at 128, for K from 1024 to 8192.
-    bool big = ((M + 255) / 256) * ((N + 255) / 256) > 128 && K >= 256;
+    bool big = many_big_tiles(M, N, K, b_nt);
     // (few tiles: the large tile again with every tile's K loop split, where that is cheaper)
     SmallPlan small{0, 0, 1};
     if (!big || !dtl_ok || env_switches().gemm_tile == 128) {

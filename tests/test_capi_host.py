@@ -388,6 +388,19 @@ def test_gemm_plan_few_tiles_stay_split_where_224_divides_n(lib, M, N, K):
     assert p["tile_n"] == 256 and p["tail_tiles"] == (M // 256) * (N // 256) and p["tail_splits"] > 1
 
 
+@pytest.mark.parametrize("M,N,K,b_t,tile", [
+    (4096, 4672, 416, True, 128), (4096, 4672, 632, True, 128),      # 304 tiles of 256 x 256: a second round of 48
+    (4096, 4672, 416, False, 256), (4096, 4672, 384, True, 256), (4096, 4672, 640, True, 256), (4096, 4672, 648, True, 256),
+    (4096, 5120, 416, True, 128), (4096, 5376, 416, True, 256),      # 320, 336 tiles
+])
+def test_gemm_plan_of_a_short_ragged_k(lib, M, N, K, b_t, tile):
+    """Transposed B, K below 640 and no multiple of 64: 128 x 128 tiles unless the rounds of large ones are 5/8 full."""
+    need = lib.kr_gemm_workspace_bytes(M, N, K)
+    p = _lib.gemm_plan(M, N, K, b_t, 3, M, workspace_bytes=need)
+    assert p["tile"] == tile and p["k_splits"] == 1
+    assert p == _lib.gemm_plan(M, N, K, b_t, 3, M, workspace_bytes=1 << 40)
+
+
 @pytest.mark.parametrize("M,N,K,b_t,few", [
     (64, 2048, 4096, True, True), (64, 2048, 4104, True, False), (64, 2040, 4104, True, True), (33, 2048, 4104, True, False),
     (64, 2048, 3584, False, True), (64, 2048, 3592, False, False), (64, 2040, 3592, False, True),
