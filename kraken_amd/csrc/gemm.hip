@@ -542,6 +542,9 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool pee
             best = c;
             p.splits = (int)s;
         }
+    // (gemm_reduce_kernel has room for a second workgroup on a compute unit, which the model does not count: with 129 to
+    // 256 tiles it pays once the K loop is long, 0.86 of the time of one pass with 144 tiles from K = 12288 on, 0.94 with 208)
+    if (b_nt && p.splits == 1 && tiles > 128 && tiles <= 256 && K >= 12288) p.splits = 2;
     if (may_big && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
         int tail, ts;
         const int64_t big_tiles = (M / 256) * (N / 256);

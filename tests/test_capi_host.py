@@ -401,6 +401,20 @@ def test_gemm_plan_of_a_short_ragged_k(lib, M, N, K, b_t, tile):
     assert p == _lib.gemm_plan(M, N, K, b_t, 3, M, workspace_bytes=1 << 40)
 
 
+@pytest.mark.parametrize("M,N,K,b_t,splits", [
+    (1280, 2304, 14224, True, 2), (1272, 2304, 12288, True, 2), (1272, 2304, 12280, True, 1), (1280, 2304, 14224, False, 1),
+    (2048, 2048, 12296, True, 2), (2048, 2056, 12296, True, 1),      # 256, 272 tiles
+])
+def test_gemm_plan_long_k_with_up_to_256_tiles(lib, M, N, K, b_t, splits):
+    """Transposed B: two workgroups per tile, on one compute unit, from K = 12288 on."""
+    need = lib.kr_gemm_workspace_bytes(M, N, K)
+    p = _lib.gemm_plan(M, N, K, b_t, 1, M, workspace_bytes=need)
+    assert (p["tile"], p["k_splits"]) == (128, splits)
+    assert splits * M * N * 4 <= need or splits == 1
+    assert p == _lib.gemm_plan(M, N, K, b_t, 1, M, workspace_bytes=1 << 40)
+    assert _lib.gemm_plan(M, N, K, b_t, 1, M)["k_splits"] == 1       # no workspace
+
+
 @pytest.mark.parametrize("M,N,K,b_t,few", [
     (64, 2048, 4096, True, True), (64, 2048, 4104, True, False), (64, 2040, 4104, True, True), (33, 2048, 4104, True, False),
     (64, 2048, 3584, False, True), (64, 2048, 3592, False, False), (64, 2040, 3592, False, True),
