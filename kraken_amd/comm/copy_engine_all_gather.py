@@ -8,10 +8,13 @@ import torch
 from .. import _lib
 from ._common import PeerBuffers
 
-# Up to here the sixteen launches of eight copies and flags bound the call (all_gather_matmul, K = 8192, N = 3584: eight
-# shards of 4 .. 128 rows 212 us, in one launch 114; 256 rows, 32 MiB gathered, 225 / 180; 512 rows 233 / 235).  Above,
-# the product does, and copies that come one behind the other leave it more of the memory (1024 rows 405 / 438;
-# the same kernel once per chunk 424).
+# Up to here all copies and flags of a gather are one launch.  What that gives depends on how long the product takes beside
+# the launches of the loop (about 120 us of host time and 9 per chunk).  all_gather_matmul, time in one launch over time
+# with a copy and a flag per chunk, 2, 4 and 8 ranks, 4 to 47 MiB, K = 1024 to 8192, N = 1024 to 28672, one and two chunks a rank:
+# a call that is waited for 0.39 to 1.00 at all 216 shapes (W = 8, 1024 x 1024, N = 1024 0.59; N = 28672 0.87); calls one
+# behind the other 0.38 to 0.9 where the launches are the longer part, 0.94 to 1.03 where the product is, up to 1.07 with two
+# or four ranks and N = 7168 (2 x 1024 x 8192 200 -> 215 us, alone 284 -> 260).  Above, copies that come one behind the other leave
+# the product more of the memory (8 x 1024 x 8192, N = 3584 405 / 438 us; the same kernel once per chunk 424).
 ONE_LAUNCH_BYTES = 48 << 20
 
 _backend_streams: dict[int, torch.cuda.Stream] = {}
