@@ -530,7 +530,7 @@ int kr_all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, in
 /*
  * The same two products for any number of rows, N and K multiples of 16, K >= 128 (edge tiles and a last
  * k-step that is not full are handled by the kernel).  The Python layer calls them for whole tiles only,
- * because of the precision stated above; other shapes are widened there.  kr_gemm_fp8_ws: with a workspace of
+ * because of the precision stated above; other shapes go to kr_gemm_fp8_wide_ws.  kr_gemm_fp8_ws: with a workspace of
  * kr_gemm_fp8_workspace_bytes bytes (0: none needed), shapes with few tiles share each tile's K loop
  * between workgroups, whose fp32 parts meet there and are summed in a fixed order; contents are scratch,
  * and calls that may overlap need one each.
@@ -542,6 +542,17 @@ int kr_all_gather_matmul_fp8_ragged(const void* A, int64_t lda, const void* A_lo
                                     int64_t ldb, int64_t M, int64_t N, int64_t K, int W, int rank, int splits_per_rank,
                                     const uint32_t* progress, int64_t wait_limit_us, int32_t* status, void* out,
                                     int out_kind, void* stream);
+
+/*
+ * kr_gemm_fp8_ws with an fp8 result (out_kind 2) and sums of 24 bits instead of 16: the operands are widened to bf16, which
+ * is exact, between LDS and the matrix cores (kraken/fused/all_gather_matmul.py:53,121,213).
+ *   N, K multiples of 16; lda, ldb >= K and multiples of 16; pointers 16-byte aligned; 256 * max(lda, ldb) < 2^31 - 1;
+ *   tile_pivot: row whose tiles are computed first; workspace of kr_gemm_fp8_wide_workspace_bytes bytes (0: none needed),
+ *   contents are scratch, calls that may overlap need one each.
+ */
+int64_t kr_gemm_fp8_wide_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int kr_gemm_fp8_wide_ws(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                        void* out, int64_t tile_pivot, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * kr_gemm_reduce_ptrs_ws_bf16 for fp32 operands (the operands of test/test_gemm_allreduce.py:57-58, which the

@@ -129,6 +129,9 @@ _SIGNATURES = {
                                c_void_p]),
     "kr_all_gather_matmul_fp8_ragged": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,
                                                 c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_void_p]),
+    "kr_gemm_fp8_wide_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
+    "kr_gemm_fp8_wide_ws": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,
+                                    c_int64, c_void_p]),
     "kr_gemm_plan": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, c_int64, c_int, c_int, c_int64, c_void_p]),
     "kr_probe_read": (c_int, [c_void_p, c_int64, c_void_p, c_void_p]),
     "kr_probe_copy": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),

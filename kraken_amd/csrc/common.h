@@ -133,6 +133,7 @@ struct EnvSwitches {
     int gemm_tailsplit;  // KRAKEN_AMD_GEMM_TAILSPLIT=<n>
     int gemm_n224;       // KRAKEN_AMD_GEMM_N224=0|1
     int gemm_ks;         // KRAKEN_AMD_GEMM_KS=0|1
+    int gemm_w8;         // KRAKEN_AMD_GEMM_W8=<parts> | 1000 * (columns / 32) of the narrow tiles + panels of 256 columns
     int gemm_skinny;     // KRAKEN_AMD_GEMM_SKINNY=0 (off) | 100 * (columns / 16) + parts
 };
 const EnvSwitches& env_switches();   // status.hip

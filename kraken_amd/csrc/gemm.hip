@@ -484,6 +484,66 @@ static void fp8_split_plan(int64_t M, int64_t N, int64_t K, int* tail_out, int* 
     }
 }
 
+// fp8 operands widened to bf16 in registers (gemm_w8.hip): the columns as `panels` panels of 256, then narrower ones of
+// 32 nb2 (nb2 = 0: none), or with at most 128 tiles of 256x256 every tile's K loop in `splits` parts.
+// Widths: whole rounds of 256-column tiles and the narrow ones behind them, the pair that ends first.  A round costs, in
+// 0.01 us, 4 us to start and finish its tiles and per k-step of 128 and 256 columns 2.05 us with up to 160 compute units
+// busy, 2.56 with all of them (the power limit), 3 % more per 32 columns less.  Measured, us, 256-column tiles / 224 / the
+// choice: 4000 x 6656 x 4096 164 / 150.5 / 146.2 (16 panels, then 160 columns), 8000 x 3584 x 8192 308.6 / 299.3 / 299.3,
+// 2400 x 4992 x 8192 143.6 / 139.3 / 139.3, 8192 x 4096 x 8192 335.8 / 413.4 / 335.8.
+struct W8Plan {
+    int panels, nb2, splits;
+};
+static W8Plan plan_w8(int64_t M, int64_t N, int64_t K, bool may_split, int64_t workspace_bytes) {
+    const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, tiles = tm * tn, steps = (K + 127) / 128;
+    W8Plan p{(int)tn, 0, 1};
+    if (const int v = env_switches().gemm_w8; v >= 0) {   // testing and tuning
+        const int64_t nb2 = v / 1000, panels = std::min<int64_t>(v % 1000, N / 256);
+        if (nb2 >= 4 && nb2 <= 7) return W8Plan{(int)panels, N > panels * 256 ? (int)nb2 : 0, 1};
+        if (nb2 == 0 && v > 1 && may_split && v <= steps && tiles * v * (256 * 256 * 4) <= workspace_bytes) p.splits = v;
+        return p;
+    }
+    if (tiles <= 128) {
+        int64_t best = 500 + 210 * steps;
+        for (int64_t s = 2; may_split && s <= kMaxSplits && s * tiles <= 256 && 2 * s <= steps && tiles * s * (256 * 256 * 4) <= workspace_bytes; ++s) {
+            const int64_t cost = 900 + 210 * ((steps + s - 1) / s) + s * M * N * 8 / 50000;
+            if (cost < best) {
+                best = cost;
+                p.splits = (int)s;
+            }
+        }
+        return p;
+    }
+    auto round_cost = [&](int64_t nb, int64_t busy) {
+        return 400 + steps * (205 + (busy > 160 ? 51 * (busy - 160) / 96 : 0)) * nb * (100 + 3 * (8 - nb)) / 800;
+    };
+    auto rounds_cost = [&](int64_t nb, int64_t n) { return n / 256 * round_cost(nb, 256) + (n % 256 > 0 ? round_cost(nb, n % 256) : 0); };
+    int64_t best = rounds_cost(8, tiles);
+    for (int64_t panels = 0; panels * 256 < N; ++panels) {
+        for (int64_t nb = 4; nb < 8; ++nb) {
+            const int64_t wide = tm * panels, narrow = tm * ((N - panels * 256 + 32 * nb - 1) / (32 * nb));
+            const int64_t early_end = wide / 256 * round_cost(8, 256), late = wide % 256;
+            int64_t end = early_end;
+            if (late == 0) {
+                end += rounds_cost(nb, narrow);
+            } else {
+                // `late` compute units are free one wide tile after the others: i narrow tiles on each of the others
+                const int64_t late_end = early_end + round_cost(8, 256), c = round_cost(nb, 256);
+                end = late_end;
+                for (int64_t i = 1, done = 0; done < narrow; ++i) {
+                    end = std::max(end, early_end + i * c);
+                    done = i * (256 - late) + (end - late_end) / c * late;
+                }
+            }
+            if (end < best) {
+                best = end;
+                p.panels = (int)panels;
+                p.nb2 = (int)nb;
+            }
+        }
+    }
+    return p;
+}
 // workspace of the two-pass form: S fp32 partial products of the whole [M, N] result
 static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (int64_t)S * M * N * 4; }
 
@@ -1113,6 +1173,54 @@ extern "C" int64_t kr_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K) 
 extern "C" int kr_gemm_fp8_ws(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
                               void* out, int out_kind, void* workspace, int64_t workspace_bytes, void* stream) {
     return gemm_fp8(A, lda, Bt, ldb, M, N, K, out, out_kind, stream, nullptr, false, workspace, workspace_bytes);
+}
+
+// The same product with sums of 24 bits: the operands are widened to bf16 on their way to the matrix cores (gemm_w8.hip).
+static int gemm_fp8_wide(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K, void* out,
+                         int64_t tile_pivot, void* workspace, int64_t workspace_bytes, void* stream) {
+    if (M < 0 || N < 0 || K < 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return KR_ERR_BAD_DIM;
+    if (N % 16 != 0 || K % 16 != 0) return KR_ERR_BAD_DIM;
+    if (M == 0 || N == 0) return KR_OK;
+    if (K == 0) return KR_ERR_BAD_DIM;
+    if (A == nullptr || Bt == nullptr || out == nullptr) return KR_ERR_NULL_POINTER;
+    if (lda < K || ldb < K) return KR_ERR_LAYOUT;
+    if (lda % 16 != 0 || ldb % 16 != 0 || !aligned16(A) || !aligned16(Bt) || !aligned16(out) || !aligned16(workspace)) return KR_ERR_ALIGNMENT;
+    // (a tile's panels are addressed with 32-bit byte offsets from their first row)
+    if (256 * std::max(lda, ldb) >= 0x7fffffffLL) return KR_ERR_LAYOUT;
+    GemmArgs g{};
+    peer_tab_stacked(g.peer, A, 0, 0);
+    g.A = (const uint16_t*)A;
+    g.B = (const uint16_t*)Bt;
+    g.lda = lda / 2;
+    g.ldb = ldb / 2;
+    g.M = (int)M; g.N = (int)N; g.K = (int)(K / 2);
+    g.comm_rows = 1;
+    g.count_rows = 1;
+    g.band_rows = (int)M;
+    g.out = out;
+    g.out_fp8 = 1;
+    g.mi16 = 1;
+    const W8Plan p = plan_w8(M, N, K, workspace != nullptr, workspace_bytes);
+    g.tiles_m = (int)((M + 255) / 256);
+    g.wide_panels = p.panels;
+    g.tiles_n = p.panels + (p.nb2 > 0 ? (int)((N - 256 * (int64_t)p.panels + 32 * p.nb2 - 1) / (32 * p.nb2)) : 0);
+    if ((int64_t)g.tiles_m * g.tiles_n > 0x7fffffffLL) return KR_ERR_BAD_DIM;
+    g.pivot_tiles = (int)(((tile_pivot / 256) % g.tiles_m + g.tiles_m) % g.tiles_m);
+    g.group_n = env_switches().gemm_group > 0 ? env_switches().gemm_group : 4;
+    g.k_splits = p.splits;
+    if (p.splits > 1) g.tail_tiles = g.tiles_m * g.tiles_n;
+    return (int)launch_gemm_w8(g, p.nb2, (hipStream_t)stream, workspace);
+}
+
+extern "C" int64_t kr_gemm_fp8_wide_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const W8Plan p = plan_w8(M, N, K, true, kMaxPartsBytes);
+    return p.splits > 1 ? ((M + 255) / 256) * ((N + 255) / 256) * p.splits * (256 * 256 * 4) : 0;
+}
+
+extern "C" int kr_gemm_fp8_wide_ws(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                   void* out, int64_t tile_pivot, void* workspace, int64_t workspace_bytes, void* stream) {
+    return gemm_fp8_wide(A, lda, Bt, ldb, M, N, K, out, tile_pivot, workspace, workspace_bytes, stream);
 }
 
 static int all_gather_matmul_fp8(const void* A, int64_t lda, const void* A_local, int64_t lda_local, const void* Bt,

@@ -39,6 +39,7 @@ struct GemmArgs {
     // launch runs the first tiles_m*tiles_n - tail_tiles tiles of the schedule, a second launch
     // the remaining ones with k_splits workgroups per tile, a third sums the parts
     int tail_tiles;
+    int wide_panels;     // gemm_w8_kernel: column panels of 256, the first of the tiles_n; the others are narrower
     int group_n;         // column panels per scheduling group (tile_schedule)
     int peers_on_mfma;   // 256x256 kernel: add whole-band tiles' peers through the matrix cores
     int mi16;            // 256x256 kernel: k loop and peer phase on 16x16x32 MFMA blocks
@@ -68,6 +69,8 @@ inline hipError_t lds_opt_in(const void* fn, int bytes, std::atomic<uint64_t>& d
 bool gemm_dtl_supported(const GemmArgs& g);
 hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* workspace);
 hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace);   // fp8 operands (gemm_dtl.hip)
+hipError_t launch_tail_finish(const GemmArgs& g, hipStream_t st, const void* workspace);   // sums the parts of split 256x256 tiles
+hipError_t launch_gemm_w8(const GemmArgs& g, int nb2, hipStream_t st, void* workspace);   // fp8 operands widened to bf16 (gemm_w8.hip)
 
 hipError_t launch_gemm_ks(const GemmArgs& g, bool b_nt, hipStream_t st);           // 128x128 tiles, k divided between waves (gemm_ks.hip)
 hipError_t launch_gemm_f32(const GemmArgs& g, bool b_nt, hipStream_t st);          // fp32 operands (gemm_f32.hip); A, B, lda, ldb in fp32 elements
@@ -144,36 +147,41 @@ __device__ __forceinline__ int64_t wave_uniform(int64_t v) {
 // [x * ntiles/8, (x+1) * ntiles/8) and a launch over fewer tiles takes the first count/8 of each
 // range (`first` skips positions an earlier launch has taken).  Where 8 does not divide the count, the
 // first ntiles % 8 XCDs own one position more (launches over all tiles only).
+// (the plain form: a launch over all of `ntiles`)
+__device__ __forceinline__ int xcd_position(int wg, int ntiles) {
+    const int x = wg % kXcds;
+    return x * (ntiles / kXcds) + min(x, ntiles % kXcds) + wg / kXcds;
+}
 __device__ __forceinline__ int schedule_position(const GemmArgs& g, int wg, int first = 0) {
     const int ntiles = g.tiles_m * g.tiles_n;
-    if (ntiles % kXcds != 0 && (g.tail_tiles == 0 || g.tail_tiles == ntiles)) {
-        const int x = wg % kXcds;
-        return x * (ntiles / kXcds) + min(x, ntiles % kXcds) + wg / kXcds;
-    }
+    if (ntiles % kXcds != 0 && (g.tail_tiles == 0 || g.tail_tiles == ntiles)) return xcd_position(wg, ntiles);
     if (ntiles % kXcds != 0 || first % kXcds != 0) return first + wg;
     return (wg % kXcds) * (ntiles / kXcds) + first / kXcds + wg / kXcds;
 }
 
 // Map a position in the tile order to its tile (tile_m, tile_n).
-__device__ __forceinline__ void tile_schedule(const GemmArgs& g, int pid, int& tile_m_out, int& tile_n_out) {
+__device__ __forceinline__ void tile_in_order(int pid, int tiles_m, int tiles_n, int group_n, int pivot_tiles, int& tile_m_out, int& tile_n_out) {
     // ---- tile schedule -------------------------------------------------------------------
-    // Tiles are ordered in groups of g.group_n column panels, M fastest in steps of g.group_n
+    // Tiles are ordered in groups of group_n column panels, M fastest in steps of group_n
     // columns: the ~32 tiles an XCD runs at a time form a (32 / group_n) x group_n block that
     // shares its A and B panels through the XCD's L2 (a dozen panels for 32 tiles), and every
     // XCD works on all row bands -- the rows of the reduce band (whose tiles also stream the
     // peers' partial sums) are spread over all XCDs instead of landing on one.  The M order is
     // rotated by the pivot, so the band's (or the local shard's) tiles are the first ones of
     // every XCD.
-    const int per_group = g.group_n * g.tiles_m;
+    const int per_group = group_n * tiles_m;
     const int group = pid / per_group;
-    const int first_n = group * g.group_n;
-    const int gsz = min(g.tiles_n - first_n, g.group_n);
+    const int first_n = group * group_n;
+    const int gsz = min(tiles_n - first_n, group_n);
     const int tile_n = first_n + (pid % per_group) % gsz;
     int tile_m = (pid % per_group) / gsz;
-    tile_m += g.pivot_tiles;
-    if (tile_m >= g.tiles_m) tile_m -= g.tiles_m;
+    tile_m += pivot_tiles;
+    if (tile_m >= tiles_m) tile_m -= tiles_m;
     tile_m_out = tile_m;
     tile_n_out = tile_n;
+}
+__device__ __forceinline__ void tile_schedule(const GemmArgs& g, int pid, int& tile_m_out, int& tile_n_out) {
+    tile_in_order(pid, g.tiles_m, g.tiles_n, g.group_n, g.pivot_tiles, tile_m_out, tile_n_out);
 }
 
 // Fused epilogue of one workgroup tile.  `acc` are this wave's 32x32 MFMA accumulators (TM x TN
@@ -462,6 +470,49 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+    }
+}
+
+// fp32 -> fp8 (e4m3fn) of two values into one half of a word: nearest even; magnitudes from 448 on
+// (infinities included) give +-448, NaN stays NaN -- the conversion kr_cast_f32_to_fp8 defines.  The
+// clamp is explicit, so the instruction's own overflow handling never comes into play.
+template <bool HIGH_HALF>
+__device__ __forceinline__ uint32_t pack2_e4m3(float a, float b, uint32_t old) {
+    const float ca = __builtin_fminf(__builtin_fmaxf(a, -448.0f), 448.0f), cb = __builtin_fminf(__builtin_fmaxf(b, -448.0f), 448.0f);
+    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a != a ? a : ca, b != b ? b : cb, (int)old, HIGH_HALF);
+}
+
+// fp8 store of a wave's 128 x 16 NB part of a tile held as 8 x NB accumulator blocks of 16 x 16 (lane l:
+// row l%16, columns 4(l/16) .. +3 of a block): per 16-row slab a lane's four values of a block become
+// one word of a per-wave LDS patch [16][16 NB + 16] bytes (with NB = 8 the pad keeps the 64 word stores of a block on
+// 64 banks), and the slab leaves as 16-byte chunks of whole rows.  `dst`: the wave's first
+// row and column; ld in bytes.  MASKED: only the first `rows` rows and `cols` columns (a multiple of 16) exist.
+template <int NB, bool MASKED>
+__device__ __forceinline__ void store_tile_fp8_blocks(const f32x4 (&acc16)[8][NB], unsigned char* smem, uint8_t* dst, int64_t ld,
+                                                      int lane, int wave, int rows, int cols) {
+    constexpr int LD = NB * 16 + 16;
+    static_assert(16 * LD <= 4096 && NB <= 8, "patch of a wave, two chunks per lane and slab");
+    unsigned char* patch = smem + wave * 4096;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            // (pinned here: copies the compiler may hoist would keep all blocks' values alive at once)
+            float x0, x1, x2, x3;
+            asm volatile("v_accvgpr_read_b32 %0, %2\n\tv_accvgpr_read_b32 %1, %3" : "=&v"(x0), "=&v"(x1) : "a"(acc16[i][j][0]), "a"(acc16[i][j][1]));
+            asm volatile("v_accvgpr_read_b32 %0, %2\n\tv_accvgpr_read_b32 %1, %3" : "=&v"(x2), "=&v"(x3) : "a"(acc16[i][j][2]), "a"(acc16[i][j][3]));
+            const uint32_t w = pack2_e4m3<true>(x2, x3, pack2_e4m3<false>(x0, x1, 0u));
+            *(uint32_t*)(patch + (lane & 15) * LD + 16 * j + 4 * (lane >> 4)) = w;
+        }
+        asm volatile("" ::: "memory");   // the reads below see the stores above (different types, same bytes)
+#pragma unroll
+        for (int it = 0; it < (16 * NB + 63) / 64; ++it) {
+            const int idx = it * 64 + lane, r = idx / NB, c = idx % NB;
+            if (16 * NB % 64 != 0 && idx >= 16 * NB) continue;
+            const u32x4 v = *(const u32x4*)(patch + r * LD + c * 16);
+            if (!MASKED || (16 * i + r < rows && c * 16 < cols)) st_stream((u32x4*)(dst + (int64_t)(16 * i + r) * ld + c * 16), v);
+        }
+        asm volatile("" ::: "memory");   // the next slab's stores stay behind these reads
     }
 }
 

@@ -94,48 +94,6 @@ __device__ __forceinline__ void store_tile_bf16_blocks(const f32x4 (&acc16)[2 * 
     }
 }
 
-// fp32 -> fp8 (e4m3fn) of two values into one half of a word: nearest even; magnitudes from 448 on
-// (infinities included) give +-448, NaN stays NaN -- the conversion kr_cast_f32_to_fp8 defines.  The
-// clamp is explicit, so the instruction's own overflow handling never comes into play.
-template <bool HIGH_HALF>
-__device__ __forceinline__ uint32_t pack2_e4m3(float a, float b, uint32_t old) {
-    const float ca = __builtin_fminf(__builtin_fmaxf(a, -448.0f), 448.0f), cb = __builtin_fminf(__builtin_fmaxf(b, -448.0f), 448.0f);
-    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a != a ? a : ca, b != b ? b : cb, (int)old, HIGH_HALF);
-}
-
-// fp8 store of a wave's 128 x 128 part of a tile held as 8 x 8 accumulator blocks of 16 x 16 (lane l:
-// row l%16, columns 4(l/16) .. +3 of a block): per 16-row slab a lane's four values of a block become
-// one word of a per-wave LDS patch [16][128 + 16] bytes (the pad keeps the 64 word stores of a block on
-// 64 banks), and the slab leaves as 16-byte chunks of whole 128-byte rows.  `dst`: the wave's first
-// row and column; ld in bytes.  MASKED: only the first `rows` rows and `cols` columns (a multiple of 16) exist.
-template <bool MASKED>
-__device__ __forceinline__ void store_tile_fp8_blocks(const f32x4 (&acc16)[2 * TM][2 * TN], unsigned char* smem, uint8_t* dst, int64_t ld,
-                                                      int lane, int wave, int rows, int cols) {
-    constexpr int COLS = 2 * TN * 16, LD = COLS + 16, CPR = COLS / 16;
-    static_assert(16 * CPR == 128, "two chunks per lane and slab");
-    unsigned char* patch = smem + wave * 4096;
-#pragma unroll
-    for (int i = 0; i < 2 * TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < 2 * TN; ++j) {
-            // (pinned here: copies the compiler may hoist would keep all blocks' values alive at once)
-            float x0, x1, x2, x3;
-            asm volatile("v_accvgpr_read_b32 %0, %2\n\tv_accvgpr_read_b32 %1, %3" : "=&v"(x0), "=&v"(x1) : "a"(acc16[i][j][0]), "a"(acc16[i][j][1]));
-            asm volatile("v_accvgpr_read_b32 %0, %2\n\tv_accvgpr_read_b32 %1, %3" : "=&v"(x2), "=&v"(x3) : "a"(acc16[i][j][2]), "a"(acc16[i][j][3]));
-            const uint32_t w = pack2_e4m3<true>(x2, x3, pack2_e4m3<false>(x0, x1, 0u));
-            *(uint32_t*)(patch + (lane & 15) * LD + 16 * j + 4 * (lane >> 4)) = w;
-        }
-        asm volatile("" ::: "memory");   // the reads below see the stores above (different types, same bytes)
-#pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int idx = it * 64 + lane, r = idx / CPR, c = idx % CPR;
-            const u32x4 v = *(const u32x4*)(patch + r * LD + c * 16);
-            if (!MASKED || (16 * i + r < rows && c * 16 < cols)) st_stream((u32x4*)(dst + (int64_t)(16 * i + r) * ld + c * 16), v);
-        }
-        asm volatile("" ::: "memory");   // the next slab's stores stay behind these reads
-    }
-}
-
 // One workgroup tile.  PEERS_FIRST picks the order of the two accumulation phases (peers'
 // partial sums, k loop) for tiles whose peers are added on the matrix cores.
 // SPLIT: the workgroup is one of g.k_splits that share a tile of the last partial round: it
@@ -940,8 +898,8 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     if (F8 && g.out_fp8) {
         if constexpr (F8) {
             uint8_t* dst = (uint8_t*)g.out + (int64_t)(m0 + wm * WTM) * g.N + n0 + wn * WTN;
-            if (full_tile) store_tile_fp8_blocks<false>(acc16, smem, dst, g.N, lane, wave, 0, 0);
-            else if constexpr (RAGGED) store_tile_fp8_blocks<true>(acc16, smem, dst, g.N, lane, wave, g.M - m0 - wm * WTM, g.N - n0 - wn * WTN);
+            if (full_tile) store_tile_fp8_blocks<2 * TN, false>(acc16, smem, dst, g.N, lane, wave, 0, 0);
+            else if constexpr (RAGGED) store_tile_fp8_blocks<2 * TN, true>(acc16, smem, dst, g.N, lane, wave, g.M - m0 - wm * WTM, g.N - n0 - wn * WTN);
         }
     } else if constexpr (NB != 2 * TN) {
         // 224-column tile of a plain product: every row goes to `out`
@@ -1022,6 +980,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
     int tile_m, tile_n;
     tile_schedule(g, schedule_position(g, u, g.tiles_m * g.tiles_n - g.tail_tiles), tile_m, tile_n);
     const int m0 = tile_m * BM + (wave / WN) * WTM + slab * 32, n0 = tile_n * BN + (wave % WN) * WTN;
+    if (m0 >= g.M || n0 >= g.N) return;   // edge tiles: nothing of this slab is in the matrix
     // this thread's quads are 16 slab + 4 jw .. +3 of the wave's 64
     const f32x4* p = parts + ((int64_t)u * S * NQ + slab * 16 + 4 * jw) * T + wave * 64 + lane;
     f32x4 sum[4];
@@ -1109,7 +1068,7 @@ bool gemm_dtl_supported(const GemmArgs& g) {
 }
 
 // The third launch: `workspace` holds g.k_splits parts of each of the last g.tail_tiles tiles.
-static hipError_t launch_tail_finish(const GemmArgs& g, hipStream_t st, const void* workspace) {
+hipError_t launch_tail_finish(const GemmArgs& g, hipStream_t st, const void* workspace) {
     hipLaunchKernelGGL(gemm_dtl_tail_finish_kernel, dim3((unsigned)(g.tail_tiles * WM * WN * TM)), dim3(WM * WN * 64), 0, st, g,
                        (const f32x4*)workspace);
     return hipGetLastError();

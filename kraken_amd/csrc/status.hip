@@ -24,6 +24,7 @@ static EnvSwitches read_env() {
     e.gemm_n224 = num("KRAKEN_AMD_GEMM_N224");
     e.gemm_ks = num("KRAKEN_AMD_GEMM_KS");
     e.gemm_skinny = num("KRAKEN_AMD_GEMM_SKINNY");
+    e.gemm_w8 = num("KRAKEN_AMD_GEMM_W8");
     return e;
 }
 static EnvSwitches& env_storage() {

@@ -43,13 +43,13 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
     fp8 once.  Shapes of whole tiles (M, N multiples of 256, K of 128) run on
     the fp8 matrix-core instruction (``kr_gemm_fp8_ws``, or ``kr_all_gather_matmul_fp8`` for ``gather=True``: the
     shards are copied chunk by chunk on a side stream while the tiles wait for their chunk's flag, as in the
-    bf16 form); others are widened to bf16 (exact), multiplied by the bf16 kernels with an fp32 result, and
-    rounded by ``kr_cast_f32_to_fp8`` after the gather has finished.  ``fp8_kernel=False`` forces the widening path.
+    bf16 form); others run on the bf16 instruction, their operands widened in registers (``kr_gemm_fp8_wide_ws``), after
+    the gather has finished.  ``fp8_kernel=False`` forces the widening kernel.
 
     The two differ in the precision of the sums: the fp8 instruction keeps about 16 bits of them (1.2e-5 in the
     2-norm against 64 bits, K = 128 .. 16384; both the 16x16x32 and the 16x16x128 form, to the same bits), the bf16
     instruction all 24 (2e-9 at K = 4096), so ragged shapes are not sent to the fp8 kernel although its C entry points
-    take them: 4000 x 6656 x 4096 takes 83 us there and 250 us here, with 5e-4 of the results one fp8 step off."""
+    take them: 4000 x 6656 x 4096 takes 83 us there and 146 us here, with 5e-4 of the results one fp8 step off."""
     fp8 = torch.float8_e4m3fn
     W = peers.W
     m, K = peers.slice(0).shape
@@ -116,14 +116,11 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
         _lib.check(lib.kr_gemm_fp8_ws(a_full.data_ptr(), K, b.T.data_ptr(), K, M, N, K, c.data_ptr(), 2, ws_ptr, ws_bytes, stream),
                    "all_gather_matmul(fp8)")
         return a_out, c
-    a16 = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
-    bt16 = torch.empty((N, K), dtype=torch.bfloat16, device=dev)           # b.T is contiguous: memory [N, K]
-    _lib.check(lib.kr_cast_fp8_to_bf16(a_full.data_ptr(), M * K, a16.data_ptr(), stream), "cast_fp8_to_bf16(a)")
-    _lib.check(lib.kr_cast_fp8_to_bf16(b.T.data_ptr(), N * K, bt16.data_ptr(), stream), "cast_fp8_to_bf16(b)")
-    c32 = torch.empty((M, N), dtype=torch.float32, device=dev)
-    _gemm.launch("all_gather_matmul", a16, bt16.T, M, N, None, 0, 0, None, 0, M, None, c32, rank * m)
     c = torch.empty((M, N), dtype=fp8, device=dev)
-    _lib.check(lib.kr_cast_f32_to_fp8(c32.data_ptr(), M * N, c.data_ptr(), stream), "cast_f32_to_fp8(c)")
+    ws = _gemm.workspace(dev, lib.kr_gemm_fp8_wide_workspace_bytes(M, N, K))
+    ws_ptr, ws_bytes = (ws.data_ptr(), ws.numel()) if ws is not None else (None, 0)
+    _lib.check(lib.kr_gemm_fp8_wide_ws(a_full.data_ptr(), K, b.T.data_ptr(), K, M, N, K, c.data_ptr(), rank * m, ws_ptr, ws_bytes, stream),
+               "all_gather_matmul(fp8)")
     return a_out, c
 
 
@@ -170,9 +167,9 @@ def all_gather_matmul(
     (nearest even, magnitudes of 448 and more saturate to 448), in both modes.
     With M and N multiples of 256 and K of 128 the product runs on the fp8
     matrix-core instruction, whose sums keep about 16 bits; other sizes (multiples of 16,
-    and ``fp8_kernel=False``) are widened to bf16 by one conversion pass per operand
-    (exact: every e4m3 value is a bf16 value), multiplied by the bf16 kernels with an
-    fp32 result and rounded to fp8 by a third pass, after the gather has finished.
+    and ``fp8_kernel=False``) run on the bf16 instruction, after the gather has finished, their
+    operands widened to bf16 in registers (exact: every e4m3 value is a bf16 value) and the
+    fp32 sums rounded to fp8 once.
     ``a_gathered`` stays fp8.
     """
     fp8 = torch.float8_e4m3fn

@@ -502,6 +502,29 @@ def test_fp8_cast_argument_errors(lib):
         assert f(None, 0, None, None) == 0
 
 
+def test_gemm_fp8_wide_argument_errors(lib):
+    f = lib.kr_gemm_fp8_wide_ws
+    base = dict(A=FAKE, lda=512, Bt=FAKE, ldb=512, M=100, N=272, K=496, out=FAKE, pivot=0, ws=None, bytes=0, stream=None)
+    def call(**kw):
+        args = dict(base); args.update(kw)
+        return f(*args.values())
+    assert call(N=264) == _lib.KR_ERR_BAD_DIM
+    assert call(K=488) == _lib.KR_ERR_BAD_DIM
+    assert call(K=0) == _lib.KR_ERR_BAD_DIM
+    assert call(M=-1) == _lib.KR_ERR_BAD_DIM
+    assert call(Bt=None) == _lib.KR_ERR_NULL_POINTER
+    assert call(lda=480) == _lib.KR_ERR_LAYOUT
+    assert call(ldb=1 << 23) == _lib.KR_ERR_LAYOUT       # 256 rows beyond the reach of 32-bit offsets
+    assert call(lda=520) == _lib.KR_ERR_ALIGNMENT
+    assert call(out=FAKE + 8) == _lib.KR_ERR_ALIGNMENT
+    assert call(ws=FAKE + 8) == _lib.KR_ERR_ALIGNMENT
+    assert call(M=0, A=None, Bt=None, out=None) == 0
+    need = lib.kr_gemm_fp8_wide_workspace_bytes
+    assert need(0, 256, 256) == 0 and need(4000, 6656, 4096) == 0
+    for M, N, K in ((1, 16, 16), (8, 8192, 16384), (512, 4096, 4096), (2000, 2048, 8192), (1, 16, 1 << 20)):
+        assert 0 <= need(M, N, K) <= 64 << 20
+
+
 def test_gemm_fp8_argument_errors(lib):
     f = lib.kr_gemm_fp8
     ok = (FAKE, 512, FAKE, 512, 256, 256, 512, FAKE, 2, None)

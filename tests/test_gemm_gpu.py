@@ -1244,6 +1244,54 @@ def test_fp8_kernel_ragged_shapes(dev, M, N, K, split):
         assert (out[M].float() == 0).all()                     # nothing past the last row
 
 
+@pytest.mark.parametrize("plan", [None, 0, 3, 4000, 5001, 6000, 7002])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (255, 272, 112), (257, 528, 1040), (300, 1040, 528), (513, 816, 384)])
+def test_fp8_wide_kernel_shapes(dev, monkeypatch, M, N, K, plan):
+    """kr_gemm_fp8_wide_ws on sizes no tile divides, by its own choice of tiles, with 256-column tiles only, with every K
+    loop in three parts, and with narrow tiles of every width behind 0, 1 or 2 panels of 256 columns; odd and even
+    numbers of k-steps, the last one full or not.  Small integers and halves: every fp32 sum is exact, the fp8 result is the
+    rounded product (saturated where it is large, NaN in the row of a NaN); what lies between the rows is not read."""
+    fp8 = torch.float8_e4m3fn
+    g = torch.Generator().manual_seed(M + N + K)
+    lda, ldb = K + 16, K + 32
+    a, b = torch.full((M, lda), float("nan")).to(fp8), torch.full((N, ldb), float("nan")).to(fp8)
+    a[:, :K] = torch.randint(-2, 3, (M, K), generator=g).float().to(fp8)
+    b[:, :K] = (torch.randint(-3, 4, (N, K), generator=g).float() * 0.5).to(fp8)
+    a[0, :K], b[0, :K] = 4.0, 16.0
+    ad, bd = a.to(dev), b.to(dev)
+    want = (ad[:, :K].float() @ bd[:, :K].float().T).clamp(-448.0, 448.0)
+    if M > 1:
+        ad[M - 1, K - 1] = float("nan")
+        want[M - 1] = float("nan")
+    if plan is not None:
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_W8", str(plan))
+    lib = _lib.load()
+    ws = torch.empty(4 * -(-M // 256) * -(-N // 256) * 256 * 256 * 4, dtype=torch.uint8, device=dev)
+    out = torch.zeros(M + 1, N, dtype=torch.float32, device=dev).to(fp8)
+    rc = lib.kr_gemm_fp8_wide_ws(ad.data_ptr(), lda, bd.data_ptr(), ldb, M, N, K, out.data_ptr(), M // 2, ws.data_ptr(), ws.numel(),
+                                 torch.cuda.current_stream(dev).cuda_stream)
+    assert rc == 0, _lib.strerror(rc)
+    assert torch.equal(torch.nan_to_num(out[:M].float(), nan=1000.0), torch.nan_to_num(want.to(fp8).float(), nan=1000.0))
+    assert (out[M].float() == 0).all()                     # nothing past the last row
+
+
+def test_fp8_wide_kernel_widens_every_code(dev):
+    """Each of the 256 e4m3 codes on both sides of a product with 1.0: the conversion on the way to the matrix cores is
+    exact, subnormals, both zeros and NaN included."""
+    fp8 = torch.float8_e4m3fn
+    codes = torch.arange(256, dtype=torch.uint8).repeat_interleave(1).view(256, 1)
+    x = torch.zeros(256, 128, dtype=torch.uint8)
+    x[torch.arange(256), torch.arange(256) % 128] = codes[:, 0]      # row r: code r at k = r % 128
+    ones = torch.full((16, 128), 1.0).to(fp8)
+    lib, stream = _lib.load(), torch.cuda.current_stream(dev).cuda_stream
+    xd, od = x.to(dev).view(fp8), ones.to(dev)
+    want = codes.view(fp8).float().expand(256, 16)
+    for a, b, w in ((xd, od, want), (od, xd, want.T)):
+        out = torch.empty(a.shape[0], b.shape[0], dtype=fp8, device=dev)
+        assert lib.kr_gemm_fp8_wide_ws(a.data_ptr(), 128, b.data_ptr(), 128, a.shape[0], b.shape[0], 128, out.data_ptr(), 0, None, 0, stream) == 0
+        assert torch.equal(torch.nan_to_num(out.cpu().float(), nan=1000.0), torch.nan_to_num(w, nan=1000.0))
+
+
 @pytest.mark.parametrize("gather", [False, True])
 @pytest.mark.parametrize("m,K,N", [(250, 144, 528), (33, 208, 4112), (256, 144, 512), (250, 128, 512)])
 def test_all_gather_matmul_fp8_ragged_sums_keep_their_bits(dev, m, K, N, gather):
