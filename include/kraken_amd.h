@@ -362,6 +362,20 @@ int kr_all_gather_matmul_bf16(const void* A, int64_t lda_m, const void* A_local,
                               void* C, void* stream);
 
 /*
+ * The same two results without flags: C = concat_r(shards[r]) @ B and A_out = concat_r(shards[r]) in one launch.  Tiles
+ * read their rows where the shards lie and write a share of what they read to A_out
+ * (kraken/fused/all_gather_matmul.py:222-325 with every shard readable from the start).
+ *   shards: host array of W device pointers, each [rows_per_shard, K] bf16 contiguous; A_out [W*rows_per_shard, K]
+ *   contiguous, which may hold a shard in its own place but overlaps none otherwise; B transposed-contiguous, ldb elements
+ *   between its columns; all 16-byte aligned; rank: whose rows are computed first.
+ * kr_gather_matmul_direct says (1 / 0) whether a shape can be called: rows_per_shard a multiple of 256, K and N of 8, and
+ * more than 128 tiles of 256 x 256.
+ */
+int kr_gather_matmul_direct(int W, int64_t rows_per_shard, int64_t N, int64_t K);
+int kr_gather_matmul_bf16(const void* const* shards, int W, int rank, int64_t rows_per_shard, void* A_out, const void* B,
+                          int64_t ldb, int64_t N, int64_t K, void* C, void* stream);
+
+/*
  * Stream-ordered flag write: *addr = value once everything enqueued on `stream` before this call
  * has completed, with its results visible to kernels that read the flag (release at system scope).
  * Replaces symm_mem_hdl.stream_write_value32 as used behind every chunk copy of the

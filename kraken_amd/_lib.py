@@ -99,6 +99,8 @@ _SIGNATURES = {
         [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64,
          c_int, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p],
     ),
+    "kr_gather_matmul_direct": (c_int, [c_int, c_int64, c_int64, c_int64]),
+    "kr_gather_matmul_bf16": (c_int, [c_void_p, c_int, c_int, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p]),
     "kr_stream_write_value32": (c_int, [c_void_p, ctypes.c_uint32, c_void_p]),
     "kr_gemm_producer_bf16": (
         c_int,

@@ -876,6 +876,9 @@ struct GatherSpec {
     uint32_t* band_counter;
     uint32_t* band_signal;
     int64_t count_rows;
+    const void* const* shards;   // gather inside the product: the W shards (comm_rows rows each) and the gathered matrix
+    int n_shards;
+    void* gather_out;
 };
 
 // Everything of the entry points except the peers: argument checks in the documented
@@ -954,6 +957,12 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
         g.band_signal = gather->band_signal;
         g.count_rows = (int)gather->count_rows;
     }
+    g.gather_out = nullptr;
+    if (gather != nullptr && gather->shards != nullptr) {
+        if (const int rc = peer_tab_from_ptrs(g.peer, gather->shards, gather->n_shards); rc != KR_OK) return rc;
+        g.gather_out = (uint16_t*)gather->gather_out;
+        g.comm_rows = (int)gather->comm_rows;
+    }
     g.bias = (const uint16_t*)bias;
     g.band_row0 = (int)band_row0;
     g.band_rows = (int)band_rows;
@@ -972,6 +981,7 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
                                     g.progress != nullptr || g.band_counter != nullptr,
                                     gemm_dtl_supported(g) && (g.a_local == nullptr || (int64_t)256 * g.lda_local * 2 < 0x7fffffffLL), skinny_ok);
     const bool dtl = plan.tile == 256;
+    if (g.gather_out != nullptr && !dtl) return KR_ERR_BAD_DIM;   // (kr_gather_matmul_direct says which shapes)
     // The 128x128 kernels address a tile's operand panels with 32-bit byte offsets from the
     // panel's first row (through a 2 GiB buffer descriptor): row strides beyond that reach are
     // refused rather than read as zeros.  (gemm_skinny_kernel, which has fewer rows, would reach
@@ -981,7 +991,7 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
         if ((128 * reach + std::max(K, N)) * (f32 ? 4 : 2) >= 0x7fffffffLL) return KR_ERR_LAYOUT;
     }
     g.peers_on_mfma = plan.peers_on_mfma;
-    g.mi16 = plan.mi16;
+    g.mi16 = plan.mi16 || g.gather_out != nullptr;
     g.n224 = plan.n224;
     const int bm = plan.tile, bn = plan.n224 ? 224 : bm;
     g.tiles_m = (int)((M + bm - 1) / bm);
@@ -1076,6 +1086,35 @@ extern "C" int kr_all_gather_matmul_bf16(const void* A, int64_t lda_m, const voi
     // no reduce: the band is every row, no peers, no bias; tile order rotated to the local shard
     return gemm_reduce(A, lda_m, 1, B, ldb_k, ldb_n, M, N, K, nullptr, 0, nullptr, 0, nullptr, 0, M, nullptr, C, 0,
                        gs.local_row0, stream, &gs);
+}
+
+// Rows gathered by the product itself: shapes with enough tiles for one-pass workgroups of 256 rows, each inside one shard.
+// Time of this form over copies on a side stream with the tiles waiting for their flags: see all_gather_matmul.
+extern "C" int kr_gather_matmul_direct(int W, int64_t rows_per_shard, int64_t N, int64_t K) {
+    if (W < 1 || W > KR_MAX_WORLD || rows_per_shard <= 0 || rows_per_shard % 256 != 0 || rows_per_shard > 0x7fffffffLL / W) return 0;
+    if (N <= 0 || N > 0x7fffffffLL || K > 0x7fffffffLL || K % 8 != 0 || N % 8 != 0) return 0;
+    GemmArgs g{};
+    g.K = (int)K;
+    g.lda = g.ldb = K;
+    if (!gemm_dtl_supported(g) || env_switches().gemm_tile == 128) return 0;
+    return many_big_tiles(W * rows_per_shard, N, K, true) ? 1 : 0;
+}
+
+extern "C" int kr_gather_matmul_bf16(const void* const* shards, int W, int rank, int64_t rows_per_shard, void* A_out, const void* B,
+                                     int64_t ldb, int64_t N, int64_t K, void* C, void* stream) {
+    if (W < 1 || W > KR_MAX_WORLD) return KR_ERR_WORLD_SIZE;
+    if (rank < 0 || rank >= W) return KR_ERR_STRIPE;
+    if (shards == nullptr || A_out == nullptr) return KR_ERR_NULL_POINTER;
+    if (!aligned16(A_out)) return KR_ERR_ALIGNMENT;
+    if (!kr_gather_matmul_direct(W, rows_per_shard, N, K)) return KR_ERR_BAD_DIM;
+    GatherSpec gs{};
+    gs.comm_rows = rows_per_shard;
+    gs.shards = shards;
+    gs.n_shards = W;
+    gs.gather_out = A_out;
+    const int64_t M = W * rows_per_shard;
+    return gemm_reduce(shards[0], K, 1, B, 1, ldb, M, N, K, nullptr, 0, nullptr, 0, nullptr, 0, M, nullptr, C, 0,
+                       rank * rows_per_shard, stream, &gs);
 }
 
 extern "C" int kr_gemm_producer_bf16(const void* A, int64_t lda_m, int64_t lda_k, const void* B, int64_t ldb_k,

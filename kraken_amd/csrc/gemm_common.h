@@ -32,6 +32,9 @@ struct GemmArgs {
     int local_row0, local_rows;
     uint64_t wait_ticks;        // bound of one tile's wait, in ticks of the 100 MHz constant clock
     int* status;                // set to 1 + block index by a tile whose wait ran out (may be nullptr)
+    // gather inside the product (gather_out == nullptr: off): rows [r*comm_rows, (r+1)*comm_rows) of A are peer.p[r], and
+    // the tiles write what they read to gather_out, [M, K] contiguous
+    uint16_t* gather_out;
     // split K loop of the 128x128 kernel (k_splits == 1: off)
     int k_splits;               // workgroups per tile, each with its share of the k-steps (grid y)
     int64_t split_out_stride;   // elements between the fp32 outputs of consecutive splits (0: one output)

@@ -109,13 +109,19 @@ __device__ __forceinline__ void store_tile_bf16_blocks(const f32x4 (&acc16)[2 * 
 // partial last round of compute units while 224-column tiles fill whole rounds (8192 x 3584: 448
 // tiles = 1.75 rounds against 512 = 2).  Per flop the narrower tile reads 7 % more of A from LDS
 // and L2, which two full rounds more than pay for.
-template <bool B_NT, bool PEERS_FIRST, bool SPLIT = false, bool RAGGED = false, bool MI16 = false, int NB = 2 * TN, bool F8 = false>
+// GATHER: the rows of A are spread over the W shards g.peer.p[r] (of g.comm_rows rows, a multiple of 256), and the matrix they
+// form, g.gather_out, is a result too.  Every tile of a row panel reads the whole panel anyway, so each writes its
+// share of the panel's k-steps out of LDS while it multiplies: no copy in front of the product, nothing to wait for.  Copies
+// on a side stream need compute units that only a finished tile gives back: 8 shards of 1024 x 8192, N = 3584 (134 MB
+// gathered) 397 us with them, 346 so; 8 x 512 x 4096, N = 4096 159 -> 106; 2 x 2048 x 4096, N = 8192 235 -> 203.
+template <bool B_NT, bool PEERS_FIRST, bool SPLIT = false, bool RAGGED = false, bool MI16 = false, int NB = 2 * TN, bool F8 = false, bool GATHER = false>
 __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* smem) {
     static_assert(NB == 2 * TN || (NB == 7 && MI16 && B_NT && !SPLIT && !RAGGED && !PEERS_FIRST), "224-column tile: plain NT products only");
     // F8: the operands are fp8 (e4m3fn) and g describes them as bf16 matrices of half the width (g.K, g.lda, g.ldb in
     // two-byte units), so a stage still holds 128-byte rows -- 128 k now -- and every load and LDS address below is unchanged;
     // only the k-step differs (k_step8: 16x16x128 MFMAs on the same 16 x 16 accumulator blocks).
     static_assert(!F8 || (MI16 && B_NT && !PEERS_FIRST && NB == 2 * TN), "fp8: plain NT products");
+    static_assert(!GATHER || (MI16 && B_NT && !PEERS_FIRST && !SPLIT && !F8), "gather: plain NT products");
     constexpr int BNX = WN * NB * 16;                            // columns of the workgroup tile
     constexpr int WTNX = NB * 16;                                // columns of a wave
     constexpr int LOADS_B = BNX * BKD * 2 / 1024 / (WM * WN);    // LDS-DMA loads of B per wave per k-step: 8 or 7
@@ -144,7 +150,13 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     const int k_begin = kt_begin * BKD;
     const uint16_t* a_tile;   // first row of the tile's A panel (gathered matrix or local shard)
     int64_t lda;
-    gathered_a_tile(g, m0, BM, a_tile, lda);
+    if constexpr (GATHER) {
+        const int shard = m0 / g.comm_rows;
+        a_tile = (const uint16_t*)g.peer.p[shard] + (int64_t)(m0 - shard * g.comm_rows) * g.lda;
+        lda = g.lda;
+    } else {
+        gathered_a_tile(g, m0, BM, a_tile, lda);
+    }
     // (the choice above is the same for the whole workgroup; the descriptor below wants it in
     // scalar registers)
     a_tile = (const uint16_t*)wave_uniform((int64_t)a_tile) + k_begin;
@@ -373,7 +385,7 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     const int band_lo = g.band_row0;
     const bool full_tile = !RAGGED || (m0 + BM <= g.M && n0 + BN <= g.N);
     const bool tile_in_band = full_tile && m0 >= band_lo && m0 + BM <= band_lo + g.band_rows;
-    const bool mfma_peers = !SPLIT && NB == 2 * TN && g.peers_on_mfma && g.n_peers > 0 && tile_in_band;
+    const bool mfma_peers = !SPLIT && !GATHER && NB == 2 * TN && g.peers_on_mfma && g.n_peers > 0 && tile_in_band;
     const bool bias_in_acc = !SPLIT && g.bias != nullptr && tile_in_band && (g.n_peers == 0 || mfma_peers);
     f32x16 acc[TM][TN];
     {
@@ -722,7 +734,31 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     // 118.2 -> 117.2 us; with the early barrier alone and the loads still 64 cycles apart nothing moves.
     // (224-column tile, NB = 7: 56 MFMAs per sub-step; barrier (b) behind MFMA 39, the same 16 slots
     // behind it for the 7 + 4 fragments of the next step; 15 fragments of sub-step 1 to read in sub-step 0)
+    // GATHER: in a step with COPY the wave also reads the eight 1 KiB chunks of A it requested itself (slots of sub-step 0
+    // that no fragment takes) and, once barrier (a) has handed the stage on, stores them to the gathered matrix between the
+    // loads of step t+2.  The stores are younger than the loads of step t+1, so the wait of barrier (b) lets them pass.
+    u32x4 copied[GATHER ? LOADS_A : 1];
+    uint32_t copy_voff = 0, copy_voff_tail = 0;
+    i32x4 copy_rsrc = {0, 0, 0, 0};
+    if constexpr (GATHER) {
+        copy_rsrc = make_rsrc(g.gather_out + (int64_t)m0 * g.K);
+        copy_voff = (uint32_t)(((int64_t)(lane >> 3) * g.K + (((lane & 7) ^ dma_sw) << 3)) * 2);
+        copy_voff_tail = RAGGED && a_voff_tail == kOob ? kOob : copy_voff;   // pieces past K: out of range, not stored
+    }
+    auto copy_read = [&](int q, uint32_t stage_off) __attribute__((always_inline)) {
+        typedef const __attribute__((address_space(3))) u32x4* lds_u32x4;
+        copied[q] = *(lds_u32x4)(size_t)(stage_off + (wave + 4 * q) * 1024 + lane * 16);
+    };
+    auto copy_store = [&](int t, int q) __attribute__((always_inline)) {
+        const uint32_t voff = RAGGED && t == t_tail ? copy_voff_tail : copy_voff;
+        asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen nt"
+                     :
+                     : "v"(copied[q]), "v"(voff), "s"(copy_rsrc), "s"((int)(((int64_t)8 * (wave + 4 * q) * g.K + t * BKD) * 2))
+                     : "memory");
+    };
     constexpr int NM16 = 2 * TM * NB;
+    constexpr int kStore0 = kBarA0 + 2 + kLoadGap16 / 2;   // slot of the first store, the others kLoadGap16 apart
+    static_assert(!GATHER || (kStore0 + kLoadGap16 * (LOADS_A - 1) <= NM16 + NM16 - 17 && 3 + 4 * (LOADS_A - 1) < kBarA0), "stores in front of barrier (b), reads in front of (a)");
     auto read_frag16 = [&](int buf, int r, int ks2, uint32_t stage_off) __attribute__((always_inline)) {
         if (r < NB) read_b16(buf, r, ks2, stage_off);
         else read_a16(buf, r - NB, ks2, stage_off);
@@ -732,7 +768,8 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     constexpr int kLoadsBeforeB = (NM16 + kBarB - kBarA0 - 2) / kLoadGap16 + 1 < kInStep ? (NM16 + kBarB - kBarA0 - 2) / kLoadGap16 + 1 : kInStep;
     static_assert(!MI16 || (kBarA0 < NM16 && kBarA0 + 2 + kLoadGap16 * (LOADS_TILE - 1) - kSlots16 < kBarA0 + 2),
                   "a step's late loads go out before the next step's first ones");
-    auto k_step16 = [&](int t, auto stage_c) __attribute__((always_inline)) {
+    auto k_step16 = [&](int t, auto stage_c, auto copy_c) __attribute__((always_inline)) {
+        constexpr bool COPY = GATHER && decltype(copy_c)::value;
         const uint32_t stage_cur = stage_c;
         const uint32_t stage_nxt = stage_cur ^ 1u;
         const uint32_t st_cur = stage_cur * A_ST, st_nxt = stage_nxt * A_ST;
@@ -754,6 +791,7 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
                 if (ks2 == 0) {
                     if (s % 2 == 0 && s / 2 < kFrags16) read_frag16(nxt, s / 2, 1, st_cur);
                     if (s % 8 == 1 && s / 8 + 4 < 2 * TM) read_a16(cur, s / 8 + 4, 0, st_cur);
+                    if (COPY && s % 4 == 3 && s / 4 < LOADS_A) copy_read(s / 4, st_cur);
                     if (s == kBarA0) {
                         KR_SCHED_FENCE();
                         __builtin_amdgcn_s_waitcnt(kLgkm0);
@@ -762,10 +800,11 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
                 }
                 if (lq >= 0 && lq % kLoadGap16 == 0 && lq / kLoadGap16 < kInStep) issue_load(t + 2, stage_cur, lq / kLoadGap16);
                 if (lw % kLoadGap16 == 0 && lw / kLoadGap16 >= kInStep && lw / kLoadGap16 < LOADS_TILE) issue_load(t + 1, stage_nxt, lw / kLoadGap16);
+                if (COPY && slot >= kStore0 && (slot - kStore0) % kLoadGap16 == 0 && (slot - kStore0) / kLoadGap16 < LOADS_A) copy_store(t, (slot - kStore0) / kLoadGap16);
                 if (ks2 == 1) {
                     if (s == kBarB) {
                         KR_SCHED_FENCE();
-                        __builtin_amdgcn_s_waitcnt(vmcnt_imm(kLoadsBeforeB));
+                        __builtin_amdgcn_s_waitcnt(vmcnt_imm(kLoadsBeforeB + (COPY ? LOADS_A : 0)));
                         __builtin_amdgcn_s_barrier();
                     }
                     // B blocks and A blocks 0..3 of k-step t+1: slots 48, 50, ..., 62; 63; 51, 55, 59
@@ -845,13 +884,30 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
         pin_accumulators();
         if (t < kt_total) k_step8(t, std::integral_constant<uint32_t, 0>{});
     } else if constexpr (MI16) {
+        auto trips = [&](int end, auto copy_c) __attribute__((always_inline)) {
 #pragma nounroll
-        for (; t + 2 <= kt_total; t += 2) {
-            k_step16(t, std::integral_constant<uint32_t, 0>{});
-            k_step16(t + 1, std::integral_constant<uint32_t, 1>{});
+            for (; t + 2 <= end; t += 2) {
+                k_step16(t, std::integral_constant<uint32_t, 0>{}, copy_c);
+                k_step16(t + 1, std::integral_constant<uint32_t, 1>{}, copy_c);
+            }
+            pin_accumulators();
+        };
+        if constexpr (GATHER) {
+            // this tile's share of the panel's k-steps, in pairs
+            trips(2 * (int)((int64_t)(kt_total / 2) * tile_n / g.tiles_n), std::false_type{});
+            trips(2 * (int)((int64_t)(kt_total / 2) * (tile_n + 1) / g.tiles_n), std::true_type{});
         }
-        pin_accumulators();
-        if (t < kt_total) k_step16(t, std::integral_constant<uint32_t, 0>{});
+        trips(kt_total, std::false_type{});
+        if (t < kt_total) k_step16(t, std::integral_constant<uint32_t, 0>{}, std::false_type{});
+        if constexpr (GATHER) {
+            // an odd last k-step is copied by itself
+            if ((kt_total & 1) && tile_n == g.tiles_n - 1) {
+                const int k = (kt_total - 1) * BKD + 8 * (tid & 7);
+#pragma unroll 4
+                for (int r = tid >> 3; r < BM; r += WM * WN * 8)
+                    if (!RAGGED || k < g.K) st_stream((u32x4*)(g.gather_out + (int64_t)(m0 + r) * g.K + k), *(const u32x4*)(a_tile + (int64_t)r * lda + k));
+            }
+        }
     } else {
 #pragma nounroll
         for (; t + 2 <= kt_total; t += 2) {
@@ -942,6 +998,13 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl16_kernel(const GemmArgs 
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl16n7_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     gemm_dtl_tile<true, false, false, false, true, 7>(g, smem);
+}
+
+// A as shards that the tiles also gather into one matrix.
+template <int NB, bool RAGGED>
+__global__ __launch_bounds__(WM* WN * 64) void gemm_dtl16_gather_kernel(const GemmArgs g) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    gemm_dtl_tile<true, false, false, RAGGED, true, NB, false, true>(g, smem);
 }
 
 // fp8 (e4m3fn) operands, transposed-contiguous B; the result is fp8, bf16 or fp32.
@@ -1091,6 +1154,19 @@ hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* w
     static std::atomic<uint64_t> opted[8];
     if (hipError_t e = lds_opt_in(kfn, LDS_BYTES, opted[(g.mi16 ? 4 : 0) + (b_nt ? 2 : 0) + (ragged ? 1 : 0)]); e != hipSuccess)
         return e;
+    if (g.gather_out != nullptr) {
+        static std::atomic<uint64_t> gopted[3];
+#define KR_LAUNCH(NB, RG, SLOT)                                                                                                       \
+    do {                                                                                                                              \
+        if (hipError_t e = lds_opt_in((const void*)gemm_dtl16_gather_kernel<NB, RG>, LDS_BYTES, gopted[SLOT]); e != hipSuccess) return e; \
+        hipLaunchKernelGGL((gemm_dtl16_gather_kernel<NB, RG>), grid, block, LDS_BYTES, st, g);                                        \
+    } while (0)
+        if (g.n224) KR_LAUNCH(7, false, 0);
+        else if (ragged) KR_LAUNCH(2 * TN, true, 1);
+        else KR_LAUNCH(2 * TN, false, 2);
+#undef KR_LAUNCH
+        return hipGetLastError();
+    }
     if (g.n224) {
         static std::atomic<uint64_t> nopted;
         if (hipError_t e = lds_opt_in((const void*)gemm_dtl16n7_kernel, LDS_BYTES, nopted); e != hipSuccess) return e;

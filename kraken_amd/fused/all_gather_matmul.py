@@ -1,11 +1,13 @@
 """All-gather + matmul, local arithmetic (``kraken/fused/all_gather_matmul.py``)."""
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib, _waits
 from ..comm._common import PeerBuffers
-from ..comm.copy_engine_all_gather import _copy_engine_all_gather_w_progress
+from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress
 from . import _gemm
 
 
@@ -36,6 +38,18 @@ def _matmul_w_progress(a, a_local, b, progress, configs, status=None) -> torch.T
     )
     _lib.check(rc, "all_gather_matmul")
     return c
+
+
+def _direct(sources: list[int], shard: torch.Tensor, a_out: torch.Tensor, b: torch.Tensor, W: int, m: int, N: int, K: int) -> bool:
+    """Whether the product gathers the shards itself (``kr_gather_matmul_bf16``): enough large tiles, each inside one
+    shard, and no shard that overlaps the gathered matrix other than in its own place (a tile may read a row
+    after another one has written it)."""
+    if W > _lib.KR_MAX_WORLD or not _lib.load().kr_gather_matmul_direct(W, m, N, K):
+        return False
+    out, size = a_out.data_ptr(), shard.numel() * shard.element_size()
+    if any(p % 16 != 0 for p in (out, b.data_ptr(), *sources)):
+        return False
+    return all(p + size <= out or p >= out + W * size or p == out + r * size for r, p in enumerate(sources))
 
 
 def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **kwargs):
@@ -143,8 +157,13 @@ def all_gather_matmul(
       the gathered matrix, so ``a_gathered`` is its zero-copy ``[W*m, K]`` view
       (copied into ``a_out`` when one is passed), ``progress`` is set to 1
       everywhere and the GEMM waits for nothing.
-    * ``gather=True`` (default for a list of shards): the reference's overlap.
-      The shards are copied chunk by chunk into ``a_out`` on a side stream,
+    * ``gather=True`` (default for a list of shards): the reference's overlap.  With more than 128
+      tiles of 256 x 256 and shards of whole tiles the product gathers the shards itself
+      (``kr_gather_matmul_bf16``): tiles read their rows where the shards lie and write what they
+      read to ``a_out`` while they multiply; the flags of ``progress`` are set behind it, no tile waits and
+      ``status`` is not touched.  8 shards of 1024 x 8192, N = 3584: 397 us with copies and flags, 346 so.
+      Otherwise, and with ``copy_engine=True``,
+      the shards are copied chunk by chunk into ``a_out`` on a side stream,
       each chunk followed by its flag in ``progress`` (``:308-311``), while the
       GEMM on the current stream consumes them: tiles of the local shard
       (``rank``) read it in place, every other tile waits for its chunk's flag
@@ -215,6 +234,18 @@ def all_gather_matmul(
         a_out = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
     else:
         assert tuple(a_out.shape) == (M, K) and a_out.dtype == torch.bfloat16 and a_out.is_contiguous()
+    sources = peers.pointers()
+    if not kwargs.get("copy_engine", False) and _direct(sources, shard, a_out, b, W, m, N, K):
+        if progress is not None:
+            _check_progress(progress, W * splits)
+            progress.fill_(0)
+        c = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+        rc = _lib.load().kr_gather_matmul_bf16((ctypes.c_void_p * W)(*sources), W, rank, m, a_out.data_ptr(), b.data_ptr(), b.stride(1),
+                                               N, K, c.data_ptr(), _lib.current_stream(dev))
+        _lib.check(rc, "all_gather_matmul")
+        if progress is not None:
+            progress.view(-1)[:W * splits].fill_(1)
+        return a_out, c
     if progress is None:
         progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)
     else:

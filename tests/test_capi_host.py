@@ -502,6 +502,29 @@ def test_fp8_cast_argument_errors(lib):
         assert f(None, 0, None, None) == 0
 
 
+def test_gather_matmul_argument_errors(lib):
+    import ctypes
+    f, direct = lib.kr_gather_matmul_bf16, lib.kr_gather_matmul_direct
+    table = (ctypes.c_void_p * 8)(*[FAKE] * 8)
+    base = dict(shards=table, W=8, rank=1, rows=512, A_out=FAKE, B=FAKE, ldb=256, N=4096, K=256, C=FAKE, stream=None)
+    def call(**kw):
+        args = dict(base); args.update(kw)
+        return f(*args.values())
+    assert direct(8, 512, 4096, 256) == 1
+    for W, rows, N, K in ((0, 512, 4096, 256), (17, 512, 4096, 256), (8, 500, 4096, 256), (8, 0, 4096, 256), (8, 256, 1024, 256),
+                          (8, 512, 4096, 64), (8, 512, 4100, 256), (8, 512, 4096, 260), (8, 1 << 40, 4096, 256), (8, 512, 4096, 1 << 22)):
+        assert direct(W, rows, N, K) == 0
+    assert call(W=17) == _lib.KR_ERR_WORLD_SIZE
+    assert call(rank=8) == _lib.KR_ERR_STRIPE
+    assert call(shards=None) == _lib.KR_ERR_NULL_POINTER
+    assert call(A_out=None) == _lib.KR_ERR_NULL_POINTER
+    assert call(A_out=FAKE + 8) == _lib.KR_ERR_ALIGNMENT
+    assert call(rows=500) == _lib.KR_ERR_BAD_DIM
+    assert call(C=None) == _lib.KR_ERR_NULL_POINTER
+    assert call(ldb=128) == _lib.KR_ERR_LAYOUT
+    assert call(shards=(ctypes.c_void_p * 8)(*[FAKE] * 7, FAKE + 2)) == _lib.KR_ERR_ALIGNMENT
+
+
 def test_gemm_fp8_wide_argument_errors(lib):
     f = lib.kr_gemm_fp8_wide_ws
     base = dict(A=FAKE, lda=512, Bt=FAKE, ldb=512, M=100, N=272, K=496, out=FAKE, pivot=0, ws=None, bytes=0, stream=None)

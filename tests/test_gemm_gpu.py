@@ -1244,6 +1244,57 @@ def test_fp8_kernel_ragged_shapes(dev, M, N, K, split):
         assert (out[M].float() == 0).all()                     # nothing past the last row
 
 
+# 256-column tiles; an odd number of k-steps; ragged K (last step 8 or 56 of 64) and N; 224-column tiles with an odd number
+# of steps; one column panel, so that a tile copies all it reads
+@pytest.mark.parametrize("W,m,N,K", [(8, 512, 4096, 256), (4, 1024, 4096, 320), (8, 512, 4104, 1032), (2, 2304, 4096, 696),
+                                     (16, 256, 7168, 320), (8, 512, 7168, 384), (2, 16640, 256, 256)])
+def test_gather_inside_the_product(dev, W, m, N, K):
+    """kr_gather_matmul_bf16: the gathered matrix is the shards bit for bit, nothing is written behind it, and the product has
+    the bits of the product of the gathered matrix and of the form with copies and flags; with shards in separate
+    buffers, in one stack, and with a shard in its own place of the gathered matrix."""
+    rank = W - 1
+    g = torch.Generator().manual_seed(N + K)
+    a = (torch.rand(W, m, K, generator=g) - 0.5).to(BF16).to(dev)
+    bT = (torch.rand(N, K, generator=g) - 0.5).to(BF16).to(dev)
+    assert _lib.load().kr_gather_matmul_direct(W, m, N, K) == 1
+    full = a.reshape(W * m, K)
+    _, want = fused.all_gather_matmul(a, bT.T, rank=rank, gather=False)
+    torch.testing.assert_close(want[::97].float(), full[::97].float() @ bT.float().T, **TOL)
+    shards = [t.clone() for t in a]
+    mem = torch.full((W * m * K + 64,), 7.0, dtype=BF16, device=dev)
+    a_out = mem[:W * m * K].view(W * m, K)
+    progress = torch.full((W + 1,), 5, dtype=torch.int32, device=dev)
+    got, c = fused.all_gather_matmul(shards, bT.T, a_out, progress, rank=rank)
+    assert got is a_out and torch.equal(a_out, full) and (mem[W * m * K:] == 7.0).all()
+    assert torch.equal(c, want) and progress.tolist() == [1] * W + [0]
+    got, c = fused.all_gather_matmul(a, bT.T, rank=rank, gather=True)
+    assert torch.equal(got, full) and torch.equal(c, want)
+    got, c = fused.all_gather_matmul(shards, bT.T, rank=rank, copy_engine=True)       # copies and flags
+    assert torch.equal(got, full) and torch.equal(c, want)
+    a_out.zero_()
+    a_out[rank * m:] = shards[rank]
+    shards[rank] = a_out[rank * m:]
+    got, c = fused.all_gather_matmul(shards, bT.T, a_out, rank=rank)
+    assert torch.equal(got, full) and torch.equal(c, want)
+
+
+def test_gather_inside_the_product_is_for_shards_apart(dev):
+    """A shard that lies in another one's place of the gathered matrix, and shards that are not 16-byte aligned, take the
+    copies; shapes of few tiles, or whose shards are no whole tiles, as well."""
+    from kraken_amd.fused.all_gather_matmul import _direct
+    W, m, N, K = 8, 512, 4096, 256
+    a_out, b = torch.zeros(W * m, K, dtype=BF16, device=dev), torch.zeros(N, K, dtype=BF16, device=dev).T
+    size, base = m * K * 2, torch.zeros(W, m, K, dtype=BF16, device=dev).data_ptr()
+    apart = [base + r * size for r in range(W)]
+    shard = a_out[:m]
+    assert _direct(apart, shard, a_out, b, W, m, N, K)
+    assert _direct([a_out.data_ptr()] + apart[1:], shard, a_out, b, W, m, N, K)
+    assert not _direct([a_out.data_ptr() + size] + apart[1:], shard, a_out, b, W, m, N, K)
+    assert not _direct([a_out.data_ptr() - 16] + apart[1:], shard, a_out, b, W, m, N, K)
+    assert not _direct([base + 8] + apart[1:], shard, a_out, b, W, m, N, K)
+    assert not _direct(apart, shard, a_out, b, W, 500, N, K) and not _direct(apart, shard, a_out, b, W, 256, 1024, K)
+
+
 @pytest.mark.parametrize("plan", [None, 0, 3, 4000, 5001, 6000, 7002])
 @pytest.mark.parametrize("M,N,K", [(1, 16, 16), (255, 272, 112), (257, 528, 1040), (300, 1040, 528), (513, 816, 384)])
 def test_fp8_wide_kernel_shapes(dev, monkeypatch, M, N, K, plan):
