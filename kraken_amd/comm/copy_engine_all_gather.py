@@ -8,13 +8,14 @@ import torch
 from .. import _lib
 from ._common import PeerBuffers
 
-# Up to here all copies and flags of a gather are one launch.  What that gives depends on how long the product takes beside
-# the launches of the loop (about 120 us of host time and 9 per chunk).  all_gather_matmul, time in one launch over time
+# Up to here all copies and flags of a gather on a side stream are one launch.  What that gives depends on how long the product
+# beside it takes next to the launches of the loop (about 120 us of host time and 9 per chunk).  Time in one launch over time
 # with a copy and a flag per chunk, 2, 4 and 8 ranks, 4 to 47 MiB, K = 1024 to 8192, N = 1024 to 28672, one and two chunks a rank:
 # a call that is waited for 0.39 to 1.00 at all 216 shapes (W = 8, 1024 x 1024, N = 1024 0.59; N = 28672 0.87); calls one
 # behind the other 0.38 to 0.9 where the launches are the longer part, 0.94 to 1.03 where the product is, up to 1.07 with two
 # or four ranks and N = 7168 (2 x 1024 x 8192 200 -> 215 us, alone 284 -> 260).  Above, copies that come one behind the other leave
 # the product more of the memory (8 x 1024 x 8192, N = 3584 405 / 438 us; the same kernel once per chunk 424).
+# (all_gather_matmul takes this way only for copies that the caller wants on the copy engines, or that one launch cannot take.)
 ONE_LAUNCH_BYTES = 48 << 20
 
 _backend_streams: dict[int, torch.cuda.Stream] = {}
@@ -31,6 +32,20 @@ def _get_backend_stream(dev: torch.device) -> torch.cuda.Stream:
 def _check_progress(progress: torch.Tensor, n: int) -> None:
     assert progress.dtype in (torch.int32, torch.uint32), "progress must be a 32-bit integer tensor"
     assert progress.is_contiguous() and progress.numel() >= n
+
+
+def gather_chunks(output: torch.Tensor, peers: PeerBuffers, progress: torch.Tensor, splits: int, rank: int, stream: int) -> bool:
+    """All chunks and flags in one launch (``kr_gather_chunks``) on the stream given; False, and nothing launched, where
+    addresses or chunks are no multiples of 16 bytes.  Of the arguments' checks only these are made here."""
+    W = peers.W
+    chunk_bytes = peers.cap // splits * output.element_size()
+    sources = peers.pointers()
+    if W > _lib.KR_MAX_WORLD or chunk_bytes % 16 != 0 or output.data_ptr() % 16 != 0 or any(p % 16 != 0 for p in sources):
+        return False
+    rc = _lib.load().kr_gather_chunks((ctypes.c_void_p * W)(*sources), W, splits, rank, chunk_bytes, output.data_ptr(),
+                                      progress.data_ptr(), stream)
+    _lib.check(rc, "gather_chunks")
+    return True
 
 
 def _copy_engine_all_gather_w_progress(
@@ -78,14 +93,11 @@ def _copy_engine_all_gather_w_progress(
     lib = _lib.load()
     chunk = peers.cap // splits_per_rank
     flat_out = output.view(-1)
-    backend_stream.wait_stream(torch.cuda.current_stream(dev))
-    chunk_bytes = chunk * output.element_size()
-    sources = [peers.slice(r).data_ptr() for r in range(W)]
-    if (not copy_engine and chunk_bytes * n_chunks <= ONE_LAUNCH_BYTES and W <= _lib.KR_MAX_WORLD and chunk_bytes % 16 == 0 and output.data_ptr() % 16 == 0
-            and all(p % 16 == 0 for p in sources)):
-        rc = lib.kr_gather_chunks((ctypes.c_void_p * W)(*sources), W, splits_per_rank, rank, chunk_bytes,
-                                  output.data_ptr(), progress.data_ptr(), backend_stream.cuda_stream)
-        _lib.check(rc, "gather_chunks")
+    current = torch.cuda.current_stream(dev)
+    if backend_stream != current:
+        backend_stream.wait_stream(current)
+    if (not copy_engine and output.numel() * output.element_size() <= ONE_LAUNCH_BYTES
+            and gather_chunks(output, peers, progress, splits_per_rank, rank, backend_stream.cuda_stream)):
         return backend_stream
     with torch.cuda.stream(backend_stream):
         for step in range(W):
@@ -110,7 +122,8 @@ def all_gather_w_progress(a_shared, a_out: torch.Tensor | None = None, progress:
     Counterpart of ``all_gather_w_progress``
     (``kraken/comm/copy_engine_all_gather.py:63-120``): allocates ``a_out`` and
     ``progress`` when not given, zeroes ``progress`` (``:108``), runs the chunked
-    copy on the side stream and makes the current stream wait for it.  kwargs:
+    copy.  The current stream would wait for a side stream at once, so the copies run on it
+    (``copy_engine=True``: on the side stream).  kwargs:
     ``splits_per_rank`` (default 1), ``rank`` (default 0), ``copy_engine`` (default False).
     """
     peers = PeerBuffers(a_shared)
@@ -125,7 +138,9 @@ def all_gather_w_progress(a_shared, a_out: torch.Tensor | None = None, progress:
         progress = torch.zeros(peers.W * splits, dtype=torch.int32, device=dev)
     else:
         progress.fill_(0)
-    stream = _copy_engine_all_gather_w_progress(a_out, a_shared, progress, splits, rank=rank,
-                                                copy_engine=kwargs.get("copy_engine", False))
-    torch.cuda.current_stream(dev).wait_stream(stream)
+    copy_engine, current = kwargs.get("copy_engine", False), torch.cuda.current_stream(dev)
+    stream = _copy_engine_all_gather_w_progress(a_out, a_shared, progress, splits, None if copy_engine else current, rank=rank,
+                                                copy_engine=copy_engine)
+    if stream != current:
+        current.wait_stream(stream)
     return a_out

@@ -7,7 +7,7 @@ import torch
 
 from .. import _lib, _waits
 from ..comm._common import PeerBuffers
-from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress
+from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress, gather_chunks
 from . import _gemm
 
 
@@ -40,25 +40,46 @@ def _matmul_w_progress(a, a_local, b, progress, configs, status=None) -> torch.T
     return c
 
 
-def _direct(sources: list[int], shard: torch.Tensor, a_out: torch.Tensor, b: torch.Tensor, W: int, m: int, N: int, K: int) -> bool:
-    """Whether the product gathers the shards itself (``kr_gather_matmul_bf16``): enough large tiles, each inside one
-    shard, and no shard that overlaps the gathered matrix other than in its own place (a tile may read a row
-    after another one has written it)."""
-    if W > _lib.KR_MAX_WORLD or not _lib.load().kr_gather_matmul_direct(W, m, N, K):
-        return False
-    out, size = a_out.data_ptr(), shard.numel() * shard.element_size()
-    if any(p % 16 != 0 for p in (out, b.data_ptr(), *sources)):
-        return False
+def _apart(sources: list[int], a_out: torch.Tensor) -> bool:
+    """No shard overlaps the gathered matrix other than in its own place."""
+    W = len(sources)
+    out, size = a_out.data_ptr(), a_out.numel() * a_out.element_size() // W
     return all(p + size <= out or p >= out + W * size or p == out + r * size for r, p in enumerate(sources))
+
+
+def _direct(sources: list[int], a_out: torch.Tensor, b: torch.Tensor, W: int, m: int, N: int, K: int) -> bool:
+    """Whether the product gathers the shards itself (``kr_gather_matmul_bf16``): enough large tiles, each inside one
+    shard, and shards apart from the gathered matrix (a tile may read a row after another one has written it)."""
+    return (W <= _lib.KR_MAX_WORLD and _lib.load().kr_gather_matmul_direct(W, m, N, K) == 1
+            and all(p % 16 == 0 for p in (a_out.data_ptr(), b.data_ptr(), *sources)) and _apart(sources, a_out))
+
+
+def _gathered_first(a_out, peers: PeerBuffers, progress, splits: int, rank: int, dev) -> bool:
+    """Gather on the current stream in one launch, in front of a product that then waits for nothing and may be any;
+    False, and nothing done, where ``kr_gather_chunks`` does not take the addresses or a shard overlaps the gathered matrix.
+
+    On one GPU nothing is gained by the side stream: its copies wait for compute units of the running product, and
+    its events, flags and status word cost the host 100 us.  Calls one behind the other, us, with the side stream /
+    in front: W = 8, 1 x 1024, N = 1024 125 / 38; 8 x 130 x 8192, N = 8192 205 / 176; 8 x 500 x 4096, N = 6656 232 / 188;
+    8 x 1000 x 8192, N = 1024 286 / 185, N = 3584 450 / 389; 2 x 1000 x 16384, N = 8192 429 / 393."""
+    if not _apart(peers.pointers(), a_out):
+        return False
+    flags = progress
+    if progress is None:
+        flags = torch.empty(peers.W * splits, dtype=torch.int32, device=dev)     # counted in, read by nobody
+    else:
+        _check_progress(progress, peers.W * splits)
+        progress.fill_(0)
+    return gather_chunks(a_out, peers, flags, splits, rank, _lib.current_stream(dev))
 
 
 def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **kwargs):
     """The fp8 branch of ``all_gather_matmul`` (``all_gather_matmul.py:53,121,213``): fp8 product, rounded to
     fp8 once.  Shapes of whole tiles (M, N multiples of 256, K of 128) run on
-    the fp8 matrix-core instruction (``kr_gemm_fp8_ws``, or ``kr_all_gather_matmul_fp8`` for ``gather=True``: the
-    shards are copied chunk by chunk on a side stream while the tiles wait for their chunk's flag, as in the
-    bf16 form); others run on the bf16 instruction, their operands widened in registers (``kr_gemm_fp8_wide_ws``), after
-    the gather has finished.  ``fp8_kernel=False`` forces the widening kernel.
+    the fp8 matrix-core instruction (``kr_gemm_fp8_ws``, or ``kr_all_gather_matmul_fp8`` where ``gather=True`` takes the
+    side stream: the tiles wait for their chunk's flag, as in the
+    bf16 form); others run on the bf16 instruction, their operands widened in registers (``kr_gemm_fp8_wide_ws``).  The
+    shards are gathered in front of it.  ``fp8_kernel=False`` forces the widening kernel.
 
     The two differ in the precision of the sums: the fp8 instruction keeps about 16 bits of them (1.2e-5 in the
     2-norm against 64 bits, K = 128 .. 16384; both the 16x16x32 and the 16x16x128 form, to the same bits), the bf16
@@ -89,29 +110,30 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
             a_out = torch.empty((M, K), dtype=fp8, device=dev)
         else:
             assert tuple(a_out.shape) == (M, K) and a_out.dtype == fp8 and a_out.is_contiguous()
-        if progress is None:
-            progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)
-        else:
-            progress.fill_(0)
-        backend_stream = _copy_engine_all_gather_w_progress(a_out, a_shared, progress, splits, rank=rank,
-                                                            copy_engine=kwargs.get("copy_engine", False))
-        if native:
-            status = kwargs.get("status")
-            own_status = status is None
-            if own_status:
-                status = _waits.new_status(dev)
-            a_local = peers.slice(rank)
-            assert a_local.stride(1) == 1
-            c = torch.empty((M, N), dtype=fp8, device=dev)
-            rc = lib.kr_all_gather_matmul_fp8(
-                a_out.data_ptr(), K, a_local.data_ptr(), a_local.stride(0), b.T.data_ptr(), K, M, N, K, W, rank, splits,
-                progress.data_ptr(), int(kwargs.get("wait_limit_us", 0)), _lib.ptr(status), c.data_ptr(), 2, stream)
-            _lib.check(rc, "all_gather_matmul(fp8)")
-            torch.cuda.current_stream(dev).wait_stream(backend_stream)
-            if own_status:
-                _waits.watch(status, "all_gather_matmul")
-            return a_out, c
-        torch.cuda.current_stream(dev).wait_stream(backend_stream)   # no overlap on the widening path
+        if kwargs.get("copy_engine", False) or not _gathered_first(a_out, peers, progress, splits, rank, dev):
+            if progress is None:
+                progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)
+            else:
+                progress.fill_(0)
+            backend_stream = _copy_engine_all_gather_w_progress(a_out, a_shared, progress, splits, rank=rank,
+                                                                copy_engine=kwargs.get("copy_engine", False))
+            if native:
+                status = kwargs.get("status")
+                own_status = status is None
+                if own_status:
+                    status = _waits.new_status(dev)
+                a_local = peers.slice(rank)
+                assert a_local.stride(1) == 1
+                c = torch.empty((M, N), dtype=fp8, device=dev)
+                rc = lib.kr_all_gather_matmul_fp8(
+                    a_out.data_ptr(), K, a_local.data_ptr(), a_local.stride(0), b.T.data_ptr(), K, M, N, K, W, rank, splits,
+                    progress.data_ptr(), int(kwargs.get("wait_limit_us", 0)), _lib.ptr(status), c.data_ptr(), 2, stream)
+                _lib.check(rc, "all_gather_matmul(fp8)")
+                torch.cuda.current_stream(dev).wait_stream(backend_stream)
+                if own_status:
+                    _waits.watch(status, "all_gather_matmul")
+                return a_out, c
+            torch.cuda.current_stream(dev).wait_stream(backend_stream)   # no overlap on the widening path
         a_full = a_out
     else:
         assert stacked, "gather=False needs the shards as one contiguous [W, m, K] tensor"
@@ -162,7 +184,8 @@ def all_gather_matmul(
       (``kr_gather_matmul_bf16``): tiles read their rows where the shards lie and write what they
       read to ``a_out`` while they multiply; the flags of ``progress`` are set behind it, no tile waits and
       ``status`` is not touched.  8 shards of 1024 x 8192, N = 3584: 397 us with copies and flags, 346 so.
-      Otherwise, and with ``copy_engine=True``,
+      Other shapes are gathered by one launch in front of the product.
+      With ``copy_engine=True``, and where shards are not 16-byte aligned or overlap ``a_out``,
       the shards are copied chunk by chunk into ``a_out`` on a side stream,
       each chunk followed by its flag in ``progress`` (``:308-311``), while the
       GEMM on the current stream consumes them: tiles of the local shard
@@ -173,8 +196,7 @@ def all_gather_matmul(
       ``c`` is then invalid; without ``status`` the wrapper keeps a word of its own
       and the next call of an overlap function (or ``kraken_amd._waits.check()``)
       raises once the failed call has finished.
-      The copies are ordinary copy kernels, which share the compute units with
-      the GEMM; ``copy_engine=True`` hands them to the GPU's copy engines.
+      ``copy_engine=True`` hands the copies to the GPU's copy engines.
 
     In both modes the order of the M tiles is rotated so that the shard of
     ``rank`` (kwarg, default 0) is consumed first and the others in the order
@@ -235,7 +257,7 @@ def all_gather_matmul(
     else:
         assert tuple(a_out.shape) == (M, K) and a_out.dtype == torch.bfloat16 and a_out.is_contiguous()
     sources = peers.pointers()
-    if not kwargs.get("copy_engine", False) and _direct(sources, shard, a_out, b, W, m, N, K):
+    if not kwargs.get("copy_engine", False) and _direct(sources, a_out, b, W, m, N, K):
         if progress is not None:
             _check_progress(progress, W * splits)
             progress.fill_(0)
@@ -245,6 +267,10 @@ def all_gather_matmul(
         _lib.check(rc, "all_gather_matmul")
         if progress is not None:
             progress.view(-1)[:W * splits].fill_(1)
+        return a_out, c
+    if not kwargs.get("copy_engine", False) and _gathered_first(a_out, peers, progress, splits, rank, dev):
+        c = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+        _gemm.launch("all_gather_matmul", a_out, b, M, N, None, 0, 0, None, 0, M, None, c, rank * m)
         return a_out, c
     if progress is None:
         progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)

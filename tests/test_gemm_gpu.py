@@ -369,6 +369,36 @@ def test_all_gather_matmul_overlapped_with_the_copies(dev, tile, rank, splits, a
     assert torch.equal(c, c_plain)
 
 
+@pytest.mark.parametrize("how", ["copy_engine", "misaligned"])
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+def test_all_gather_matmul_on_the_side_stream(dev, tile, how, dtype):
+    """The form with copies and flags on a side stream (asked for, or shards that one launch cannot take): the
+    results of the form that gathers in front of the product, every flag at 1, no wait run out."""
+    from kraken_amd import _waits
+    W, m, K, N, rank, splits = 4, 256, 384, 512, 2, 2
+    dt = BF16 if dtype == "bf16" else torch.float8_e4m3fn
+    g = torch.Generator().manual_seed(3)
+    a = torch.randn(W, m, K, generator=g).to(dt).to(dev)
+    bT = (torch.randn(N, K, generator=g) * 0.05).to(dt).to(dev)
+    bits = torch.int16 if dtype == "bf16" else torch.uint8
+    want_a, want = fused.all_gather_matmul([t.clone() for t in a], bT.T, rank=rank, splits_per_rank=splits)
+    assert torch.equal(want_a.view(bits), a.reshape(W * m, K).view(bits))
+    shards = [t.clone() for t in a]
+    if how == "misaligned":
+        for r in range(W):
+            mem = torch.empty(m * K + 8, dtype=dt, device=dev)
+            shards[r] = mem[4:4 + m * K].view(m, K)
+            shards[r].copy_(a[r])
+        assert all(t.data_ptr() % 16 for t in shards)
+        shards[rank] = a[rank].clone()            # (tiles read the local shard in place)
+    progress = torch.full((W * splits,), 7, dtype=torch.int32, device=dev)
+    got, c = fused.all_gather_matmul(shards, bT.T, None, progress, rank=rank, splits_per_rank=splits, copy_engine=how == "copy_engine")
+    torch.cuda.synchronize()
+    _waits.check(block=True)
+    assert torch.equal(got.view(bits), a.reshape(W * m, K).view(bits)) and (progress == 1).all()
+    assert torch.equal(c.view(bits), want.view(bits))
+
+
 def test_all_gather_w_progress(dev):
     # test/test_allgather.py:50-75: gathered tensor exact, every flag set
     W, m, K = 8, 64, 128
@@ -1286,13 +1316,12 @@ def test_gather_inside_the_product_is_for_shards_apart(dev):
     a_out, b = torch.zeros(W * m, K, dtype=BF16, device=dev), torch.zeros(N, K, dtype=BF16, device=dev).T
     size, base = m * K * 2, torch.zeros(W, m, K, dtype=BF16, device=dev).data_ptr()
     apart = [base + r * size for r in range(W)]
-    shard = a_out[:m]
-    assert _direct(apart, shard, a_out, b, W, m, N, K)
-    assert _direct([a_out.data_ptr()] + apart[1:], shard, a_out, b, W, m, N, K)
-    assert not _direct([a_out.data_ptr() + size] + apart[1:], shard, a_out, b, W, m, N, K)
-    assert not _direct([a_out.data_ptr() - 16] + apart[1:], shard, a_out, b, W, m, N, K)
-    assert not _direct([base + 8] + apart[1:], shard, a_out, b, W, m, N, K)
-    assert not _direct(apart, shard, a_out, b, W, 500, N, K) and not _direct(apart, shard, a_out, b, W, 256, 1024, K)
+    assert _direct(apart, a_out, b, W, m, N, K)
+    assert _direct([a_out.data_ptr()] + apart[1:], a_out, b, W, m, N, K)
+    assert not _direct([a_out.data_ptr() + size] + apart[1:], a_out, b, W, m, N, K)
+    assert not _direct([a_out.data_ptr() - 16] + apart[1:], a_out, b, W, m, N, K)
+    assert not _direct([base + 8] + apart[1:], a_out, b, W, m, N, K)
+    assert not _direct(apart, a_out, b, W, 500, N, K) and not _direct(apart, a_out, b, W, 256, 1024, K)
 
 
 @pytest.mark.parametrize("plan", [None, 0, 3, 4000, 5001, 6000, 7002])
