@@ -100,6 +100,17 @@ def _readable_in_place(bands: list[torch.Tensor], written: list[torch.Tensor]) -
     return all(hi <= r_lo or r_hi <= lo for lo, hi in map(_byte_range, written) for r_lo, r_hi in reads)
 
 
+def _sends_direct(sent, a: torch.Tensor, b: torch.Tensor, world_size: int, m_per_rank: int, N: int) -> bool:
+    """Whether the GEMM may store the other ranks' bands in ``sent`` itself: one matrix of contiguous bands, apart from
+    the operands, and nothing autograd would have to know of."""
+    if not (isinstance(sent, torch.Tensor) and tuple(sent.shape) == (world_size, m_per_rank, N) and sent.is_contiguous()
+            and sent.dtype == a.dtype and sent.device == a.device and sent.data_ptr() % 16 == 0
+            and not sent.requires_grad):
+        return False
+    lo, hi = _byte_range(sent)
+    return all(hi <= t_lo or t_hi <= lo for t_lo, t_hi in (_byte_range(a), _byte_range(b)))
+
+
 def _reduce_bands(bands: list[torch.Tensor], rows: int, N: int, output: torch.Tensor, configs: dict) -> torch.Tensor:
     """``reduce`` of W bands in buffers of their own."""
     dev = _lib.require_device(output, *bands)
@@ -182,7 +193,9 @@ def gemm_reduce_scatter_ce_persistent(
     GEMM writes the full bf16 ``C = a @ b`` on the current stream and flags every
     band as it completes; with the kwarg ``sent`` (``[W, M/W, N]`` tensor or sequence) a side
     stream, which first waits for the current stream (``:345-346``), copies the flagged band of
-    every other rank r to ``sent[r]`` (``:367-368``).  What the other ranks would push is in the
+    every other rank r to ``sent[r]`` (``:367-368``).  A contiguous ``sent`` tensor takes no copies: the GEMM
+    stores the other ranks' bands there, nothing is flagged or waited for, and ``wait_limit_us`` and ``status``
+    stay unused.  What the other ranks would push is in the
     pre-staged ``peers`` (kwarg, ``[W-1, M/W, N]`` or a sequence, the other ranks in ascending
     order).  The reduce (``:258-279``) sums the W bands starting at ``rank + 1`` and reads them where
     they are, the peers in their own buffers and the own band in ``C``, instead of through a
@@ -204,16 +217,21 @@ def gemm_reduce_scatter_ce_persistent(
     assert P == world_size - 1
     dev = _lib.require_device(a, b)
     _waits.check()      # an earlier call's failed wait is reported before anything of this call is enqueued
-    gemm_out = torch.empty((M, N), dtype=a.dtype, device=dev)
     output = torch.empty((m_per_rank, N), dtype=a.dtype, device=dev)
     configs = {"RANK": rank, "WORLD_SIZE": world_size, "fp32_acc": kwargs.get("fp32_acc", False)}
     if M == 0 or N == 0:
         return output
     sent = kwargs.get("sent")
     dests = [None if sent is None or r == rank else sent[r] for r in range(world_size)]
-    bands = list(peers) if peers is not None else []
-    bands.insert(rank, gemm_out[rank * m_per_rank:(rank + 1) * m_per_rank])
     written = [t for t in dests if t is not None]
+    direct = bool(written) and not kwargs.get("copy_engine", False) and _sends_direct(sent, a, b, world_size, m_per_rank, N)
+    if direct:
+        gemm_out, own = None, torch.empty((m_per_rank, N), dtype=a.dtype, device=dev)
+    else:
+        gemm_out = torch.empty((M, N), dtype=a.dtype, device=dev)
+        own = gemm_out[rank * m_per_rank:(rank + 1) * m_per_rank]
+    bands = list(peers) if peers is not None else []
+    bands.insert(rank, own)
 
     if not _readable_in_place(bands, written):
         scatter_out = torch.empty((world_size, m_per_rank, N), dtype=a.dtype, device=dev)
@@ -221,6 +239,17 @@ def gemm_reduce_scatter_ce_persistent(
             if r != rank:
                 scatter_out[r].copy_(t)
                 bands[r] = scatter_out[r]
+    # Destinations that make up one matrix: the GEMM stores every tile where it has to go, the own band in a buffer of its
+    # own (the reduce-scatter epilogue without peers), and may be any.  On one GPU the copies find compute units only as
+    # the last tiles end, and their order costs the product its best tile order.  W = 8, all bands sent, us, copies
+    # behind the bands' flags (one round of tiles: behind the GEMM) / stores of the GEMM:
+    # 8192 x 4096 x 14336 735 / 658, 8192 x 8192 x 3584 (row-major B) 434 / 363, 4096 x 4096 x 4096 120 / 103,
+    # 2704 x 2816 x 2304 71 / 56, 8 x 1600 x 768 73 / 58.
+    if direct:
+        _gemm.launch("gemm_reduce_scatter_ce_persistent", *_gemm.prepare_operands(a, b), M, N, None, 0, 0, None,
+                     rank * m_per_rank, m_per_rank, sent.view(M, N), own, ((rank + 1) % world_size) * m_per_rank)
+        torch.autograd.graph.increment_version(sent)
+        return _reduce_bands(bands, m_per_rank, N, output, configs)
     # One round of tiles or less: all bands finish together, so they leave behind the GEMM in stream order, without
     # flags, and the GEMM may be any (W = 8, 2048 x 4096 x 4096 with all bands sent: 219 us with a wait and a copy per
     # band on a side stream, 74 us with two copies).

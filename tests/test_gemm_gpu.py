@@ -967,6 +967,46 @@ def test_ce_reduce_reads_the_bands_in_place(dev, M, N, K, form):
     assert torch.equal(out, fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers.to(dev), rank=rank, sent=list(plain)))
 
 
+# bands of whole tiles; of parts of one; of 1 row; K loop in parts; few rows; more than a round, bands inside a tile
+@pytest.mark.parametrize("M,N,K,W", [(1024, 512, 256, 4), (600, 1048, 264, 4), (8, 1024, 512, 8), (504, 776, 4096, 8), (40, 2048, 1024, 2),
+                                     (2320, 8192, 128, 8)])
+@pytest.mark.parametrize("b_t", [False, True])
+def test_ce_bands_stored_by_the_product(dev, M, N, K, W, b_t):
+    """Destinations in one matrix: the product stores the bands there itself.  Integers up to 4 times integers up to 2
+    are exact in every order of the sums (K * 8 < 2^24), so bands and result are those of the product rounded once."""
+    g = torch.Generator().manual_seed(M)
+    a = torch.randint(-4, 5, (M, K), generator=g).to(BF16)
+    b = torch.randint(-2, 3, (K, N), generator=g).to(BF16)
+    m = M // W
+    ad, bd = a.to(dev), b.T.contiguous().to(dev).T if b_t else b.to(dev)
+    c = (a.float() @ b.float()).to(BF16)
+    for rank in (0, W - 1):
+        peers = torch.stack([orc.randn_bf16((m, N), 100 + j, 30.0) for j in range(W - 1)])
+        sent = torch.full((W, m, N), float("nan"), dtype=BF16, device=dev)
+        version = sent._version
+        out = fused.gemm_reduce_scatter_ce_persistent(ad, bd, peers=peers.to(dev), rank=rank, sent=sent)
+        assert sent._version > version
+        for r in range(W):
+            assert torch.isnan(sent[r]).all() if r == rank else torch.equal(sent[r].cpu(), c[r * m:(r + 1) * m]), (rank, r)
+        bands = list(peers)
+        bands.insert(rank, c[rank * m:(rank + 1) * m])
+        assert torch.equal(out.cpu(), orc.reduce_rotated(torch.cat(bands, 0), W, rank, acc_bf16=True))
+
+
+def test_ce_bands_sent_over_an_operand(dev):
+    """Destinations in the memory of the left operand (its rows are those of the product, N = K): not stored by the
+    product, which still reads them, but copied behind it."""
+    M, N, K, W, rank = 512, 256, 256, 4, 1
+    a, b, peers = mk(M, N, K, W - 1, True, seed=4)
+    a, b, peers = a.to(dev), b.to(dev), peers[:, :M // W].contiguous().to(dev)
+    apart = torch.zeros(W, M // W, N, dtype=BF16, device=dev)
+    want = fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers, rank=rank, sent=apart)
+    out = fused.gemm_reduce_scatter_ce_persistent(a, b, peers=peers, rank=rank, sent=a.view(W, M // W, N))
+    assert torch.equal(out, want)
+    for r in range(W):
+        assert r == rank or torch.equal(a.view(W, M // W, N)[r], apart[r])
+
+
 @pytest.mark.parametrize("M,N,K", [(512, 1024, 256), (2048, 8192, 256)])   # bands together; one by one
 @pytest.mark.parametrize("form", ["expanded", "list"])
 def test_ce_bands_sent_into_one_scratch_band(dev, M, N, K, form):
