@@ -23,7 +23,7 @@ import time
 
 import torch
 
-from ._lib import KrakenAmdError
+from ._lib import KrakenAmdError, current_stream
 
 _lock = threading.Lock()
 # (event behind the mirror copy, pinned host mirror, device word, what, the stream the work is on)
@@ -44,7 +44,7 @@ def new_status(dev: torch.device, stream_handle: int | None = None) -> torch.Ten
     has run out and has not been reported yet).  Every wait of one call shares it: the first wait
     that runs out makes the later ones give up at once instead of each running to the limit."""
     if stream_handle is None:
-        stream_handle = torch.cuda.current_stream(dev).cuda_stream
+        stream_handle = current_stream(dev)
     key = (dev.index if dev.index is not None else torch.cuda.current_device(), stream_handle)
     with _lock:
         word = _words.get(key)
@@ -58,10 +58,14 @@ def watch(status: torch.Tensor, what: str, min_interval_s: float = 0.0) -> None:
     """Register ``status`` to be read once everything enqueued so far on the current stream is done.
     ``min_interval_s`` > 0: skip the registration if this word was registered less than that long
     ago (for calls of a few microseconds; the word is sticky, so a later look still finds a failure)."""
+    now = 0.0
+    if min_interval_s > 0.0:
+        now = time.monotonic()
+        if now - _last_watch.get(id(status), -1e30) < min_interval_s:
+            return      # (the common case of short calls; looked at again below, under the lock)
     if torch.cuda.is_current_stream_capturing():
         return          # a captured call cannot be read back here; its caller passes a status of its own
     if min_interval_s > 0.0:
-        now = time.monotonic()
         with _lock:
             if now - _last_watch.get(id(status), -1e30) < min_interval_s:
                 return

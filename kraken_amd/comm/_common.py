@@ -10,7 +10,7 @@ from .. import _lib, _waits
 
 
 class PeerBuffers:
-    """The W buffers a reduce reads: one per rank, all on this GPU.
+    """The W buffers a reduce reads: one per rank, all on this GPU (``shape``: of one of them).
 
     Stands in for the peers' symmetric-memory buffers of the reference
     (``symm_mem_hdl.buffer_ptrs_dev``, ``kraken/comm/one_shot_all_reduce.py:96-99``).
@@ -37,19 +37,24 @@ class PeerBuffers:
             self.stride = buffers.stride(0) if self.W > 1 else self.cap
             self.stacked = buffers
             self.tensors = [buffers]
+            self.shape = buffers.shape[1:]
         else:
             bufs = list(buffers)
             assert len(bufs) >= 1, "expected W >= 1 buffers"
+            assert isinstance(bufs[0], torch.Tensor), "expected a tensor or a sequence of tensors"
+            dtype, shape = bufs[0].dtype, bufs[0].shape
+            assert dtype in dtypes, "Only bfloat16 is supported for now."
             for t in bufs:
                 assert isinstance(t, torch.Tensor), "expected a tensor or a sequence of tensors"
-                assert t.dtype in dtypes and t.dtype == bufs[0].dtype, "Only bfloat16 is supported for now."
+                assert t.dtype == dtype, "Only bfloat16 is supported for now."
                 assert t.is_contiguous(), "each of the W buffers must be contiguous"
-                assert t.shape == bufs[0].shape, "the W buffers must have one shape"
+                assert t.shape == shape, "the W buffers must have one shape"
             self.W = len(bufs)
             self.cap = bufs[0].numel()
             self.stride = None
             self.stacked = None
             self.tensors = bufs
+            self.shape = bufs[0].shape
 
     def slice(self, rank: int) -> torch.Tensor:
         """Buffer of rank ``rank``."""
@@ -99,10 +104,7 @@ class PeerBuffers:
             rc = lib.kr_reduce_rmsnorm_ptrs_ws_bf16(self._table(0), self.W, rows, D, bias_ptr, bias_is_vector,
                                                     w_ptr, eps, y_ptr, ws_ptr, ws_bytes, _lib.ptr(status), stream)
         if status is not None and rc == 0:
-            # (the word is sticky and these calls take microseconds: mirroring it to the host now and
-            # then is enough to report a time-out, every call would cost more than the kernel)
-            _waits.watch(status, "reduce + RMSNorm of a few long rows (rows spread over many compute units)",
-                         min_interval_s=0.05)
+            row_watch(status)
         return rc
 
 
@@ -125,6 +127,18 @@ def row_workspace(dev: torch.device, nbytes: int, stream_handle: int) -> torch.T
         entry = (torch.zeros(nbytes, dtype=torch.uint8, device=dev), torch.cuda.current_stream(dev))
         _row_workspaces[key] = entry
     return entry[0]
+
+
+def row_exchange(index: int, nbytes: int, stream_handle: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """Workspace and status word of the split-row kernel for a device index and stream."""
+    dev = torch.device("cuda", index)
+    return row_workspace(dev, nbytes, stream_handle), _waits.new_status(dev, stream_handle)
+
+
+def row_watch(status: torch.Tensor) -> None:
+    # (the word is sticky and these calls take microseconds: mirroring it to the host now and
+    # then is enough to report a time-out, every call would cost more than the kernel)
+    _waits.watch(status, "reduce + RMSNorm of a few long rows (rows spread over many compute units)", min_interval_s=0.05)
 
 
 def _zero_row_workspaces() -> None:
@@ -182,6 +196,7 @@ class _Sources(PeerBuffers):
         self.stride = None
         self.stacked = None
         self.tensors = peers.tensors
+        self.shape = peers.shape
         self._pointers = pointers
 
     def pointers(self) -> list[int]:

@@ -83,10 +83,10 @@ def _copy_engine_all_gather_w_progress(
     assert peers.cap % splits_per_rank == 0
     n_chunks = W * splits_per_rank
     _check_progress(progress, n_chunks)
-    out_shape = list(peers.slice(0).shape)
+    out_shape = list(peers.shape)
     out_shape[0] *= W
     assert list(output.shape) == out_shape, (list(output.shape), out_shape)
-    assert output.is_contiguous() and output.dtype == peers.slice(0).dtype
+    assert output.is_contiguous() and output.dtype == peers.tensors[0].dtype
     dev = _lib.require_device(*peers.tensors, output, progress)
     if backend_stream is None:
         backend_stream = _get_backend_stream(dev)
@@ -130,7 +130,7 @@ def all_gather_w_progress(a_shared, a_out: torch.Tensor | None = None, progress:
     splits = kwargs.get("splits_per_rank", 1)
     rank = kwargs.get("rank", 0)
     dev = _lib.require_device(*peers.tensors)
-    shape = list(peers.slice(0).shape)
+    shape = list(peers.shape)
     shape[0] *= peers.W
     if a_out is None:
         a_out = torch.empty(shape, dtype=torch.bfloat16, device=dev)

@@ -22,11 +22,14 @@ def one_shot_all_reduce(tensor, **kwargs) -> torch.Tensor:
     ``max_num_blocks``, ``num_warps`` and ``BLOCK_SIZE`` are accepted for
     signature compatibility and ignored: the launch is sized to fill the GPU.
     """
+    out = _lib.calls().all_reduce(tensor)
+    if out is not None:
+        return out
     peers = check_stack(tensor)
     numel = peers.cap
     assert numel % 8 == 0, "The number of elements must be 128-bit aligned."
     dev = _lib.require_device(*peers.tensors)
-    out = torch.empty(peers.slice(0).shape, dtype=torch.bfloat16, device=dev)
+    out = torch.empty(peers.shape, dtype=torch.bfloat16, device=dev)
     rc = peers.reduce(0, numel, None, 0, 0, 1, out.data_ptr(), _lib.current_stream(dev))
     _lib.check(rc, "one_shot_all_reduce")
     return out

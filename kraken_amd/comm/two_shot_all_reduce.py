@@ -7,12 +7,10 @@ from .. import _lib
 from ._common import check_stack
 
 
-def _share_rows(one: torch.Tensor, rank: int, W: int) -> tuple[int, int, tuple[int, ...]]:
-    """Contiguous 1/W chunk of a slice ``one``: (offset, numel, shape)."""
-    numel = one.numel()
+def _share_rows(shape: tuple[int, ...], numel: int, rank: int, W: int) -> tuple[int, int, tuple[int, ...]]:
+    """Contiguous 1/W chunk of a slice of the given shape: (offset, numel, shape)."""
     assert numel % W == 0, "the number of elements must be divisible by the world size"
     share = numel // W
-    shape = tuple(one.shape)
     if len(shape) >= 1 and shape[0] % W == 0:
         out_shape = (shape[0] // W, *shape[1:])
     else:
@@ -41,19 +39,23 @@ def two_shot_all_reduce(tensor, **kwargs) -> torch.Tensor:
     ``tensor`` is the ``[W, ...]`` stack or a list of W separate tensors.
     ``max_num_blocks`` and ``num_warps`` are accepted and ignored.
     """
-    peers = check_stack(tensor)
-    W, numel = peers.W, peers.cap
-    assert numel % 8 == 0, "The number of elements must be 128-bit aligned."
     rank = kwargs.get("rank", 0)
     layout = kwargs.get("layout", "rows")
     block = kwargs.get("BLOCK_SIZE", 2048)
+    if layout in ("rows", "striped"):
+        out = _lib.calls().two_shot_share(tensor, rank, layout == "striped", block)
+        if out is not None:
+            return out
+    peers = check_stack(tensor)
+    W, numel = peers.W, peers.cap
+    assert numel % 8 == 0, "The number of elements must be 128-bit aligned."
     assert block % W == 0, "BLOCK_SIZE must be divisible by world_size for two-shot all-reduce"
     assert layout in ("rows", "striped")
     dev = _lib.require_device(*peers.tensors)
     lib = _lib.load()
     stream = _lib.current_stream(dev)
     if rank is None:
-        out = torch.empty(peers.slice(0).shape, dtype=torch.bfloat16, device=dev)
+        out = torch.empty(peers.shape, dtype=torch.bfloat16, device=dev)
         rc = peers.reduce(0, numel, None, 0, 0, 0, out.data_ptr(), stream)
         _lib.check(rc, "two_shot_all_reduce")
         return out
@@ -65,7 +67,7 @@ def two_shot_all_reduce(tensor, **kwargs) -> torch.Tensor:
         rc = peers.reduce_striped(numel, None, block, rank, out.data_ptr(), stream)
         _lib.check(rc, "two_shot_all_reduce")
         return out
-    off, share, out_shape = _share_rows(peers.slice(0), rank, W)
+    off, share, out_shape = _share_rows(peers.shape, numel, rank, W)
     assert share % 8 == 0, "each rank's share must be 128-bit aligned"
     out = torch.empty(out_shape, dtype=torch.bfloat16, device=dev)
     rc = peers.reduce(off, share, None, 0, 0, 0, out.data_ptr(), stream)

@@ -122,11 +122,15 @@ def workspace(dev: torch.device, nbytes: int) -> torch.Tensor | None:
     buffer per stream keeps calls on different streams from sharing one)."""
     if nbytes <= 0:
         return None
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(dev).cuda_stream)
+    return stream_workspace(dev.index if dev.index is not None else torch.cuda.current_device(), nbytes, _lib.current_stream(dev))
+
+
+def stream_workspace(index: int, nbytes: int, stream: int) -> torch.Tensor:
+    """``workspace`` for a device index and the handle of its current stream."""
+    key = (index, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=torch.device("cuda", index))
         _workspaces[key] = ws
     return ws
 
@@ -211,6 +215,6 @@ def check_peers(peers, rows: int, N: int) -> tuple[int, int]:
     assert peers.dim() == 3 and tuple(peers.shape[1:]) == (rows, N), (
         f"peers must have shape [W-1, {rows}, {N}], got {tuple(peers.shape)}"
     )
-    assert peers[0].is_contiguous()
     P = peers.shape[0]
+    assert (P > 0 and peers.is_contiguous()) or peers[0].is_contiguous()
     return P, (peers.stride(0) if P > 1 else rows * N)

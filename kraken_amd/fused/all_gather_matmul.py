@@ -87,7 +87,7 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
     take them: 4000 x 6656 x 4096 takes 83 us there and 146 us here, with 5e-4 of the results one fp8 step off."""
     fp8 = torch.float8_e4m3fn
     W = peers.W
-    m, K = peers.slice(0).shape
+    m, K = peers.shape
     assert b.dtype == fp8, "fp8 shards need an fp8 b"
     assert b.dim() == 2 and b.shape[0] == K
     if not b.T.is_contiguous():
@@ -215,13 +215,12 @@ def all_gather_matmul(
     """
     fp8 = torch.float8_e4m3fn
     peers = PeerBuffers(a_shared, dtypes=(torch.bfloat16, fp8))
-    if peers.slice(0).dtype == fp8:
+    if peers.tensors[0].dtype == fp8:
         return _all_gather_matmul_fp8(a_shared, peers, b, a_out, progress, **kwargs)
     W = peers.W
-    shard = peers.slice(0)
-    assert shard.dim() == 2, "expected shards of shape [m, K]"
+    assert len(peers.shape) == 2, "expected shards of shape [m, K]"
     assert b.dtype == torch.bfloat16, "Only bfloat16 is supported for now."
-    m, K = shard.shape
+    m, K = peers.shape
     assert b.dim() == 2 and b.shape[0] == K
     if not b.T.is_contiguous():
         raise ValueError("b.T must be contiguous")
@@ -244,9 +243,11 @@ def all_gather_matmul(
             a_out = a_full
         if progress is not None:
             progress.fill_(1)
-        a2, b2 = _gemm.prepare_operands(a_full, b)
-        c = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-        _gemm.launch("all_gather_matmul", a2, b2, M, N, None, 0, 0, None, 0, M, None, c, rank * m)
+        c = _lib.calls().gemm(a_full, b, None, None, None, 0, M, False, rank * m)
+        if c is None:
+            a2, b2 = _gemm.prepare_operands(a_full, b)
+            c = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+            _gemm.launch("all_gather_matmul", a2, b2, M, N, None, 0, 0, None, 0, M, None, c, rank * m)
         return a_out, c
 
     assert K % 8 == 0, "K must be a multiple of 8"
@@ -269,8 +270,10 @@ def all_gather_matmul(
             progress.view(-1)[:W * splits].fill_(1)
         return a_out, c
     if not kwargs.get("copy_engine", False) and _gathered_first(a_out, peers, progress, splits, rank, dev):
-        c = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-        _gemm.launch("all_gather_matmul", a_out, b, M, N, None, 0, 0, None, 0, M, None, c, rank * m)
+        c = _lib.calls().gemm(a_out, b, None, None, None, 0, M, False, rank * m)
+        if c is None:
+            c = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+            _gemm.launch("all_gather_matmul", a_out, b, M, N, None, 0, 0, None, 0, M, None, c, rank * m)
         return a_out, c
     if progress is None:
         progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)

@@ -3,6 +3,7 @@ from __future__ import annotations
 
 import torch
 
+from .. import _lib
 from . import _gemm
 
 
@@ -25,12 +26,16 @@ def gemm_one_shot_all_reduce(a: torch.Tensor, b: torch.Tensor, **kwargs) -> torc
     ``group``, ``BLOCK_SIZE_M/N/K``, ``GROUP_SIZE_M``, ``num_warps`` and
     ``num_stages`` are accepted and ignored.
     """
-    a, b = _gemm.prepare_operands(a, b, keep_fp32=True)
-    M, N = a.shape[0], b.shape[1]
-    assert N % 8 == 0, "N must be a multiple of 8"
     peers = kwargs.get("peers")
     bias = kwargs.get("bias")
     out_dtype = kwargs.get("out_dtype", torch.float32)
+    if out_dtype in (torch.float32, torch.bfloat16):
+        out = _lib.calls().gemm(a, b, peers, bias, None, 0, a.shape[0] if a.dim() == 2 else 0, out_dtype == torch.float32, 0)
+        if out is not None:
+            return out
+    a, b = _gemm.prepare_operands(a, b, keep_fp32=True)
+    M, N = a.shape[0], b.shape[1]
+    assert N % 8 == 0, "N must be a multiple of 8"
     assert out_dtype in (torch.float32, torch.bfloat16)
     P, pstride = _gemm.check_peers(peers, M, N)
     if bias is not None:

@@ -86,8 +86,8 @@ def _one_round(dev: torch.device, M: int, N: int) -> bool:
 
 def _byte_range(t: torch.Tensor) -> tuple[int, int]:
     """First and past-the-last byte a tensor's elements lie in."""
-    if t.numel() == 0:
-        return t.data_ptr(), t.data_ptr()
+    if t.is_contiguous():
+        return t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()
     last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
     return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
 
@@ -111,15 +111,32 @@ def _sends_direct(sent, a: torch.Tensor, b: torch.Tensor, world_size: int, m_per
     return all(hi <= t_lo or t_hi <= lo for t_lo, t_hi in (_byte_range(a), _byte_range(b)))
 
 
-def _reduce_bands(bands: list[torch.Tensor], rows: int, N: int, output: torch.Tensor, configs: dict) -> torch.Tensor:
-    """``reduce`` of W bands in buffers of their own."""
-    dev = _lib.require_device(output, *bands)
+def _stacked_peers_apart(peers, sent: torch.Tensor, rows: int, N: int) -> list[int] | None:
+    """Addresses of the peers' bands where they come as one tensor that the reduce may read in place whatever is
+    written to ``sent``; ``None`` where that needs a closer look (a view per band costs the host more than the launch)."""
+    if not isinstance(peers, torch.Tensor) or peers.device != sent.device:
+        return None
+    base, step, P = peers.data_ptr(), 2 * peers.stride(0), peers.shape[0]
+    end, (lo, hi) = base + (P - 1) * step + 2 * rows * N, _byte_range(sent)
+    if base % 16 != 0 or step % 16 != 0 or (base < hi and lo < end):
+        return None
+    return [base + r * step for r in range(P)]
+
+
+def _reduce_sources(sources: list[int], rows: int, N: int, output: torch.Tensor, configs: dict) -> torch.Tensor:
+    """``reduce`` of W bands given by their addresses, all on the device of ``output``."""
     rc = _lib.load().kr_reduce_rotated_ptrs_bf16(
-        (ctypes.c_void_p * len(bands))(*[t.data_ptr() for t in bands]), len(bands), rows, N, configs["RANK"],
-        int(not configs["fp32_acc"]), output.data_ptr(), _lib.current_stream(dev),
+        (ctypes.c_void_p * len(sources))(*sources), len(sources), rows, N, configs["RANK"],
+        int(not configs["fp32_acc"]), output.data_ptr(), _lib.current_stream(output.device),
     )
     _lib.check(rc, "gemm_reduce_scatter_ce_persistent")
     return output
+
+
+def _reduce_bands(bands: list[torch.Tensor], rows: int, N: int, output: torch.Tensor, configs: dict) -> torch.Tensor:
+    """``reduce`` of W bands in buffers of their own."""
+    _lib.require_device(output, *bands)
+    return _reduce_sources([t.data_ptr() for t in bands], rows, N, output, configs)
 
 
 def copy_engine_scatter(
@@ -222,16 +239,34 @@ def gemm_reduce_scatter_ce_persistent(
     if M == 0 or N == 0:
         return output
     sent = kwargs.get("sent")
+    # Destinations that make up one matrix: the GEMM stores every tile where it has to go, the own band in a buffer of its
+    # own (the reduce-scatter epilogue without peers), and may be any.  On one GPU the copies find compute units only as
+    # the last tiles end, and bands that finish one by one cost the product its best tile order.  W = 8, all bands sent, us, copies
+    # behind the bands' flags (one round of tiles: behind the GEMM) / stores of the GEMM:
+    # 8192 x 4096 x 14336 735 / 658, 8192 x 8192 x 3584 (row-major B) 434 / 363, 4096 x 4096 x 4096 120 / 103,
+    # 2704 x 2816 x 2304 71 / 56, 8 x 1600 x 768 73 / 58.
+    direct = world_size > 1 and not kwargs.get("copy_engine", False) and _sends_direct(sent, a, b, world_size, m_per_rank, N)
+    if direct:
+        pivot = ((rank + 1) % world_size) * m_per_rank
+        sources = _stacked_peers_apart(peers, sent, m_per_rank, N)
+        if sources is None:
+            bands = list(peers)
+            if not _readable_in_place([a, *bands], [sent[r] for r in range(world_size) if r != rank]):
+                bands = [torch.empty((m_per_rank, N), dtype=a.dtype, device=dev).copy_(t) for t in bands]
+            sources = [t.data_ptr() for t in bands]
+        own = _lib.calls().gemm(a, b, None, None, sent.view(M, N), rank * m_per_rank, m_per_rank, False, pivot)
+        if own is None:
+            own = torch.empty((m_per_rank, N), dtype=a.dtype, device=dev)
+            _gemm.launch("gemm_reduce_scatter_ce_persistent", *_gemm.prepare_operands(a, b), M, N, None, 0, 0, None,
+                         rank * m_per_rank, m_per_rank, sent.view(M, N), own, pivot)
+        torch.autograd.graph.increment_version(sent)
+        sources.insert(rank, own.data_ptr())
+        return _reduce_sources(sources, m_per_rank, N, output, configs)
     dests = [None if sent is None or r == rank else sent[r] for r in range(world_size)]
     written = [t for t in dests if t is not None]
-    direct = bool(written) and not kwargs.get("copy_engine", False) and _sends_direct(sent, a, b, world_size, m_per_rank, N)
-    if direct:
-        gemm_out, own = None, torch.empty((m_per_rank, N), dtype=a.dtype, device=dev)
-    else:
-        gemm_out = torch.empty((M, N), dtype=a.dtype, device=dev)
-        own = gemm_out[rank * m_per_rank:(rank + 1) * m_per_rank]
+    gemm_out = torch.empty((M, N), dtype=a.dtype, device=dev)
     bands = list(peers) if peers is not None else []
-    bands.insert(rank, own)
+    bands.insert(rank, gemm_out[rank * m_per_rank:(rank + 1) * m_per_rank])
 
     if not _readable_in_place(bands, written):
         scatter_out = torch.empty((world_size, m_per_rank, N), dtype=a.dtype, device=dev)
@@ -239,17 +274,6 @@ def gemm_reduce_scatter_ce_persistent(
             if r != rank:
                 scatter_out[r].copy_(t)
                 bands[r] = scatter_out[r]
-    # Destinations that make up one matrix: the GEMM stores every tile where it has to go, the own band in a buffer of its
-    # own (the reduce-scatter epilogue without peers), and may be any.  On one GPU the copies find compute units only as
-    # the last tiles end, and their order costs the product its best tile order.  W = 8, all bands sent, us, copies
-    # behind the bands' flags (one round of tiles: behind the GEMM) / stores of the GEMM:
-    # 8192 x 4096 x 14336 735 / 658, 8192 x 8192 x 3584 (row-major B) 434 / 363, 4096 x 4096 x 4096 120 / 103,
-    # 2704 x 2816 x 2304 71 / 56, 8 x 1600 x 768 73 / 58.
-    if direct:
-        _gemm.launch("gemm_reduce_scatter_ce_persistent", *_gemm.prepare_operands(a, b), M, N, None, 0, 0, None,
-                     rank * m_per_rank, m_per_rank, sent.view(M, N), own, ((rank + 1) % world_size) * m_per_rank)
-        torch.autograd.graph.increment_version(sent)
-        return _reduce_bands(bands, m_per_rank, N, output, configs)
     # One round of tiles or less: all bands finish together, so they leave behind the GEMM in stream order, without
     # flags, and the GEMM may be any (W = 8, 2048 x 4096 x 4096 with all bands sent: 219 us with a wait and a copy per
     # band on a side stream, 74 us with two copies).

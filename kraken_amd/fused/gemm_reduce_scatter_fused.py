@@ -3,7 +3,18 @@ from __future__ import annotations
 
 import torch
 
+from .. import _lib
 from . import _gemm
+
+
+def _common_form(a, b, peers=None, rank=0, world_size=None, c_scratch=None, **_) -> torch.Tensor | None:
+    """The call in native code where its arguments are of the common form: all peers in one tensor, a scratch to write to."""
+    if not (isinstance(peers, torch.Tensor) and isinstance(c_scratch, torch.Tensor) and a.dim() == 2):
+        return None
+    W, M = len(peers) + 1, len(a)
+    if world_size not in (None, W) or M % W != 0 or not 0 <= rank < W:
+        return None
+    return _lib.calls().gemm(a, b, peers, None, c_scratch, rank * (M // W), M // W, False, rank * (M // W))
 
 
 def gemm_reduce_scatter(a: torch.Tensor, b: torch.Tensor, **kwargs) -> torch.Tensor:
@@ -28,6 +39,9 @@ def gemm_reduce_scatter(a: torch.Tensor, b: torch.Tensor, **kwargs) -> torch.Ten
     Returns ``[M/W, N]`` in ``a.dtype``.  Tile-size kwargs are ignored.
     """
     in_dtype = a.dtype
+    out = _common_form(a, b, **kwargs)
+    if out is not None:
+        return out
     a, b = _gemm.prepare_operands(a, b, keep_fp32=True)
     M, N = a.shape[0], b.shape[1]
     assert N % 8 == 0, "N must be a multiple of 8"

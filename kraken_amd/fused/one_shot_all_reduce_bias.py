@@ -38,6 +38,8 @@ def one_shot_all_reduce_bias(
     """
     if symm_mem_buffer is None:
         raise ValueError("symm_mem_buffer much be a valid symmetric memory tensor.")
+    if not stage and _lib.calls().all_reduce_bias(symm_mem_buffer, input_tensor, bias, output, rank):
+        return
     peers = check_stack(symm_mem_buffer)
     W, cap = peers.W, peers.cap
     ref = input_tensor if input_tensor is not None else output

@@ -14,6 +14,9 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float = 1.0e-5) -> torch.Ten
     Counterpart of ``kraken.fused.rms_norm`` (``kraken/fused/rms_norm.py:46-72``;
     arithmetic ``:34-43``).
     """
+    y = _lib.calls().rms_norm(x, w, eps)
+    if y is not None:
+        return y
     D = x.shape[-1]
     assert w.is_contiguous()
     assert w.shape == (D,)

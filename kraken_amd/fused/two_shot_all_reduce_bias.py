@@ -40,6 +40,9 @@ def two_shot_all_reduce_bias(
     copies it into slice ``rank`` first, the reference's copy-in ``:43-50``), else ``numel`` if passed, else ``bias.numel()`` for a
     full-shape bias, else the slice size.  Returns ``output``.
     """
+    if not stage and layout in ("rows", "striped") and _lib.calls().two_shot_bias(
+            symm_mem_input, input_tensor, bias, output, BLOCK_SIZE, rank, layout == "striped", numel):
+        return output
     peers = check_stack(symm_mem_input)
     W, cap = peers.W, peers.cap
     assert BLOCK_SIZE % W == 0
@@ -57,8 +60,7 @@ def two_shot_all_reduce_bias(
     assert n % 8 == 0, "The number of elements must be 128-bit aligned."
     assert n <= cap, "the message does not fit in one slice of the stacked buffer"
     assert output.dtype == torch.bfloat16 and output.is_contiguous()
-    ref = input_tensor if input_tensor is not None else peers.slice(0)
-    D = ref.shape[-1]
+    D = (input_tensor.shape if input_tensor is not None else peers.shape)[-1]
     if bias is not None:
         assert bias.dtype == torch.bfloat16 and bias.is_contiguous()
     dev = _lib.require_device(*peers.tensors, input_tensor, bias, output)

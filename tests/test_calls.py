@@ -1,0 +1,167 @@
+"""The native form of the common calls (csrc/calls.cpp) against the general path: the same results and the same errors,
+whichever of the two takes a call."""
+import itertools
+
+import pytest
+import torch
+
+from kraken_amd import _lib, comm, fused
+from oracle import oracle as orc
+
+BF16 = torch.bfloat16
+FUNCTIONS = {"all_reduce": 1, "all_reduce_bias": 5, "two_shot_share": 4, "two_shot_bias": 8, "reduce_rms_norm": 7, "rms_norm": 3, "gemm": 9}
+
+
+class _General:
+    """Stands in for the native module: takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+@pytest.mark.parametrize("name", FUNCTIONS)
+def test_what_is_not_of_the_common_form_is_left_to_the_general_path(name):
+    fn, n = getattr(_lib.calls(), name), FUNCTIONS[name]
+    host = torch.zeros(2, 8, dtype=BF16)
+    sub = host.as_subclass(type("Sub", (torch.Tensor,), {}))
+    for value in (host, sub, None, [host, host], 1, 1.0, "x", host.to_sparse(), host.to("meta")):
+        for count in (n, n - 1, n + 1, 0):
+            assert fn(*[value] * count) is None
+
+
+def _both(monkeypatch, call):
+    """``call()`` as it is and through the general path: two results, or two exceptions' types."""
+    got = []
+    for general in (False, True):
+        with monkeypatch.context() as m:
+            if general:
+                _lib.calls()
+                m.setattr(_lib, "_calls", _General())
+            try:
+                got.append(call())
+            except Exception as e:        # noqa: BLE001 (the type is what is compared)
+                got.append(type(e))
+    return got
+
+
+def _same(monkeypatch, call, what):
+    one, two = _both(monkeypatch, call)
+    if isinstance(one, type) or isinstance(two, type):
+        assert one is two, (what, one, two)
+        return False
+    for x, y in zip(one, two, strict=True):
+        assert x.shape == y.shape and x.stride() == y.stride() and x.dtype == y.dtype, what
+        assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), what
+    return True
+
+
+def _stacks(dev, W, rows, D):
+    """Forms a stack comes in: contiguous, with room behind each slice, strided, transposed, a list, of another type, misaligned."""
+    g = torch.Generator(device=dev).manual_seed(W * rows + D)
+    big = torch.randn(W, rows + 2, D, generator=g, device=dev).to(BF16)
+    plain = big[:, :rows].contiguous()
+    yield "plain", plain
+    yield "roomy", big
+    yield "strided", big[:, :rows]
+    yield "transposed", plain.transpose(1, 2).contiguous().transpose(1, 2)
+    yield "list", list(plain)
+    yield "fp32", plain.float()
+    yield "misaligned", torch.cat([torch.zeros(1, dtype=BF16, device=dev), plain.flatten()])[1:].view(W, rows, D)
+    yield "flat", plain.view(W, rows * D)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,rows,D", [(1, 3, 64), (2, 8, 1024), (3, 6, 136), (8, 16, 8192), (8, 8, 512), (16, 4, 72), (17, 2, 64), (4, 5, 20), (2, 1, 4096)])
+def test_row_calls_take_both_paths_alike(dev, monkeypatch, W, rows, D):
+    g = torch.Generator(device=dev).manual_seed(7)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(BF16)      # noqa: E731
+    x, full, vec, w = rnd(rows, D), rnd(rows, D), rnd(D), rnd(D)
+    xs = {"none": None, "own": x, "wide": rnd(rows, 2 * D)[:, :D], "off": rnd(rows * D + 1)[1:].view(rows, D), "fp32": x.float(), "short": x[:1],
+          "column": rnd(D, rows).T}
+    ok = 0
+    for (form, stack), (xf, xv), (bf, bias), rank in itertools.product(
+            _stacks(dev, W, rows, D), xs.items(), {"none": None, "full": full, "vec": vec, "bad": rnd(D + 8)}.items(), (0, W - 1, W)):
+        if rank == W and (xf, bf) != ("none", "vec"):
+            continue
+        what = (form, xf, bf, rank)
+
+        def rms():
+            y = torch.empty(rows, D, dtype=BF16, device=dev)
+            fused.one_shot_all_reduce_bias_rms_norm(stack, xv, bias, w, y, rank=rank)
+            return [y]
+
+        def one_shot():
+            out = torch.empty(rows, D, dtype=BF16, device=dev)
+            fused.one_shot_all_reduce_bias(stack, xv, bias, out, rank=rank)
+            return [out]
+
+        ok += _same(monkeypatch, rms, ("rms", what)) + _same(monkeypatch, one_shot, ("bias", what))
+        for layout, block, numel in (("rows", 48 * W, None), ("striped", 48 * W, rows * D), ("striped", 8 * W, None), ("rows", 16, rows * D), ("other", 16, None)):
+            sizes = {rows * D, rows * D // W, rows * D // W + 8}
+            if layout == "striped" and rows * D % 8 == 0 and W <= 16 and rank < W:
+                sizes.add(max(8, _lib.load().kr_striped_share_numel(rows * D, W, block, rank)))
+            for size in sizes:
+                def two_shot():
+                    out = torch.zeros(size, dtype=BF16, device=dev)
+                    return [fused.two_shot_all_reduce_bias(stack, xv, bias, out, BLOCK_SIZE=block, rank=rank, layout=layout, numel=numel)]
+
+                _same(monkeypatch, two_shot, ("two-shot", what, layout, block, numel, size))
+        if (xf, bf) == ("none", "none"):
+            ok += _same(monkeypatch, lambda: [comm.one_shot_all_reduce(stack)], what)
+            for layout, block in (("rows", 2048), ("striped", 8 * W), ("striped", 2048), ("other", 8 * W)):
+                _same(monkeypatch, lambda: [comm.two_shot_all_reduce(stack, rank=rank, layout=layout, BLOCK_SIZE=block)], (what, layout, block))
+    assert (ok > 0) == (W <= 16 and D % 8 == 0)
+    for v in (x, xs["wide"], xs["off"], xs["column"], x.float(), x[:0]):
+        for wv in (w, w[:-8], w.float(), rnd(2 * D)[::2]):
+            _same(monkeypatch, lambda: [fused.rms_norm(v, wv)], ("rms_norm", v.shape, v.stride(), wv.shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,W", [(8, 256, 128, 4), (1, 64, 72, 2), (512, 264, 4096, 8), (40, 20, 64, 2), (24, 64, 60, 3), (32, 128, 64, 1)])
+def test_products_take_both_paths_alike(dev, monkeypatch, M, N, K, W):
+    g = torch.Generator(device=dev).manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(BF16)      # noqa: E731
+    a, b = rnd(M, K), rnd(K, N)
+    left = {"plain": a, "wide": rnd(M, 2 * K)[:, :K], "column": rnd(K, M).T, "off": rnd(M * K + 1)[1:].view(M, K), "fp32": a.float(), "odd": rnd(M, K + 1)[:, :K]}
+    right = {"rows": b, "columns": rnd(N, K).T, "wide": rnd(K, 2 * N)[:, :N], "off": rnd(K * N + 1)[1:].view(K, N), "fp32": b.float(), "long": rnd(K + 8, N)}
+    ok = 0
+    for (af, av), (bf, bv) in itertools.product(left.items(), right.items()):
+        for rows, fn in ((M, "ar"), (M // W, "rs")):
+            whole = rnd(max(W - 1, 1), rows, N)
+            for pf, pv in {"none": None, "stack": whole[:W - 1], "list": list(whole[:W - 1]), "gap": rnd(max(W - 1, 1), rows + 1, N)[:W - 1, :rows],
+                           "fp32": whole.float(), "flat": whole.flatten(1)}.items():
+                what = (af, bf, fn, pf)
+                if fn == "ar":
+                    for bias, dtype in ((None, BF16), (rnd(N), torch.float32), (rnd(N).float(), BF16), (rnd(1, N), BF16), (None, torch.float16)):
+                        ok += _same(monkeypatch, lambda: [fused.gemm_one_shot_all_reduce_fused(av, bv, peers=pv, bias=bias, out_dtype=dtype)], (what, dtype))
+                else:
+                    for rank, kw in ((0, {}), (W - 1, {"world_size": W}), (W, {}), (0, {"world_size": W + 1})):
+                        def rs():
+                            c = torch.zeros(M, N, dtype=BF16, device=dev)
+                            return [fused.gemm_reduce_scatter(av, bv, peers=pv, rank=rank, c_scratch=c, **kw), c]
+
+                        ok += _same(monkeypatch, rs, (what, rank, kw))
+    assert (ok > 0) == (N % 8 == 0)
+
+
+@pytest.mark.gpu
+def test_native_calls_run_on_the_current_stream_and_in_a_graph(dev):
+    stack, w = orc.make_stack(8, (16, 8192)).to(dev), torch.ones(8192, dtype=BF16, device=dev)
+    y = torch.empty(16, 8192, dtype=BF16, device=dev)
+    want = orc.reduce_bias_rms_norm(stack.cpu(), torch.zeros(8192, dtype=BF16), w.cpu())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        fused.one_shot_all_reduce_bias_rms_norm(stack, None, None, w, y)     # the stream's workspace, outside the capture
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            fused.one_shot_all_reduce_bias_rms_norm(stack, None, None, w, y)
+            out = comm.one_shot_all_reduce(stack)
+    for _ in range(3):
+        y.zero_()
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        torch.testing.assert_close(y.cpu(), want, rtol=2e-2, atol=2e-2)
+        assert torch.equal(out.cpu(), orc.reduce(stack.cpu()))
