@@ -36,8 +36,7 @@ __device__ __forceinline__ void add_group(const LOAD& at, int r0, float (&acc)[k
 
 // The same for all W buffers of a run-time W: groups of eight, and what is left in one group of its size (the
 // branches are uniform).  One buffer at a time is a chain of W round trips to memory: W = 16 on 1024 x 8192
-// 48.2 -> 43.4 us, W = 3 on 4096 x 4096 24.1 -> 22.4, W = 6 on 1000 x 5120 15.3 -> 14.3 (the striped kernel keeps the
-// simple loop: with eight loads together W = 8 on 16384 x 8192 goes from 47.4 to 49.6 us).
+// 48.2 -> 43.4 us, W = 3 on 4096 x 4096 24.1 -> 22.4, W = 6 on 1000 x 5120 15.3 -> 14.3.
 template <int kUnroll, class LOAD>
 __device__ __forceinline__ void add_all(const LOAD& at, int W, float (&acc)[kUnroll][8]) {
     int r = 0;
@@ -129,31 +128,52 @@ __global__ __launch_bounds__(kThreads) void reduce_kernel(
 
 // Striped ownership: output vector j (compact) comes from input vector
 //   (j / blk_v) * blk_v * W + rank * blk_v + (j % blk_v).
-template <class SRC>
-__global__ __launch_bounds__(kThreads) void reduce_striped_kernel(
-    const SRC src, int W, int64_t share_nvec,
+// One vector per thread in single-wave workgroups.  TOGETHER: all of a thread's loads are requested before the first add; one
+// after the other they are a chain of W round trips to memory, which is what a share of up to some thousand
+// workgroups takes (kernel time, W = 8, chain / together: 256 x 4096 6.0 / 2.35 us, 2047 x 5120 with a bias 7.6 / 5.7, 8000 x 5120 19.6 / 17.8).
+// Above kChainVecs the chip is full of waves either way, and with W = 8 the chain keeps HBM a little busier (16384 x 8192 48.1 /
+// 49.3; W = 4 and 2 level).  256 threads a workgroup are 1 to 3 % slower in both forms at 16384 rows.
+constexpr int kStripedThreads = kWave;
+constexpr int64_t kChainVecs = 1 << 20;
+
+template <class SRC, int WT, bool TOGETHER>
+__global__ __launch_bounds__(kStripedThreads) void reduce_striped_kernel(
+    const SRC src, int w_rt, int64_t share_nvec,
     const u32x4* __restrict__ bias, uint32_t blk_v, int rank, u32x4* __restrict__ out) {
-    const int64_t j = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    const int W = WT > 0 ? WT : w_rt;
+    const int64_t j = (int64_t)blockIdx.x * kStripedThreads + threadIdx.x;
     if (j >= share_nvec) return;
     const int64_t stripe = j / blk_v;
     const int64_t i = (stripe * W + rank) * blk_v + (j - stripe * blk_v);
-    float acc[8];
-    zero8(acc);
-    add8(ld_stream(src.at(0) + i), acc);
-    for (int r = 1; r < W; ++r) add8(ld_stream(src.at(r) + i), acc);
-    if (bias != nullptr) add8(ld_stream(bias + i), acc);
-    st_stream(out + j, pack8(acc));
+    float acc[1][8];
+    zero8(acc[0]);
+    u32x4 bv = {0, 0, 0, 0};
+    if constexpr (TOGETHER) {
+        if (bias != nullptr) bv = ld_stream(bias + i);
+        add_all<1>([&](int r, int) { return ld_stream(src.at(r) + i); }, W, acc);
+    } else {
+#pragma unroll 1
+        for (int r = 0; r < W; ++r) add8(ld_stream(src.at(r) + i), acc[0]);
+        if (bias != nullptr) bv = ld_stream(bias + i);
+    }
+    if (bias != nullptr) add8(bv, acc[0]);
+    st_stream(out + j, pack8(acc[0]));
 }
 
 // Rotated-order tile reduce of the copy-engine reduce-scatter variant:
 // out[v] = sum_i band_{(i + rank + 1) % W}[v], optionally rounding
 // the running sum to bf16 after every add.  Up to eight bands are requested together.  The bands are
 // the slices of one tensor or buffers of their own (SRC, common.h), so what the other ranks sent is read where it is.
-template <class SRC, bool ACC_BF16>
-__global__ __launch_bounds__(kThreads) void reduce_rotated_kernel(
-    const SRC src, int W, int64_t band_v, int rank, u32x4* __restrict__ out) {
+// W known at compile time and single-wave workgroups: no branch between the requests (kernel time, W = 8: 1 x 1600 2.6 -> 2.3 us,
+// 18 x 1728 2.8 -> 2.5, 1024 x 4096 level, 1024 x 8192 28.4 -> 27.4).
+constexpr int kRotatedThreads = kWave;
+
+template <class SRC, bool ACC_BF16, int WT>
+__global__ __launch_bounds__(kRotatedThreads) void reduce_rotated_kernel(
+    const SRC src, int w_rt, int64_t band_v, int rank, u32x4* __restrict__ out) {
+    const int W = WT > 0 ? WT : w_rt;
     constexpr int G = 8;
-    const int64_t v = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    const int64_t v = (int64_t)blockIdx.x * kRotatedThreads + threadIdx.x;
     if (v >= band_v) return;
     float acc[8];
     const int first = (rank + 1) % W;
@@ -327,10 +347,17 @@ static int launch_striped(const SRC& tab, int W, int64_t share, const void* bias
                           int rank, void* out, void* stream) {
     if (bias != nullptr && !aligned16(bias)) return KR_ERR_ALIGNMENT;
     const int64_t nvec = share / 8;
-    const int64_t blocks = (nvec + kThreads - 1) / kThreads;
+    const int64_t blocks = (nvec + kStripedThreads - 1) / kStripedThreads;
     if (blocks > 0x7fffffffLL || stripe_block / 8 > 0xffffffffLL) return KR_ERR_BAD_DIM;
-    hipLaunchKernelGGL(reduce_striped_kernel<SRC>, dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, tab,
-                       W, nvec, (const u32x4*)bias, (uint32_t)(stripe_block / 8), rank, (u32x4*)out);
+#define KR_LAUNCH(WT, TOGETHER)                                                                                                   \
+    hipLaunchKernelGGL((reduce_striped_kernel<SRC, WT, TOGETHER>), dim3((unsigned)blocks), dim3(kStripedThreads), 0, (hipStream_t)stream, tab, \
+                       W, nvec, (const u32x4*)bias, (uint32_t)(stripe_block / 8), rank, (u32x4*)out)
+    if (nvec > kChainVecs) KR_LAUNCH(0, false);
+    else if (W == 8) KR_LAUNCH(8, true);
+    else if (W == 4) KR_LAUNCH(4, true);
+    else if (W == 2) KR_LAUNCH(2, true);
+    else KR_LAUNCH(0, true);
+#undef KR_LAUNCH
     return (int)hipGetLastError();
 }
 
@@ -361,14 +388,24 @@ extern "C" int kr_reduce_striped_ptrs_bf16(const void* const* bufs, int W, int64
 
 template <class SRC>
 static int launch_rotated(const SRC& src, int W, int64_t band_v, int rank, int acc_bf16, void* out, void* stream) {
-    const int64_t blocks = (band_v + kThreads - 1) / kThreads;
+    const int64_t blocks = (band_v + kRotatedThreads - 1) / kRotatedThreads;
     if (blocks > 0x7fffffffLL) return KR_ERR_BAD_DIM;
-    if (acc_bf16)
-        hipLaunchKernelGGL((reduce_rotated_kernel<SRC, true>), dim3((unsigned)blocks), dim3(kThreads), 0,
-                           (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);
-    else
-        hipLaunchKernelGGL((reduce_rotated_kernel<SRC, false>), dim3((unsigned)blocks), dim3(kThreads), 0,
-                           (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);
+#define KR_LAUNCH(WT)                                                                                                                       \
+    do {                                                                                                                                    \
+        if (acc_bf16)                                                                                                                       \
+            hipLaunchKernelGGL((reduce_rotated_kernel<SRC, true, WT>), dim3((unsigned)blocks), dim3(kRotatedThreads), 0,                    \
+                               (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);                                                     \
+        else                                                                                                                                \
+            hipLaunchKernelGGL((reduce_rotated_kernel<SRC, false, WT>), dim3((unsigned)blocks), dim3(kRotatedThreads), 0,                   \
+                               (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);                                                     \
+    } while (0)
+    switch (W) {
+        case 2: KR_LAUNCH(2); break;
+        case 4: KR_LAUNCH(4); break;
+        case 8: KR_LAUNCH(8); break;
+        default: KR_LAUNCH(0); break;
+    }
+#undef KR_LAUNCH
     return (int)hipGetLastError();
 }
 

@@ -233,6 +233,47 @@ def test_rotated_band_reduce(dev):
             assert same_bits(out, orc.reduce_rotated(inp, W, rank, acc_bf16=not fp32_acc))
 
 
+@pytest.mark.parametrize("W", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("numel", [8, 504, 8 * 64 * 9, 8 * 1001])
+def test_striped_and_rotated_reduce_by_world_size(dev, W, numel):
+    """Sums of one vector per thread, W known to the kernel or not, less and more than a wavefront: bit for bit, infinities, NaN and
+    negative zeros among the inputs."""
+    from kraken_amd.fused.gemm_reduce_scatter_ce_persistent import reduce as rotated_reduce
+
+    def alike(x, y):       # (which NaN it is, is not stated)
+        x, nan = x.cpu().flatten(), y.flatten().isnan()
+        return torch.equal(x.isnan(), nan) and same_bits(x[~nan], y.flatten()[~nan])
+
+    stack = orc.make_stack(W, (numel,))
+    stack[:, 3], stack[0, 5], stack[W - 1, 6] = -0.0, float("inf"), float("nan")
+    bias = orc.randn_bf16((numel,), 9)
+    for rank in {0, W // 2, W - 1}:
+        for b in (None, bias):
+            idx = orc.striped_indices(numel, W, 8 * W, rank)
+            out = torch.empty(idx.numel(), dtype=BF16, device=dev)
+            if idx.numel():
+                fused.two_shot_all_reduce_bias(stack.to(dev), None, None if b is None else b.to(dev), out, BLOCK_SIZE=8 * W, rank=rank,
+                                               layout="striped", numel=numel)
+            if out.numel() != numel:
+                assert alike(out, orc.reduce_striped(stack, b, 8 * W, rank))
+        for fp32_acc in (False, True):
+            got = torch.empty(1, numel, dtype=BF16, device=dev)
+            rotated_reduce(stack.to(dev), got, {"RANK": rank, "WORLD_SIZE": W, "fp32_acc": fp32_acc})
+            assert alike(got, orc.reduce_rotated(stack, W, rank, acc_bf16=not fp32_acc))
+
+
+@pytest.mark.parametrize("more", [0, 8])      # the largest share whose loads go out together, and one vector more
+def test_striped_share_at_a_million_vectors(dev, more):
+    W, rank, block = 2, 0, 2048
+    numel = W * 8 * (1 << 20) + more
+    g = torch.Generator(device=dev).manual_seed(3)
+    stack = torch.randn(W, numel, generator=g, device=dev).to(BF16)
+    share = comm.two_shot_all_reduce(stack, rank=rank, layout="striped", BLOCK_SIZE=block)
+    assert share.numel() == 8 * (1 << 20) + more
+    idx = torch.from_numpy(orc.striped_indices(numel, W, block, rank).numpy()).to(dev)
+    assert torch.equal(share, (stack[0, idx].float() + stack[1, idx].float()).to(BF16))
+
+
 def test_full_size_config2(dev):
     """benchmark config 2: stack [8,4096,4096] -> [4096,4096], and the two-shot 1/8 row chunk.
     Checked exactly against the oracle on sampled row bands, and by linearity on the whole."""
