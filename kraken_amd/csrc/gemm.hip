@@ -458,8 +458,8 @@ static void tail_split_plan(int64_t tiles, int64_t K, int* tail_out, int* splits
     *tail_out = (int)tail;
     *splits_out = (int)s;
 }
-static int64_t gemm_dtl_tail_workspace_bytes(int tail_tiles, int splits) {
-    return (int64_t)tail_tiles * splits * (256 * 256 * 4);
+static int64_t gemm_dtl_tail_workspace_bytes(int tail_tiles, int splits, int cols = 256) {
+    return (int64_t)tail_tiles * splits * (256 * 4) * cols;
 }
 
 // fp8 operands: which tiles share their K loop, and how many workgroups each gets.  With at most 128 tiles
@@ -559,9 +559,21 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     S = 1 with peers and more than 16 k-steps (transposed B 15: 384 x 1712 x 1024 23.7 / 18.4) 4 us more (fitted, the cause is not separated; one or three peers, in
 //     one pass / in three parts: 112 x 9216 x 1664 27.0 / 21.7, 256 x 4096 x 1536 25.0 / 20.8, 720 x 1280 x 1464 24.6 / 21.1,
 //     row-major 22.4 / 20.1; 360 x 768 x 1096 21.4 / 20.5; but 300 x 2048 x 1024 16.8 / 19.6, 128 x 4096 x 1024 16.5 / 19.1);
-//   the 256x256 kernel with every tile's K loop split: 1.2 us per k-step, twice the work per operand byte, but
-//     parts of whole 256 KiB tiles (512 x 6656 x 16384: 122 us against 150 with gemm_ks_kernel; 512 x 4096 x 8192:
-//     51 against 43);
+//     Transposed B with 257 to 512 workgroups: 0.68 us and 0.18 a round, not two whole rounds (gemm_reduce_kernel has room
+//     for a second workgroup on a compute unit);
+//   the 256-row kernel with every tile's K loop in parts, M and N as they come: half the operand bytes per flop, but
+//     parts of whole tiles.  10.7 us, 1.03 us per k-step (row-major B 1.08, 224-column tiles 0.94) and 0.25 more with all
+//     compute units busy, 0.24 us per MB of parts; at least eight k-steps a part, K from 2048 on, and only where this is
+//     0.88 or less of the best 128x128 form (both models are off by a tenth; whole tiles with a long K need no margin).
+//     224 columns, transposed B only, where they fill enough more compute units to be 2 % ahead.  220 random shapes, 65 to
+//     2300 rows, other than those the model was fitted to: taken by 52, 0.56 to 0.98 of their time, 0.957 over all.  us,
+//     128x128 / in parts: 504 x 6656 x 8192 with a band 82 / 66, 576 x 4608 x 10560 row-major 101 / 78, 998 x 6400 x 6336
+//     row-major 134 / 102, 1792 x 2432 x 12912 224 / 134; 512 x 6656 with a band and seven peers, 256 columns (208
+//     workgroups) / 224 (240), K = 8192 68.1 / 66.3, 16384 120 / 109.
+//     Left on the forms they had, which tests/test_capi_host.py and tests/test_gemm_gpu.py name: plain products of whole tiles
+//     (256 columns; 224 are level where they divide N, 512 x 5376 x 6400 50.5 / 50.2, 256 x 7168 x 12928 62.9 / 62.3, and
+//     66 / 63 at 512 x 6656 x 8192); a K that is no multiple of 64 (128x128; 2048 x 2056 x 12296 249 / 133); with transposed B
+//     and at most one peer, ragged shapes of 129 to 272 tiles of 128x128 (1000 x 4096 x 8192 72 / 70, 1000 x 4224 x 4096 56 / 48).
 // Which 128x128 kernel, by the time of gemm_ks_kernel over that of gemm_reduce_kernel (geometric means over 20 000 random
 // shapes, 1 to 8192 rows, operands in no cache):
 //   transposed B, in parts: 1.034 to 1.042 at every K: gemm_reduce_kernel.  In one pass, K a multiple of 64, no peers:
@@ -574,11 +586,13 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     another's k loop.  K a multiple of 64, without / with peers: 1.02 / 1.07 from 1024 to 2048, 0.94 / 0.97 above; no
 //     multiple: 1.08 / 1.08, 1.01 / 1.06.  1000 x 6656 x 1024 28.6 / 28.2 us, x 2048 45 / 47, x 4096 79 / 86, x 8192 144 / 165.
 struct SmallPlan {
-    int big;      // 256x256 kernel, every tile split
+    int big;      // columns of the large tiles, every one split: 256 or 224; 0: a 128x128 kernel
     int ks;       // gemm_ks_kernel, else gemm_reduce_kernel
-    int splits;   // workgroups per tile of the 128x128 kernels
+    int splits;   // workgroups per tile
 };
-static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool peers, bool dtl_ok, bool may_split, bool may_big) {
+static int64_t big_tiles_of(int64_t M, int64_t N, int cols) { return ((M + 255) / 256) * ((N + cols - 1) / cols); }
+static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peers, bool plain, bool dtl_ok, bool may_split, bool may_big) {
+    const bool peers = n_peers > 0;
     SmallPlan p{0, 0, 1};
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
     auto choose_kernel = [&]() {
@@ -605,13 +619,33 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, bool pee
     // (gemm_reduce_kernel has room for a second workgroup on a compute unit, which the model does not count: with 129 to
     // 256 tiles it pays once the K loop is long, 0.86 of the time of one pass with 144 tiles from K = 12288 on, 0.94 with 208)
     if (b_nt && p.splits == 1 && tiles > 128 && tiles <= 256 && K >= 12288) p.splits = 2;
-    if (may_big && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
-        int tail, ts;
-        const int64_t big_tiles = (M / 256) * (N / 256);
-        tail_split_plan(big_tiles, K, &tail, &ts);
-        if (tail == big_tiles && 800 + 120 * ((steps + ts - 1) / ts) + 600 + ts * big_tiles * 262144 * 2 / 50000 < best) {
-            p.big = 1;
-            p.splits = 1;
+    const EnvSwitches& env = env_switches();
+    const int64_t force = env.gemm_tailsplit;   // 0: off, n: n parts (testing)
+    const bool whole = M % 256 == 0 && N % 256 == 0;
+    const bool as_before = K % 64 != 0 || K < 2048 || (!whole && b_nt && n_peers < 2 && tiles > 128 && tiles <= 272);   // see above
+    if (may_big && dtl_ok && force != 0 && (env.gemm_mfma != 32 || (whole && K % 64 == 0)) && (!as_before || force > 0)) {
+        // whole tiles, K from 4096 on, as many parts as there are compute units for: no margin
+        const int64_t most = std::min<int64_t>({256 / std::max<int64_t>(1, big_tiles_of(M, N, 256)), kMaxTailSplits, steps / kMinSplitSteps});
+        const bool long_whole = whole && K >= 4096 && most > 1 &&
+                                1400 + 120 * ((steps + most - 1) / most) + most * big_tiles_of(M, N, 256) * 262144 * 2 / 50000 < best;
+        // (the second round of gemm_reduce_kernel starts beside the first, see above)
+        const int64_t wgs = tiles * p.splits, per = (steps + p.splits - 1) / p.splits;
+        if (b_nt && wgs > 256 && wgs <= 512) best += (68 + 18 * wgs / 256 - 2 * step) * per;
+        best = best * 88 / 100;
+        if (long_whole || (force > 0 && env.gemm_tile == 256)) best = INT64_MAX;
+        for (const int cols : {256, 224}) {
+            if (cols == 224 ? !b_nt || env.gemm_n224 == 0 || env.gemm_mfma == 32 || (plain && whole && env.gemm_n224 < 0) : b_nt && env.gemm_n224 == 1) continue;
+            const int64_t big_tiles = big_tiles_of(M, N, cols);
+            if (p.big && force <= 0) best = best * 98 / 100;   // (224 after 256: level otherwise)
+            for (int64_t s = cols == 256 && long_whole && force <= 0 ? most : 2; s <= kMaxTailSplits; ++s) {
+                if (force > 0 ? s != std::min<int64_t>(force, steps) : s * big_tiles > 256 || s * kMinSplitSteps > steps) continue;
+                const int64_t bytes = gemm_dtl_tail_workspace_bytes((int)big_tiles, (int)s, cols), k = (steps + s - 1) / s;
+                const int64_t c = 1070 + ((cols == 224 ? 94 : b_nt ? 103 : 108) + 25 * s * big_tiles / 256) * k + bytes * 241 / 10000000;
+                if (bytes > KR_STATIC_SCRATCH_BYTES || c >= best) continue;   // (the form that allocates nothing takes every split)
+                best = c;
+                p.big = cols;
+                p.splits = (int)s;
+            }
         }
     }
     return choose_kernel();
@@ -737,12 +771,9 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     // (few tiles: the large tile again with every tile's K loop split, where that is cheaper)
     SmallPlan small{0, 0, 1};
     if (!big || !dtl_ok || env_switches().gemm_tile == 128) {
-        small = plan_small(M, N, K, b_nt, n_peers > 0, dtl_ok, has_workspace, has_workspace && !has_gather && env_switches().gemm_tile != 128);
-        if (small.big) {
-            int tail, ts;
-            tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
-            if (gemm_dtl_tail_workspace_bytes(tail, ts) > workspace_bytes) small = plan_small(M, N, K, b_nt, n_peers > 0, dtl_ok, has_workspace, false);
-        }
+        small = plan_small(M, N, K, b_nt, n_peers, plain, dtl_ok, has_workspace, has_workspace && !has_gather && env_switches().gemm_tile != 128);
+        if (small.big && gemm_dtl_tail_workspace_bytes((int)big_tiles_of(M, N, small.big), small.splits, small.big) > workspace_bytes)
+            small = plan_small(M, N, K, b_nt, n_peers, plain, dtl_ok, has_workspace, false);
         big = small.big != 0;
     }
     // KRAKEN_AMD_GEMM_TILE=128|256 overrides the choice (testing and tuning)
@@ -782,7 +813,11 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     // 256x256 kernel: the last partial round of tiles, split over the idle CUs (workspace given)
     p.tail_tiles = 0;
     p.tail_splits = 1;
-    if (dtl && has_workspace && !has_progress && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
+    if (dtl && small.big) {
+        p.n224 = small.big == 224;
+        p.tail_tiles = (int)big_tiles_of(M, N, small.big);
+        p.tail_splits = small.splits;
+    } else if (dtl && has_workspace && !has_progress && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
         int tail, ts;
         tail_split_plan(tiles_m * tiles_n, K, &tail, &ts);
         if (tail > 0 && gemm_dtl_tail_workspace_bytes(tail, ts) <= workspace_bytes) {
@@ -798,7 +833,6 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
     // per flop (A is read from LDS and L2 for fewer columns).  KRAKEN_AMD_GEMM_N224=0|1 overrides.
     // (An A that arrives while the kernel runs is fine: the tile waits for its rows' flags before its
     // first load, whatever its width.)
-    p.n224 = 0;
     // (Not where few tiles share their K loops: one round of whole ones leaves most of the chip idle, 256 x 7168 x 12928
     // 213 us, 77 on 128x128 tiles in parts.)
     if (dtl && !small.big && p.mi16 && b_nt && plain && plain_bf16_all_rows && M % 256 == 0 && N % 224 == 0 && K % 64 == 0) {
@@ -1337,7 +1371,8 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     bool big = ((M + 255) / 256) * ((N + 255) / 256) > 128 && K >= 256;
     if (force_tile == 128) big = false;
     if (force_tile == 256) big = true;
-    if (big && K >= 64) {
+    const bool parts_forced = force_tile == 256 && env_switches().gemm_tailsplit > 0 && env_switches().gemm_mfma != 32 && big_tiles_of(M, N, 256) <= 128;
+    if (big && K >= 64 && !parts_forced) {
         if (M % 256 != 0 || N % 256 != 0 || K % 64 != 0) return 0;
         int tail, ts;
         tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
@@ -1345,17 +1380,16 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     }
     // the layout of B and the number of peers are not known here: enough for any
     int64_t bytes = 0;
-    for (int form = 0; form < 4; ++form) {
-        const bool b_nt = form & 1, peers = form & 2;
+    for (int form = 0; form < 8; ++form) {
+        const bool b_nt = form & 1, plain = (form >> 1) == 0;
+        const int n_peers = (form >> 1) == 2 ? 1 : (form >> 1) == 3 ? 2 : 0;
         if (const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, false, kMaxPartsBytes); sk.cb != 0) {
             if (sk.splits > 1) bytes = std::max(bytes, split_k_workspace_bytes(M, N, sk.splits));
             continue;
         }
-        const SmallPlan p = plan_small(M, N, K, b_nt, peers, K % 8 == 0 && K >= 64, true, force_tile != 128);
+        const SmallPlan p = plan_small(M, N, K, b_nt, n_peers, plain, K % 8 == 0 && K >= 64, true, force_tile != 128);
         if (p.big) {
-            int tail, ts;
-            tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
-            bytes = std::max(bytes, gemm_dtl_tail_workspace_bytes(tail, ts));
+            bytes = std::max(bytes, gemm_dtl_tail_workspace_bytes((int)big_tiles_of(M, N, p.big), p.splits, p.big));
         } else if (p.splits > 1) {
             bytes = std::max(bytes, split_k_workspace_bytes(M, N, p.splits));
         }

@@ -116,7 +116,7 @@ __device__ __forceinline__ void store_tile_bf16_blocks(const f32x4 (&acc16)[2 * 
 // gathered) 397 us with them, 346 so; 8 x 512 x 4096, N = 4096 159 -> 106; 2 x 2048 x 4096, N = 8192 235 -> 203.
 template <bool B_NT, bool PEERS_FIRST, bool SPLIT = false, bool RAGGED = false, bool MI16 = false, int NB = 2 * TN, bool F8 = false, bool GATHER = false>
 __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* smem) {
-    static_assert(NB == 2 * TN || (NB == 7 && MI16 && B_NT && !SPLIT && !RAGGED && !PEERS_FIRST), "224-column tile: plain NT products only");
+    static_assert(NB == 2 * TN || (NB == 7 && MI16 && B_NT && (SPLIT || !RAGGED) && !PEERS_FIRST), "224-column tile: plain NT products and parts of K");
     // F8: the operands are fp8 (e4m3fn) and g describes them as bf16 matrices of half the width (g.K, g.lda, g.ldb in
     // two-byte units), so a stage still holds 128-byte rows -- 128 k now -- and every load and LDS address below is unchanged;
     // only the k-step differs (k_step8: 16x16x128 MFMAs on the same 16 x 16 accumulator blocks).
@@ -203,7 +203,7 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     // its operand descriptors end with the last valid row, so the loads of the missing rows are
     // out of range (they fetch nothing) and the accumulators of those rows and columns, which
     // hold whatever the LDS stage held, are never stored (the epilogue masks them).
-    const int rows_a = RAGGED ? min(BM, g.M - m0) : BM, rows_b = RAGGED ? min(BN, g.N - n0) : BN;
+    const int rows_a = RAGGED ? min(BM, g.M - m0) : BM, rows_b = RAGGED ? min(BNX, g.N - n0) : BNX;
     // The LDS-DMA load is issued through inline assembly on purpose: the compiler then does not
     // know that LDS is written behind its back and leaves the ordering to the explicit
     // s_waitcnt vmcnt / s_barrier pairs below (told about it, it waits for vmcnt(0) in front of
@@ -925,13 +925,13 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     if constexpr (SPLIT) {
         // accumulators to the workspace in register order: quad q = (i, j, v/4) of thread tid at
         // [tail tile][split][q][tid], so that a wave's store is 1 KiB of consecutive addresses
-        f32x4* part = (f32x4*)g.out + ((int64_t)tail_index * g.k_splits + split) * (TM * TN * 4 * WM * WN * 64) + tid;
-        if constexpr (MI16) {   // quad q = block (i, j) of the 8 x 8
+        f32x4* part = (f32x4*)g.out + ((int64_t)tail_index * g.k_splits + split) * (2 * TM * NB * WM * WN * 64) + tid;
+        if constexpr (MI16) {   // quad q = block (i, j) of the 8 x NB
 #pragma unroll
             for (int i = 0; i < 2 * TM; ++i)
 #pragma unroll
-                for (int j = 0; j < 2 * TN; ++j)
-                    __builtin_nontemporal_store(acc16[i][j], part + (i * 2 * TN + j) * (WM * WN * 64));
+                for (int j = 0; j < NB; ++j)
+                    __builtin_nontemporal_store(acc16[i][j], part + (i * NB + j) * (WM * WN * 64));
             return;
         }
 #pragma unroll
@@ -1017,11 +1017,12 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl8_kernel(const GemmArgs g
 }  // namespace
 
 // Second launch of a call with a split tail: g.k_splits workgroups per tile of the last partial
-// round (g.out = workspace).
-template <bool B_NT, bool MI16, bool RAGGED = false, bool F8 = false>
+// round (g.out = workspace).  With few tiles every one is split and there is no launch before this one; M and N may
+// then be ragged, and the tiles 224 columns wide (NB = 7; plan_small in gemm.hip says when and what it measured).
+template <bool B_NT, bool MI16, bool RAGGED = false, bool F8 = false, int NB = 2 * TN>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_split_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gemm_dtl_tile<B_NT, false, true, RAGGED, MI16, 2 * TN, F8>(g, smem);
+    gemm_dtl_tile<B_NT, false, true, RAGGED, MI16, NB, F8>(g, smem);
 }
 
 // Third launch: sums the parts of every tail tile in the order 0..S-1 and applies the epilogue
@@ -1034,18 +1035,20 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_split_kernel(const GemmA
 // its 8-byte stores, as first written, left 32-byte pieces of a line to workgroups on different XCDs and waited for one
 // part after the other: 512 x 6656 x 8192 in four parts with a band and seven peers took 19.8 us, now 14.9 for 68 MB
 // (4.6 TB/s; parts written and read with or without the non-temporal hint: the same).
+template <int NB>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const GemmArgs g, const f32x4* __restrict__ parts) {
-    constexpr int T = WM * WN * 64, NQ = TM * TN * 4, LD = WTN + 4, kParts = 4;
+    constexpr int T = WM * WN * 64, NQ = 2 * TM * NB, WTNX = 16 * NB, LD = WTNX + 4, kParts = 4;
     __shared__ __attribute__((aligned(16))) float patch[32 * LD];
     const int tid = threadIdx.x, lane = tid & 63, jw = tid >> 6;
     const int slab = blockIdx.x % TM, wave = blockIdx.x / TM % (WM * WN), u = blockIdx.x / (TM * WM * WN);
     const int S = g.k_splits;
     int tile_m, tile_n;
     tile_schedule(g, schedule_position(g, u, g.tiles_m * g.tiles_n - g.tail_tiles), tile_m, tile_n);
-    const int m0 = tile_m * BM + (wave / WN) * WTM + slab * 32, n0 = tile_n * BN + (wave % WN) * WTN;
+    const int m0 = tile_m * BM + (wave / WN) * WTM + slab * 32, n0 = tile_n * (WN * WTNX) + (wave % WN) * WTNX;
     if (m0 >= g.M || n0 >= g.N) return;   // edge tiles: nothing of this slab is in the matrix
-    // this thread's quads are 16 slab + 4 jw .. +3 of the wave's 64
-    const f32x4* p = parts + ((int64_t)u * S * NQ + slab * 16 + 4 * jw) * T + wave * 64 + lane;
+    // this thread's quads are 4 jw .. +3 of the slab's 2 NB (NB = 7: the last wavefront's last two are not there, it reads its second again)
+    const int quads = NB == 2 * TN || jw < 3 ? 4 : 2 * NB - 12;
+    const f32x4* p = parts + ((int64_t)u * S * NQ + slab * 2 * NB + 4 * jw) * T + wave * 64 + lane;
     f32x4 sum[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1054,7 +1057,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
 #pragma unroll
         for (int sp = 0; sp < kParts; ++sp)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) x[sp][q] = __builtin_nontemporal_load(p + ((int64_t)min(s0 + sp, S - 1) * NQ + q) * T);
+            for (int q = 0; q < 4; ++q) x[sp][q] = __builtin_nontemporal_load(p + ((int64_t)min(s0 + sp, S - 1) * NQ + min(q, quads - 1)) * T);
 #pragma unroll
         for (int sp = 0; sp < kParts; ++sp) {
             if (s0 + sp >= S) break;
@@ -1069,9 +1072,9 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
         const int b = 4 * jw + q;   // quad of the slab
         // 16x16 blocks: row 16 (b / 8) + lane%16, columns 16 (b % 8) + 4(lane/16) .. +3; 32x32 blocks: row lane%32,
         // columns 32 (b / 4) + 8 (b % 4) + 4(lane/32) .. +3
-        const int r = g.mi16 ? 16 * (b >> 3) + (lane & 15) : lane & 31;
-        const int c = g.mi16 ? 16 * (b & 7) + 4 * (lane >> 4) : 8 * b + 4 * (lane >> 5);
-        *(f32x4*)(patch + r * LD + c) = sum[q];
+        const int r = g.mi16 ? 16 * (b / NB) + (lane & 15) : lane & 31;
+        const int c = g.mi16 ? 16 * (b % NB) + 4 * (lane >> 4) : 8 * b + 4 * (lane >> 5);
+        if (q < quads) *(f32x4*)(patch + r * LD + c) = sum[q];
     }
     __syncthreads();
     // The rounding of the main launch's tiles (gemm_dtl_tile): a tile that lies wholly in the band
@@ -1084,7 +1087,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int r = 16 * h + (tid >> 4), m = m0 + r, n = n0 + 8 * (tid & 15);
-        if (m >= g.M || n >= g.N) continue;   // an edge tile's missing rows and columns (N is a multiple of 8)
+        if (m >= g.M || n >= g.N || (tid & 15) >= 2 * NB) continue;   // an edge tile's missing rows and columns (N is a multiple of 8)
         float f[8];
         const f32x4 lo = *(const f32x4*)(patch + r * LD + 8 * (tid & 15)), hi = *(const f32x4*)(patch + r * LD + 8 * (tid & 15) + 4);
 #pragma unroll
@@ -1132,8 +1135,9 @@ bool gemm_dtl_supported(const GemmArgs& g) {
 
 // The third launch: `workspace` holds g.k_splits parts of each of the last g.tail_tiles tiles.
 hipError_t launch_tail_finish(const GemmArgs& g, hipStream_t st, const void* workspace) {
-    hipLaunchKernelGGL(gemm_dtl_tail_finish_kernel, dim3((unsigned)(g.tail_tiles * WM * WN * TM)), dim3(WM * WN * 64), 0, st, g,
-                       (const f32x4*)workspace);
+    const dim3 grid((unsigned)(g.tail_tiles * WM * WN * TM)), block(WM * WN * 64);
+    if (g.n224) hipLaunchKernelGGL(gemm_dtl_tail_finish_kernel<7>, grid, block, 0, st, g, (const f32x4*)workspace);
+    else hipLaunchKernelGGL(gemm_dtl_tail_finish_kernel<2 * TN>, grid, block, 0, st, g, (const f32x4*)workspace);
     return hipGetLastError();
 }
 
@@ -1167,7 +1171,7 @@ hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* w
 #undef KR_LAUNCH
         return hipGetLastError();
     }
-    if (g.n224) {
+    if (g.n224 && g.tail_tiles == 0) {
         static std::atomic<uint64_t> nopted;
         if (hipError_t e = lds_opt_in((const void*)gemm_dtl16n7_kernel, LDS_BYTES, nopted); e != hipSuccess) return e;
         hipLaunchKernelGGL(gemm_dtl16n7_kernel, grid, block, LDS_BYTES, st, g);
@@ -1191,24 +1195,30 @@ hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* w
         else hipLaunchKernelGGL((gemm_dtl_kernel<false, false>), grid, block, LDS_BYTES, st, g);
     }
     if (g.tail_tiles > 0) {
+        const bool split_ragged = g.M % BM != 0 || g.N % (g.n224 ? 224 : BN) != 0 || g.K % BKD != 0;
         // the tiles of the last partial round: k_splits workgroups each, parts to the workspace,
         // then the sum and the epilogue
-        static std::atomic<uint64_t> split_opted[4];
-        const void* sfn = g.mi16 ? (b_nt ? (const void*)gemm_dtl_split_kernel<true, true> : (const void*)gemm_dtl_split_kernel<false, true>)
-                                 : (b_nt ? (const void*)gemm_dtl_split_kernel<true, false> : (const void*)gemm_dtl_split_kernel<false, false>);
-        if (hipError_t e2 = lds_opt_in(sfn, LDS_BYTES, split_opted[(g.mi16 ? 2 : 0) + (b_nt ? 1 : 0)]); e2 != hipSuccess) return e2;
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         GemmArgs gs = g;
         gs.out = workspace;
         const dim3 sgrid((unsigned)(g.tail_tiles * g.k_splits));
-        if (g.mi16) {
-            if (b_nt) hipLaunchKernelGGL((gemm_dtl_split_kernel<true, true>), sgrid, block, LDS_BYTES, st, gs);
-            else hipLaunchKernelGGL((gemm_dtl_split_kernel<false, true>), sgrid, block, LDS_BYTES, st, gs);
+#define KR_LAUNCH(...)                                                                                                          \
+    do {                                                                                                                        \
+        static std::atomic<uint64_t> split_opted{0};                                                                            \
+        if (hipError_t e2 = lds_opt_in((const void*)gemm_dtl_split_kernel<__VA_ARGS__>, LDS_BYTES, split_opted); e2 != hipSuccess) return e2; \
+        hipLaunchKernelGGL((gemm_dtl_split_kernel<__VA_ARGS__>), sgrid, block, LDS_BYTES, st, gs);                              \
+    } while (0)
+        if (g.n224) {
+            if (split_ragged) KR_LAUNCH(true, true, true, false, 7); else KR_LAUNCH(true, true, false, false, 7);
+        } else if (!g.mi16) {   // (whole tiles only)
+            if (b_nt) KR_LAUNCH(true, false); else KR_LAUNCH(false, false);
+        } else if (split_ragged) {
+            if (b_nt) KR_LAUNCH(true, true, true); else KR_LAUNCH(false, true, true);
         } else {
-            if (b_nt) hipLaunchKernelGGL((gemm_dtl_split_kernel<true, false>), sgrid, block, LDS_BYTES, st, gs);
-            else hipLaunchKernelGGL((gemm_dtl_split_kernel<false, false>), sgrid, block, LDS_BYTES, st, gs);
+            if (b_nt) KR_LAUNCH(true, true); else KR_LAUNCH(false, true);
         }
+#undef KR_LAUNCH
         e = hipGetLastError();
         if (e != hipSuccess) return e;
         return launch_tail_finish(g, st, workspace);

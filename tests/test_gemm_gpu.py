@@ -546,6 +546,53 @@ def test_split_parts_of_very_few_k_steps(dev, monkeypatch, b_t, mfma):
         torch.testing.assert_close(out.cpu(), a.float() @ b.float(), rtol=1e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("cols", [256, 224])
+@pytest.mark.parametrize("M,N,K,S", [(513, 776, 576, 3), (255, 224, 128, 2), (264, 456, 1024, 8), (512, 448, 320, 5), (8, 8, 192, 2), (520, 680, 64 * 17, 4)])
+def test_ragged_tiles_in_parts(dev, monkeypatch, M, N, K, S, cols):
+    """Every 256 x 256 or 256 x 224 tile's K loop in parts, with edge tiles of one row, one 16-byte piece or all but one:
+    all rows with peers and bias, and a band that starts inside a tile.  Small integers: every fp32 sum is exact."""
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_TILE", "256")
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_TAILSPLIT", str(S))
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_N224", str(int(cols == 224)))
+    _lib.reload_env()
+    g = torch.Generator().manual_seed(K + N)
+    a, b = torch.randint(-4, 5, (M, K), generator=g).float(), torch.randint(-4, 5, (K, N), generator=g).float()
+    peers = torch.randint(-8, 9, (9, M, N), generator=g).to(BF16)
+    bias = torch.randint(-8, 9, (N,), generator=g).to(BF16)
+    for b_t in (True,) if cols == 224 else (False, True):
+        p = _lib.gemm_plan(M, N, K, b_t, 9, M, workspace_bytes=1 << 40)
+        assert (p["tile_n"], p["tail_tiles"], p["tail_splits"]) == (cols, -(-M // 256) * -(-N // cols), S)
+        ad, bd = a.to(BF16).to(dev), b.T.contiguous().to(BF16).to(dev).T if b_t else b.to(BF16).to(dev)
+        out = fused.gemm_one_shot_all_reduce_fused(ad, bd, peers=peers.to(dev), bias=bias.to(dev))
+        assert torch.equal(out.cpu(), a @ b + peers.float().sum(0) + bias.float())
+        if M % 4 == 0:
+            c = torch.zeros(M, N, dtype=BF16, device=dev)
+            rows = slice(M // 4, M // 2)
+            got = fused.gemm_reduce_scatter(ad, bd, peers=peers[:3, :M // 4].contiguous().to(dev), rank=1, c_scratch=c).cpu()
+            product, summed = a @ b, peers[:3, :M // 4].float().sum(0)
+            # (a tile wholly in the band rounds once, others round the product first)
+            once, twice = (product[rows] + summed).to(BF16), (product[rows].to(BF16).float() + summed).to(BF16)
+            assert ((got == once) | (got == twice)).all()
+            c = c.cpu()
+            assert (c[rows] == 0).all()
+            c[rows] = product[rows].to(BF16)
+            assert torch.equal(c, product.to(BF16))
+
+
+@pytest.mark.parametrize("M,N,K,b_t,cols", [(500, 6656, 8192, True, 224), (576, 4608, 5120, False, 256), (300, 1032, 4096, True, 128)])
+def test_ragged_tiles_in_parts_where_the_rule_takes_them(dev, M, N, K, b_t, cols):
+    """Nothing forced: seven peers, bf16 result, against the exact sums."""
+    plan = _lib.gemm_plan(M, N, K, b_t, 7, M, workspace_bytes=_lib.load().kr_gemm_workspace_bytes(M, N, K))
+    assert plan["tile_n"] == cols and (plan["tail_splits"] > 1) == (cols != 128)
+    g = torch.Generator().manual_seed(K)
+    a = torch.randint(-2, 3, (M, K), generator=g).float().to(dev)
+    b = torch.randint(-1, 2, (K, N), generator=g).float().to(dev)
+    peers = torch.randint(-8, 9, (7, M, N), generator=g).to(BF16).to(dev)
+    b16 = b.T.contiguous().to(BF16).T if b_t else b.to(BF16)
+    out = fused.gemm_one_shot_all_reduce_fused(a.to(BF16), b16, peers=peers)
+    assert torch.equal(out, a @ b + peers.float().sum(0))
+
+
 def _band_tile_counts(M, N, W, bm):
     rows = M // W
     return [(((r + 1) * rows - 1) // bm - (r * rows) // bm + 1) * -(-N // bm) for r in range(W)]
