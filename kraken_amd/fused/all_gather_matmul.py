@@ -47,6 +47,11 @@ def _apart(sources: list[int], a_out: torch.Tensor) -> bool:
     return all(p + size <= out or p >= out + W * size or p == out + r * size for r, p in enumerate(sources))
 
 
+def _recorded(peers: PeerBuffers, a_out: torch.Tensor) -> bool:
+    """Whether autograd has to know of the gather: the copies of the side-stream form tell it, a kernel does not."""
+    return torch.is_grad_enabled() and (a_out.requires_grad or any(t.requires_grad for t in peers.tensors))
+
+
 def _direct(sources: list[int], a_out: torch.Tensor, b: torch.Tensor, W: int, m: int, N: int, K: int) -> bool:
     """Whether the product gathers the shards itself (``kr_gather_matmul_bf16``): enough large tiles, each inside one
     shard, and shards apart from the gathered matrix (a tile may read a row after another one has written it)."""
@@ -70,7 +75,10 @@ def _gathered_first(a_out, peers: PeerBuffers, progress, splits: int, rank: int,
     else:
         _check_progress(progress, peers.W * splits)
         progress.fill_(0)
-    return gather_chunks(a_out, peers, flags, splits, rank, _lib.current_stream(dev))
+    if not gather_chunks(a_out, peers, flags, splits, rank, _lib.current_stream(dev)):
+        return False
+    torch.autograd.graph.increment_version(a_out)
+    return True
 
 
 def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **kwargs):
@@ -110,7 +118,7 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
             a_out = torch.empty((M, K), dtype=fp8, device=dev)
         else:
             assert tuple(a_out.shape) == (M, K) and a_out.dtype == fp8 and a_out.is_contiguous()
-        if kwargs.get("copy_engine", False) or not _gathered_first(a_out, peers, progress, splits, rank, dev):
+        if kwargs.get("copy_engine", False) or _recorded(peers, a_out) or not _gathered_first(a_out, peers, progress, splits, rank, dev):
             if progress is None:
                 progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)
             else:
@@ -185,7 +193,8 @@ def all_gather_matmul(
       read to ``a_out`` while they multiply; the flags of ``progress`` are set behind it, no tile waits and
       ``status`` is not touched.  8 shards of 1024 x 8192, N = 3584: 397 us with copies and flags, 346 so.
       Other shapes are gathered by one launch in front of the product.
-      With ``copy_engine=True``, and where shards are not 16-byte aligned or overlap ``a_out``,
+      With ``copy_engine=True``, and where shards are not 16-byte aligned, overlap ``a_out`` or (with gradients
+      enabled) require a gradient,
       the shards are copied chunk by chunk into ``a_out`` on a side stream,
       each chunk followed by its flag in ``progress`` (``:308-311``), while the
       GEMM on the current stream consumes them: tiles of the local shard
@@ -258,7 +267,8 @@ def all_gather_matmul(
     else:
         assert tuple(a_out.shape) == (M, K) and a_out.dtype == torch.bfloat16 and a_out.is_contiguous()
     sources = peers.pointers()
-    if not kwargs.get("copy_engine", False) and _direct(sources, a_out, b, W, m, N, K):
+    side_stream = kwargs.get("copy_engine", False) or _recorded(peers, a_out)
+    if not side_stream and _direct(sources, a_out, b, W, m, N, K):
         if progress is not None:
             _check_progress(progress, W * splits)
             progress.fill_(0)
@@ -266,10 +276,11 @@ def all_gather_matmul(
         rc = _lib.load().kr_gather_matmul_bf16((ctypes.c_void_p * W)(*sources), W, rank, m, a_out.data_ptr(), b.data_ptr(), b.stride(1),
                                                N, K, c.data_ptr(), _lib.current_stream(dev))
         _lib.check(rc, "all_gather_matmul")
+        torch.autograd.graph.increment_version(a_out)
         if progress is not None:
             progress.view(-1)[:W * splits].fill_(1)
         return a_out, c
-    if not kwargs.get("copy_engine", False) and _gathered_first(a_out, peers, progress, splits, rank, dev):
+    if not side_stream and _gathered_first(a_out, peers, progress, splits, rank, dev):
         c = _lib.calls().gemm(a_out, b, None, None, None, 0, M, False, rank * m)
         if c is None:
             c = torch.empty((M, N), dtype=torch.bfloat16, device=dev)

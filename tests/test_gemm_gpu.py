@@ -1395,6 +1395,25 @@ def test_gather_inside_the_product(dev, W, m, N, K):
     assert torch.equal(got, full) and torch.equal(c, want)
 
 
+@pytest.mark.parametrize("m,N,dtype", [(512, 4096, BF16), (5, 1024, BF16), (5, 1024, torch.float8_e4m3fn)])
+def test_gathered_matrix_is_known_to_be_written(dev, m, N, dtype):
+    """Autograd sees that the gathered matrix changed, whether the product or a launch in front of it gathers; shards
+    that require a gradient take the side stream, whose copies are recorded, with that form's results."""
+    W, K = 8, 256
+    shards = [torch.randn(m, K, device=dev).to(dtype) for _ in range(W)]
+    b = torch.randn(N, K, device=dev).to(dtype).T
+    a_out = torch.zeros(W * m, K, device=dev).to(dtype)
+    version = a_out._version
+    fused.all_gather_matmul(shards, b, a_out)
+    assert a_out._version > version
+    if dtype == BF16:
+        # (the product behind the flags; one behind a launch that gathers may add in another order)
+        _, want = fused.all_gather_matmul(shards, b, copy_engine=True)
+        followed = [t.clone().requires_grad_() for t in shards]
+        got, c = fused.all_gather_matmul(followed, b)
+        assert torch.equal(got, torch.cat(shards)) and torch.equal(c, want)
+
+
 def test_gather_inside_the_product_is_for_shards_apart(dev):
     """A shard that lies in another one's place of the gathered matrix, and shards that are not 16-byte aligned, take the
     copies; shapes of few tiles, or whose shards are no whole tiles, as well."""
