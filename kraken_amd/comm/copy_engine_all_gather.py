@@ -34,6 +34,17 @@ def _check_progress(progress: torch.Tensor, n: int) -> None:
     assert progress.is_contiguous() and progress.numel() >= n
 
 
+def followed(output: torch.Tensor, peers: PeerBuffers) -> bool:
+    """Whether autograd has to know of the gather: copies by torch tell it, a kernel or a copy engine does not."""
+    return torch.is_grad_enabled() and (output.requires_grad or any(t.requires_grad for t in peers.tensors))
+
+
+def _takes_copies(output: torch.Tensor) -> bool:
+    """Whether torch copies into ``output`` while gradients are enabled (not into a leaf that requires one, nor a view of it)."""
+    base = output._base if output._is_view() else output
+    return not (base.is_leaf and base.requires_grad)
+
+
 def gather_chunks(output: torch.Tensor, peers: PeerBuffers, progress: torch.Tensor, splits: int, rank: int, stream: int) -> bool:
     """All chunks and flags in one launch (``kr_gather_chunks``) on the stream given; False, and nothing launched, where
     addresses or chunks are no multiples of 16 bytes.  Of the arguments' checks only these are made here."""
@@ -45,6 +56,7 @@ def gather_chunks(output: torch.Tensor, peers: PeerBuffers, progress: torch.Tens
     rc = _lib.load().kr_gather_chunks((ctypes.c_void_p * W)(*sources), W, splits, rank, chunk_bytes, output.data_ptr(),
                                       progress.data_ptr(), stream)
     _lib.check(rc, "gather_chunks")
+    torch.autograd.graph.increment_version(output)
     return True
 
 
@@ -70,12 +82,13 @@ def _copy_engine_all_gather_w_progress(
     flag write (``:47-53``).  The side stream first waits for the current
     stream (``:35``); the caller makes the current stream wait for the returned
     stream when it needs the gathered tensor (``:118``).  All chunks and flags
-    of a gather of up to ``ONE_LAUNCH_BYTES`` are one launch (``kr_gather_chunks``); larger ones, and
-    chunks that are no multiple of 16 bytes, are copied one by one by ordinary device-to-device copy
-    kernels with a flag write behind each; ``copy_engine=True`` hands them to the GPU's
+    of a gather of up to ``ONE_LAUNCH_BYTES`` are one launch (``kr_gather_chunks``); larger ones,
+    chunks that are no multiple of 16 bytes, and (with gradients enabled) shards that require a gradient
+    are copied one by one by ordinary device-to-device copies, which autograd records,
+    with a flag write behind each; ``copy_engine=True`` hands them to the GPU's
     copy engines (``kr_copy_engine_memcpy``), which take no compute units but
-    are slower within one GPU.  ``progress`` must have been zeroed on the current
-    stream beforehand.
+    are slower within one GPU and, like the one launch, only mark ``output`` as written.  ``progress``
+    must have been zeroed on the current stream beforehand.
     """
     peers = PeerBuffers(inp, dtypes=(torch.bfloat16, torch.float8_e4m3fn))
     W = peers.W
@@ -92,13 +105,17 @@ def _copy_engine_all_gather_w_progress(
         backend_stream = _get_backend_stream(dev)
     lib = _lib.load()
     chunk = peers.cap // splits_per_rank
-    flat_out = output.view(-1)
     current = torch.cuda.current_stream(dev)
     if backend_stream != current:
         backend_stream.wait_stream(current)
-    if (not copy_engine and output.numel() * output.element_size() <= ONE_LAUNCH_BYTES
+    recorded = not copy_engine and followed(output, peers)
+    if (not copy_engine and output.numel() * output.element_size() <= ONE_LAUNCH_BYTES and not (recorded and _takes_copies(output))
             and gather_chunks(output, peers, progress, splits_per_rank, rank, backend_stream.cuda_stream)):
         return backend_stream
+    if (recorded and output.grad_fn is not None and not output._is_view()
+            and all(t.untyped_storage().data_ptr() != output.untyped_storage().data_ptr() for t in peers.tensors)):
+        output.detach_()     # every element is written below: a matrix that is kept does not keep the history of earlier gathers
+    flat_out = output.view(-1)
     with torch.cuda.stream(backend_stream):
         for step in range(W):
             src_rank = (rank + step + 1) % W
@@ -112,6 +129,8 @@ def _copy_engine_all_gather_w_progress(
                     dst_c.copy_(src_c)
                 rc = lib.kr_stream_write_value32(progress.data_ptr() + 4 * c, 1, backend_stream.cuda_stream)
                 _lib.check(rc, "stream_write_value32")
+    if copy_engine:
+        torch.autograd.graph.increment_version(output)
     return backend_stream
 
 

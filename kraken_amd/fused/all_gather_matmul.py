@@ -7,7 +7,7 @@ import torch
 
 from .. import _lib, _waits
 from ..comm._common import PeerBuffers
-from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress, gather_chunks
+from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress, followed, gather_chunks
 from . import _gemm
 
 
@@ -47,11 +47,6 @@ def _apart(sources: list[int], a_out: torch.Tensor) -> bool:
     return all(p + size <= out or p >= out + W * size or p == out + r * size for r, p in enumerate(sources))
 
 
-def _recorded(peers: PeerBuffers, a_out: torch.Tensor) -> bool:
-    """Whether autograd has to know of the gather: the copies of the side-stream form tell it, a kernel does not."""
-    return torch.is_grad_enabled() and (a_out.requires_grad or any(t.requires_grad for t in peers.tensors))
-
-
 def _direct(sources: list[int], a_out: torch.Tensor, b: torch.Tensor, W: int, m: int, N: int, K: int) -> bool:
     """Whether the product gathers the shards itself (``kr_gather_matmul_bf16``): enough large tiles, each inside one
     shard, and shards apart from the gathered matrix (a tile may read a row after another one has written it)."""
@@ -75,10 +70,7 @@ def _gathered_first(a_out, peers: PeerBuffers, progress, splits: int, rank: int,
     else:
         _check_progress(progress, peers.W * splits)
         progress.fill_(0)
-    if not gather_chunks(a_out, peers, flags, splits, rank, _lib.current_stream(dev)):
-        return False
-    torch.autograd.graph.increment_version(a_out)
-    return True
+    return gather_chunks(a_out, peers, flags, splits, rank, _lib.current_stream(dev))
 
 
 def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **kwargs):
@@ -118,7 +110,7 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
             a_out = torch.empty((M, K), dtype=fp8, device=dev)
         else:
             assert tuple(a_out.shape) == (M, K) and a_out.dtype == fp8 and a_out.is_contiguous()
-        if kwargs.get("copy_engine", False) or _recorded(peers, a_out) or not _gathered_first(a_out, peers, progress, splits, rank, dev):
+        if kwargs.get("copy_engine", False) or followed(a_out, peers) or not _gathered_first(a_out, peers, progress, splits, rank, dev):
             if progress is None:
                 progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)
             else:
@@ -267,7 +259,7 @@ def all_gather_matmul(
     else:
         assert tuple(a_out.shape) == (M, K) and a_out.dtype == torch.bfloat16 and a_out.is_contiguous()
     sources = peers.pointers()
-    side_stream = kwargs.get("copy_engine", False) or _recorded(peers, a_out)
+    side_stream = kwargs.get("copy_engine", False) or followed(a_out, peers)
     if not side_stream and _direct(sources, a_out, b, W, m, N, K):
         if progress is not None:
             _check_progress(progress, W * splits)

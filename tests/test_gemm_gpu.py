@@ -1414,6 +1414,36 @@ def test_gathered_matrix_is_known_to_be_written(dev, m, N, dtype):
         assert torch.equal(got, torch.cat(shards)) and torch.equal(c, want)
 
 
+def test_gathers_of_any_form_are_known_to_autograd(dev):
+    """Below the size up to which a gather is one launch: shards that require a gradient get it back from the gathered matrix, a
+    matrix that is kept does not keep earlier gathers, and every other form marks it as written."""
+    W, m, K, N = 4, 40, 256, 1024
+    b = torch.randn(N, K, device=dev).to(BF16).T
+    def shards(grad):
+        return [torch.randn(m, K, device=dev).to(BF16).requires_grad_(grad) for _ in range(W)]
+    calls = {"matmul": lambda s, out, **kw: fused.all_gather_matmul(s, b, out, **kw)[0], "gather": lambda s, out, **kw: comm.all_gather_w_progress(s, out, **kw)}
+    for what, call in calls.items():
+        kept, first, second = torch.empty(W * m, K, dtype=BF16, device=dev), shards(True), shards(True)
+        for s in (first, second):
+            got = call(s, kept)
+            assert got is kept and torch.equal(got, torch.cat(s)) and got.grad_fn is not None, what
+        weight = torch.randn(W * m, K, device=dev).to(BF16)
+        kept.backward(weight)
+        assert all(t.grad is None for t in first) and torch.equal(torch.cat([t.grad for t in second]), weight), what
+        call(shards(False), kept)
+        assert not kept.requires_grad, what
+        with torch.no_grad():
+            assert not call(shards(True), None).requires_grad, what
+        # (a leaf takes no recorded copies)
+        leaf = torch.empty(W * m, K, dtype=BF16, device=dev, requires_grad=True)
+        version, s = leaf._version, shards(False)
+        assert torch.equal(call(s, leaf), torch.cat(s)) and leaf._version > version, what
+        out = torch.zeros(W * m, K, dtype=BF16, device=dev)
+        for kw in ({}, {"copy_engine": True}):
+            version, s = out._version, shards(False)
+            assert torch.equal(call(s, out, **kw), torch.cat(s)) and out._version > version, (what, kw)
+
+
 def test_gather_inside_the_product_is_for_shards_apart(dev):
     """A shard that lies in another one's place of the gathered matrix, and shards that are not 16-byte aligned, take the
     copies; shapes of few tiles, or whose shards are no whole tiles, as well."""
