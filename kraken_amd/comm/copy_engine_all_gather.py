@@ -45,13 +45,22 @@ def _takes_copies(output: torch.Tensor) -> bool:
     return not (base.is_leaf and base.requires_grad)
 
 
+def in_own_place(sources: list[int], output: torch.Tensor) -> list[bool]:
+    """For each shard's address whether it overlaps the gathered matrix nowhere but in its own place."""
+    W = len(sources)
+    out, size = output.data_ptr(), output.numel() * output.element_size() // W
+    return [p + size <= out or p >= out + W * size or p == out + r * size for r, p in enumerate(sources)]
+
+
 def gather_chunks(output: torch.Tensor, peers: PeerBuffers, progress: torch.Tensor, splits: int, rank: int, stream: int) -> bool:
     """All chunks and flags in one launch (``kr_gather_chunks``) on the stream given; False, and nothing launched, where
-    addresses or chunks are no multiples of 16 bytes.  Of the arguments' checks only these are made here."""
+    addresses or chunks are no multiples of 16 bytes, or a shard lies where another one's copy goes (its workgroups
+    run in no order).  Of the arguments' checks only these are made here."""
     W = peers.W
     chunk_bytes = peers.cap // splits * output.element_size()
     sources = peers.pointers()
-    if W > _lib.KR_MAX_WORLD or chunk_bytes % 16 != 0 or output.data_ptr() % 16 != 0 or any(p % 16 != 0 for p in sources):
+    if (W > _lib.KR_MAX_WORLD or chunk_bytes % 16 != 0 or output.data_ptr() % 16 != 0 or any(p % 16 != 0 for p in sources)
+            or not all(in_own_place(sources, output))):
         return False
     rc = _lib.load().kr_gather_chunks((ctypes.c_void_p * W)(*sources), W, splits, rank, chunk_bytes, output.data_ptr(),
                                       progress.data_ptr(), stream)
@@ -83,7 +92,8 @@ def _copy_engine_all_gather_w_progress(
     stream (``:35``); the caller makes the current stream wait for the returned
     stream when it needs the gathered tensor (``:118``).  All chunks and flags
     of a gather of up to ``ONE_LAUNCH_BYTES`` are one launch (``kr_gather_chunks``); larger ones,
-    chunks that are no multiple of 16 bytes, and (with gradients enabled) shards that require a gradient
+    chunks that are no multiple of 16 bytes, shards that lie in another one's place of ``output`` (they are
+    set aside first) and (with gradients enabled) shards that require a gradient
     are copied one by one by ordinary device-to-device copies, which autograd records,
     with a flag write behind each; ``copy_engine=True`` hands them to the GPU's
     copy engines (``kr_copy_engine_memcpy``), which take no compute units but
@@ -117,9 +127,10 @@ def _copy_engine_all_gather_w_progress(
         output.detach_()     # every element is written below: a matrix that is kept does not keep the history of earlier gathers
     flat_out = output.view(-1)
     with torch.cuda.stream(backend_stream):
+        shards = [peers.slice(r) if kept else peers.slice(r).clone() for r, kept in enumerate(in_own_place(peers.pointers(), output))]
         for step in range(W):
             src_rank = (rank + step + 1) % W
-            src = peers.slice(src_rank).reshape(-1)
+            src = shards[src_rank].reshape(-1)
             for split_id in range(splits_per_rank):
                 c = src_rank * splits_per_rank + split_id
                 dst_c, src_c = flat_out[c * chunk:(c + 1) * chunk], src[split_id * chunk:(split_id + 1) * chunk]

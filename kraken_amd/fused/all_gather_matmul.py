@@ -7,7 +7,7 @@ import torch
 
 from .. import _lib, _waits
 from ..comm._common import PeerBuffers
-from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress, followed, gather_chunks
+from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress, followed, gather_chunks, in_own_place
 from . import _gemm
 
 
@@ -40,18 +40,17 @@ def _matmul_w_progress(a, a_local, b, progress, configs, status=None) -> torch.T
     return c
 
 
-def _apart(sources: list[int], a_out: torch.Tensor) -> bool:
-    """No shard overlaps the gathered matrix other than in its own place."""
-    W = len(sources)
-    out, size = a_out.data_ptr(), a_out.numel() * a_out.element_size() // W
-    return all(p + size <= out or p >= out + W * size or p == out + r * size for r, p in enumerate(sources))
-
-
 def _direct(sources: list[int], a_out: torch.Tensor, b: torch.Tensor, W: int, m: int, N: int, K: int) -> bool:
     """Whether the product gathers the shards itself (``kr_gather_matmul_bf16``): enough large tiles, each inside one
     shard, and shards apart from the gathered matrix (a tile may read a row after another one has written it)."""
     return (W <= _lib.KR_MAX_WORLD and _lib.load().kr_gather_matmul_direct(W, m, N, K) == 1
-            and all(p % 16 == 0 for p in (a_out.data_ptr(), b.data_ptr(), *sources)) and _apart(sources, a_out))
+            and all(p % 16 == 0 for p in (a_out.data_ptr(), b.data_ptr(), *sources)) and all(in_own_place(sources, a_out)))
+
+
+def _local_shard(peers: PeerBuffers, rank: int, a_out: torch.Tensor) -> torch.Tensor | None:
+    """The shard that tiles read without waiting; ``None`` where another one's copy overwrites it meanwhile (its tiles then
+    wait for their flags and read ``a_out``)."""
+    return peers.slice(rank) if in_own_place(peers.pointers(), a_out)[rank] else None
 
 
 def _gathered_first(a_out, peers: PeerBuffers, progress, splits: int, rank: int, dev) -> bool:
@@ -62,8 +61,6 @@ def _gathered_first(a_out, peers: PeerBuffers, progress, splits: int, rank: int,
     its events, flags and status word cost the host 100 us.  Calls one behind the other, us, with the side stream /
     in front: W = 8, 1 x 1024, N = 1024 125 / 38; 8 x 130 x 8192, N = 8192 205 / 176; 8 x 500 x 4096, N = 6656 232 / 188;
     8 x 1000 x 8192, N = 1024 286 / 185, N = 3584 450 / 389; 2 x 1000 x 16384, N = 8192 429 / 393."""
-    if not _apart(peers.pointers(), a_out):
-        return False
     flags = progress
     if progress is None:
         flags = torch.empty(peers.W * splits, dtype=torch.int32, device=dev)     # counted in, read by nobody
@@ -122,11 +119,11 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
                 own_status = status is None
                 if own_status:
                     status = _waits.new_status(dev)
-                a_local = peers.slice(rank)
-                assert a_local.stride(1) == 1
+                a_local = _local_shard(peers, rank, a_out)
+                assert a_local is None or a_local.stride(1) == 1
                 c = torch.empty((M, N), dtype=fp8, device=dev)
                 rc = lib.kr_all_gather_matmul_fp8(
-                    a_out.data_ptr(), K, a_local.data_ptr(), a_local.stride(0), b.T.data_ptr(), K, M, N, K, W, rank, splits,
+                    a_out.data_ptr(), K, _lib.ptr(a_local), 0 if a_local is None else a_local.stride(0), b.T.data_ptr(), K, M, N, K, W, rank, splits,
                     progress.data_ptr(), int(kwargs.get("wait_limit_us", 0)), _lib.ptr(status), c.data_ptr(), 2, stream)
                 _lib.check(rc, "all_gather_matmul(fp8)")
                 torch.cuda.current_stream(dev).wait_stream(backend_stream)
@@ -290,7 +287,7 @@ def all_gather_matmul(
     own_status = status is None
     if own_status:
         status = _waits.new_status(dev)
-    c = _matmul_w_progress(a_out, peers.slice(rank), b, progress, configs, status)
+    c = _matmul_w_progress(a_out, _local_shard(peers, rank, a_out), b, progress, configs, status)
     torch.cuda.current_stream(dev).wait_stream(backend_stream)
     if own_status:
         _waits.watch(status, "all_gather_matmul")

@@ -707,3 +707,23 @@ def test_bench_refuses_more_than_one_gpu():
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 2
     assert "--gpus 2 is not supported" in r.stderr and r.stdout == ""
+
+
+def test_shards_in_each_others_places_take_no_single_launch(monkeypatch):
+    """The workgroups of kr_gather_chunks run in no order: it is not launched where a shard lies where another one's copy goes."""
+    from kraken_amd.comm import copy_engine_all_gather as ag
+    from kraken_amd.comm._common import PeerBuffers
+
+    launched = []
+
+    class Lib:
+        def kr_gather_chunks(self, *args):
+            launched.append(args)
+            return 0
+
+    monkeypatch.setattr(_lib, "load", Lib)
+    W, m, K = 4, 6, 64
+    out, progress, own = torch.zeros(W * m, K, dtype=torch.bfloat16), torch.zeros(W, dtype=torch.int32), torch.zeros(W, m, K, dtype=torch.bfloat16)
+    for first, taken in ((own[0], True), (out[:m], True), (out[m:2 * m], False), (out[1:m + 1], False), (out[(W - 1) * m:], False)):
+        launched.clear()
+        assert ag.gather_chunks(out, PeerBuffers([first, *own[1:]]), progress, 1, 0, 0) == taken == bool(launched)

@@ -1460,6 +1460,27 @@ def test_gather_inside_the_product_is_for_shards_apart(dev):
     assert not _direct(apart, a_out, b, W, 500, N, K) and not _direct(apart, a_out, b, W, 256, 1024, K)
 
 
+@pytest.mark.parametrize("m,N,K,dtype", [(40, 264, 256, BF16), (512, 4096, 256, BF16), (512, 1024, 128, torch.float8_e4m3fn), (6, 48, 48, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("copy_engine", [False, True])
+def test_shards_in_each_others_places_are_gathered_whole(dev, m, N, K, dtype, copy_engine):
+    """Shards that lie in the gathered matrix, rotated by one place, one of them across two: every row comes out as the shard
+    held it at the call, and so does the product.  One shard in its own place, one outside."""
+    W, rank = 4, 1
+    b = torch.randn(N, K, device=dev).to(dtype).T
+    rows = torch.randn(W * m, K, device=dev).to(dtype)
+    for places in ((1, 2, 3, 0), (0, 2, 1.5, None), (2.5, 0.5, None, 3)):
+        a_out = rows.clone()
+        shards = [rows[:m].clone() if p is None else a_out[int(p * m):int(p * m) + m] for p in places]
+        full = torch.cat([s.view(torch.uint8) for s in shards]).view(dtype)
+        _, want = fused.all_gather_matmul(full.view(W, m, K), b, gather=False)
+        got, c = fused.all_gather_matmul(shards, b, a_out, rank=rank, copy_engine=copy_engine)
+        assert got is a_out and torch.equal(got.view(torch.uint8), full.view(torch.uint8)), places
+        torch.testing.assert_close(c.float(), want.float(), rtol=2e-2 if dtype == BF16 else 0.13, atol=2e-2)
+        if dtype == BF16:
+            a_out.copy_(rows)
+            assert torch.equal(comm.all_gather_w_progress(shards, a_out, rank=rank, copy_engine=copy_engine), full), places
+
+
 @pytest.mark.parametrize("plan", [None, 0, 3, 4000, 5001, 6000, 7002])
 @pytest.mark.parametrize("M,N,K", [(1, 16, 16), (255, 272, 112), (257, 528, 1040), (300, 1040, 528), (513, 816, 384)])
 def test_fp8_wide_kernel_shapes(dev, monkeypatch, M, N, K, plan):
