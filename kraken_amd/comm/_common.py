@@ -5,6 +5,7 @@ import ctypes
 from typing import Sequence
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib, _waits
 
@@ -149,6 +150,11 @@ def _zero_row_workspaces() -> None:
 
 
 _waits.on_failure(_zero_row_workspaces)
+
+
+def has_tangent(*tensors: torch.Tensor) -> bool:
+    """Whether a tensor carries a forward-mode tangent: only copies by torch hand it on, or clear it."""
+    return forward_ad._current_level >= 0 and any(forward_ad.unpack_dual(t).tangent is not None for t in tensors)
 
 
 def check_stack(stacked: torch.Tensor | Sequence[torch.Tensor]) -> PeerBuffers:

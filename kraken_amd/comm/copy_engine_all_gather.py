@@ -6,7 +6,7 @@ import ctypes
 import torch
 
 from .. import _lib
-from ._common import PeerBuffers
+from ._common import PeerBuffers, has_tangent
 
 # Up to here all copies and flags of a gather on a side stream are one launch.  What that gives depends on how long the product
 # beside it takes next to the launches of the loop (about 120 us of host time and 9 per chunk).  Time in one launch over time
@@ -36,13 +36,14 @@ def _check_progress(progress: torch.Tensor, n: int) -> None:
 
 def followed(output: torch.Tensor, peers: PeerBuffers) -> bool:
     """Whether autograd has to know of the gather: copies by torch tell it, a kernel or a copy engine does not."""
-    return torch.is_grad_enabled() and (output.requires_grad or any(t.requires_grad for t in peers.tensors))
+    return ((torch.is_grad_enabled() and (output.requires_grad or any(t.requires_grad for t in peers.tensors)))
+            or has_tangent(output, *peers.tensors))
 
 
 def _takes_copies(output: torch.Tensor) -> bool:
-    """Whether torch copies into ``output`` while gradients are enabled (not into a leaf that requires one, nor a view of it)."""
+    """Whether torch copies into ``output`` (with gradients enabled, not into a leaf that requires one, nor a view of it)."""
     base = output._base if output._is_view() else output
-    return not (base.is_leaf and base.requires_grad)
+    return not (torch.is_grad_enabled() and base.is_leaf and base.requires_grad)
 
 
 def in_own_place(sources: list[int], output: torch.Tensor) -> list[bool]:
@@ -93,7 +94,7 @@ def _copy_engine_all_gather_w_progress(
     stream when it needs the gathered tensor (``:118``).  All chunks and flags
     of a gather of up to ``ONE_LAUNCH_BYTES`` are one launch (``kr_gather_chunks``); larger ones,
     chunks that are no multiple of 16 bytes, shards that lie in another one's place of ``output`` (they are
-    set aside first) and (with gradients enabled) shards that require a gradient
+    set aside first) and shards that autograd follows (they require a gradient, or carry a forward-mode tangent)
     are copied one by one by ordinary device-to-device copies, which autograd records,
     with a flag write behind each; ``copy_engine=True`` hands them to the GPU's
     copy engines (``kr_copy_engine_memcpy``), which take no compute units but
@@ -122,7 +123,7 @@ def _copy_engine_all_gather_w_progress(
     if (not copy_engine and output.numel() * output.element_size() <= ONE_LAUNCH_BYTES and not (recorded and _takes_copies(output))
             and gather_chunks(output, peers, progress, splits_per_rank, rank, backend_stream.cuda_stream)):
         return backend_stream
-    if (recorded and output.grad_fn is not None and not output._is_view()
+    if (recorded and torch.is_grad_enabled() and output.grad_fn is not None and not output._is_view()
             and all(t.untyped_storage().data_ptr() != output.untyped_storage().data_ptr() for t in peers.tensors)):
         output.detach_()     # every element is written below: a matrix that is kept does not keep the history of earlier gathers
     flat_out = output.view(-1)

@@ -182,8 +182,8 @@ def all_gather_matmul(
       read to ``a_out`` while they multiply; the flags of ``progress`` are set behind it, no tile waits and
       ``status`` is not touched.  8 shards of 1024 x 8192, N = 3584: 397 us with copies and flags, 346 so.
       Other shapes are gathered by one launch in front of the product.
-      With ``copy_engine=True``, and where shards are not 16-byte aligned, overlap ``a_out`` or (with gradients
-      enabled) require a gradient,
+      With ``copy_engine=True``, and where shards are not 16-byte aligned, overlap ``a_out`` or are followed by autograd
+      (they require a gradient, with gradients enabled, or carry a forward-mode tangent),
       the shards are copied chunk by chunk into ``a_out`` on a side stream,
       each chunk followed by its flag in ``progress`` (``:308-311``), while the
       GEMM on the current stream consumes them: tiles of the local shard

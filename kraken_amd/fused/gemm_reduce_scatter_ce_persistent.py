@@ -6,6 +6,7 @@ import ctypes
 import torch
 
 from .. import _lib, _waits
+from ..comm._common import has_tangent
 from ..comm.copy_engine_all_gather import _get_backend_stream
 from . import _gemm
 
@@ -105,7 +106,7 @@ def _sends_direct(sent, a: torch.Tensor, b: torch.Tensor, world_size: int, m_per
     the operands, and nothing autograd would have to know of."""
     if not (isinstance(sent, torch.Tensor) and tuple(sent.shape) == (world_size, m_per_rank, N) and sent.is_contiguous()
             and sent.dtype == a.dtype and sent.device == a.device and sent.data_ptr() % 16 == 0
-            and not sent.requires_grad):
+            and not sent.requires_grad and not has_tangent(sent)):
         return False
     lo, hi = _byte_range(sent)
     return all(hi <= t_lo or t_hi <= lo for t_lo, t_hi in (_byte_range(a), _byte_range(b)))

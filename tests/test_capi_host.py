@@ -727,3 +727,27 @@ def test_shards_in_each_others_places_take_no_single_launch(monkeypatch):
     for first, taken in ((own[0], True), (out[:m], True), (out[m:2 * m], False), (out[1:m + 1], False), (out[(W - 1) * m:], False)):
         launched.clear()
         assert ag.gather_chunks(out, PeerBuffers([first, *own[1:]]), progress, 1, 0, 0) == taken == bool(launched)
+
+
+def test_tangents_keep_gathers_and_sends_from_the_kernels():
+    """A forward-mode tangent is handed on, or cleared, by torch's copies only, whether gradients are enabled or not."""
+    import torch.autograd.forward_ad as fw
+
+    from kraken_amd.comm import copy_engine_all_gather as ag
+    from kraken_amd.comm._common import PeerBuffers
+    from kraken_amd.fused.gemm_reduce_scatter_ce_persistent import _sends_direct
+
+    W, m, K = 2, 4, 16
+    out, a, b = torch.zeros(W * m, K, dtype=BF16), torch.zeros(W * m, K, dtype=BF16), torch.zeros(K, K, dtype=BF16)
+    shards, sent = [torch.zeros(m, K, dtype=BF16) for _ in range(W)], torch.zeros(W, m, K, dtype=BF16)
+    with fw.dual_level():
+        assert not ag.followed(out, PeerBuffers(shards)) and _sends_direct(sent, a, b, W, m, K)
+        for grad in (torch.no_grad, torch.enable_grad):
+            with grad():
+                dual = fw.make_dual(shards[1], torch.ones_like(shards[1]))
+                assert ag.followed(out, PeerBuffers([shards[0], dual]))
+                assert ag.followed(fw.make_dual(out, torch.ones_like(out)), PeerBuffers(shards))
+                assert not _sends_direct(fw.make_dual(sent, torch.ones_like(sent)), a, b, W, m, K)
+    with torch.no_grad():
+        assert ag._takes_copies(out.requires_grad_())
+    assert not ag._takes_copies(out)

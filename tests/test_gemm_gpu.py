@@ -1460,6 +1460,28 @@ def test_gather_inside_the_product_is_for_shards_apart(dev):
     assert not _direct(apart, a_out, b, W, 500, N, K) and not _direct(apart, a_out, b, W, 256, 1024, K)
 
 
+@pytest.mark.parametrize("m,N", [(40, 1024), (512, 4096)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_gathers_hand_tangents_on(dev, m, N, grad):
+    """Forward mode: the gathered matrix has the shards' tangents, and none of an earlier gather, also where the product or one launch would gather."""
+    import torch.autograd.forward_ad as fw
+    W, K = 8, 256
+    b = torch.randn(N, K, device=dev).to(BF16).T
+    shards, tangents = ([torch.randn(m, K, device=dev).to(BF16) for _ in range(W)] for _ in range(2))
+    calls = (lambda s, out: fused.all_gather_matmul(s, b, out)[0], comm.all_gather_w_progress)
+    with fw.dual_level(), torch.set_grad_enabled(grad):
+        duals = [fw.make_dual(s, t) if r != 2 else s for r, (s, t) in enumerate(zip(shards, tangents))]
+        for call in calls:
+            out = torch.zeros(W * m, K, dtype=BF16, device=dev)
+            primal, tangent = fw.unpack_dual(call(duals, out))
+            assert torch.equal(primal, torch.cat(shards))
+            assert torch.equal(tangent, torch.cat([t if r != 2 else torch.zeros_like(t) for r, t in enumerate(tangents)]))
+            assert not fw.unpack_dual(call(shards, out)).tangent.any()
+        sent = fw.make_dual(torch.zeros(2, 8, N, dtype=BF16, device=dev), torch.ones(2, 8, N, dtype=BF16, device=dev))
+        fused.gemm_reduce_scatter_ce_persistent(shards[0][:16], b, peers=torch.zeros(1, 8, N, dtype=BF16, device=dev), rank=1, sent=sent)
+        assert not fw.unpack_dual(sent).tangent[0].any()
+
+
 @pytest.mark.parametrize("m,N,K,dtype", [(40, 264, 256, BF16), (512, 4096, 256, BF16), (512, 1024, 128, torch.float8_e4m3fn), (6, 48, 48, torch.float8_e4m3fn)])
 @pytest.mark.parametrize("copy_engine", [False, True])
 def test_shards_in_each_others_places_are_gathered_whole(dev, m, N, K, dtype, copy_engine):
