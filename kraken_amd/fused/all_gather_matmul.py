@@ -6,7 +6,7 @@ import ctypes
 import torch
 
 from .. import _lib, _waits
-from ..comm._common import PeerBuffers
+from ..comm._common import PeerBuffers, has_tangent
 from ..comm.copy_engine_all_gather import _check_progress, _copy_engine_all_gather_w_progress, followed, gather_chunks, in_own_place
 from . import _gemm
 
@@ -45,6 +45,12 @@ def _direct(sources: list[int], a_out: torch.Tensor, b: torch.Tensor, W: int, m:
     shard, and shards apart from the gathered matrix (a tile may read a row after another one has written it)."""
     return (W <= _lib.KR_MAX_WORLD and _lib.load().kr_gather_matmul_direct(W, m, N, K) == 1
             and all(p % 16 == 0 for p in (a_out.data_ptr(), b.data_ptr(), *sources)) and all(in_own_place(sources, a_out)))
+
+
+def _copies_stream(peers: PeerBuffers, a_out: torch.Tensor, copy_engine: bool, dev: torch.device) -> torch.cuda.Stream | None:
+    """The stream of the copies, ``None`` for the side stream.  Copies that make a tangent of ``a_out`` run on the caller's, whose
+    memory it then is."""
+    return torch.cuda.current_stream(dev) if not copy_engine and has_tangent(a_out, *peers.tensors) else None
 
 
 def _local_shard(peers: PeerBuffers, rank: int, a_out: torch.Tensor) -> torch.Tensor | None:
@@ -107,13 +113,14 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
             a_out = torch.empty((M, K), dtype=fp8, device=dev)
         else:
             assert tuple(a_out.shape) == (M, K) and a_out.dtype == fp8 and a_out.is_contiguous()
-        if kwargs.get("copy_engine", False) or followed(a_out, peers) or not _gathered_first(a_out, peers, progress, splits, rank, dev):
+        copy_engine = kwargs.get("copy_engine", False)
+        if copy_engine or followed(a_out, peers) or not _gathered_first(a_out, peers, progress, splits, rank, dev):
             if progress is None:
                 progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)
             else:
                 progress.fill_(0)
-            backend_stream = _copy_engine_all_gather_w_progress(a_out, a_shared, progress, splits, rank=rank,
-                                                                copy_engine=kwargs.get("copy_engine", False))
+            backend_stream = _copy_engine_all_gather_w_progress(
+                a_out, a_shared, progress, splits, _copies_stream(peers, a_out, copy_engine, dev), rank=rank, copy_engine=copy_engine)
             if native:
                 status = kwargs.get("status")
                 own_status = status is None
@@ -256,7 +263,8 @@ def all_gather_matmul(
     else:
         assert tuple(a_out.shape) == (M, K) and a_out.dtype == torch.bfloat16 and a_out.is_contiguous()
     sources = peers.pointers()
-    side_stream = kwargs.get("copy_engine", False) or followed(a_out, peers)
+    copy_engine = kwargs.get("copy_engine", False)
+    side_stream = copy_engine or followed(a_out, peers)
     if not side_stream and _direct(sources, a_out, b, W, m, N, K):
         if progress is not None:
             _check_progress(progress, W * splits)
@@ -279,8 +287,8 @@ def all_gather_matmul(
         progress = torch.zeros(W * splits, dtype=torch.int32, device=dev)
     else:
         progress.fill_(0)
-    backend_stream = _copy_engine_all_gather_w_progress(a_out, a_shared, progress, splits, rank=rank,
-                                                        copy_engine=kwargs.get("copy_engine", False))
+    backend_stream = _copy_engine_all_gather_w_progress(
+        a_out, a_shared, progress, splits, _copies_stream(peers, a_out, copy_engine, dev), rank=rank, copy_engine=copy_engine)
     configs = {"RANK": rank, "WORLD_SIZE": W, "SPLITS_PER_RANK": splits,
                "wait_limit_us": kwargs.get("wait_limit_us", 0)}
     status = kwargs.get("status")

@@ -1,6 +1,7 @@
 """GPU parity of the bf16 MFMA GEMM with fused reduce(+bias) epilogue against the CPU oracle.
 Gate: rtol = atol = 2e-2 for bf16 outputs vs the fp32-accumulated oracle."""
 import ctypes
+import importlib
 import os
 
 import pytest
@@ -1462,13 +1463,15 @@ def test_gather_inside_the_product_is_for_shards_apart(dev):
 
 @pytest.mark.parametrize("m,N", [(40, 1024), (512, 4096)])
 @pytest.mark.parametrize("grad", [False, True])
-def test_gathers_hand_tangents_on(dev, m, N, grad):
+def test_gathers_hand_tangents_on(dev, monkeypatch, m, N, grad):
     """Forward mode: the gathered matrix has the shards' tangents, and none of an earlier gather, also where the product or one launch would gather."""
     import torch.autograd.forward_ad as fw
     W, K = 8, 256
     b = torch.randn(N, K, device=dev).to(BF16).T
     shards, tangents = ([torch.randn(m, K, device=dev).to(BF16) for _ in range(W)] for _ in range(2))
     calls = (lambda s, out: fused.all_gather_matmul(s, b, out)[0], comm.all_gather_w_progress)
+    # (the tangent is memory of the caller's stream: no copy runs on another one)
+    monkeypatch.setattr(importlib.import_module("kraken_amd.comm.copy_engine_all_gather"), "_get_backend_stream", lambda dev: 1 / 0)
     with fw.dual_level(), torch.set_grad_enabled(grad):
         duals = [fw.make_dual(s, t) if r != 2 else s for r, (s, t) in enumerate(zip(shards, tangents))]
         for call in calls:
