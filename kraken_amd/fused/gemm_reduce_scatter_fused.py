@@ -7,12 +7,14 @@ from .. import _lib
 from . import _gemm
 
 
-def _common_form(a, b, peers=None, rank=0, world_size=None, c_scratch=None, **_) -> torch.Tensor | None:
+def _common_form(a, b, peers=None, rank=0, c_scratch=None, **kwargs) -> torch.Tensor | None:
     """The call in native code where its arguments are of the common form: all peers in one tensor, a scratch to write to."""
-    if not (isinstance(peers, torch.Tensor) and isinstance(c_scratch, torch.Tensor) and a.dim() == 2):
+    if not (isinstance(peers, torch.Tensor) and peers.dim() == 3 and isinstance(c_scratch, torch.Tensor) and a.dim() == 2):
         return None
     W, M = len(peers) + 1, len(a)
-    if world_size not in (None, W) or M % W != 0 or not 0 <= rank < W:
+    # (a world_size that is passed is a number of ranks, or an error of the general path: None and 8.0 are no defaults)
+    world_size = kwargs.get("world_size", W)
+    if type(world_size) is not int or world_size != W or M % W != 0 or not 0 <= rank < W:
         return None
     return _lib.calls().gemm(a, b, peers, None, c_scratch, rank * (M // W), M // W, False, rank * (M // W))
 

@@ -29,6 +29,22 @@ def test_what_is_not_of_the_common_form_is_left_to_the_general_path(name):
             assert fn(*[value] * count) is None
 
 
+def test_world_size_of_the_reduce_scatter_is_a_number_of_ranks(monkeypatch):
+    """What the general path refuses is not taken by the native one: ``world_size`` absent or the number of ranks, nothing else."""
+    class Takes:
+        def gemm(self, *args):
+            return args
+
+    monkeypatch.setattr(_lib, "_calls", Takes())
+    a, b, peers, c = (torch.zeros(*s, dtype=BF16) for s in ((8, 16), (16, 8), (3, 2, 8), (8, 8)))
+    for kw, taken in (({}, True), ({"world_size": 4}, True), ({"world_size": None}, False), ({"world_size": 4.0}, False), ({"world_size": 2}, False)):
+        try:
+            out = fused.gemm_reduce_scatter(a, b, peers=peers, c_scratch=c, **kw)
+        except Exception:        # noqa: BLE001 (the general path's)
+            out = None
+        assert isinstance(out, tuple) == taken, kw
+
+
 def _both(monkeypatch, call):
     """``call()`` as it is and through the general path: two results, or two exceptions' types."""
     got = []
