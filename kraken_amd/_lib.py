@@ -3,12 +3,14 @@ from __future__ import annotations
 
 import ctypes
 import importlib.util
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from pathlib import Path
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libkraken_amd.so"
+CALLS_PATH = LIB_PATH.with_name("_calls.so")
 
 # negative return codes of the library (include/kraken_amd.h)
 KR_OK = 0
@@ -170,22 +172,41 @@ def load() -> ctypes.CDLL:
 _calls = None
 
 
+class _NoCalls:
+    """Stands in for the native form of the common calls: takes none, so each goes through its wrapper's general path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_calls():
+    from .comm._common import row_exchange, row_watch
+    from .fused._gemm import stream_workspace
+
+    lib = load()
+    spec = importlib.util.spec_from_file_location("kraken_amd._calls", CALLS_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    built_for = getattr(module, "torch_version", None)
+    if built_for != str(torch.__version__):      # (it reads torch's objects by their layout)
+        raise ImportError(f"built for torch {built_for}, not {torch.__version__}")
+    module.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in EXPORTS},
+                torch._C._cuda_getCurrentRawStream, row_exchange, row_watch, stream_workspace)
+    return module
+
+
 def calls():
-    """The native form of the common calls (``csrc/calls.cpp``), loaded once and bound to the library."""
+    """The native form of the common calls (``csrc/calls.cpp``), loaded once and bound to the library.  It only makes them
+    shorter: where it is missing or belongs to another torch, all calls take the general path, with one warning."""
     global _calls
     if _calls is None:
-        from .comm._common import row_exchange, row_watch
-        from .fused._gemm import stream_workspace
-
-        lib, path = load(), LIB_PATH.with_name("_calls.so")
-        if not path.exists():
-            raise RuntimeError(f"{path} is missing: build it with `python -m kraken_amd.build`")
-        spec = importlib.util.spec_from_file_location("kraken_amd._calls", path)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        module.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in EXPORTS},
-                    torch._C._cuda_getCurrentRawStream, row_exchange, row_watch, stream_workspace)
-        _calls = module
+        load()
+        try:
+            _calls = _load_calls()
+        except (ImportError, OSError) as e:
+            warnings.warn(f"kraken_amd: short calls cost the host more than they need to, {CALLS_PATH} is not usable ({e}): "
+                          "build it with `python -m kraken_amd.build`", RuntimeWarning, stacklevel=3)
+            _calls = _NoCalls()
     return _calls
 
 

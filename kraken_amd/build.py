@@ -62,7 +62,7 @@ def _build_calls() -> None:
 
     tmp = CALLS_PATH.with_suffix(".so.tmp")
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           "-DUSE_ROCM", *(f"-isystem{p}" for p in include_paths()), f"-isystem{sysconfig.get_paths()['include']}",
+           "-DUSE_ROCM", f'-DKR_TORCH_VERSION="{torch.__version__}"', *(f"-isystem{p}" for p in include_paths()), f"-isystem{sysconfig.get_paths()['include']}",
            str(CSRC / "calls.cpp"), f"-L{Path(torch.__file__).parent / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

@@ -432,4 +432,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__calls() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__calls() {
+    PyObject* m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", KR_TORCH_VERSION) != 0) Py_CLEAR(m);
+    return m;
+}

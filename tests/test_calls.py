@@ -12,11 +12,24 @@ BF16 = torch.bfloat16
 FUNCTIONS = {"all_reduce": 1, "all_reduce_bias": 5, "two_shot_share": 4, "two_shot_bias": 8, "reduce_rms_norm": 7, "rms_norm": 3, "gemm": 9}
 
 
-class _General:
-    """Stands in for the native module: takes no call."""
+_General = _lib._NoCalls      # stands in for the native module: takes no call
 
-    def __getattr__(self, name):
-        return lambda *args: None
+
+@pytest.mark.parametrize("fault", ["missing", "no library", "another torch"])
+def test_without_the_native_form_every_call_takes_the_general_path(monkeypatch, tmp_path, fault):
+    other = tmp_path / "_calls.so"
+    if fault == "no library":
+        other.write_bytes(b"\x7fELF")
+    monkeypatch.setattr(_lib, "_calls", None)
+    if fault == "another torch":
+        monkeypatch.setattr(_lib.torch, "__version__", "0.0")
+    else:
+        monkeypatch.setattr(_lib, "CALLS_PATH", other)
+    with pytest.warns(RuntimeWarning, match="not usable"):
+        native = _lib.calls()
+    assert native is _lib.calls() and all(getattr(native, name)(*[None] * n) is None for name, n in FUNCTIONS.items())
+    with pytest.raises(RuntimeError, match="run on a HIP device only"):
+        comm.one_shot_all_reduce(torch.zeros(2, 8, dtype=BF16))
 
 
 @pytest.mark.parametrize("name", FUNCTIONS)
