@@ -593,12 +593,13 @@ int kr_gemm_reduce_f32_ws(const void* A, int64_t lda_m, int64_t lda_k, const voi
  *   plan[0] workgroup tile: 256 (256x256 tile, global->LDS loads without registers) or 128
  *   plan[1] matrix-core block of the k loop: 16 (v_mfma_f32_16x16x32_bf16) or 32 (32x32x16)
  *   plan[2] 128 tile: workgroups per tile that share its K loop (1: one pass)
- *   plan[3] 256 tile: tiles of the last partial round that are split, plan[4] parts of each
+ *   plan[3] 256 tile: tiles whose K loops are split (those of the last partial round, or with few tiles all of them, and
+ *           then no other launch runs in front of the split one), plan[4] parts of each
  *   plan[5] column panels per scheduling group
  *   plan[6] 1: tiles that lie wholly in the reduce band add the peers on the matrix cores
  *   plan[7] bit 0: M or N is not a multiple of the tile or K of 64 (bounds-checked edges); bit 1: the
- *           tile is 256 x 224 (a plain product with transposed-contiguous B that fills whole rounds
- *           of the compute units with 224-column tiles and not with 256-column ones); bit 2: at most 64
+ *           tile is 256 x 224 (transposed-contiguous B: a plain product that fills whole rounds of the compute
+ *           units with 224-column tiles and not with 256-column ones, or few tiles, all split); bit 2: at most 64
  *           rows, gemm_skinny_kernel (16 to 64 columns per workgroup instead of tiles); bit 3: 128x128
  *           tiles in gemm_ks_kernel (no bit of 2 and 3: those of gemm_reduce_kernel)
  */

@@ -221,7 +221,9 @@ def gemm_plan(M: int, N: int, K: int, b_transposed: bool, n_peers: int = 0, band
     tile, block, splits, tail, tail_splits, group_n, mfma_peers, ragged = list(plan)
     n224, skinny, ks = bool(ragged & 2), bool(ragged & 4), bool(ragged & 8)
     ragged &= 1
-    if tile == 256:
+    if tile == 256 and tail == -(-M // 256) * -(-N // (224 if n224 else 256)):
+        kernel = "gemm_dtl_split_kernel"      # (followed by gemm_dtl_tail_finish_kernel, as every split tail is)
+    elif tile == 256:
         kernel = "gemm_dtl16n7_kernel" if n224 else "gemm_dtl16_kernel" if block == 16 else "gemm_dtl_kernel"
     else:
         kernel = "gemm_skinny_kernel" if skinny else "gemm_ks_kernel" if ks else "gemm_reduce_kernel"

@@ -1357,7 +1357,7 @@ extern "C" int kr_gemm_plan(int64_t M, int64_t N, int64_t K, int b_transposed, i
     plan[4] = p.tail_splits;
     plan[5] = p.group_n;
     plan[6] = whole_band_peers ? 1 : 0;
-    plan[7] = (M % p.tile != 0 || N % p.tile != 0 || K % 64 != 0) ? 1 : 0;
+    plan[7] = (M % p.tile != 0 || N % (p.n224 ? 224 : p.tile) != 0 || K % 64 != 0) ? 1 : 0;
     if (p.n224) plan[7] |= 2;   // bit 1: 256 x 224 tiles
     if (p.skinny) plan[7] |= 4;   // bit 2: gemm_skinny_kernel
     if (p.ks) plan[7] |= 8;   // bit 3: gemm_ks_kernel

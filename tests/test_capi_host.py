@@ -388,6 +388,16 @@ def test_gemm_plan_few_tiles_stay_split_where_224_divides_n(lib, M, N, K):
     assert p["tile_n"] == 256 and p["tail_tiles"] == (M // 256) * (N // 256) and p["tail_splits"] > 1
 
 
+@pytest.mark.parametrize("M,N,K,b_t,P,cols,ragged", [
+    (512, 6656, 8192, True, 7, 224, True), (512, 6720, 8192, True, 7, 224, False), (512, 6656, 8192, False, 7, 256, False),
+    (500, 6656, 8192, False, 7, 256, True),
+])
+def test_gemm_plan_names_the_launch_of_tiles_that_are_all_split(lib, M, N, K, b_t, P, cols, ragged):
+    p = _lib.gemm_plan(M, N, K, b_t, P, M // 8, False, True, workspace_bytes=lib.kr_gemm_workspace_bytes(M, N, K))
+    assert p["tail_tiles"] == -(-M // 256) * -(-N // cols) and p["tail_splits"] > 1
+    assert (p["kernel"], p["tile_n"], p["ragged"]) == ("gemm_dtl_split_kernel", cols, ragged)
+
+
 @pytest.mark.parametrize("M,N,K,b_t,tile", [
     (4096, 4672, 416, True, 128), (4096, 4672, 632, True, 128),      # 304 tiles of 256 x 256: a second round of 48
     (4096, 4672, 416, False, 256), (4096, 4672, 384, True, 256), (4096, 4672, 640, True, 256), (4096, 4672, 648, True, 256),
