@@ -565,8 +565,14 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     parts of whole tiles.  10.7 us, 1.03 us per k-step (row-major B 1.08, 224-column tiles 0.94) and 0.25 more with all
 //     compute units busy, 0.24 us per MB of parts; at least eight k-steps a part, K from 2048 on, and only where this is
 //     0.88 or less of the best 128x128 form (both models are off by a tenth; whole tiles with a long K need no margin).
-//     224 columns, transposed B only, where they fill enough more compute units to be 2 % ahead.  220 random shapes, 65 to
-//     2300 rows, other than those the model was fitted to: taken by 52, 0.56 to 0.98 of their time, 0.957 over all.  us,
+//     224 columns, transposed B only, where they fill enough more compute units to be 2 % ahead.
+//     Row-major B where the 128x128 form is one round of workgroups, which that model takes for up to a quarter dearer than
+//     it is, has to be 2 % ahead by a second one as well, fitted to 660 such shapes: in parts 25.4 us, 0.18 us per k-step and
+//     1.24 more with all compute units busy, 0.044 us per MB of operands; on 128x128 2.9 us, 0.53 us per k-step, 0.101 us per MB of
+//     operands, parts 0.9 us and 0.42 per MB.  1422 x 1088 x 7424 (40.7 us / 47.1 in parts), 632 x 2304 x 6208 with a band
+//     (37.7 / 42.2) and 640 x 4608 x 5120 (50.4 / 57.2) stay on 128x128; 330 other
+//     shapes that it leaves in parts take 0.60 to 1.033 of the 128x128 form's time there, 0.825 in the mean (without it 27 of 129 were
+//     slower, up to 1.16).  Shapes of the other kinds, 1360: 0.52 to 1.05, 15 of them slower.  us,
 //     128x128 / in parts: 504 x 6656 x 8192 with a band 82 / 66, 576 x 4608 x 10560 row-major 101 / 78, 998 x 6400 x 6336
 //     row-major 134 / 102, 1792 x 2432 x 12912 224 / 134; 512 x 6656 with a band and seven peers, 256 columns (208
 //     workgroups) / 224 (240), K = 8192 68.1 / 66.3, 16384 120 / 109.
@@ -631,6 +637,7 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, int n_pe
         // (the second round of gemm_reduce_kernel starts beside the first, see above)
         const int64_t wgs = tiles * p.splits, per = (steps + p.splits - 1) / p.splits;
         if (b_nt && wgs > 256 && wgs <= 512) best += (68 + 18 * wgs / 256 - 2 * step) * per;
+        const int small_splits = p.splits;
         best = best * 88 / 100;
         if (long_whole || (force > 0 && env.gemm_tile == 256)) best = INT64_MAX;
         for (const int cols : {256, 224}) {
@@ -645,6 +652,16 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, int n_pe
                 best = c;
                 p.big = cols;
                 p.splits = (int)s;
+            }
+        }
+        if (p.big && !b_nt && wgs <= 256 && !long_whole && force <= 0) {   // (see above)
+            const int64_t operands = 2 * (M + N) * K, parts = small_splits > 1 ? 4 * small_splits * M * N : 0;
+            const int64_t k = (steps + p.splits - 1) / p.splits, busy = p.splits * big_tiles_of(M, N, 256);
+            const int64_t in_parts = 2540 + (18 + 124 * busy / 256) * k + operands * 44 / 10000000;
+            const int64_t on_128 = 286 + 53 * per + (parts > 0 ? 89 : 0) + parts * 424 / 10000000 + operands * 101 / 10000000;
+            if (in_parts >= on_128 * 98 / 100) {
+                p.big = 0;
+                p.splits = small_splits;
             }
         }
     }

@@ -398,6 +398,17 @@ def test_gemm_plan_names_the_launch_of_tiles_that_are_all_split(lib, M, N, K, b_
     assert (p["kernel"], p["tile_n"], p["ragged"]) == ("gemm_dtl_split_kernel", cols, ragged)
 
 
+@pytest.mark.parametrize("M,N,K,b_t,P,band", [
+    (1422, 1088, 7424, False, 0, 1),      # us, 128 x 128 tiles / 256 x 256 in parts: 40.7 / 47.1
+    (632, 2304, 6208, False, 7, 8),       # 37.7 / 42.2
+    (1208, 1216, 5696, False, 7, 8),      # 34.0 / 39.0
+    (640, 4608, 5120, False, 7, 1),       # 50.4 / 57.2
+])
+def test_gemm_plan_keeps_small_tiles_where_large_ones_in_parts_are_slower(lib, M, N, K, b_t, P, band):
+    p = _lib.gemm_plan(M, N, K, b_t, P, M // band, False, band > 1, workspace_bytes=lib.kr_gemm_workspace_bytes(M, N, K))
+    assert p["tail_splits"] == 1
+
+
 @pytest.mark.parametrize("M,N,K,b_t,tile", [
     (4096, 4672, 416, True, 128), (4096, 4672, 632, True, 128),      # 304 tiles of 256 x 256: a second round of 48
     (4096, 4672, 416, False, 256), (4096, 4672, 384, True, 256), (4096, 4672, 640, True, 256), (4096, 4672, 648, True, 256),

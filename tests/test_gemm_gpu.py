@@ -580,7 +580,7 @@ def test_ragged_tiles_in_parts(dev, monkeypatch, M, N, K, S, cols):
             assert torch.equal(c, product.to(BF16))
 
 
-@pytest.mark.parametrize("M,N,K,b_t,cols", [(500, 6656, 8192, True, 224), (576, 4608, 5120, False, 256), (300, 1032, 4096, True, 128)])
+@pytest.mark.parametrize("M,N,K,b_t,cols", [(500, 6656, 8192, True, 224), (576, 4608, 10560, False, 256), (300, 1032, 4096, True, 128)])
 def test_ragged_tiles_in_parts_where_the_rule_takes_them(dev, M, N, K, b_t, cols):
     """Nothing forced: seven peers, bf16 result, against the exact sums."""
     plan = _lib.gemm_plan(M, N, K, b_t, 7, M, workspace_bytes=_lib.load().kr_gemm_workspace_bytes(M, N, K))
