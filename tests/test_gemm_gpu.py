@@ -548,10 +548,11 @@ def test_split_parts_of_very_few_k_steps(dev, monkeypatch, b_t, mfma):
 
 
 @pytest.mark.parametrize("cols", [256, 224])
-@pytest.mark.parametrize("M,N,K,S", [(513, 776, 576, 3), (255, 224, 128, 2), (264, 456, 1024, 8), (512, 448, 320, 5), (8, 8, 192, 2), (520, 680, 64 * 17, 4)])
+@pytest.mark.parametrize("M,N,K,S", [(513, 776, 576, 3), (255, 224, 128, 2), (264, 456, 1024, 8), (512, 448, 320, 5), (8, 8, 192, 2), (520, 680, 64 * 17, 4),
+                                     (513, 776, 600, 3), (264, 456, 1032, 5), (512, 448, 328, 2), (256, 256, 72, 2)])
 def test_ragged_tiles_in_parts(dev, monkeypatch, M, N, K, S, cols):
-    """Every 256 x 256 or 256 x 224 tile's K loop in parts, with edge tiles of one row, one 16-byte piece or all but one:
-    all rows with peers and bias, and a band that starts inside a tile.  Small integers: every fp32 sum is exact."""
+    """Every 256 x 256 or 256 x 224 tile's K loop in parts, with edge tiles of one row, one 16-byte piece or all but one,
+    and a last k-step of one 16-byte piece or more that is not full: all rows with peers and bias, and a band that starts inside a tile.  Small integers: every fp32 sum is exact."""
     monkeypatch.setenv("KRAKEN_AMD_GEMM_TILE", "256")
     monkeypatch.setenv("KRAKEN_AMD_GEMM_TAILSPLIT", str(S))
     monkeypatch.setenv("KRAKEN_AMD_GEMM_N224", str(int(cols == 224)))
