@@ -571,7 +571,7 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     1.24 more with all compute units busy, 0.044 us per MB of operands; on 128x128 2.9 us, 0.53 us per k-step, 0.101 us per MB of
 //     operands, parts 0.9 us and 0.42 per MB.  1422 x 1088 x 7424 (40.7 us / 47.1 in parts), 632 x 2304 x 6208 with a band
 //     (37.7 / 42.2) and 640 x 4608 x 5120 (50.4 / 57.2) stay on 128x128; 330 other
-//     shapes that it leaves in parts take 0.60 to 1.033 of the 128x128 form's time there, 0.825 in the mean (without it 27 of 129 were
+//     shapes that it leaves in parts take 0.63 to 1.033 of the 128x128 form's time there, 0.825 in the mean (without it 27 of 129 were
 //     slower, up to 1.16).  Shapes of the other kinds, 1360: 0.52 to 1.05, 15 of them slower.  us,
 //     128x128 / in parts: 504 x 6656 x 8192 with a band 82 / 66, 576 x 4608 x 10560 row-major 101 / 78, 998 x 6400 x 6336
 //     row-major 134 / 102, 1792 x 2432 x 12912 224 / 134; 512 x 6656 with a band and seven peers, 256 columns (208

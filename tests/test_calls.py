@@ -100,6 +100,58 @@ def _stacks(dev, W, rows, D):
 
 
 @pytest.mark.gpu
+def test_the_common_form_is_taken(dev, monkeypatch):
+    """Every native function takes its call in the common form, with each of its options, and gives the general path's bits
+    (that both paths agree, above and below, says nothing of which one ran)."""
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(BF16)      # noqa: E731
+    native, W, rows, D, rank = _lib.calls(), 8, 16, 8192, 3
+    stack, x, full, vec, w = rnd(W, rows, D), rnd(rows, D), rnd(rows, D), rnd(D), rnd(D)
+    reduced = orc.reduce(stack.cpu())
+
+    def own(t):                     # the stack with one rank's slice replaced
+        s = stack.clone()
+        s[rank] = t
+        return s
+
+    assert torch.equal(native.all_reduce(stack).cpu(), reduced)
+    for xv, bias in itertools.product((None, x), (None, full, vec)):
+        source = (stack if xv is None else own(xv)).cpu()
+        b32 = None if bias is None else bias.cpu()
+        y = torch.zeros(rows, D, dtype=BF16, device=dev)
+        assert native.all_reduce_bias(stack, xv, bias, y, rank) is True
+        want = torch.zeros_like(y)
+        fused.one_shot_all_reduce_bias(list(own(xv) if xv is not None else stack), None, bias, want)
+        assert torch.equal(y, want) and (bias is not None or torch.equal(y.cpu(), orc.reduce(source)))
+        assert native.reduce_rms_norm(stack, xv, bias, w, y, 1e-5, rank) is True
+        zero = torch.zeros(D, dtype=BF16) if b32 is None else b32
+        torch.testing.assert_close(y.cpu(), orc.reduce_bias_rms_norm(source, zero, w.cpu()), rtol=2e-2, atol=2e-2)
+    assert torch.equal(native.two_shot_share(stack, rank, False, 2048).cpu(), reduced.view(W, rows // W, D)[rank])
+    share = native.two_shot_share(stack, rank, True, 2048)
+    blocks = reduced.view(-1, W, 2048)[:, rank].reshape(-1)
+    assert torch.equal(share.cpu(), blocks)
+    for xv, bias, striped in itertools.product((None, x), (None, full), (False, True)):
+        out, want = torch.zeros(rows * D // W, dtype=BF16, device=dev), torch.zeros(rows * D // W, dtype=BF16, device=dev)
+        assert native.two_shot_bias(stack, xv, bias, out, 2048, rank, striped, rows * D) is True
+        fused.two_shot_all_reduce_bias(list(own(xv) if xv is not None else stack), None, bias, want, BLOCK_SIZE=2048, rank=rank,
+                                       layout="striped" if striped else "rows", numel=rows * D)
+        assert torch.equal(out, want)
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "_calls", _General())
+        normed = fused.rms_norm(x, w, 1e-5)
+    assert torch.equal(native.rms_norm(x, w, 1e-5), normed)
+    M, N, K = 64, 256, 512
+    for b in (rnd(K, N), rnd(N, K).T):
+        a, peers, c = rnd(M, K), rnd(3, M // 4, N), torch.zeros(M, N, dtype=BF16, device=dev)
+        for fp32 in (False, True):
+            out = native.gemm(a, b, None, vec[:N], None, 0, M, fp32, 0)
+            assert out.dtype == (torch.float32 if fp32 else BF16)
+            torch.testing.assert_close(out.float(), a.float() @ b.float() + vec[:N].float(), rtol=2e-2, atol=2e-2)
+        out, want = native.gemm(a, b, peers, None, c, M // 4, M // 4, False, M // 4), torch.zeros_like(c)
+        assert torch.equal(out, fused.gemm_reduce_scatter(a, b, peers=list(peers), rank=1, c_scratch=want)) and torch.equal(c, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W,rows,D", [(1, 3, 64), (2, 8, 1024), (3, 6, 136), (8, 16, 8192), (8, 8, 512), (16, 4, 72), (17, 2, 64), (4, 5, 20), (2, 1, 4096)])
 def test_row_calls_take_both_paths_alike(dev, monkeypatch, W, rows, D):
     g = torch.Generator(device=dev).manual_seed(7)
