@@ -488,8 +488,8 @@ static void fp8_split_plan(int64_t M, int64_t N, int64_t K, int* tail_out, int* 
 // 32 nb2 (nb2 = 0: none), or with at most 128 tiles of 256x256 every tile's K loop in `splits` parts.
 // Widths: whole rounds of 256-column tiles and the narrow ones behind them, the pair that ends first.  A round costs, in
 // 0.01 us, 4 us to start and finish its tiles and per k-step of 128 and 256 columns 2.05 us with up to 160 compute units
-// busy, 2.56 with all of them (the power limit), 3 % more per 32 columns less.  Measured, us, 256-column tiles / 224 / the
-// choice: 4000 x 6656 x 4096 164 / 150.5 / 146.2 (16 panels, then 160 columns), 8000 x 3584 x 8192 308.6 / 299.3 / 299.3,
+// busy, 2.56 with all of them (the power limit), 3 % more per 32 columns less.  Measured in turn, on a card of the slower ones
+// (the first call's choice takes 137 to 146 us on different cards), us, 256-column tiles / 224 / the choice: 4000 x 6656 x 4096 164 / 150.5 / 146.2 (16 panels, then 160 columns), 8000 x 3584 x 8192 308.6 / 299.3 / 299.3,
 // 2400 x 4992 x 8192 143.6 / 139.3 / 139.3, 8192 x 4096 x 8192 335.8 / 413.4 / 335.8.
 struct W8Plan {
     int panels, nb2, splits;
@@ -874,7 +874,9 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
 }
 
 // fp32 operands split in registers (gemm_f32.hip): 128x128 tiles, S workgroups per tile by the same kind of model
-// as plan_small: 7 us to start and finish, 0.9 us per step of 64 k and round of 256 workgroups.
+// as plan_small: 7 us to start and finish, 0.9 us per step of 64 k and round of 256 workgroups.  These choose the parts, they
+// do not give the time: 256 workgroups in one pass measure 1.6 us per step and 13.5 us outside the k loop with row-major B, 1.45
+// and 12 with transposed B, three peers 4 to 5 us more (1000 x 4096, K = 512 .. 8192: 26.6, 40.1, 66.4, 118.6, 216 us).
 static int split_f32(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
     if (const int v = env_switches().gemm_splitk; v >= 1 && v <= kMaxSplits) return (int)std::min<int64_t>(v, steps);   // testing and tuning
@@ -1140,7 +1142,12 @@ extern "C" int kr_all_gather_matmul_bf16(const void* A, int64_t lda_m, const voi
 }
 
 // Rows gathered by the product itself: shapes with enough tiles for one-pass workgroups of 256 rows, each inside one shard.
-// Time of this form over copies on a side stream with the tiles waiting for their flags: see all_gather_matmul.
+// us, copies on a side stream with tiles that wait for their flags / a gather launch in front of the product / this form,
+// W = 2, 4 and 8, 136 to 448 tiles, K = 1024 to 16384 (72 shapes): this form 0.31 to 0.99 of the first.  Of the second 0.82 to 0.95
+// at K = 1024 and 0.84 to 0.98 at K = 4096 and 8192 (8 x 512 x 4096, N = 4096 155 / 115 / 101; 8 x 1024 x 8192, N = 3584
+// 404 / 369 / 345), but for 257 to 352 tiles from K = 4096 on, 0.95 to 1.38: a product with a workspace splits its last round
+// (8 x 512, N = 4352: K = 4096 220 / 142 / 170, 8192 366 / 243 / 320, 16384 682 / 465 / 639); at K = 16384 and other counts
+// 0.97 to 1.16 (8 x 1024, N = 1280 481 / 390 / 454).
 extern "C" int kr_gather_matmul_direct(int W, int64_t rows_per_shard, int64_t N, int64_t K) {
     if (W < 1 || W > KR_MAX_WORLD || rows_per_shard <= 0 || rows_per_shard % 256 != 0 || rows_per_shard > 0x7fffffffLL / W) return 0;
     if (N <= 0 || N > 0x7fffffffLL || K > 0x7fffffffLL || K % 8 != 0 || N % 8 != 0) return 0;

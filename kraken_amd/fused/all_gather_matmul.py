@@ -66,7 +66,9 @@ def _gathered_first(a_out, peers: PeerBuffers, progress, splits: int, rank: int,
     On one GPU nothing is gained by the side stream: its copies wait for compute units of the running product, and
     its events, flags and status word cost the host 100 us.  Calls one behind the other, us, with the side stream /
     in front: W = 8, 1 x 1024, N = 1024 125 / 38; 8 x 130 x 8192, N = 8192 205 / 176; 8 x 500 x 4096, N = 6656 232 / 188;
-    8 x 1000 x 8192, N = 1024 286 / 185, N = 3584 450 / 389; 2 x 1000 x 16384, N = 8192 429 / 393."""
+    8 x 1000 x 8192, N = 1024 286 / 185, N = 3584 450 / 389; 2 x 1000 x 16384, N = 8192 429 / 393.
+    fp8 of whole tiles, whose product could follow the flags: 8 x 32 x 1024, N = 1024 104 / 29; 8 x 1024 x 4096, N = 3584 153 / 106,
+    K = 8192 266 / 184; N = 8192, K = 16384 760 / 722; 63 shapes 0.25 to 0.96."""
     flags = progress
     if progress is None:
         flags = torch.empty(peers.W * splits, dtype=torch.int32, device=dev)     # counted in, read by nobody
@@ -87,7 +89,7 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
     The two differ in the precision of the sums: the fp8 instruction keeps about 16 bits of them (1.2e-5 in the
     2-norm against 64 bits, K = 128 .. 16384; both the 16x16x32 and the 16x16x128 form, to the same bits), the bf16
     instruction all 24 (2e-9 at K = 4096), so ragged shapes are not sent to the fp8 kernel although its C entry points
-    take them: 4000 x 6656 x 4096 takes 83 us there and 146 us here, with 5e-4 of the results one fp8 step off."""
+    take them: 4000 x 6656 x 4096 takes 83 us there and 139 us here, with 5e-4 of the results one fp8 step off."""
     fp8 = torch.float8_e4m3fn
     W = peers.W
     m, K = peers.shape
