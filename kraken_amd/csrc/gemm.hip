@@ -1277,6 +1277,8 @@ static int gemm_fp8_wide(const void* A, int64_t lda, const void* Bt, int64_t ldb
                          int64_t tile_pivot, void* workspace, int64_t workspace_bytes, void* stream) {
     if (M < 0 || N < 0 || K < 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return KR_ERR_BAD_DIM;
     if (N % 16 != 0 || K % 16 != 0) return KR_ERR_BAD_DIM;
+    // (an operand with elements has to be aligned whether or not there is a product)
+    if (K > 0 && ((M > 0 && !aligned16(A)) || (N > 0 && !aligned16(Bt)))) return KR_ERR_ALIGNMENT;
     if (M == 0 || N == 0) return KR_OK;
     if (K == 0) return KR_ERR_BAD_DIM;
     if (A == nullptr || Bt == nullptr || out == nullptr) return KR_ERR_NULL_POINTER;

@@ -772,3 +772,10 @@ def test_tangents_keep_gathers_and_sends_from_the_kernels():
     with torch.no_grad():
         assert ag._takes_copies(out.requires_grad_())
     assert not ag._takes_copies(out)
+
+
+def test_fp8_wide_empty_products_check_the_operand_that_has_elements(lib):
+    f = lib.kr_gemm_fp8_wide_ws
+    for off, M, N, want in ((8, 0, 64, 0), (8, 16, 0, _lib.KR_ERR_ALIGNMENT), (0, 16, 0, 0), (0, 0, 64, 0)):
+        assert f(FAKE + off, 64, FAKE, 64, M, N, 64, FAKE, 0, None, 0, None) == want
+        assert f(FAKE, 64, FAKE + off, 64, N, M, 64, FAKE, 0, None, 0, None) == want
