@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "gemm_common.h"
@@ -566,13 +567,19 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     compute units busy, 0.24 us per MB of parts; at least eight k-steps a part, K from 2048 on, and only where this is
 //     0.88 or less of the best 128x128 form (both models are off by a tenth; whole tiles with a long K need no margin).
 //     224 columns, transposed B only, where they fill enough more compute units to be 2 % ahead.
-//     Row-major B where the 128x128 form is one round of workgroups, which that model takes for up to a quarter dearer than
-//     it is, has to be 2 % ahead by a second one as well, fitted to 660 such shapes: in parts 25.4 us, 0.18 us per k-step and
-//     1.24 more with all compute units busy, 0.044 us per MB of operands; on 128x128 2.9 us, 0.53 us per k-step, 0.101 us per MB of
-//     operands, parts 0.9 us and 0.42 per MB.  1422 x 1088 x 7424 (40.7 us / 47.1 in parts), 632 x 2304 x 6208 with a band
-//     (37.7 / 42.2) and 640 x 4608 x 5120 (50.4 / 57.2) stay on 128x128; 330 other
-//     shapes that it leaves in parts take 0.63 to 1.033 of the 128x128 form's time there, 0.825 in the mean (without it 27 of 129 were
-//     slower, up to 1.16).  Shapes of the other kinds, 1360: 0.52 to 1.05, 15 of them slower.  us,
+//     Two kinds of shapes where the 128x128 forms are cheaper than that model says have to clear a second bar (calls one behind
+//     the other, four sets of operands in turn, 1700 shapes in all):
+//     * M and N multiples of 128: those forms have no edge tiles then, and a short K does not pay for the second launch.  The bar
+//       rises with the doublings of K from 2048 on: one round of 128x128 workgroups 0.51 + 0.14 a doubling (transposed B 0.51 + 0.19),
+//       more 0.67 + 0.11 (0.83 + 0.04).  1180 shapes: of the 890 below the bar 64 are slower in parts, 33 by more than 3 %, up
+//       to 1.16, 0.844 in the mean; above it 222 of 290 are, up to 1.33, 1.077 in the mean.  512 x 4352 x 4096 row-major with a band
+//       (32.4 us / 39.2 in parts), x 3072 transposed (29.5 / 33.9), 2816 x 2560 x 3072 row-major (52.9 / 63.5) stay on 128x128;
+//     * other shapes with row-major B and one round of 128x128 workgroups: 6 % ahead by a closer fit of both: in parts 25.4 us, 0.18 us
+//       per k-step and 1.24 more with all compute units busy, 0.044 us per MB of operands; on 128x128 2.9 us, 0.53 us per k-step,
+//       0.101 us per MB of operands, parts 0.9 us and 0.42 per MB.  93 shapes: 4 of the 58 below the bar are slower in parts, up to
+//       1.04, 25 of the 35 above it, up to 1.15 (1422 x 1088 x 7424 40.7 / 47.1, 632 x 2304 x 6208 with a band 37.7 / 42.2).
+//     The rest, 427 shapes: 0.55 to 1.05, 0.797 in the mean, 4 of them slower.  540 shapes of all kinds drawn after the bars were set and
+//     left in parts: 25 slower, 14 by more than 3 %, up to 1.09, 0.827 in the mean.  us,
 //     128x128 / in parts: 504 x 6656 x 8192 with a band 82 / 66, 576 x 4608 x 10560 row-major 101 / 78, 998 x 6400 x 6336
 //     row-major 134 / 102, 1792 x 2432 x 12912 224 / 134; 512 x 6656 with a band and seven peers, 256 columns (208
 //     workgroups) / 224 (240), K = 8192 68.1 / 66.3, 16384 120 / 109.
@@ -637,7 +644,9 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, int n_pe
         // (the second round of gemm_reduce_kernel starts beside the first, see above)
         const int64_t wgs = tiles * p.splits, per = (steps + p.splits - 1) / p.splits;
         if (b_nt && wgs > 256 && wgs <= 512) best += (68 + 18 * wgs / 256 - 2 * step) * per;
+        const int64_t small_cost = best;
         const int small_splits = p.splits;
+        int64_t big_cost = 0;
         best = best * 88 / 100;
         if (long_whole || (force > 0 && env.gemm_tile == 256)) best = INT64_MAX;
         for (const int cols : {256, 224}) {
@@ -649,20 +658,28 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, int n_pe
                 const int64_t bytes = gemm_dtl_tail_workspace_bytes((int)big_tiles, (int)s, cols), k = (steps + s - 1) / s;
                 const int64_t c = 1070 + ((cols == 224 ? 94 : b_nt ? 103 : 108) + 25 * s * big_tiles / 256) * k + bytes * 241 / 10000000;
                 if (bytes > KR_STATIC_SCRATCH_BYTES || c >= best) continue;   // (the form that allocates nothing takes every split)
-                best = c;
+                best = big_cost = c;
                 p.big = cols;
                 p.splits = (int)s;
             }
         }
-        if (p.big && !b_nt && wgs <= 256 && !long_whole && force <= 0) {   // (see above)
+        // where that model is too kind to the parts (see above)
+        bool ahead = true;
+        if (p.big && M % 128 == 0 && N % 128 == 0) {
+            const double doublings = std::log2((double)K / 2048);
+            const double limit = b_nt ? (wgs <= 256 ? 0.51 + 0.19 * doublings : 0.83 + 0.04 * doublings)
+                                      : (wgs <= 256 ? 0.51 + 0.14 * doublings : 0.67 + 0.11 * doublings);
+            ahead = big_cost < limit * small_cost;
+        } else if (p.big && !b_nt && wgs <= 256) {
             const int64_t operands = 2 * (M + N) * K, parts = small_splits > 1 ? 4 * small_splits * M * N : 0;
             const int64_t k = (steps + p.splits - 1) / p.splits, busy = p.splits * big_tiles_of(M, N, 256);
             const int64_t in_parts = 2540 + (18 + 124 * busy / 256) * k + operands * 44 / 10000000;
             const int64_t on_128 = 286 + 53 * per + (parts > 0 ? 89 : 0) + parts * 424 / 10000000 + operands * 101 / 10000000;
-            if (in_parts >= on_128 * 98 / 100) {
-                p.big = 0;
-                p.splits = small_splits;
-            }
+            ahead = in_parts < on_128 * 94 / 100;
+        }
+        if (!ahead && !long_whole && force <= 0) {
+            p.big = 0;
+            p.splits = small_splits;
         }
     }
     return choose_kernel();

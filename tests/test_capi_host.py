@@ -403,6 +403,9 @@ def test_gemm_plan_names_the_launch_of_tiles_that_are_all_split(lib, M, N, K, b_
     (632, 2304, 6208, False, 7, 8),       # 37.7 / 42.2
     (1208, 1216, 5696, False, 7, 8),      # 34.0 / 39.0
     (640, 4608, 5120, False, 7, 1),       # 50.4 / 57.2
+    (512, 4352, 4096, False, 7, 8),       # 32.4 / 39.2
+    (512, 4352, 3072, True, 7, 8),        # 29.5 / 33.9
+    (2816, 2560, 3072, False, 7, 8),      # 52.9 / 63.5
 ])
 def test_gemm_plan_keeps_small_tiles_where_large_ones_in_parts_are_slower(lib, M, N, K, b_t, P, band):
     p = _lib.gemm_plan(M, N, K, b_t, P, M // band, False, band > 1, workspace_bytes=lib.kr_gemm_workspace_bytes(M, N, K))
