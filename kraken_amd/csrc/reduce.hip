@@ -133,15 +133,18 @@ __global__ __launch_bounds__(kThreads) void reduce_kernel(
 // workgroups takes (kernel time, W = 8, chain / together: 256 x 4096 6.0 / 2.35 us, 2047 x 5120 with a bias 7.6 / 5.7, 8000 x 5120 19.6 / 17.8).
 // Above kChainVecs the chip is full of waves either way, and with W = 8 the chain keeps HBM a little busier (16384 x 8192 48.1 /
 // 49.3; W = 4 and 2 level).  256 threads a workgroup are 1 to 3 % slower in both forms at 16384 rows.
-constexpr int kStripedThreads = kWave;
-constexpr int64_t kChainVecs = 1 << 20;
+// In between four and sixteen buffers, whose slices lie a power of two apart in many calls, are read faster by a chain in
+// workgroups of 256 threads, from kTogetherVecs on: W = 4, 2^18, 2^19 and 2^20 vectors 5.5 us / 6.0 together, 8.6 / 9.9, 16.3 / 17.5,
+// sizes that are no power of two 0.95 to 1.06; W = 16, half as many again (below it is slower), 2^19 and 2^20 23.9 / 25.9, 45.9 / 48.2.
+// The mean over 256 k to 1 M vectors of together over chain with W = 6, 8, 9, 13: 0.97 to 1.00.
+constexpr int64_t kTogetherVecs = 1 << 18, kChainVecs = 1 << 20;
 
-template <class SRC, int WT, bool TOGETHER>
-__global__ __launch_bounds__(kStripedThreads) void reduce_striped_kernel(
+template <class SRC, int WT, bool TOGETHER, int THREADS>
+__global__ __launch_bounds__(THREADS) void reduce_striped_kernel(
     const SRC src, int w_rt, int64_t share_nvec,
     const u32x4* __restrict__ bias, uint32_t blk_v, int rank, u32x4* __restrict__ out) {
     const int W = WT > 0 ? WT : w_rt;
-    const int64_t j = (int64_t)blockIdx.x * kStripedThreads + threadIdx.x;
+    const int64_t j = (int64_t)blockIdx.x * THREADS + threadIdx.x;
     if (j >= share_nvec) return;
     const int64_t stripe = j / blk_v;
     const int64_t i = (stripe * W + rank) * blk_v + (j - stripe * blk_v);
@@ -151,9 +154,14 @@ __global__ __launch_bounds__(kStripedThreads) void reduce_striped_kernel(
     if constexpr (TOGETHER) {
         if (bias != nullptr) bv = ld_stream(bias + i);
         add_all<1>([&](int r, int) { return ld_stream(src.at(r) + i); }, W, acc);
-    } else {
+    } else if constexpr (THREADS == kWave) {
 #pragma unroll 1
         for (int r = 0; r < W; ++r) add8(ld_stream(src.at(r) + i), acc[0]);
+        if (bias != nullptr) bv = ld_stream(bias + i);
+    } else {
+        // (the first buffer in front of the loop and the loop left to the compiler: 1 to 5 % at these sizes)
+        add8(ld_stream(src.at(0) + i), acc[0]);
+        for (int r = 1; r < W; ++r) add8(ld_stream(src.at(r) + i), acc[0]);
         if (bias != nullptr) bv = ld_stream(bias + i);
     }
     if (bias != nullptr) add8(bv, acc[0]);
@@ -347,16 +355,16 @@ static int launch_striped(const SRC& tab, int W, int64_t share, const void* bias
                           int rank, void* out, void* stream) {
     if (bias != nullptr && !aligned16(bias)) return KR_ERR_ALIGNMENT;
     const int64_t nvec = share / 8;
-    const int64_t blocks = (nvec + kStripedThreads - 1) / kStripedThreads;
-    if (blocks > 0x7fffffffLL || stripe_block / 8 > 0xffffffffLL) return KR_ERR_BAD_DIM;
-#define KR_LAUNCH(WT, TOGETHER)                                                                                                   \
-    hipLaunchKernelGGL((reduce_striped_kernel<SRC, WT, TOGETHER>), dim3((unsigned)blocks), dim3(kStripedThreads), 0, (hipStream_t)stream, tab, \
-                       W, nvec, (const u32x4*)bias, (uint32_t)(stripe_block / 8), rank, (u32x4*)out)
-    if (nvec > kChainVecs) KR_LAUNCH(0, false);
-    else if (W == 8) KR_LAUNCH(8, true);
-    else if (W == 4) KR_LAUNCH(4, true);
-    else if (W == 2) KR_LAUNCH(2, true);
-    else KR_LAUNCH(0, true);
+    if ((nvec + kWave - 1) / kWave > 0x7fffffffLL || stripe_block / 8 > 0xffffffffLL) return KR_ERR_BAD_DIM;
+#define KR_LAUNCH(WT, TOGETHER, THREADS)                                                                                         \
+    hipLaunchKernelGGL((reduce_striped_kernel<SRC, WT, TOGETHER, THREADS>), dim3((unsigned)((nvec + THREADS - 1) / THREADS)), dim3(THREADS), 0, \
+                       (hipStream_t)stream, tab, W, nvec, (const u32x4*)bias, (uint32_t)(stripe_block / 8), rank, (u32x4*)out)
+    if (nvec > kChainVecs) KR_LAUNCH(0, false, kWave);
+    else if ((W == 4 && nvec >= kTogetherVecs) || (W == 16 && 2 * nvec >= 3 * kTogetherVecs)) KR_LAUNCH(0, false, kThreads);
+    else if (W == 8) KR_LAUNCH(8, true, kWave);
+    else if (W == 4) KR_LAUNCH(4, true, kWave);
+    else if (W == 2) KR_LAUNCH(2, true, kWave);
+    else KR_LAUNCH(0, true, kWave);
 #undef KR_LAUNCH
     return (int)hipGetLastError();
 }

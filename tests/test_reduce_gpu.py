@@ -274,6 +274,25 @@ def test_striped_share_at_a_million_vectors(dev, more):
     assert torch.equal(share, (stack[0, idx].float() + stack[1, idx].float()).to(BF16))
 
 
+@pytest.mark.parametrize("W,nvec", [(4, (1 << 18) - 1), (4, 1 << 18), (4, (1 << 18) + 65), (16, (3 << 17) - 1), (16, 3 << 17)])
+@pytest.mark.parametrize("as_list", [False, True])
+def test_striped_share_where_loads_become_a_chain(dev, W, nvec, as_list):
+    """The largest share of four and sixteen buffers whose loads go out together and the smallest ones read by a chain, with a bias."""
+    g = torch.Generator(device=dev).manual_seed(W)
+    block, whole = 8 * W, (nvec - 1) // W               # rank 0: `whole` blocks and a last one that may be cut
+    numel = W * block * whole + 8 * (nvec - W * whole)
+    stack = torch.randn(W, numel, generator=g, device=dev, dtype=BF16)
+    bias = torch.randn(numel, generator=g, device=dev, dtype=BF16)
+    share = torch.empty(8 * nvec, device=dev, dtype=BF16)
+    fused.two_shot_all_reduce_bias(list(stack) if as_list else stack, None, bias, share, BLOCK_SIZE=block, rank=0, layout="striped", numel=numel)
+    i = torch.arange(8 * nvec, device=dev)
+    i = i // block * (W * block) + i % block
+    want = stack[0][i].float()
+    for r in range(1, W):
+        want = want + stack[r][i].float()
+    assert torch.equal(share, (want + bias[i].float()).to(BF16))
+
+
 def test_full_size_config2(dev):
     """benchmark config 2: stack [8,4096,4096] -> [4096,4096], and the two-shot 1/8 row chunk.
     Checked exactly against the oracle on sampled row bands, and by linearity on the whole."""
