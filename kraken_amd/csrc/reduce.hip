@@ -174,14 +174,17 @@ __global__ __launch_bounds__(THREADS) void reduce_striped_kernel(
 // the slices of one tensor or buffers of their own (SRC, common.h), so what the other ranks sent is read where it is.
 // W known at compile time and single-wave workgroups: no branch between the requests (kernel time, W = 8: 1 x 1600 2.6 -> 2.3 us,
 // 18 x 1728 2.8 -> 2.5, 1024 x 4096 level, 1024 x 8192 28.4 -> 27.4).
-constexpr int kRotatedThreads = kWave;
+// Bands of kRotatedWide to kRotatedFull vectors, W = 4 and 8, lie a power of two apart in many calls: workgroups of 256 threads (us, single
+// waves / 256 threads, W = 8: 256 x 4096 5.9 / 4.8, 512 x 4096 9.15 / 8.4, 768 x 4096 11.7 / 10.9, 256 x 5120 5.5 / 5.6; W = 4 5.1 / 4.9 at
+// 512 x 4096); above single waves again (W = 8, 1000 x 4096 14.2 / 14.6, 1024 x 6144 20.5 / 21.8).
+constexpr int64_t kRotatedWide = 1 << 17, kRotatedFull = 15 << 15;
 
-template <class SRC, bool ACC_BF16, int WT>
-__global__ __launch_bounds__(kRotatedThreads) void reduce_rotated_kernel(
+template <class SRC, bool ACC_BF16, int WT, int THREADS>
+__global__ __launch_bounds__(THREADS) void reduce_rotated_kernel(
     const SRC src, int w_rt, int64_t band_v, int rank, u32x4* __restrict__ out) {
     const int W = WT > 0 ? WT : w_rt;
     constexpr int G = 8;
-    const int64_t v = (int64_t)blockIdx.x * kRotatedThreads + threadIdx.x;
+    const int64_t v = (int64_t)blockIdx.x * THREADS + threadIdx.x;
     if (v >= band_v) return;
     float acc[8];
     const int first = (rank + 1) % W;
@@ -396,22 +399,21 @@ extern "C" int kr_reduce_striped_ptrs_bf16(const void* const* bufs, int W, int64
 
 template <class SRC>
 static int launch_rotated(const SRC& src, int W, int64_t band_v, int rank, int acc_bf16, void* out, void* stream) {
-    const int64_t blocks = (band_v + kRotatedThreads - 1) / kRotatedThreads;
-    if (blocks > 0x7fffffffLL) return KR_ERR_BAD_DIM;
-#define KR_LAUNCH(WT)                                                                                                                       \
-    do {                                                                                                                                    \
-        if (acc_bf16)                                                                                                                       \
-            hipLaunchKernelGGL((reduce_rotated_kernel<SRC, true, WT>), dim3((unsigned)blocks), dim3(kRotatedThreads), 0,                    \
-                               (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);                                                     \
-        else                                                                                                                                \
-            hipLaunchKernelGGL((reduce_rotated_kernel<SRC, false, WT>), dim3((unsigned)blocks), dim3(kRotatedThreads), 0,                   \
-                               (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out);                                                     \
+    if ((band_v + kWave - 1) / kWave > 0x7fffffffLL) return KR_ERR_BAD_DIM;
+    const bool wide = band_v >= kRotatedWide && band_v < kRotatedFull;
+#define KR_LAUNCH(WT, THREADS)                                                                                                     \
+    do {                                                                                                                           \
+        const dim3 grid((unsigned)((band_v + THREADS - 1) / THREADS)), block(THREADS);                                             \
+        if (acc_bf16)                                                                                                              \
+            hipLaunchKernelGGL((reduce_rotated_kernel<SRC, true, WT, THREADS>), grid, block, 0, (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out); \
+        else                                                                                                                       \
+            hipLaunchKernelGGL((reduce_rotated_kernel<SRC, false, WT, THREADS>), grid, block, 0, (hipStream_t)stream, src, W, band_v, rank, (u32x4*)out); \
     } while (0)
     switch (W) {
-        case 2: KR_LAUNCH(2); break;
-        case 4: KR_LAUNCH(4); break;
-        case 8: KR_LAUNCH(8); break;
-        default: KR_LAUNCH(0); break;
+        case 2: KR_LAUNCH(2, kWave); break;
+        case 4: if (wide) KR_LAUNCH(4, kThreads); else KR_LAUNCH(4, kWave); break;
+        case 8: if (wide) KR_LAUNCH(8, kThreads); else KR_LAUNCH(8, kWave); break;
+        default: KR_LAUNCH(0, kWave); break;
     }
 #undef KR_LAUNCH
     return (int)hipGetLastError();

@@ -274,6 +274,23 @@ def test_striped_share_at_a_million_vectors(dev, more):
     assert torch.equal(share, (stack[0, idx].float() + stack[1, idx].float()).to(BF16))
 
 
+@pytest.mark.parametrize("W", [4, 8])
+@pytest.mark.parametrize("nvec", [(1 << 17) - 1, 1 << 17, (1 << 17) + 1, (15 << 15) - 1, 15 << 15])
+def test_rotated_reduce_where_workgroups_become_wider(dev, W, nvec):
+    """The bands on either side of both lines between single waves and 256 threads, the order of the sum and its roundings."""
+    from kraken_amd.fused.gemm_reduce_scatter_ce_persistent import reduce as rotated_reduce
+    g = torch.Generator(device=dev).manual_seed(W)
+    inp, rank = torch.randn(W, 8 * nvec, generator=g, device=dev, dtype=BF16), W - 2
+    for fp32_acc in (False, True):
+        out = torch.empty(1, 8 * nvec, device=dev, dtype=BF16)
+        rotated_reduce(inp, out, {"RANK": rank, "WORLD_SIZE": W, "fp32_acc": fp32_acc})
+        want = torch.zeros(8 * nvec, device=dev)
+        for i in range(W):
+            want = want + inp[(i + rank + 1) % W].float()
+            want = want if fp32_acc else want.to(BF16).float()
+        assert torch.equal(out[0], want.to(BF16))
+
+
 @pytest.mark.parametrize("W,nvec", [(4, (1 << 18) - 1), (4, 1 << 18), (4, (1 << 18) + 65), (16, (3 << 17) - 1), (16, 3 << 17)])
 @pytest.mark.parametrize("as_list", [False, True])
 def test_striped_share_where_loads_become_a_chain(dev, W, nvec, as_list):
