@@ -490,7 +490,7 @@ static void fp8_split_plan(int64_t M, int64_t N, int64_t K, int* tail_out, int* 
 // Widths: whole rounds of 256-column tiles and the narrow ones behind them, the pair that ends first.  A round costs, in
 // 0.01 us, 4 us to start and finish its tiles and per k-step of 128 and 256 columns 2.05 us with up to 160 compute units
 // busy, 2.56 with all of them (the power limit), 3 % more per 32 columns less.  Measured in turn, on a card of the slower ones
-// (the first call's choice takes 137 to 146 us on different cards), us, 256-column tiles / 224 / the choice: 4000 x 6656 x 4096 164 / 150.5 / 146.2 (16 panels, then 160 columns), 8000 x 3584 x 8192 308.6 / 299.3 / 299.3,
+// (the first call's choice takes 135 to 146 us on different cards), us, 256-column tiles / 224 / the choice: 4000 x 6656 x 4096 164 / 150.5 / 146.2 (16 panels, then 160 columns), 8000 x 3584 x 8192 308.6 / 299.3 / 299.3,
 // 2400 x 4992 x 8192 143.6 / 139.3 / 139.3, 8192 x 4096 x 8192 335.8 / 413.4 / 335.8.
 struct W8Plan {
     int panels, nb2, splits;

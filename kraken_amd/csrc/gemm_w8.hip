@@ -1,7 +1,7 @@
 // Product of fp8 (e4m3fn) operands whose sums keep all 24 bits: the operands stay fp8 in memory and in LDS and are widened
 // to bf16 (exactly) in registers, between LDS and the bf16 matrix cores.  The fp8 matrix-core instruction keeps about 16
 // bits of a sum, so shapes that promise 24 used to take two conversion passes, a bf16 product with an fp32 result
-// and a third pass: 4000 x 6656 x 4096 in 257 us, now 139 (137 to 146 on different cards); 64 x 8192 x 8192 96 -> 37; 700 x 7168 x 8192 164 -> 78.
+// and a third pass: 4000 x 6656 x 4096 in 257 us, now 139 (135 to 146 on different cards); 64 x 8192 x 8192 96 -> 37; 700 x 7168 x 8192 164 -> 78.
 //
 // Bound by the bf16 matrix cores.  Tile, waves, LDS stages and loads are those of the 256x256 kernel (gemm_dtl.hip):
 // 256 rows, four wavefronts of 128 x 16 NB, rows of 128 bytes per stage -- 128 k here, so a stage lasts four sub-steps of
