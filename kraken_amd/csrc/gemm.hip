@@ -451,6 +451,9 @@ static void tail_split_plan(int64_t tiles, int64_t K, int* tail_out, int* splits
     const int64_t tail = tiles % 256;
     // (measured: 16..64 tail tiles gain 5-25 % from K = 4096 on; 128 tail tiles at K = 2048 lose
     // 12 %: half a round saved does not pay for two more launches and 64 MiB of parts)
+    // Ragged shapes the same, us, whole rounds / in parts, transposed B unless said: 5486 x 3456 x 9984 397 / 310 (308 tiles),
+    // 4900 x 3648 x 4096 172 / 152, row-major 188 / 157, 2312 x 8000 x 6144 271 / 218, 4584 x 7744 x 5376 348 / 324; below K = 4096
+    // transposed B gains little and less with a K of 2048: 4600 x 4096 x 3072 131 / 124, x 2048 88 / 95.
     if (tail == 0 || (tail > 96 && tiles > 128) || (K < 4096 && force <= 0)) return;
     int64_t s = std::min<int64_t>(256 / tail, kMaxTailSplits);
     s = std::min<int64_t>(s, (K / 64) / kMinSplitSteps);
@@ -851,7 +854,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
         p.n224 = small.big == 224;
         p.tail_tiles = (int)big_tiles_of(M, N, small.big);
         p.tail_splits = small.splits;
-    } else if (dtl && has_workspace && !has_progress && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
+    } else if (dtl && has_workspace && !has_progress && (p.mi16 || (M % 256 == 0 && N % 256 == 0 && K % 64 == 0))) {
         int tail, ts;
         tail_split_plan(tiles_m * tiles_n, K, &tail, &ts);
         if (tail > 0 && gemm_dtl_tail_workspace_bytes(tail, ts) <= workspace_bytes) {
@@ -1416,9 +1419,8 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (force_tile == 256) big = true;
     const bool parts_forced = force_tile == 256 && env_switches().gemm_tailsplit > 0 && env_switches().gemm_mfma != 32 && big_tiles_of(M, N, 256) <= 128;
     if (big && K >= 64 && !parts_forced) {
-        if (M % 256 != 0 || N % 256 != 0 || K % 64 != 0) return 0;
         int tail, ts;
-        tail_split_plan((M / 256) * (N / 256), K, &tail, &ts);
+        tail_split_plan(((M + 255) / 256) * ((N + 255) / 256), K, &tail, &ts);
         return tail > 0 ? gemm_dtl_tail_workspace_bytes(tail, ts) : 0;
     }
     // the layout of B and the number of peers are not known here: enough for any

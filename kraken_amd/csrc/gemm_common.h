@@ -149,7 +149,8 @@ __device__ __forceinline__ int64_t wave_uniform(int64_t v) {
 // re-numbered to give every XCD a contiguous range of the order: XCD x owns positions
 // [x * ntiles/8, (x+1) * ntiles/8) and a launch over fewer tiles takes the first count/8 of each
 // range (`first` skips positions an earlier launch has taken).  Where 8 does not divide the count, the
-// first ntiles % 8 XCDs own one position more (launches over all tiles only).
+// first ntiles % 8 XCDs own one position more (launches over all tiles), or the ranges are those of the launch over the
+// first ntiles - tail_tiles, a multiple of 256, and the tiles behind it follow in order.
 // (the plain form: a launch over all of `ntiles`)
 __device__ __forceinline__ int xcd_position(int wg, int ntiles) {
     const int x = wg % kXcds;
@@ -158,6 +159,7 @@ __device__ __forceinline__ int xcd_position(int wg, int ntiles) {
 __device__ __forceinline__ int schedule_position(const GemmArgs& g, int wg, int first = 0) {
     const int ntiles = g.tiles_m * g.tiles_n;
     if (ntiles % kXcds != 0 && (g.tail_tiles == 0 || g.tail_tiles == ntiles)) return xcd_position(wg, ntiles);
+    if (ntiles % kXcds != 0 && first == 0) return xcd_position(wg, ntiles - g.tail_tiles);
     if (ntiles % kXcds != 0 || first % kXcds != 0) return first + wg;
     return (wg % kXcds) * (ntiles / kXcds) + first / kXcds + wg / kXcds;
 }

@@ -1848,3 +1848,30 @@ def test_gather_over_the_flags_of_an_earlier_one(dev, rows):
         torch.cuda.current_stream(dev).wait_stream(_copy_engine_all_gather_w_progress(out, shards, progress, 1, rank=2))
         assert torch.equal(out, shards.view(W * rows, K))
         assert progress.tolist() == [1] * W
+
+
+def _small_integers(shape, seed, density, dev):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    v = torch.randint(-1, 2, shape, generator=g, device=dev).to(BF16)
+    return v * (torch.rand(shape, generator=g, device=dev) < density)
+
+
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K,W,rank", [
+    (4136, 4104, 4104, 2, 1),      # 289 tiles, all edges ragged, a K that is no multiple of 64: the tiles beyond the first round in parts
+    (4400, 4096, 4160, 8, 7),      # 288 tiles, ragged rows only
+    (2312, 4104, 264, 8, 3),       # the band's tiles ahead of the others, both its edges inside a tile
+    (2312, 4104, 264, 8, 7),       # ... the last band, which ends with the matrix
+    (3000, 3000, 72, 4, 0), (6144, 3072, 128, 2, 1), (2560, 4096, 64, 2, 0)])
+def test_reduce_scatter_of_many_tiles(dev, M, N, K, W, rank, b_t):
+    """More than 128 tiles of 256 x 256.  Operands of -1, 0, 1 (a quarter of b's are not zero): every sum is an integer far
+    below 256 (six standard deviations at K = 4160: 160, seven peers 7), so product, sum and rounding are exact."""
+    a, b = _small_integers((M, K), 1, 1.0, dev), _small_integers((K, N), 2, 0.25, dev)
+    peers = _small_integers((W - 1, M // W, N), 3, 1.0, dev)
+    c = torch.full((M, N), float("nan"), dtype=BF16, device=dev)
+    out = fused.gemm_reduce_scatter(a, b.T.contiguous().T if b_t else b, peers=peers, rank=rank, c_scratch=c)
+    want = a.float() @ b.float()
+    lo, hi = rank * (M // W), (rank + 1) * (M // W)
+    assert torch.equal(out.float(), want[lo:hi] + peers.float().sum(0))
+    assert torch.equal(c[:lo].float(), want[:lo]) and torch.equal(c[hi:].float(), want[hi:])
+    assert bool(c[lo:hi].isnan().all())      # the band's own rows are not the scratch's
