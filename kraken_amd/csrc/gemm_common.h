@@ -149,8 +149,8 @@ __device__ __forceinline__ int64_t wave_uniform(int64_t v) {
 // re-numbered to give every XCD a contiguous range of the order: XCD x owns positions
 // [x * ntiles/8, (x+1) * ntiles/8) and a launch over fewer tiles takes the first count/8 of each
 // range (`first` skips positions an earlier launch has taken).  Where 8 does not divide the count, the
-// first ntiles % 8 XCDs own one position more (launches over all tiles), or the ranges are those of the launch over the
-// first ntiles - tail_tiles, a multiple of 256, and the tiles behind it follow in order.
+// first ntiles % 8 XCDs own one position more (launches over all tiles), or the range is that of the launch over the
+// first ntiles - tail_tiles, which is a multiple of 256, and the tiles behind it follow in order.
 // (the plain form: a launch over all of `ntiles`)
 __device__ __forceinline__ int xcd_position(int wg, int ntiles) {
     const int x = wg % kXcds;
@@ -159,6 +159,7 @@ __device__ __forceinline__ int xcd_position(int wg, int ntiles) {
 __device__ __forceinline__ int schedule_position(const GemmArgs& g, int wg, int first = 0) {
     const int ntiles = g.tiles_m * g.tiles_n;
     if (ntiles % kXcds != 0 && (g.tail_tiles == 0 || g.tail_tiles == ntiles)) return xcd_position(wg, ntiles);
+    if (ntiles % kXcds != 0 && first == 0 && g.tail_tiles % kXcds == ntiles % kXcds) return xcd_position(wg, ntiles - g.tail_tiles);
     if (ntiles % kXcds != 0 && first == 0) return xcd_position(wg, ntiles - g.tail_tiles);
     if (ntiles % kXcds != 0 || first % kXcds != 0) return first + wg;
     return (wg % kXcds) * (ntiles / kXcds) + first / kXcds + wg / kXcds;
@@ -233,6 +234,8 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
     constexpr int EP_ITERS = 32 * CPR / 64; // chunks per lane per 32-row slab
     constexpr int kChunkBatch = BM >= 256 ? 4 : 2;   // the small tile keeps its register count low (occupancy)
     constexpr int kPeerGroup = 4;           // peers fetched together by the generic path
+    // a wave of an edge tile with no row or column in the matrix
+    if (!EVEN && (__builtin_amdgcn_readfirstlane(m0 + wm * WTM) >= g.M || __builtin_amdgcn_readfirstlane(n0 + wn * WTN) >= g.N)) return;
     const int band_lo = g.band_row0, band_hi = g.band_row0 + g.band_rows;
     const int lane_r = lane / CPR, lane_cc = lane % CPR;   // chunk (it*64 + lane): row it*(64/CPR) + lane_r
     const int n = n0 + wn * WTN + lane_cc * 8;             // first of the lane's 8 columns, same for every chunk
@@ -332,66 +335,99 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
     // the wave's first row, as a scalar: the classification below must branch uniformly
     const int wave_m0 = __builtin_amdgcn_readfirstlane(m0 + wm * WTM);
 
-    // ---- every row of the wave lies in the band and there are exactly 7 peers ---------------
-    // (the eight-rank case of the reference benchmarks): straight-line batches of kFastBatch
-    // chunks, peer loads double-buffered one batch ahead across slab boundaries.
-    if constexpr (!F32) {
-        constexpr int kFastPeers = 7;
-        constexpr int kFastBatch = BM >= 256 ? 2 : 1;   // chunks per batch (the small tile keeps two workgroups per CU)
-        constexpr int kFastBatches = EP_ITERS / kFastBatch;
-        static_assert(kFastBatches % 2 == 0, "the two peer buffers alternate with a static parity");
-        if (EVEN && n_peers == kFastPeers && wave_m0 >= band_lo && wave_m0 + WTM <= band_hi) {
-            u32x4 pv[2][kFastBatch][kFastPeers];
-            const int64_t peer_off = (int64_t)(wave_m0 - band_lo + lane_r) * g.N + n;
-            const int64_t chunk_step = (int64_t)(64 / CPR) * g.N;   // elements between consecutive chunks of a lane
-            auto issue = [&](auto buf_c, int chunk_abs) __attribute__((always_inline)) {
-                constexpr int buf = decltype(buf_c)::value;
+    // ---- up to seven peers, and the wave has rows of the band -----------------------------------
+    // Straight-line batches of kBatch chunks, peer loads double-buffered one batch ahead across slab boundaries.  A chunk's
+    // row goes to `out` or to c_full, lane by lane (edges of the matrix and of the band), and neither loads nor stores are
+    // under a branch, where the waits could not count them: a lane outside the band loads a valid address, a peer past the
+    // last repeats the last one and is masked, and both stores go out, out of range where they are not meant.
+    // Tiles at the edges used to take the loads behind the stores, as below, also for rows outside the band, and held up the
+    // others: 7392 x 5056 x 896 with a band and seven peers 128 -> 96 us, 2520 x 7232 x 1024 70.5 -> 51.6, 1448 x 2048 x 832
+    // 20.5 -> 16.9, fp32 results 700 x 4160 x 1024 with one peer 20.1 -> 17.8.
+    auto with_peers = [&](auto np_c) __attribute__((always_inline)) {
+        constexpr int P = decltype(np_c)::value;
+        constexpr int kBatch = (P <= 3 ? 2 : 1) * (BM >= 256 ? 2 : 1), kBatches = EP_ITERS / kBatch;
+        static_assert(EP_ITERS % kBatch == 0 && kBatches % 2 == 0, "the two peer buffers alternate with a static parity");
+        constexpr uint32_t kOob = 0x80000000u;
+        constexpr int kEl = F32 ? 4 : 2;
+        u32x4 pv[2][kBatch][P];
+        const int row_out = max(wave_m0, band_lo);   // first row of the band in this wave
+        const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (char*)g.out + ((int64_t)blockIdx.y * g.split_out_stride + (int64_t)(row_out - band_lo) * g.N) * kEl, 0, 0x7fffffff, 0x00020000);
+        const __amdgpu_buffer_rsrc_t full_rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(g.c_full + (int64_t)wave_m0 * g.N, 0, g.c_full != nullptr ? 0x7fffffff : 0, 0x00020000);
+        const int64_t safe_off = min(n, g.N - 8);
+        auto row_of = [&](int chunk_abs) __attribute__((always_inline)) { return wave_m0 + chunk_abs * (64 / CPR) + lane_r; };
+        auto inside = [&](int m) __attribute__((always_inline)) { return m >= band_lo && m < band_hi && (EVEN || n < g.N); };
+        auto issue = [&](auto buf_c, int chunk_abs) __attribute__((always_inline)) {
+            constexpr int buf = decltype(buf_c)::value;
 #pragma unroll
-                for (int c = 0; c < kFastBatch; ++c)
+            for (int c = 0; c < kBatch; ++c) {
+                const int m = row_of(chunk_abs + c);
+                const int64_t off = inside(m) ? (int64_t)(m - band_lo) * g.N + n : safe_off;
 #pragma unroll
-                    for (int q = 0; q < kFastPeers; ++q)
-                        pv[buf][c][q] =
-                            ld_stream((const u32x4*)((const uint16_t*)g.peer.p[q] + peer_off + (chunk_abs + c) * chunk_step));
-            };
-            issue(std::integral_constant<int, 0>{}, 0);
-#pragma nounroll
-            for (int i = 0; i < TM; ++i) {
-                copy_slab(i);
-                const int chunk0 = i * EP_ITERS;   // chunks are numbered through all slabs of the wave
-#pragma unroll
-                for (int b = 0; b < kFastBatches; ++b) {
-                    // unconditional (the very last batch re-fetches itself, unused): a prefetch under
-                    // a branch would make the wait below assume the shorter queue and stall on stores
-                    const int next_chunk = min(chunk0 + (b + 1) * kFastBatch, TM * EP_ITERS - kFastBatch);
-                    if (b & 1) issue(std::integral_constant<int, 0>{}, next_chunk);
-                    else issue(std::integral_constant<int, 1>{}, next_chunk);
-                    float f[kFastBatch][8];
-#pragma unroll
-                    for (int c = 0; c < kFastBatch; ++c) read_chunk(b * kFastBatch + c, f[c]);
-#pragma unroll
-                    for (int c = 0; c < kFastBatch; ++c) {
-#pragma unroll
-                        for (int q = 0; q < kFastPeers; ++q) add8(pv[b & 1][c][q], f[c]);
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) f[c][e] += bias_f[e];
-                    }
-#pragma unroll
-                    for (int c = 0; c < kFastBatch; ++c) {
-                        const int m = wave_m0 + (chunk0 + b * kFastBatch + c) * (64 / CPR) + lane_r;
-                        store_out((int64_t)(m - band_lo) * g.N + n, f[c]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+                for (int q = 0; q < P; ++q) pv[buf][c][q] = ld_stream((const u32x4*)((const uint16_t*)g.peer.p[min(q, n_peers - 1)] + off));
             }
-            return;
+        };
+        issue(std::integral_constant<int, 0>{}, 0);
+#pragma nounroll
+        for (int i = 0; i < TM; ++i) {
+            copy_slab(i);
+            const int chunk0 = i * EP_ITERS;
+#pragma unroll
+            for (int b = 0; b < kBatches; ++b) {
+                // (the very last batch re-fetches itself, unused)
+                const int next_chunk = min(chunk0 + (b + 1) * kBatch, TM * EP_ITERS - kBatch);
+                if (b & 1) issue(std::integral_constant<int, 0>{}, next_chunk);
+                else issue(std::integral_constant<int, 1>{}, next_chunk);
+                float f[kBatch][8];
+                u32x4 product[kBatch];   // as c_full gets it
+#pragma unroll
+                for (int c = 0; c < kBatch; ++c) {
+                    read_chunk(b * kBatch + c, f[c]);
+                    product[c] = pack8(f[c]);
+                }
+#pragma unroll
+                for (int c = 0; c < kBatch; ++c) {
+#pragma unroll
+                    for (int q = 0; q < P; ++q) {
+                        const uint32_t keep = q < n_peers ? 0xffffffffu : 0u;
+                        const u32x4 v = pv[b & 1][c][q];
+                        add8(u32x4{v.x & keep, v.y & keep, v.z & keep, v.w & keep}, f[c]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) f[c][e] += bias_f[e];
+                }
+#pragma unroll
+                for (int c = 0; c < kBatch; ++c) {
+                    const int m = row_of(chunk0 + b * kBatch + c);
+                    const bool in = inside(m), full = !in && (EVEN || (m < g.M && n < g.N));
+                    const uint32_t o = in ? (uint32_t)(((m - row_out) * g.N + n) * kEl) : kOob;
+                    const uint32_t q = full ? (uint32_t)(((m - wave_m0) * g.N + n) * 2) : kOob;
+                    constexpr int kNt = 2;   // non-temporal
+                    if constexpr (F32) {
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{f[c][0], f[c][1], f[c][2], f[c][3]}), out_rsrc, o, 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{f[c][4], f[c][5], f[c][6], f[c][7]}), out_rsrc, in ? o + 16 : kOob, 0, 0);
+                    } else {
+                        __builtin_amdgcn_raw_buffer_store_b128(pack8(f[c]), out_rsrc, o, 0, kNt);
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b128(product[c], full_rsrc, q, 0, kNt);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+    };
+    // (the stores' offsets are 32 bits from the wave's first row)
+    if (n_peers > 0 && n_peers <= 7 && wave_m0 < band_hi && wave_m0 + WTM > band_lo && (int64_t)WTM * g.N * 4 < 0x7fffffffLL) {
+        if (n_peers > 3) with_peers(std::integral_constant<int, 7>{});
+        else with_peers(std::integral_constant<int, 3>{});
+        return;
     }
 
     // ---- every other case, one slab at a time ------------------------------------------------
+    const bool whole = EVEN || (wave_m0 + WTM <= g.M && __builtin_amdgcn_readfirstlane(n0 + wn * WTN) + WTN <= g.N);
     // One batch of kChunkBatch chunks of the current slab.  NP == 0: every row of the slab lies
-    // in the band and there are no peers; NP == -2: no row of the slab lies in the band (both
-    // straight-line code without loads); NP == -1: generic per-lane handling (band edge inside
-    // the slab, ragged tile, any peer count).
+    // in the band (or below the matrix) and there are no peers; NP == -2: no row of the slab lies in the band (both
+    // without loads); NP == -1: generic per-lane handling (band edge inside the slab, any peer count).
     auto slab_batch = [&](auto np_c, int slab_m0, int b0) __attribute__((always_inline)) {
         constexpr int NP = decltype(np_c)::value;
         int64_t off[kChunkBatch];
@@ -400,7 +436,7 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
         for (int c = 0; c < kChunkBatch; ++c) {
             const int m = slab_m0 + (b0 + c) * (64 / CPR) + lane_r;
             valid[c] = EVEN || (m < g.M && n < g.N);
-            in_band[c] = NP == 0 ? true : NP == -2 ? false : (valid[c] && m >= band_lo && m < band_hi);
+            in_band[c] = NP == 0 ? valid[c] : NP == -2 ? false : (valid[c] && m >= band_lo && m < band_hi);
             off[c] = in_band[c] ? (int64_t)(m - band_lo) * g.N + n : (int64_t)m * g.N + n;
         }
         if constexpr (!F32 && NP != -1) {
@@ -408,8 +444,17 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
             if (NP == -2 || !has_bias) {
                 if (NP == 0 || g.c_full != nullptr) {
                     uint16_t* dst = NP == 0 ? (uint16_t*)g.out : g.c_full;
+                    u32x4 raw[kChunkBatch];
 #pragma unroll
-                    for (int c = 0; c < kChunkBatch; ++c) st_stream((u32x4*)(dst + off[c]), read_raw(b0 + c));
+                    for (int c = 0; c < kChunkBatch; ++c) raw[c] = read_raw(b0 + c);
+                    if (whole) {
+#pragma unroll
+                        for (int c = 0; c < kChunkBatch; ++c) st_stream((u32x4*)(dst + off[c]), raw[c]);
+                    } else {
+#pragma unroll
+                        for (int c = 0; c < kChunkBatch; ++c)
+                            if (valid[c]) st_stream((u32x4*)(dst + off[c]), raw[c]);
+                    }
                 }
                 return;
             }
@@ -462,8 +507,8 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
     for (int i = 0; i < TM; ++i) {
         copy_slab(i);
         const int slab_m0 = wave_m0 + i * 32;
-        const bool all_in = EVEN && slab_m0 >= band_lo && slab_m0 + 32 <= band_hi;
-        const bool all_out = EVEN && (slab_m0 + 32 <= band_lo || slab_m0 >= band_hi);
+        const bool all_in = slab_m0 >= band_lo && (slab_m0 + 32 <= band_hi || (!EVEN && band_hi == g.M));
+        const bool all_out = slab_m0 + 32 <= band_lo || slab_m0 >= band_hi;
 #pragma unroll
         for (int b0 = 0; b0 < EP_ITERS; b0 += kChunkBatch) {
             if (all_out) {

@@ -961,17 +961,11 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
         // 224-column tile of a plain product: every row goes to `out`
         store_tile_bf16_blocks<NB>(acc16, smem, (uint16_t*)g.out + (int64_t)(m0 + wm * WTM) * g.N + n0 + wn * WTNX, g.N, lane, wave);
     } else if constexpr (MI16) {
-        if (full_tile) {
-            gemm_epilogue<BM, WTM, WTN, TM, TN, true, EP_WAVE>(g, mfma_peers ? 0 : g.n_peers, bias_in_acc ? nullptr : g.bias, acc16,
-                                                               smem, m0, n0, wm, wn, lane, wave);
-        } else if constexpr (RAGGED) {
-            gemm_epilogue<BM, WTM, WTN, TM, TN, false, EP_WAVE>(g, g.n_peers, g.bias, acc16, smem, m0, n0, wm, wn, lane, wave);
-        }
-    } else if (full_tile) {
-        gemm_epilogue<BM, WTM, WTN, TM, TN, true, EP_WAVE>(g, mfma_peers ? 0 : g.n_peers, bias_in_acc ? nullptr : g.bias,
-                                                           acc, smem, m0, n0, wm, wn, lane, wave);
-    } else if constexpr (RAGGED) {   // edge tile: every access checked against M and N
-        gemm_epilogue<BM, WTM, WTN, TM, TN, false, EP_WAVE>(g, g.n_peers, g.bias, acc, smem, m0, n0, wm, wn, lane, wave);
+        gemm_epilogue<BM, WTM, WTN, TM, TN, !RAGGED, EP_WAVE>(g, mfma_peers ? 0 : g.n_peers, bias_in_acc ? nullptr : g.bias, acc16, smem, m0, n0,
+                                                              wm, wn, lane, wave);
+    } else {
+        gemm_epilogue<BM, WTM, WTN, TM, TN, !RAGGED, EP_WAVE>(g, mfma_peers ? 0 : g.n_peers, bias_in_acc ? nullptr : g.bias, acc, smem, m0, n0, wm,
+                                                              wn, lane, wave);
     }
 }
 #undef KR_SCHED_FENCE

@@ -1875,3 +1875,25 @@ def test_reduce_scatter_of_many_tiles(dev, M, N, K, W, rank, b_t):
     assert torch.equal(out.float(), want[lo:hi] + peers.float().sum(0))
     assert torch.equal(c[:lo].float(), want[:lo]) and torch.equal(c[hi:].float(), want[hi:])
     assert bool(c[lo:hi].isnan().all())      # the band's own rows are not the scratch's
+
+
+@pytest.mark.parametrize("P", [1, 2, 3, 4, 7, 8])
+@pytest.mark.parametrize("M,N,K", [(264, 264, 64), (520, 328, 136), (90, 8, 64), (383, 640, 72)])
+def test_epilogue_at_the_edges(dev, tile, M, N, K, P):
+    """Peers added in the epilogue, for waves that are in the band, partly in it and outside, at the edges of the matrix, with
+    bf16 and fp32 results: integers as above, exact."""
+    a, b, bias = _small_integers((M, K), 1, 1.0, dev), _small_integers((K, N), 2, 0.25, dev), _small_integers((N,), 4, 1.0, dev)
+    peers = _small_integers((P, M, N), 3, 1.0, dev)
+    want = a.float() @ b.float()
+    for dtype in (BF16, torch.float32):
+        out = fused.gemm_one_shot_all_reduce_fused(a, b, peers=peers, bias=bias, out_dtype=dtype)
+        assert out.dtype == dtype and torch.equal(out.float(), want + peers.float().sum(0) + bias.float())
+    W = P + 1
+    rows = M // W
+    a, want = a[:rows * W], want[:rows * W]
+    for rank in (0, W // 2, W - 1):
+        c = torch.full((rows * W, N), float("nan"), dtype=BF16, device=dev)
+        out = fused.gemm_reduce_scatter(a, b, peers=peers[:, :rows].contiguous(), rank=rank, c_scratch=c)
+        lo, hi = rank * rows, (rank + 1) * rows
+        assert torch.equal(out.float(), want[lo:hi] + peers[:, :rows].float().sum(0))
+        assert torch.equal(c[:lo].float(), want[:lo]) and torch.equal(c[hi:].float(), want[hi:]) and bool(c[lo:hi].isnan().all())
