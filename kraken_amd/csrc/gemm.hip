@@ -71,7 +71,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_reduce_kernel(const GemmArgs
     const int wm = wave / WN, wn = wave % WN;
 
     int tile_m, tile_n;
-    tile_schedule(g, schedule_position(g, blockIdx.x), tile_m, tile_n);
+    tile_of(g, blockIdx.x, 0, tile_m, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const uint16_t* a_tile;   // first row of the tile's A panel (gathered matrix or local shard)
     int64_t lda;
@@ -1083,6 +1083,20 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
     if (splits > 1 && !aligned16(workspace)) return KR_ERR_ALIGNMENT;
     int64_t pt = tile_pivot / bm;
     g.pivot_tiles = (int)(((pt % g.tiles_m) + g.tiles_m) % g.tiles_m);
+    // 256-row tiles with a band: the band's tiles as a region of their own at the head of the order, dealt to all XCDs, the others behind
+    // them.  In one order the band lies with one to four of the XCDs, whose compute units are then the last to get to the tiles beyond the
+    // first round: us, one order / two regions, 6144 x 3072 x 2048 (288 tiles, one peer) 102.5 / 86.0, 3000 x 3000 x 600 34.1 / 26.7,
+    // 7392 x 5056 x 896 (580 tiles, seven peers) 96.0 / 78.6, 8192 x 4096 x 1024 72.7 / 63.6.  An XCD then works on two sets of
+    // panels at first, which a long K does not win back: 8192 x 8192 x 3584 343 / 352, 5000 x 5000 x 5000 234 / 242, 4600 x 6000 x 4096
+    // 192 / 186, 7360 x 3328 x 3072 155 / 134.
+    g.band_tile0 = g.band_tile_rows = 0;
+    if (dtl && n_peers > 0 && band_rows > 0 && band_rows < M && K <= 3328) {
+        const int64_t r0 = band_row0 / bm, rows = (band_row0 + band_rows + bm - 1) / bm - r0;
+        if (rows < g.tiles_m && rows * g.tiles_n + g.tail_tiles <= (int64_t)g.tiles_m * g.tiles_n) {
+            g.band_tile0 = (int)r0;
+            g.band_tile_rows = (int)rows;
+        }
+    }
     const bool even = (M % bm == 0 && N % bn == 0 && K % BK == 0);
     if (splits > 1) {
         // pass 1: S partial products, fp32, no epilogue work; pass 2: sum + epilogue

@@ -44,6 +44,7 @@ struct GemmArgs {
     int tail_tiles;
     int wide_panels;     // gemm_w8_kernel: column panels of 256, the first of the tiles_n; the others are narrower
     int group_n;         // column panels per scheduling group (tile_schedule)
+    int band_tile0, band_tile_rows;   // rows of tiles that touch the reduce band, ahead of all others (tile_of; 0 rows: one order)
     int peers_on_mfma;   // 256x256 kernel: add whole-band tiles' peers through the matrix cores
     int mi16;            // 256x256 kernel: k loop and peer phase on 16x16x32 MFMA blocks
     int n224;            // 256x224 tiles (tiles_n counts them), transposed-contiguous B: a plain product in whole rounds, or every tile in parts
@@ -188,6 +189,22 @@ __device__ __forceinline__ void tile_in_order(int pid, int tiles_m, int tiles_n,
 }
 __device__ __forceinline__ void tile_schedule(const GemmArgs& g, int pid, int& tile_m_out, int& tile_n_out) {
     tile_in_order(pid, g.tiles_m, g.tiles_n, g.group_n, g.pivot_tiles, tile_m_out, tile_n_out);
+}
+
+// Tile of workgroup `wg`; with `first` > 0 of a launch over the tiles from position `first` on.
+__device__ __forceinline__ void tile_of(const GemmArgs& g, int wg, int first, int& tile_m, int& tile_n) {
+    // (without branches around the choice: the compiler keeps the tile in scalar registers only so)
+    const int tiles = g.tiles_m * g.tiles_n, band = g.band_tile_rows * g.tiles_n;
+    const bool in_band = first == 0 && wg < band;
+    const int row0 = in_band ? g.band_tile0 : band > 0 ? g.band_tile0 + g.band_tile_rows : g.pivot_tiles;
+    const int rows = in_band ? g.band_tile_rows : g.tiles_m - g.band_tile_rows;
+    const int pid = band == 0 ? schedule_position(g, wg, first)
+                              : first > 0 ? first - band + wg : xcd_position(in_band ? wg : wg - band, in_band ? band : tiles - g.tail_tiles - band);
+    tile_in_order(pid, rows, g.tiles_n, g.group_n, 0, tile_m, tile_n);
+    tile_m += row0;
+    if (tile_m >= g.tiles_m) tile_m -= g.tiles_m;
+    tile_m = __builtin_amdgcn_readfirstlane(tile_m);
+    tile_n = __builtin_amdgcn_readfirstlane(tile_n);
 }
 
 // Fused epilogue of one workgroup tile.  `acc` are this wave's 32x32 MFMA accumulators (TM x TN

@@ -140,8 +140,7 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     const int first_tile = g.tiles_m * g.tiles_n - g.tail_tiles;     // SPLIT: tiles the main launch took
     const int split = SPLIT ? (int)(blockIdx.x % (unsigned)g.k_splits) : 0;
     const int tail_index = SPLIT ? (int)(blockIdx.x / (unsigned)g.k_splits) : 0;
-    tile_schedule(g, SPLIT ? schedule_position(g, tail_index, first_tile) : schedule_position(g, blockIdx.x), tile_m,
-                  tile_n);
+    tile_of(g, SPLIT ? tail_index : (int)blockIdx.x, SPLIT ? first_tile : 0, tile_m, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BNX;
     // k-steps of this workgroup: all of them, or the split's share
     const int kt_all = RAGGED ? (g.K + BKD - 1) / BKD : g.K / BKD;
@@ -1037,7 +1036,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
     const int slab = blockIdx.x % TM, wave = blockIdx.x / TM % (WM * WN), u = blockIdx.x / (TM * WM * WN);
     const int S = g.k_splits;
     int tile_m, tile_n;
-    tile_schedule(g, schedule_position(g, u, g.tiles_m * g.tiles_n - g.tail_tiles), tile_m, tile_n);
+    tile_of(g, u, g.tiles_m * g.tiles_n - g.tail_tiles, tile_m, tile_n);
     const int m0 = tile_m * BM + (wave / WN) * WTM + slab * 32, n0 = tile_n * (WN * WTNX) + (wave % WN) * WTNX;
     if (m0 >= g.M || n0 >= g.N) return;   // edge tiles: nothing of this slab is in the matrix
     // this thread's quads are 4 jw .. +3 of the slab's 2 NB (NB = 7: the last wavefront's last two are not there, it reads its second again)

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(const GemmArgs g)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int mh = wave >> 1, kh = wave & 1;   // rows 64 mh .. +63 of the tile, stage kh of a step
     int tile_m, tile_n;
-    tile_schedule(g, schedule_position(g, blockIdx.x), tile_m, tile_n);
+    tile_of(g, blockIdx.x, 0, tile_m, tile_n);
     const int m0 = tile_m * BT, n0 = tile_n * BT;
     // steps of this workgroup (64 k each): all of them, or the share of split blockIdx.y
     const int kt_all = (g.K + 2 * BKS - 1) / (2 * BKS);
