@@ -584,6 +584,25 @@ int kr_gemm_reduce_f32_ws(const void* A, int64_t lda_m, int64_t lda_k, const voi
                           int64_t workspace_bytes, void* stream);
 
 /*
+ * The same product and arithmetic in two launches, for many tiles or a long K: every element is split once, by a pass of its own,
+ * and the 256x256 kernel multiplies the parts.
+ *   kr_split_pairs_fp32: A [M, K] fp32 with k contiguous (lda floats between rows) and B [K, N] fp32 with strides (ldb_k, ldb_n),
+ *     one of them 1, to A_out [M, 2 Kp] and B_out [N, 2 Kp] bf16, Kp = K rounded up to 32: of every 32 k the 32 hi parts and then the
+ *     32 lo parts, zeros past K.  K, N multiples of 8, rows 16-byte aligned.
+ *   kr_gemm_reduce_pairs_ws: A and B as written by it; M, N, K of the fp32 operands; the rest as for kr_gemm_reduce_f32_ws.
+ *     workspace of kr_gemm_pairs_workspace_bytes bytes (0: none needed; a smaller one or none: K loops are not shared).
+ *   kr_gemm_f32_pairs: 1 where the pass pays, 0 where kr_gemm_reduce_f32_ws is faster (K below 2^20).
+ */
+int kr_split_pairs_fp32(const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n, int64_t M, int64_t N,
+                        int64_t K, void* A_out, void* B_out, void* stream);
+int kr_gemm_f32_pairs(int64_t M, int64_t N, int64_t K);
+int64_t kr_gemm_pairs_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int kr_gemm_reduce_pairs_ws(const void* A, const void* B, int64_t M, int64_t N, int64_t K, const void* const* peers,
+                            int n_peers, const void* bias, int64_t band_row0, int64_t band_rows, void* c_full,
+                            void* out, int out_is_fp32, int64_t tile_pivot, void* workspace,
+                            int64_t workspace_bytes, void* stream);
+
+/*
  * Which kernel kr_gemm_reduce_*_bf16 would run for a shape (contiguous operands), decided by the
  * same code that launches it; for benchmarks and logs that want to name the kernel they timed.
  * No counterpart in the reference (its tile sizes are keyword arguments of the wrappers,

@@ -129,6 +129,14 @@ _SIGNATURES = {
          c_void_p, c_int, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64,
          c_void_p, c_int64, c_void_p],
     ),
+    "kr_split_pairs_fp32": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p]),
+    "kr_gemm_f32_pairs": (c_int, [c_int64, c_int64, c_int64]),
+    "kr_gemm_pairs_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
+    "kr_gemm_reduce_pairs_ws": (
+        c_int,
+        [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64,
+         c_void_p, c_int64, c_void_p],
+    ),
     "kr_gemm_fp8_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "kr_gemm_fp8_ws": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p, c_int64,
                                c_void_p]),

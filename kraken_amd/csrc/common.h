@@ -131,6 +131,7 @@ struct EnvSwitches {
     int gemm_group;      // KRAKEN_AMD_GEMM_GROUP=<n>
     int gemm_splitk;     // KRAKEN_AMD_GEMM_SPLITK=<n>
     int gemm_tailsplit;  // KRAKEN_AMD_GEMM_TAILSPLIT=<n>
+    int gemm_pairs;      // KRAKEN_AMD_GEMM_PAIRS=0|1
     int gemm_n224;       // KRAKEN_AMD_GEMM_N224=0|1
     int gemm_ks;         // KRAKEN_AMD_GEMM_KS=0|1
     int gemm_w8;         // KRAKEN_AMD_GEMM_W8=<parts> | 1000 * (columns / 32) of the narrow tiles + panels of 256 columns

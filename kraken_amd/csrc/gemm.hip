@@ -1504,6 +1504,108 @@ extern "C" int kr_gemm_reduce_f32_ws(const void* A, int64_t lda_m, int64_t lda_k
                        out_is_fp32, tile_pivot, stream, nullptr, workspace, workspace_bytes, false, /*f32=*/true);
 }
 
+// fp32 operands as pairs (kPairs in gemm_dtl.hip): which tiles share their K loop.  A k-step of 32 takes 1.66 us with 192
+// compute units busy and 1.9 with 256 (1.69 PFLOP/s), 64 MiB of parts 19 us to write, read and sum.
+static void pairs_split_plan(int64_t M, int64_t N, int64_t K, int* tail_out, int* splits_out) {
+    const int64_t tiles = big_tiles_of(M, N, 256), steps = (K + 31) / 32;
+    *tail_out = 0;
+    *splits_out = 1;
+    const int64_t force = env_switches().gemm_tailsplit;   // 0: off, n: n parts (testing)
+    if (force == 0) return;
+    const int64_t tail = tiles <= 128 ? tiles : tiles % 256;
+    if (tail == 0 || (tail > 128 && force <= 0)) return;
+    int64_t best = 165 * steps;
+    for (int64_t s = 2; s <= kMaxTailSplits && s * tail <= 256 && s * 4 <= steps; ++s) {
+        if (force > 0 && s != force) continue;
+        const int64_t c = 500 + 165 * ((steps + s - 1) / s) + gemm_dtl_tail_workspace_bytes((int)tail, (int)s) * 241 / 10000000;
+        if (c >= best && force <= 0) continue;
+        best = c;
+        *tail_out = (int)tail;
+        *splits_out = (int)s;
+    }
+}
+
+// Pairs or the kernel that splits in registers (split_f32), in 0.01 us.  That one runs 256 tiles of 128x128 at a time: 17 us and
+// 1.5 per round and 64 k.  Pairs take 4 us and the pass, 8 bytes per element of both operands at 5.2 TB/s, then 8 us
+// (one pass 18, which also stores) and the k-steps, and the parts.  us, in registers / pairs, transposed and row-major B:
+// 1316 x 3136 x 9280 431 / 260, 460 / 254 (275 tiles), x 3000 155 / 113, 162 / 109; 1000 x 4096 x 8192 224 / 218, 230 / 207,
+// x 2048 64 / 85, 66 / 82; 2000 x 4096 x 2048 123 / 124, 128 / 122; 512 x 4096 x 8192 128 / 151, 129 / 145; 128 x 8192 x 8192
+// 81 / 197.  Above 512 tiles, as a bf16 product of three times the K / pairs, three peers, transposed B: 4096 x 4096 x 2048 202 /
+// 176, x 1024 113 / 104, 6000 x 6000 x 1024 281 / 246, 3000 x 8000 x 1536 255 / 233, 8192 x 2048 x 512 76 / 69.
+extern "C" int kr_gemm_f32_pairs(int64_t M, int64_t N, int64_t K) {
+    if (M <= 64 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K >= 1 << 20) return 0;   // (few rows: gemm_skinny_kernel)
+    if (const int v = env_switches().gemm_pairs; v >= 0) return v;   // testing and tuning
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+    if (tiles > 512) return 1;
+    const int64_t s = split_f32(M, N, K), k64 = (K + 63) / 64;
+    const int64_t registers = 1700 + (tiles * s + 255) / 256 * 150 * ((k64 + s - 1) / s) + (s > 1 ? 600 + s * M * N * 16 / 100000 : 0);
+    int tail, splits;
+    pairs_split_plan(M, N, K, &tail, &splits);
+    const int64_t big = big_tiles_of(M, N, 256), rounds = tail > 0 ? (big - tail) / 256 : (big + 255) / 256, k32 = (K + 31) / 32;
+    const int64_t pairs = 400 + (M + N) * K * 8 / 52000 + (rounds > 0 ? 1800 : 800) + rounds * 190 * k32 +
+                          (tail > 0 ? 300 + 190 * ((k32 + splits - 1) / splits) + gemm_dtl_tail_workspace_bytes(tail, splits) / 36000 : 0);
+    return pairs < registers * 95 / 100;
+}
+
+extern "C" int64_t kr_gemm_pairs_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    int tail, splits;
+    pairs_split_plan(M, N, K, &tail, &splits);
+    return tail > 0 ? gemm_dtl_tail_workspace_bytes(tail, splits) : 0;
+}
+
+extern "C" int kr_gemm_reduce_pairs_ws(const void* A, const void* B, int64_t M, int64_t N, int64_t K, const void* const* peers, int n_peers,
+                                       const void* bias, int64_t band_row0, int64_t band_rows, void* c_full, void* out, int out_is_fp32,
+                                       int64_t tile_pivot, void* workspace, int64_t workspace_bytes, void* stream) {
+    if (M < 0 || N < 0 || K < 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x3fffffffLL) return KR_ERR_BAD_DIM;
+    if (n_peers < 0 || n_peers >= KR_MAX_WORLD) return KR_ERR_WORLD_SIZE;
+    if (band_row0 < 0 || band_rows < 0 || band_row0 + band_rows > M) return KR_ERR_BAND;
+    if (N % 8 != 0) return KR_ERR_NUMEL_MOD8;
+    if (M == 0 || N == 0) return KR_OK;
+    if (K == 0) return KR_ERR_BAD_DIM;
+    if (A == nullptr || B == nullptr || (band_rows > 0 && out == nullptr) || (n_peers > 0 && peers == nullptr)) return KR_ERR_NULL_POINTER;
+    if (!aligned16(A) || !aligned16(B) || !aligned16(bias) || !aligned16(c_full) || !aligned16(out) || !aligned16(workspace)) return KR_ERR_ALIGNMENT;
+    GemmArgs g{};
+    if (n_peers > 0) {
+        if (const int rc = peer_tab_from_ptrs(g.peer, peers, n_peers); rc != KR_OK) return rc;
+    } else {
+        peer_tab_stacked(g.peer, A, 0, 0);
+    }
+    g.A = (const uint16_t*)A;
+    g.B = (const uint16_t*)B;
+    g.M = (int)M; g.N = (int)N; g.K = (int)((K + 31) / 32 * 64);
+    g.lda = g.ldb = g.K;
+    if (!gemm_dtl_supported(g)) return KR_ERR_LAYOUT;
+    g.n_peers = n_peers;
+    g.comm_rows = 1;
+    g.count_rows = 1;
+    g.bias = (const uint16_t*)bias;
+    g.band_row0 = (int)band_row0;
+    g.band_rows = (int)band_rows;
+    g.c_full = (uint16_t*)c_full;
+    g.out = out;
+    g.out_is_fp32 = out_is_fp32;
+    g.tiles_m = (int)((M + 255) / 256);
+    g.tiles_n = (int)((N + 255) / 256);
+    if ((int64_t)g.tiles_m * g.tiles_n > 0x7fffffffLL) return KR_ERR_BAD_DIM;
+    g.pivot_tiles = (int)(((tile_pivot / 256) % g.tiles_m + g.tiles_m) % g.tiles_m);
+    g.group_n = n_peers > 0 && band_rows * 2 >= M ? 16 : 8;
+    if (const int v = env_switches().gemm_group; v >= 1 && v <= 64) g.group_n = v;
+    g.k_splits = 1;
+    g.mi16 = 1;
+    // Peers on the matrix cores spread a value that is not finite over 16 columns: only where the bf16 product of three times
+    // the K did so too.  (In the epilogue 4096 x 4096 x 1024 takes 107 us with one peer, so 101.)
+    const bool many = ((M + 127) / 128) * ((N + 127) / 128) > 512;
+    g.peers_on_mfma = K % 64 != 0 ? 0 : env_switches().gemm_peers >= 0 ? env_switches().gemm_peers : many;
+    int tail, splits;
+    pairs_split_plan(M, N, K, &tail, &splits);
+    if (tail > 0 && workspace != nullptr && gemm_dtl_tail_workspace_bytes(tail, splits) <= workspace_bytes) {
+        g.tail_tiles = tail;
+        g.k_splits = splits;
+    }
+    return (int)launch_gemm_pairs(g, (hipStream_t)stream, workspace);
+}
+
 extern "C" int kr_gemm_reduce_noalloc_bf16(const void* A, int64_t lda_m, int64_t lda_k, const void* B,
                                            int64_t ldb_k, int64_t ldb_n, int64_t M, int64_t N, int64_t K,
                                            const void* peers, int n_peers, int64_t peers_stride,

@@ -73,6 +73,7 @@ inline hipError_t lds_opt_in(const void* fn, int bytes, std::atomic<uint64_t>& d
 bool gemm_dtl_supported(const GemmArgs& g);
 hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* workspace);
 hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace);   // fp8 operands (gemm_dtl.hip)
+hipError_t launch_gemm_pairs(const GemmArgs& g, hipStream_t st, void* workspace);  // fp32 operands as pairs of bf16 parts (gemm_dtl.hip)
 hipError_t launch_tail_finish(const GemmArgs& g, hipStream_t st, const void* workspace);   // sums the parts of split 256x256 tiles
 hipError_t launch_gemm_w8(const GemmArgs& g, int nb2, hipStream_t st, void* workspace);   // fp8 operands widened to bf16 (gemm_w8.hip)
 

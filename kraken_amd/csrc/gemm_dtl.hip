@@ -53,6 +53,8 @@ typedef const __attribute__((address_space(3))) bf16x8* lds_frag;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_tr;
 
+enum { kBf16, kFp8, kPairs };   // what the operands hold (gemm_dtl_tile)
+
 // s_waitcnt vmcnt(n) only (expcnt and lgkmcnt left at "no wait")
 constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 constexpr int kLgkm0 = 0xc07f;   // s_waitcnt lgkmcnt(0) only
@@ -114,14 +116,21 @@ __device__ __forceinline__ void store_tile_bf16_blocks(const f32x4 (&acc16)[2 * 
 // share of the panel's k-steps out of LDS while it multiplies: no copy in front of the product, nothing to wait for.  Copies
 // on a side stream need compute units that only a finished tile gives back: 8 shards of 1024 x 8192, N = 3584 (134 MB
 // gathered) 397 us with them, 346 so; 8 x 512 x 4096, N = 4096 159 -> 106; 2 x 2048 x 4096, N = 8192 235 -> 203.
-template <bool B_NT, bool PEERS_FIRST, bool SPLIT = false, bool RAGGED = false, bool MI16 = false, int NB = 2 * TN, bool F8 = false, bool GATHER = false>
+// OPER kPairs: fp32 operands that a pass of their own (split.hip) has turned into rows of 32 hi and 32 lo parts in turn, which g
+// describes as bf16 matrices of twice the width: a stage's row is 32 k, and piece q and piece 4 + q of it are the hi and the lo
+// part of the same eight values.  Loads and LDS layout are those of the bf16 form; a k-step (k_step_pairs) reads each part
+// once and multiplies it twice, hi hi, lo hi and hi lo, where a bf16 product of [hi | hi | lo] and [hi | lo | hi], three times the
+// width, loads and reads six parts for the four there are.  Bound by the matrix cores at their power limit: 1.9 us a k-step with
+// 256 tiles, 1.69 PFLOP/s; 4096 x 4096 x 2048 with its split passes and three peers 202 us as that product, 176 so (kr_gemm_f32_pairs says when).
+template <bool B_NT, bool PEERS_FIRST, bool SPLIT = false, bool RAGGED = false, bool MI16 = false, int NB = 2 * TN, int OPER = kBf16, bool GATHER = false>
 __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* smem) {
+    constexpr bool F8 = OPER == kFp8, PAIRS = OPER == kPairs;
     static_assert(NB == 2 * TN || (NB == 7 && MI16 && B_NT && (SPLIT || !RAGGED) && !PEERS_FIRST), "224-column tile: plain NT products and parts of K");
     // F8: the operands are fp8 (e4m3fn) and g describes them as bf16 matrices of half the width (g.K, g.lda, g.ldb in
     // two-byte units), so a stage still holds 128-byte rows -- 128 k now -- and every load and LDS address below is unchanged;
     // only the k-step differs (k_step8: 16x16x128 MFMAs on the same 16 x 16 accumulator blocks).
-    static_assert(!F8 || (MI16 && B_NT && !PEERS_FIRST && NB == 2 * TN), "fp8: plain NT products");
-    static_assert(!GATHER || (MI16 && B_NT && !PEERS_FIRST && !SPLIT && !F8), "gather: plain NT products");
+    static_assert(OPER == kBf16 || (MI16 && B_NT && NB == 2 * TN && (PAIRS || !PEERS_FIRST)), "fp8: plain NT products; pairs: NT products");
+    static_assert(!GATHER || (MI16 && B_NT && !PEERS_FIRST && !SPLIT && OPER == kBf16), "gather: plain NT products");
     constexpr int BNX = WN * NB * 16;                            // columns of the workgroup tile
     constexpr int WTNX = NB * 16;                                // columns of a wave
     constexpr int LOADS_B = BNX * BKD * 2 / 1024 / (WM * WN);    // LDS-DMA loads of B per wave per k-step: 8 or 7
@@ -347,7 +356,8 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     typedef const __attribute__((address_space(3))) i32x4* lds_i32x4;
     uint32_t fa8[2], fb8[2];
     i32x8 af8[2][TM], bf8[2][2 * TN];   // A: blocks 0..3 and 4..7 of the current step; B: all blocks, this step's and the next one's
-    if constexpr (F8) {
+    i32x4 ap[2][TM][2], bp[2][2 * TN][2];   // pairs: the same by halves, [0] the hi and [1] the lo parts
+    if constexpr (F8 || PAIRS) {
         const int p = lane & 15, gq = lane >> 4;
         const int sw8 = (p >> 1) & 7;
 #pragma unroll
@@ -369,6 +379,11 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
             const i32x4 v = *(lds_i32x4)(size_t)(fb8[h] + stage_off + bj * 2048);
             if (h == 0) bf8[buf][bj].lo = v; else bf8[buf][bj].hi = v;
         }
+    };
+    auto read_frag_pairs = [&](int buf, int r, uint32_t stage_off) __attribute__((always_inline)) {   // (the same order)
+        const int h = r & 1, bi = r < 2 ? 0 : (r - 16) / 2, bj = (r - 2) / 2;
+        if (r < 2 || r >= 18) ap[0][bi][h] = *(lds_i32x4)(size_t)(fa8[h] + stage_off + bi * 2048);
+        else bp[buf][bj][h] = *(lds_i32x4)(size_t)(fb8[h] + stage_off + bj * 2048);
     };
     auto read_a8_late = [&](int r, uint32_t stage_off) __attribute__((always_inline)) {   // r = 0 .. 7: halves of A blocks 4 .. 7
         const i32x4 v = *(lds_i32x4)(size_t)(fa8[r & 1] + stage_off + (4 + r / 2) * 2048);
@@ -646,7 +661,8 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     constexpr int kInStep = (kSlots16 - 1 - kBarA0 - 2) / kLoadGap16 + 1 < LOADS_TILE ? (kSlots16 - 1 - kBarA0 - 2) / kLoadGap16 + 1 : LOADS_TILE;
     constexpr int kBarA8 = 12, kBarB8 = 39, kLoadGap8 = 3;               // fp8 form (k_step8): barrier slots, slots between loads
     constexpr int kInStep8 = (63 - kBarA8 - 1) / kLoadGap8 + 1 < LOADS_TILE ? (63 - kBarA8 - 1) / kLoadGap8 + 1 : LOADS_TILE;
-    constexpr int kFirst = F8 ? kInStep8 : MI16 ? kInStep : kEarly;   // loads of step 1 the prologue issues
+    constexpr int kBarAP = 36, kBarBP = 117, kLoadGapP = 9;              // pairs (k_step_pairs)
+    constexpr int kFirst = PAIRS ? LOADS_TILE : F8 ? kInStep8 : MI16 ? kInStep : kEarly;   // loads of step 1 the prologue issues
     static_assert(NSTAGE == 2 && LOADS_PER_TILE == 16 && (LOADS_TILE == 16 || (NB == 7 && LOADS_TILE == 15)), "load schedules below");
 #pragma unroll
     for (int q = 0; q < LOADS_TILE; ++q) issue_load(0, 0, q);
@@ -655,7 +671,10 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(kFirst));
     __builtin_amdgcn_s_barrier();
     KR_SCHED_FENCE();
-    if constexpr (F8) {
+    if constexpr (PAIRS) {
+#pragma unroll
+        for (int r = 0; r < 24; ++r) read_frag_pairs(0, r, 0);
+    } else if constexpr (F8) {
 #pragma unroll
         for (int r = 0; r < 24; ++r) read_frag8(0, r, 0);
     } else if constexpr (MI16) {   // (A blocks 4..7 are read inside the first sub-step)
@@ -870,11 +889,53 @@ __device__ __forceinline__ void gemm_dtl_tile(const GemmArgs& g, unsigned char* 
             KR_SCHED_FENCE();
         }
     };
+    // The k-step on pairs: 192 v_mfma_f32_16x16x32_bf16, for each row of blocks hi hi, then lo (of B) hi, then hi lo, so that an
+    // accumulator is used once in eight slots.  The schedule is that of k_step8, in slots of 16 instead of 32 cycles and half
+    // as many again: A blocks 4..7 in the first 22 slots (needed from slot 96 on), barrier (a) behind slot kBarAP, the loads
+    // of step t+2 one per kLoadGapP slots, barrier (b) behind slot kBarBP, the fragments of step t+1 one per three slots.
+    constexpr int kLoadsBeforeBP = (kBarBP - kBarAP - 1) / kLoadGapP + 1;   // loads of step t+2 in slots <= kBarBP
+    static_assert(kBarAP > 22 && kBarAP + 1 + kLoadGapP * (LOADS_PER_TILE - 1) < 192 && kBarBP + 1 + 3 * 23 < 192, "pairs k-step schedule");
+    auto k_step_pairs = [&](int t, auto stage_c) __attribute__((always_inline)) {
+        const uint32_t stage_cur = stage_c;
+        const uint32_t stage_nxt = stage_cur ^ 1u;
+        const uint32_t st_cur = stage_cur * A_ST, st_nxt = stage_nxt * A_ST;
+        const int cur = stage_c, nxt = cur ^ 1;
+#pragma unroll
+        for (int s = 0; s < 192; ++s) {
+            const int i = s / 24, part = s % 24 / 8, j = s % 8;
+            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                         : "+a"(acc16[i][j])
+                         : "v"(bp[cur][j][part == 1 ? 1 : 0]), "v"(ap[i >> 2][i & 3][part == 2 ? 1 : 0]));
+            if (s % 3 == 1 && s / 3 < 8) ap[1][s / 6][s / 3 & 1] = *(lds_i32x4)(size_t)(fa8[s / 3 & 1] + st_cur + (4 + s / 6) * 2048);
+            if (s == kBarAP) {
+                KR_SCHED_FENCE();
+                __builtin_amdgcn_s_waitcnt(kLgkm0);
+                __builtin_amdgcn_s_barrier();
+            }
+            if (s > kBarAP && (s - kBarAP - 1) % kLoadGapP == 0 && (s - kBarAP - 1) / kLoadGapP < LOADS_PER_TILE)
+                issue_load(t + 2, stage_cur, (s - kBarAP - 1) / kLoadGapP);
+            if (s == kBarBP) {
+                KR_SCHED_FENCE();
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(kLoadsBeforeBP));
+                __builtin_amdgcn_s_barrier();
+            }
+            if (s > kBarBP && (s - kBarBP - 1) % 3 == 0 && (s - kBarBP - 1) / 3 < 24) read_frag_pairs(nxt, (s - kBarBP - 1) / 3, st_nxt);
+            KR_SCHED_FENCE();
+        }
+    };
     // Main part: one trip = two k-steps, so every LDS stage offset is a compile-time constant
     // (immediate offsets on the fragment reads) and the loop branch is taken once per 128 MFMAs;
     // an odd last step follows.
     int t = 0;
-    if constexpr (F8) {
+    if constexpr (PAIRS) {
+#pragma nounroll
+        for (; t + 2 <= kt_total; t += 2) {
+            k_step_pairs(t, std::integral_constant<uint32_t, 0>{});
+            k_step_pairs(t + 1, std::integral_constant<uint32_t, 1>{});
+        }
+        pin_accumulators();
+        if (t < kt_total) k_step_pairs(t, std::integral_constant<uint32_t, 0>{});
+    } else if constexpr (F8) {
 #pragma nounroll
         for (; t + 2 <= kt_total; t += 2) {
             k_step8(t, std::integral_constant<uint32_t, 0>{});
@@ -997,14 +1058,22 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl16n7_kernel(const GemmArg
 template <int NB, bool RAGGED>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl16_gather_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gemm_dtl_tile<true, false, false, RAGGED, true, NB, false, true>(g, smem);
+    gemm_dtl_tile<true, false, false, RAGGED, true, NB, kBf16, true>(g, smem);
 }
 
 // fp8 (e4m3fn) operands, transposed-contiguous B; the result is fp8, bf16 or fp32.
 template <bool RAGGED>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl8_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gemm_dtl_tile<true, false, false, RAGGED, true, 2 * TN, true>(g, smem);
+    gemm_dtl_tile<true, false, false, RAGGED, true, 2 * TN, kFp8>(g, smem);
+}
+
+// fp32 operands as pairs of bf16 parts (kPairs above).
+template <bool RAGGED>
+__global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_pairs_kernel(const GemmArgs g) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    if (g.peers_on_mfma && g.n_peers > 0 && (g.peers_on_mfma == 1 ? ((blockIdx.x >> 3) & 1) : g.peers_on_mfma == 2)) gemm_dtl_tile<true, true, false, RAGGED, true, 2 * TN, kPairs>(g, smem);
+    else gemm_dtl_tile<true, false, false, RAGGED, true, 2 * TN, kPairs>(g, smem);
 }
 
 }  // namespace
@@ -1012,10 +1081,10 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl8_kernel(const GemmArgs g
 // Second launch of a call with a split tail: g.k_splits workgroups per tile of the last partial
 // round (g.out = workspace).  With few tiles every one is split and there is no launch before this one; M and N may
 // then be ragged, and the tiles 224 columns wide (NB = 7; plan_small in gemm.hip says when and what it measured).
-template <bool B_NT, bool MI16, bool RAGGED = false, bool F8 = false, int NB = 2 * TN>
+template <bool B_NT, bool MI16, bool RAGGED = false, int OPER = kBf16, int NB = 2 * TN>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_split_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gemm_dtl_tile<B_NT, false, true, RAGGED, MI16, NB, F8>(g, smem);
+    gemm_dtl_tile<B_NT, false, true, RAGGED, MI16, NB, OPER>(g, smem);
 }
 
 // Third launch: sums the parts of every tail tile in the order 0..S-1 and applies the epilogue
@@ -1203,7 +1272,7 @@ hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* w
         hipLaunchKernelGGL((gemm_dtl_split_kernel<__VA_ARGS__>), sgrid, block, LDS_BYTES, st, gs);                              \
     } while (0)
         if (g.n224) {
-            if (split_ragged) KR_LAUNCH(true, true, true, false, 7); else KR_LAUNCH(true, true, false, false, 7);
+            if (split_ragged) KR_LAUNCH(true, true, true, kBf16, 7); else KR_LAUNCH(true, true, false, kBf16, 7);
         } else if (!g.mi16) {   // (whole tiles only)
             if (b_nt) KR_LAUNCH(true, false); else KR_LAUNCH(false, false);
         } else if (split_ragged) {
@@ -1219,31 +1288,38 @@ hipError_t launch_gemm_dtl(const GemmArgs& g, bool b_nt, hipStream_t st, void* w
     return hipGetLastError();
 }
 
-// g as for the bf16 kernel with the fp8 operands described in two-byte units (K, lda, ldb halved);
+// Operands described to the kernel as bf16 matrices: fp8 in two-byte units (K, lda, ldb halved), pairs as twice the width.
 // g.tail_tiles tiles are split over g.k_splits workgroups each, as for the bf16 kernel.
-hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace) {
+template <int OPER>
+static hipError_t launch_gemm_units(const GemmArgs& g, hipStream_t st, void* workspace, const void* whole_fn, const void* ragged_fn) {
     const bool ragged = g.M % BM != 0 || g.N % BN != 0 || g.K % BKD != 0;
     const dim3 grid((unsigned)(g.tiles_m * g.tiles_n - g.tail_tiles)), block(WM * WN * 64);
     static std::atomic<uint64_t> opted[4];
     if (grid.x > 0) {
-        const void* kfn = ragged ? (const void*)gemm_dtl8_kernel<true> : (const void*)gemm_dtl8_kernel<false>;
+        const void* kfn = ragged ? ragged_fn : whole_fn;
         if (hipError_t e = lds_opt_in(kfn, LDS_BYTES, opted[ragged]); e != hipSuccess) return e;
-        if (ragged) hipLaunchKernelGGL(gemm_dtl8_kernel<true>, grid, block, LDS_BYTES, st, g);
-        else hipLaunchKernelGGL(gemm_dtl8_kernel<false>, grid, block, LDS_BYTES, st, g);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        GemmArgs args = g;
+        void* argv[] = {&args};
+        if (hipError_t e = hipLaunchKernel(kfn, grid, block, argv, LDS_BYTES, st); e != hipSuccess) return e;
     }
     if (g.tail_tiles > 0) {
         GemmArgs gs = g;
         gs.out = workspace;
+        void* argv[] = {&gs};
         const dim3 sgrid((unsigned)(g.tail_tiles * g.k_splits));
-        const void* sfn = ragged ? (const void*)gemm_dtl_split_kernel<true, true, true, true> : (const void*)gemm_dtl_split_kernel<true, true, false, true>;
+        const void* sfn = ragged ? (const void*)gemm_dtl_split_kernel<true, true, true, OPER> : (const void*)gemm_dtl_split_kernel<true, true, false, OPER>;
         if (hipError_t e = lds_opt_in(sfn, LDS_BYTES, opted[2 + ragged]); e != hipSuccess) return e;
-        if (ragged) hipLaunchKernelGGL((gemm_dtl_split_kernel<true, true, true, true>), sgrid, block, LDS_BYTES, st, gs);
-        else hipLaunchKernelGGL((gemm_dtl_split_kernel<true, true, false, true>), sgrid, block, LDS_BYTES, st, gs);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        if (hipError_t e = hipLaunchKernel(sfn, sgrid, block, argv, LDS_BYTES, st); e != hipSuccess) return e;
         return launch_tail_finish(g, st, workspace);
     }
     return hipGetLastError();
+}
+
+hipError_t launch_gemm_dtl8(const GemmArgs& g, hipStream_t st, void* workspace) {
+    return launch_gemm_units<kFp8>(g, st, workspace, (const void*)gemm_dtl8_kernel<false>, (const void*)gemm_dtl8_kernel<true>);
+}
+hipError_t launch_gemm_pairs(const GemmArgs& g, hipStream_t st, void* workspace) {
+    return launch_gemm_units<kPairs>(g, st, workspace, (const void*)gemm_dtl_pairs_kernel<false>, (const void*)gemm_dtl_pairs_kernel<true>);
 }
 
 }  // namespace kr

@@ -59,13 +59,20 @@ def fp32_direct(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether fp32 operands go to the kernel that splits them in registers (``kr_gemm_reduce_f32_ws``).
 
     Up to two rounds of its 128 x 128 tiles on the 256 compute units: 2000 x 4096 x 2048 takes 117 us there and 166 us
-    as a split pass and a bf16 product; with more tiles the 256 x 256 bf16 kernel wins the pass back
-    (4096 x 4096 x 1024: 135 against 104 us).  The kernel addresses 128 rows of an operand with 32-bit byte offsets: row
+    as a split pass and a bf16 product of 3K; with more tiles, and where ``fp32_pairs`` says so, 256 x 256 tiles win a
+    pass back.  The kernel addresses 128 rows of an operand with 32-bit byte offsets: row
     strides beyond that reach (from about 4.19 million elements on) take the split pass, which reads any stride.
     """
     if not (a.is_cuda and b.is_cuda) or a.shape[1] % 8 != 0 or b.shape[1] % 8 != 0:
         return False
     return -(-a.shape[0] // 128) * -(-b.shape[1] // 128) <= 512 and _fp32_in_reach(a, b)
+
+
+def fp32_pairs(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether fp32 operands are split by one pass over both and multiplied part by part (``kr_split_pairs_fp32``,
+    ``kr_gemm_reduce_pairs_ws``): many tiles or a long K (``kr_gemm_f32_pairs``)."""
+    (M, K), N = a.shape, b.shape[1]
+    return a.is_cuda and b.is_cuda and K % 8 == 0 and N % 8 == 0 and _lib.load().kr_gemm_f32_pairs(M, N, K) == 1
 
 
 def _fp32_in_reach(a: torch.Tensor, b: torch.Tensor) -> bool:
@@ -90,7 +97,7 @@ def prepare_operands(a: torch.Tensor, b: torch.Tensor, keep_fp32: bool = False) 
     stridings (the reference accepts any 2-D strides,
     ``gemm_one_shot_all_reduce_fused.py:163-166``) take one copy.  fp32 operands are split into
     bf16 parts by one kernel pass each (``split_fp32``); with ``keep_fp32``, for callers whose
-    product goes through ``launch``, they stay fp32 where it splits them itself (``fp32_direct``).
+    product goes through ``launch``, they stay fp32 where that splits them (``fp32_direct``, ``fp32_pairs``).
     K is padded to a multiple of 8 with zeros when necessary.
     """
     assert a.dim() == 2 and b.dim() == 2
@@ -98,7 +105,7 @@ def prepare_operands(a: torch.Tensor, b: torch.Tensor, keep_fp32: bool = False) 
     assert a.dtype == b.dtype, "Input tensors must have the same dtype"
     assert a.dtype in (torch.bfloat16, torch.float32), "bfloat16 (or float32) operands expected"
     if a.dtype == torch.float32:
-        if keep_fp32 and fp32_direct(a, b):
+        if keep_fp32 and (fp32_direct(a, b) or fp32_pairs(a, b)):
             return fp32_layout(a, b)
         a, b = split_fp32(a, b)
     K = a.shape[1]
@@ -145,8 +152,20 @@ def launch(name, a, b, M, N, peers, n_peers, peers_stride, bias, band_row0, band
         K = a.shape[1]
         plist = peers if isinstance(peers, (list, tuple)) else [] if peers is None else list(peers)
         dev = _lib.require_device(a, b, *plist, bias, c_full, out)
-        ws = workspace(dev, lib.kr_gemm_f32_workspace_bytes(M, N, K))
         table = (ctypes.c_void_p * max(n_peers, 1))(*[t.data_ptr() for t in plist])
+        if fp32_pairs(a, b):
+            stream = _lib.current_stream(dev)
+            width = -(-K // 32) * 64
+            pairs = torch.empty((M + N, width), dtype=torch.bfloat16, device=dev)
+            ap, bp = pairs.data_ptr(), pairs.data_ptr() + M * width * 2
+            rc = lib.kr_split_pairs_fp32(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), b.stride(1), M, N, K, ap, bp, stream)
+            _lib.check(rc, name)
+            ws = workspace(dev, lib.kr_gemm_pairs_workspace_bytes(M, N, K))
+            rc = lib.kr_gemm_reduce_pairs_ws(ap, bp, M, N, K, table, n_peers, _lib.ptr(bias), band_row0, band_rows, _lib.ptr(c_full),
+                                             _lib.ptr(out), out_fp32, pivot, _lib.ptr(ws), ws.numel() if ws is not None else 0, stream)
+            _lib.check(rc, name)
+            return
+        ws = workspace(dev, lib.kr_gemm_f32_workspace_bytes(M, N, K))
         rc = lib.kr_gemm_reduce_f32_ws(
             a.data_ptr(), a.stride(0), a.stride(1), b.data_ptr(), b.stride(0), b.stride(1), M, N, K,
             table, n_peers, _lib.ptr(bias), band_row0, band_rows, _lib.ptr(c_full), _lib.ptr(out), out_fp32, pivot,

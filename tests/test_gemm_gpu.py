@@ -1897,3 +1897,44 @@ def test_epilogue_at_the_edges(dev, tile, M, N, K, P):
         lo, hi = rank * rows, (rank + 1) * rows
         assert torch.equal(out.float(), want[lo:hi] + peers[:, :rows].float().sum(0))
         assert torch.equal(c[:lo].float(), want[:lo]) and torch.equal(c[hi:].float(), want[hi:]) and bool(c[lo:hi].isnan().all())
+
+
+@pytest.mark.parametrize("parts", [0, 3])
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,K,W,rank", [(65, 8, 8, 1, 0), (128, 264, 40, 2, 1), (256, 256, 64, 2, 0), (260, 520, 72, 4, 2), (520, 328, 1000, 8, 7)])
+def test_fp32_operands_as_pairs(dev, monkeypatch, M, N, K, W, rank, b_t, parts):
+    """kr_split_pairs_fp32 and kr_gemm_reduce_pairs_ws: a last group of 32 k that is not full (its zeros are written into a
+    buffer of NaN), edges of the 64 x 64 blocks of the pass and of the tiles, K loops in one pass and in three parts, operands whose rows
+    lie apart.  Integers up to 2^11 (hi and lo parts exact) times integers up to 8, every sum below 2^24: exact."""
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_PAIRS", "1")
+    monkeypatch.setenv("KRAKEN_AMD_GEMM_TAILSPLIT", str(parts))
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.full((M, K + 4), float("nan"), device=dev)
+    b = torch.full((N, K + 4) if b_t else (K, N + 4), float("nan"), device=dev)
+    a[:, :K] = torch.randint(-2047, 2048, (M, K), generator=g).float()
+    bv = torch.randint(-8, 9, (K, N), generator=g).float().to(dev)
+    if b_t:
+        b[:, :K] = bv.T
+        b = b[:, :K].T
+    else:
+        b[:, :N] = bv
+        b = b[:, :N]
+    a = a[:, :K]
+    assert K * 2047 * 8 < 1 << 24
+    from kraken_amd.fused import _gemm
+    assert _gemm.fp32_pairs(a, b)
+    rows = M // W
+    peers = torch.randint(-8, 9, (W - 1, M, N), generator=g).to(BF16).to(dev) if W > 1 else None
+    bias = torch.randint(-8, 9, (N,), generator=g).to(BF16).to(dev)
+    want = a.contiguous().double() @ bv.double()
+    for poison in range(2):     # (the allocator hands the pass a buffer of the last call's values)
+        out = fused.gemm_one_shot_all_reduce_fused(a, b, peers=peers, bias=bias)
+        assert torch.equal(out.double(), want + (peers.double().sum(0) if W > 1 else 0) + bias.double())
+        torch.full(((M + N) * (K // 32 + 1) * 32,), float("nan"), device=dev)
+    if M % W == 0 and W > 1:
+        c = torch.zeros((M, N), dtype=BF16, device=dev)
+        mine = peers[:, :rows].contiguous()
+        out = fused.gemm_reduce_scatter(a, b, peers=mine, rank=rank, c_scratch=c)
+        lo, hi = rank * rows, (rank + 1) * rows
+        assert out.dtype == torch.float32 and torch.equal(out.double(), want[lo:hi] + mine.double().sum(0))
+        assert torch.equal(c[:lo], want[:lo].to(BF16)) and torch.equal(c[hi:], want[hi:].to(BF16))
