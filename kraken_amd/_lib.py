@@ -189,6 +189,7 @@ class _NoCalls:
 
 def _load_calls():
     from .comm._common import row_exchange, row_watch
+    from ._waits import check as waits_check
     from .fused._gemm import stream_workspace
 
     lib = load()
@@ -199,7 +200,7 @@ def _load_calls():
     if built_for != str(torch.__version__):      # (it reads torch's objects by their layout)
         raise ImportError(f"built for torch {built_for}, not {torch.__version__}")
     module.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in EXPORTS},
-                torch._C._cuda_getCurrentRawStream, row_exchange, row_watch, stream_workspace)
+                torch._C._cuda_getCurrentRawStream, row_exchange, row_watch, stream_workspace, waits_check)
     return module
 
 

@@ -4,6 +4,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib, _waits
 from ..comm._common import PeerBuffers, has_tangent
@@ -166,6 +167,17 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
     return a_out, c
 
 
+def _common_form(a_shared, b, a_out, progress, rank=0, splits_per_rank=1, gather=None, **kwargs):
+    """The call in native code where its arguments are of the common form: nothing but sizes named, and no tangents about."""
+    if kwargs or forward_ad._current_level >= 0:
+        return None
+    if gather is None:
+        gather = not isinstance(a_shared, torch.Tensor)     # (a stack that is not contiguous goes the general way in any case)
+    if type(gather) is not bool:
+        return None
+    return _lib.calls().gather_matmul(a_shared, b, a_out, progress, rank, splits_per_rank, gather)
+
+
 def all_gather_matmul(
     a_shared,
     b: torch.Tensor,
@@ -220,6 +232,9 @@ def all_gather_matmul(
     fp32 sums rounded to fp8 once.
     ``a_gathered`` stays fp8.
     """
+    out = _common_form(a_shared, b, a_out, progress, **kwargs)
+    if out is not None:
+        return out
     fp8 = torch.float8_e4m3fn
     peers = PeerBuffers(a_shared, dtypes=(torch.bfloat16, fp8))
     if peers.tensors[0].dtype == fp8:

@@ -4,6 +4,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib, _waits
 from ..comm._common import has_tangent
@@ -197,6 +198,14 @@ def copy_engine_scatter(
         _waits.watch(status, "copy_engine_scatter")
 
 
+def _common_form(a, b, reduce_op, peers=None, rank=0, sent=None, fp32_acc=False, **kwargs):
+    """The call in native code where its arguments are of the common form: all peers in one tensor, the destinations in another,
+    nothing else named, and no tangents about."""
+    if kwargs or reduce_op != "sum" or type(fp32_acc) is not bool or forward_ad._current_level >= 0:
+        return None
+    return _lib.calls().reduce_scatter_sent(a, b, peers, sent, rank, not fp32_acc)
+
+
 def gemm_reduce_scatter_ce_persistent(
     a: torch.Tensor,
     b: torch.Tensor,
@@ -223,6 +232,9 @@ def gemm_reduce_scatter_ce_persistent(
     waits for the side stream (``:370``).  kwargs ``rank`` (default 0), ``world_size``, ``fp32_acc``,
     ``wait_limit_us``, ``status``, ``copy_engine``.
     """
+    out = _common_form(a, b, reduce_op, **kwargs)
+    if out is not None:
+        return out
     assert reduce_op == "sum", "only support sum for now"
     assert a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16, "Only bfloat16 is supported for now."
     M, N = a.shape[0], b.shape[1]

@@ -16,7 +16,7 @@ def _common_form(a, b, peers=None, rank=0, c_scratch=None, **kwargs) -> torch.Te
     world_size = kwargs.get("world_size", W)
     if type(world_size) is not int or world_size != W or M % W != 0 or not 0 <= rank < W:
         return None
-    return _lib.calls().gemm(a, b, peers, None, c_scratch, rank * (M // W), M // W, False, rank * (M // W))
+    return _lib.calls().gemm(a, b, peers, None, c_scratch, rank * (M // W), M // W, a.dtype == torch.float32, rank * (M // W))
 
 
 def gemm_reduce_scatter(a: torch.Tensor, b: torch.Tensor, **kwargs) -> torch.Tensor:

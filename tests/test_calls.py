@@ -246,3 +246,103 @@ def test_native_calls_run_on_the_current_stream_and_in_a_graph(dev):
         torch.cuda.synchronize()
         torch.testing.assert_close(y.cpu(), want, rtol=2e-2, atol=2e-2)
         assert torch.equal(out.cpu(), orc.reduce(stack.cpu()))
+
+
+@pytest.mark.parametrize("name,n", [("reduce_scatter_sent", 6), ("gather_matmul", 7)])
+def test_overlap_calls_that_are_not_of_the_common_form(name, n):
+    fn = getattr(_lib.calls(), name)
+    host = torch.zeros(2, 8, dtype=BF16)
+    for value in (host, None, [host, host], [], 1, 1.0, "x", host.to_sparse(), host.to("meta")):
+        for count in (n, n - 1, n + 1, 0):
+            assert fn(*[value] * count) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,W", [(8, 16, 8, 4), (96, 264, 72, 8), (512, 1032, 200, 2), (24, 64, 64, 3), (2304, 4096, 64, 4)])
+def test_fp32_products_are_taken(dev, monkeypatch, M, N, K, W):
+    """fp32 operands: one native step for each kernel that splits them (few rows, in registers, as pairs), the general path's bits."""
+    g = torch.Generator(device=dev).manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)      # noqa: E731
+    native, a, bias = _lib.calls(), rnd(M, K), rnd(N).to(BF16)
+    for b in (rnd(K, N), rnd(N, K).T, rnd(K, N + 4)[:, :N], rnd(N, K + 4)[:, :K].T):
+        peers, c = rnd(W - 1, M // W, N).to(BF16), torch.zeros(M, N, dtype=BF16, device=dev)
+        assert native.gemm(a, b, None, bias, None, 0, M, True, 0).dtype == torch.float32
+        assert native.gemm(a, b, peers, None, c, 0, M // W, True, 0) is not None
+        for dtype in (BF16, torch.float32):
+            assert _same(monkeypatch, lambda: [fused.gemm_one_shot_all_reduce_fused(a, b, bias=bias, out_dtype=dtype)], (b.stride(), dtype))
+        assert _same(monkeypatch, lambda: [fused.gemm_reduce_scatter(a, b, peers=peers, rank=W - 1, c_scratch=c), c.clone()], b.stride())
+    for odd in (a[:, ::2], rnd(K, M).T, rnd(M * K + 1)[1:].view(M, K), a[:1].expand(M, K), a.double(), a.to(BF16)):
+        _same(monkeypatch, lambda: [fused.gemm_one_shot_all_reduce_fused(odd, rnd(odd.shape[1], N))[:0]], odd.stride())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,W", [(16, 16, 8, 2), (96, 264, 72, 8), (512, 1032, 200, 4), (2304, 4096, 64, 4)])
+def test_reduce_scatter_with_destinations_takes_both_paths_alike(dev, monkeypatch, M, N, K, W):
+    g = torch.Generator(device=dev).manual_seed(2)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(BF16)      # noqa: E731
+    m, a = M // W, rnd(M, K)
+    room = rnd(2 * W, m, N)
+    peers = rnd(W - 1, m, N)
+    sents = {"own": lambda: torch.zeros(W, m, N, dtype=BF16, device=dev), "list": lambda: list(torch.zeros(W, m, N, dtype=BF16, device=dev)),
+             "grad": lambda: torch.zeros(W, m, N, dtype=BF16, device=dev, requires_grad=True), "short": lambda: torch.zeros(W - 1, m, N, dtype=BF16, device=dev),
+             "spaced": lambda: torch.zeros(W, m + 1, N, dtype=BF16, device=dev)[:, :m], "none": lambda: None,
+             "over the peers": lambda: room[1:W + 1]}
+    taken = _lib.calls().reduce_scatter_sent(a, rnd(K, N), peers, sents["own"](), 1, True)
+    assert taken.shape == (m, N)
+    for bf, b in (("rows", rnd(K, N)), ("columns", rnd(N, K).T)):
+        for sf, make in sents.items():
+            for rank, kw in ((0, {}), (W - 1, {"fp32_acc": True}), (1, {"world_size": W}), (W, {}), (0, {"world_size": None}), (0, {"reduce_op": "avg"})):
+                def run():
+                    room[:W - 1].copy_(peers)
+                    sent = make()
+                    mine = room[:W - 1] if sf == "over the peers" else peers
+                    versions = getattr(sent, "_version", None)
+                    out = fused.gemm_reduce_scatter_ce_persistent(a, b, peers=mine, rank=rank, sent=sent, **kw)
+                    assert sf != "own" or sent._version > versions
+                    others = [] if sent is None else [t.detach().contiguous() for r, t in enumerate(sent) if r != rank]
+                    return [out, *others]
+
+                _same(monkeypatch, run, (bf, sf, rank, kw))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,N,K,W", [(1, 16, 16, 2), (12, 272, 144, 8), (256, 512, 128, 2), (250, 1040, 272, 3), (512, 4096, 256, 5), (4, 16, 16, 17), (4, 20, 24, 2)])
+def test_gathered_products_take_both_paths_alike(dev, monkeypatch, m, N, K, W):
+    g = torch.Generator(device=dev).manual_seed(4)
+    fp8 = torch.float8_e4m3fn
+    for dtype in (BF16, fp8):
+        rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(dtype)      # noqa: E731
+        stack = rnd(W, m, K)
+        room = rnd(W + 1, m, K)
+        forms = {"stack": stack, "list": [t.clone() for t in stack.unbind()], "tuple": tuple(stack.unbind()),
+                 "columns": stack.view(torch.uint8 if dtype == fp8 else BF16).transpose(1, 2).contiguous().view(dtype).transpose(1, 2), "in the result": list(room[1:].unbind())}
+        ok = 0
+        for (form, shards), (bf, b) in itertools.product(forms.items(), {"columns": rnd(N, K).T, "wide": rnd(N, 2 * K)[:, :K].T, "rows": rnd(K, N)}.items()):
+            for kw in ({}, {"gather": True}, {"gather": False}, {"gather": True, "rank": W - 1, "splits_per_rank": 2}, {"gather": True, "splits_per_rank": 3},
+                       {"gather": True, "rank": W}, {"gather": 1}, {"gather": 0}):
+                for given in ("both", "neither", "flags", "many flags", "small"):
+                    def run():
+                        a_out = None if given in ("neither", "flags") else room[:W].reshape(W * m, K) if form == "in the result" else torch.zeros(W * m, K, device=dev).to(dtype)
+                        flags = None if given == "neither" else torch.full(((W if given == "small" else 3 * W + 5),), 7, dtype=torch.int32, device=dev)
+                        if given == "flags" or given == "both":
+                            flags = flags[:W * kw.get("splits_per_rank", 1)]
+                        if form == "in the result":
+                            room[1:].view(torch.uint8).copy_(stack.view(torch.uint8))
+                        before = None if a_out is None else a_out._version
+                        gathered, c = fused.all_gather_matmul(shards, b, a_out=a_out, progress=flags, **kw)
+                        torch.cuda.synchronize()
+                        assert a_out is None or kw.get("gather") is not True or gathered._version > before
+                        return [gathered.contiguous(), c] + ([] if flags is None else [flags])
+
+                    ok += _same(monkeypatch, run, (dtype, form, bf, kw, given))
+        assert ok > 0 or N % 16 != 0
+        if W <= 16 and N % 16 == 0:
+            a_out, flags = torch.zeros(W * m, K, device=dev).to(dtype), torch.zeros(W, dtype=torch.int32, device=dev)
+            b = rnd(N, K).T
+            assert _lib.calls().gather_matmul(forms["list"], b, a_out, flags, 0, 1, True) is not None
+            assert _lib.calls().gather_matmul(stack, b, None, None, 0, 1, False) is not None
+            if dtype == BF16:     # what autograd follows is left to it
+                forms["list"][0].requires_grad_()
+                assert _lib.calls().gather_matmul(forms["list"], b, a_out, flags, 0, 1, True) is None
+                with torch.no_grad():
+                    assert _lib.calls().gather_matmul(forms["list"], b, a_out, flags, 0, 1, True) is not None
