@@ -394,6 +394,10 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const GemmArgs g, co
         if (g.c_full != nullptr) st_stream((u32x4*)(g.c_full + (int64_t)m * g.N + n), pack8(f));
         return;
     }
+    if (g.out_fp8) {
+        store8_e4m3((uint8_t*)g.out + off, f);
+        return;
+    }
     if (!g.out_is_fp32) unpack8(pack8(f), f);   // the one-pass kernel rounds the product on its way to the epilogue
 #pragma unroll
     for (int q = 0; q < kPeers; ++q)
@@ -407,6 +411,13 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const GemmArgs g, co
     } else {
         st_stream((u32x4*)((uint16_t*)g.out + off), pack8(f));
     }
+}
+
+static hipError_t launch_splitk_finish(const GemmArgs& g, const void* parts, int S, hipStream_t st) {
+    const int64_t vecs = (int64_t)g.M * (g.N / 8);
+    const unsigned threads = vecs > 65536 ? 256 : 64;   // few rows: one wavefront per workgroup, on as many compute units as there are
+    hipLaunchKernelGGL(splitk_finish_kernel, dim3((unsigned)((vecs + threads - 1) / threads)), dim3(threads), 0, st, g, (const float*)parts, S);
+    return hipGetLastError();
 }
 
 template <int BM, int BN, int WM, int WN>
@@ -705,11 +716,12 @@ struct SkinnyPlan {
     int cb;       // columns of a workgroup / 16; 0: not for this call
     int splits;   // parts of K, summed by a second launch
 };
-static SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool b_nt, bool f32, int64_t parts_bytes) {
+static SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool b_nt, int64_t e, int64_t parts_bytes) {   // e: bytes of an element
     SkinnyPlan p{0, 1};
     const EnvSwitches& env = env_switches();
     if (M > 64 || N < 16 || env.gemm_tile > 0 || env.gemm_ks >= 0 || env.gemm_splitk >= 1 || env.gemm_skinny == 0) return p;
-    const int64_t e = f32 ? 4 : 2, units = (K * e + 127) / 128, rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+    const bool f32 = e == 4;
+    const int64_t units = (K * e + 127) / 128, rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
     parts_bytes = std::min(parts_bytes, kMaxPartsBytes);
     if (const int cb = env.gemm_skinny / 100, s = env.gemm_skinny % 100; cb > 0) {   // testing and tuning
         if (cb != 1 && cb != 2 && (cb != 4 || f32)) return p;
@@ -717,7 +729,7 @@ static SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool b_nt, bool f
         if (s >= 1 && s <= units && s * M * N * 4 <= parts_bytes) p.splits = s;
         return p;
     }
-    if (!f32 && M > 16 && N >= 2048 && K > (M > 32 ? (b_nt ? 4096 : 3584) : b_nt ? 11264 : INT64_MAX)) return p;
+    if (e == 2 && M > 16 && N >= 2048 && K > (M > 32 ? (b_nt ? 4096 : 3584) : b_nt ? 11264 : INT64_MAX)) return p;
     int64_t best = 0;
     for (int cb = 1; cb <= (f32 || M > 32 ? 2 : 4); cb *= 2) {
         for (int64_t s = 1; s <= kMaxSplits && (s == 1 || (4 * s <= units && s * M * N * 4 <= parts_bytes)); s *= 2) {
@@ -796,7 +808,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
                           bool dtl_ok, bool skinny_ok) {
     GemmPlan p{};
     if (skinny_ok && !flagged) {
-        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, false, has_workspace ? workspace_bytes : 0);
+        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, 2, has_workspace ? workspace_bytes : 0);
         if (sk.cb != 0) return plan_of_skinny(sk);
     }
     // Tile choice: the 256x256 tile of the LDS-DMA kernel (4 waves x 128x128) has the highest
@@ -912,7 +924,7 @@ static GemmPlan plan_gemm_f32(int64_t M, int64_t N, int64_t K, bool b_nt, int n_
                               bool skinny_ok) {
     GemmPlan p{};
     if (skinny_ok) {
-        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, true, workspace_bytes);
+        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, 4, workspace_bytes);
         if (sk.cb != 0) return plan_of_skinny(sk);
     }
     p.tile = 128;
@@ -1110,17 +1122,13 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
         g1.band_row0 = 0;
         g1.band_rows = (int)M;
         g1.c_full = nullptr;
-        hipError_t e = plan.skinny ? launch_gemm_skinny(g1, b_nt, f32, plan.skinny, (hipStream_t)stream)
+        hipError_t e = plan.skinny ? launch_gemm_skinny(g1, b_nt, f32 ? 4 : 2, plan.skinny, (hipStream_t)stream)
                        : f32 ? launch_gemm_f32(g1, b_nt, (hipStream_t)stream)
                        : plan.ks ? launch_gemm_ks(g1, b_nt, (hipStream_t)stream) : launch_gemm<128, 128, 2, 2>(g1, b_nt, even, (hipStream_t)stream);
         if (e != hipSuccess) return (int)e;
-        const int64_t vecs = M * (N / 8);
-        const unsigned threads = vecs > 65536 ? 256 : 64;   // few rows: one wavefront per workgroup, on as many compute units as there are
-        hipLaunchKernelGGL(splitk_finish_kernel, dim3((unsigned)((vecs + threads - 1) / threads)), dim3(threads), 0,
-                           (hipStream_t)stream, g, (const float*)workspace, splits);
-        return (int)hipGetLastError();
+        return (int)launch_splitk_finish(g, workspace, splits, (hipStream_t)stream);
     }
-    hipError_t e = plan.skinny ? launch_gemm_skinny(g, b_nt, f32, plan.skinny, (hipStream_t)stream)
+    hipError_t e = plan.skinny ? launch_gemm_skinny(g, b_nt, f32 ? 4 : 2, plan.skinny, (hipStream_t)stream)
                        : f32 ? launch_gemm_f32(g, b_nt, (hipStream_t)stream)
                        : dtl ? launch_gemm_dtl(g, b_nt, (hipStream_t)stream, workspace)
                        : plan.ks ? launch_gemm_ks(g, b_nt, (hipStream_t)stream)
@@ -1306,6 +1314,13 @@ extern "C" int kr_gemm_fp8_ws(const void* A, int64_t lda, const void* Bt, int64_
     return gemm_fp8(A, lda, Bt, ldb, M, N, K, out, out_kind, stream, nullptr, false, workspace, workspace_bytes);
 }
 
+// At most 64 rows: gemm_skinny_kernel, which reads B once, where 256-row tiles work for rows that are not there: 0.25 to 0.9 of
+// their time over 4 to 64 rows, N = 1152 to 7488, K = 1088 to 13248, and the form plan_skinny picks the best of them or level with it.
+static SkinnyPlan plan_skinny_fp8(int64_t M, int64_t N, int64_t K, int64_t parts_bytes) {
+    if (env_switches().gemm_w8 >= 0) return SkinnyPlan{0, 1};   // (testing and tuning of the other)
+    return plan_skinny(M, N, K, true, 1, parts_bytes);
+}
+
 // The same product with sums of 24 bits: the operands are widened to bf16 on their way to the matrix cores (gemm_w8.hip).
 static int gemm_fp8_wide(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K, void* out,
                          int64_t tile_pivot, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -1333,6 +1348,22 @@ static int gemm_fp8_wide(const void* A, int64_t lda, const void* Bt, int64_t ldb
     g.out = out;
     g.out_fp8 = 1;
     g.mi16 = 1;
+    if (M * lda + K + 128 < 0x7fffffffLL && 64 * ldb + K + 128 < 0x7fffffffLL && M * N * 2 < 0x7fffffffLL) {
+        if (const SkinnyPlan sk = plan_skinny_fp8(M, N, K, workspace != nullptr ? workspace_bytes : 0); sk.cb != 0) {
+            g.lda = lda;
+            g.ldb = ldb;
+            g.K = (int)K;
+            g.k_splits = sk.splits;
+            if (sk.splits == 1) return (int)launch_gemm_skinny(g, true, 1, sk.cb, (hipStream_t)stream);
+            GemmArgs parts = g;
+            parts.out = workspace;
+            parts.out_fp8 = 0;
+            parts.out_is_fp32 = 1;
+            parts.split_out_stride = M * N;
+            if (hipError_t e = launch_gemm_skinny(parts, true, 1, sk.cb, (hipStream_t)stream); e != hipSuccess) return (int)e;
+            return (int)launch_splitk_finish(g, workspace, sk.splits, (hipStream_t)stream);
+        }
+    }
     const W8Plan p = plan_w8(M, N, K, workspace != nullptr, workspace_bytes);
     g.tiles_m = (int)((M + 255) / 256);
     g.wide_panels = p.panels;
@@ -1347,8 +1378,10 @@ static int gemm_fp8_wide(const void* A, int64_t lda, const void* Bt, int64_t ldb
 
 extern "C" int64_t kr_gemm_fp8_wide_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const SkinnyPlan sk = plan_skinny_fp8(M, N, K, kMaxPartsBytes);
     const W8Plan p = plan_w8(M, N, K, true, kMaxPartsBytes);
-    return p.splits > 1 ? ((M + 255) / 256) * ((N + 255) / 256) * p.splits * (256 * 256 * 4) : 0;
+    // (strides beyond the reach of gemm_skinny_kernel, which are not known here, take the other)
+    return std::max<int64_t>(sk.cb != 0 && sk.splits > 1 ? split_k_workspace_bytes(M, N, sk.splits) : 0, p.splits > 1 ? ((M + 255) / 256) * ((N + 255) / 256) * p.splits * (256 * 256 * 4) : 0);
 }
 
 extern "C" int kr_gemm_fp8_wide_ws(const void* A, int64_t lda, const void* Bt, int64_t ldb, int64_t M, int64_t N, int64_t K,
@@ -1442,7 +1475,7 @@ extern "C" int64_t kr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     for (int form = 0; form < 8; ++form) {
         const bool b_nt = form & 1, plain = (form >> 1) == 0;
         const int n_peers = (form >> 1) == 2 ? 1 : (form >> 1) == 3 ? 2 : 0;
-        if (const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, false, kMaxPartsBytes); sk.cb != 0) {
+        if (const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, 2, kMaxPartsBytes); sk.cb != 0) {
             if (sk.splits > 1) bytes = std::max(bytes, split_k_workspace_bytes(M, N, sk.splits));
             continue;
         }
@@ -1484,7 +1517,7 @@ extern "C" int64_t kr_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) 
     int64_t skinny_bytes = 0;
     bool skinny = false;
     for (const bool b_nt : {false, true}) {
-        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, true, kMaxPartsBytes);
+        const SkinnyPlan sk = plan_skinny(M, N, K, b_nt, 4, kMaxPartsBytes);
         skinny = sk.cb != 0;
         if (skinny && sk.splits > 1) skinny_bytes = std::max(skinny_bytes, split_k_workspace_bytes(M, N, sk.splits));
     }

@@ -79,7 +79,7 @@ hipError_t launch_gemm_w8(const GemmArgs& g, int nb2, hipStream_t st, void* work
 
 hipError_t launch_gemm_ks(const GemmArgs& g, bool b_nt, hipStream_t st);           // 128x128 tiles, k divided between waves (gemm_ks.hip)
 hipError_t launch_gemm_f32(const GemmArgs& g, bool b_nt, hipStream_t st);          // fp32 operands (gemm_f32.hip); A, B, lda, ldb in fp32 elements
-hipError_t launch_gemm_skinny(const GemmArgs& g, bool b_nt, bool f32, int cb, hipStream_t st);   // at most 64 rows, 16 cb columns per workgroup (gemm_skinny.hip)
+hipError_t launch_gemm_skinny(const GemmArgs& g, bool b_nt, int esize, int cb, hipStream_t st);   // at most 64 rows, 16 cb columns per workgroup (gemm_skinny.hip)
 hipError_t load_gemm_dtl();
 hipError_t load_gemm_ks();
 hipError_t load_gemm_skinny();
@@ -548,6 +548,12 @@ template <bool HIGH_HALF>
 __device__ __forceinline__ uint32_t pack2_e4m3(float a, float b, uint32_t old) {
     const float ca = __builtin_fminf(__builtin_fmaxf(a, -448.0f), 448.0f), cb = __builtin_fminf(__builtin_fmaxf(b, -448.0f), 448.0f);
     return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a != a ? a : ca, b != b ? b : cb, (int)old, HIGH_HALF);
+}
+
+// eight consecutive values as fp8
+__device__ __forceinline__ void store8_e4m3(uint8_t* p, const float (&f)[8]) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    *(u32x2*)p = u32x2{pack2_e4m3<true>(f[2], f[3], pack2_e4m3<false>(f[0], f[1], 0u)), pack2_e4m3<true>(f[6], f[7], pack2_e4m3<false>(f[4], f[5], 0u))};
 }
 
 // fp8 store of a wave's 128 x 16 NB part of a tile held as 8 x NB accumulator blocks of 16 x 16 (lane l:

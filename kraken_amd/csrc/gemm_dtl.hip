@@ -1155,8 +1155,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[e] = lo[e], f[4 + e] = hi[e];
         if (g.out_fp8) {
-            *(u32x2*)((uint8_t*)g.out + (int64_t)m * g.N + n) = u32x2{pack2_e4m3<true>(f[2], f[3], pack2_e4m3<false>(f[0], f[1], 0u)),
-                                                                      pack2_e4m3<true>(f[6], f[7], pack2_e4m3<false>(f[4], f[5], 0u))};
+            store8_e4m3((uint8_t*)g.out + (int64_t)m * g.N + n, f);
             continue;
         }
         const int mb = m - g.band_row0;

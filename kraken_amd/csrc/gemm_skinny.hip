@@ -15,7 +15,9 @@
 // finishing pass 20.9; reading B at 6.3 TB/s 9.3), 4 x 3360 x 976 6.3 (14.1), fp32 16 x 4096 x 4096 17.6 (28.7).  What bounds
 // it: HBM for wide outputs, the 64 GB/s a compute unit takes in for narrow ones, 6 us of start and end for small ones.
 //
-// fp32 operands are split into hi and lo parts in registers and take three products (hi hi, lo hi, hi lo).
+// fp32 operands are split into hi and lo parts in registers and take three products (hi hi, lo hi, hi lo); fp8 operands are
+// widened to bf16 in registers.  us, 256-row tiles of gemm_w8.hip / here: 16 x 4672 x 4096 23.8 / 7.4, x 13248 37.1 / 21.4 (B at 6.3 TB/s: 9.8),
+// 4 x 1152 x 1088 15.6 / 5.9, 64 x 7488 x 4096 27.2 / 13.1, x 13248 45.7 / 37.4.
 #include "gemm_common.h"
 
 namespace kr {
@@ -55,17 +57,28 @@ __device__ __forceinline__ void split8(const u32x4 (&x)[2], bf16x8& hi, bf16x8& 
     lo = __builtin_bit_cast(bf16x8, l);
 }
 
+// eight fp8 (e4m3) as bf16, exactly
+__device__ __forceinline__ bf16x8 widen8(uint32_t w0, uint32_t w1) {
+    return __builtin_bit_cast(bf16x8, u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w0, 1.0f, false)),
+                                            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w0, 1.0f, true)),
+                                            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w1, 1.0f, false)),
+                                            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w1, 1.0f, true))});
+}
+
 // row-major B: slot of a k-row in LDS that holds piece 0; a fragment read then touches every bank once or twice
-template <bool F32, int CB>
+template <int E, int CB>
 __device__ __forceinline__ int swizzle(int k) {
-    if constexpr (F32) return CB > 1 ? 4 * ((k >> 2) & 1) : 0;
+    if constexpr (E == 4) return CB > 1 ? 4 * ((k >> 2) & 1) : 0;
     return CB > 2 ? 2 * ((k >> 1) & 1) + 4 * ((k >> 3) & 1) : CB > 1 ? 2 * ((k >> 3) & 1) : 0;
 }
 
-template <bool F32, bool B_NT, int MB, int CB>
+// E: bytes of an operand's element: 4 fp32, 2 bf16, 1 fp8 (transposed-contiguous B only)
+template <int E, bool B_NT, int MB, int CB>
 __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // starts at LDS address 0; one ring per wavefront
-    constexpr int E = F32 ? 4 : 2, NB = 16 * CB, LD = red_pitch(CB);
+    constexpr bool F32 = E == 4, F8 = E == 1;
+    static_assert(!F8 || B_NT, "fp8: transposed-contiguous B");
+    constexpr int NB = 16 * CB, LD = red_pitch(CB);
     constexpr int KU = 128 / E;                                // k of a unit
     constexpr int kWaves = waves_of(MB, CB), kStages = stages_of(MB, CB), kRing = ring_bytes(MB, CB);
     constexpr int kStage = (MB + CB) * kBlock, kLoads = 2 * (MB + CB);
@@ -114,7 +127,7 @@ __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(cons
             // row-major B: a load fills 1 KiB of k-rows of NB columns, their pieces permuted by swizzle(k)
             constexpr int PR = NB * E / 16, KR = 64 / PR;   // pieces of a k-row, k-rows of a load
             const int k = KR * r + lane / PR;
-            const int piece = (lane % PR) ^ swizzle<F32, CB>(k);
+            const int piece = (lane % PR) ^ swizzle<E, CB>(k);
             b_off[r] = (uint32_t)((k * g.ldb + min(piece * (16 / E), g.N - 16 / E - n0)) * E);
         }
     }
@@ -144,7 +157,7 @@ __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(cons
     for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int c = 0; c < CB; ++c) acc[i][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    u32x4 af[MB][2], bf[CB][2];   // bf16: the fragments of both 32-k halves; fp32: 8 values
+    u32x4 af[MB][2], bf[CB][2];   // bf16: the fragments of both 32-k halves; fp32: 8 values; fp8: 16 and 16 values
     auto read_unit = [&](uint32_t stage) __attribute__((always_inline)) {
         const uint32_t a = ring + stage, b = a + MB * kBlock;
 #pragma unroll
@@ -159,7 +172,7 @@ __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(cons
                 bf[c][1] = *(lds_u4)(size_t)(b + c * kBlock + f1);
             } else if constexpr (F32) {
                 // column 16c + p of k-rows 4 gq .. +3 and 16 + 4 gq .. +3
-                const uint32_t o = b + (uint32_t)(4 * gq * NB * 4 + (((4 * c + (p >> 2)) ^ swizzle<F32, CB>(4 * gq)) << 4) + (p & 3) * 4);
+                const uint32_t o = b + (uint32_t)(4 * gq * NB * 4 + (((4 * c + (p >> 2)) ^ swizzle<E, CB>(4 * gq)) << 4) + (p & 3) * 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     bf[c][0][e] = *(lds_u1)(size_t)(o + e * NB * 4);
@@ -167,7 +180,7 @@ __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(cons
                 }
             } else {
                 // transposing reads: group gq reads k-rows 32 h + 8 gq + p/4 (and 4 further on), columns 16c + 4 (p%4) .. +3
-                const uint32_t o = b + (uint32_t)((8 * gq + (p >> 2)) * NB * 2 + (((2 * c + ((p & 3) >> 1)) ^ swizzle<F32, CB>(8 * gq + (p >> 2))) << 4) + (p & 1) * 8);
+                const uint32_t o = b + (uint32_t)((8 * gq + (p >> 2)) * NB * 2 + (((2 * c + ((p & 3) >> 1)) ^ swizzle<E, CB>(8 * gq + (p >> 2))) << 4) + (p & 1) * 8);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(size_t)(o + 32 * h * NB * 2));
@@ -191,6 +204,20 @@ __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(cons
                     acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b_hi, a_hi[i], acc[i][c], 0, 0, 0);
                     acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b_lo, a_hi[i], acc[i][c], 0, 0, 0);
                     acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b_hi, a_lo[i], acc[i][c], 0, 0, 0);
+                }
+            }
+        } else if constexpr (F8) {
+            // (16 k of a piece in two halves of 8: both operands take their k in this order)
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                bf16x8 a8[MB];
+#pragma unroll
+                for (int i = 0; i < MB; ++i) a8[i] = widen8(af[i][h / 2][2 * (h % 2)], af[i][h / 2][2 * (h % 2) + 1]);
+#pragma unroll
+                for (int c = 0; c < CB; ++c) {
+                    const bf16x8 b8 = widen8(bf[c][h / 2][2 * (h % 2)], bf[c][h / 2][2 * (h % 2) + 1]);
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b8, a8[i], acc[i][c], 0, 0, 0);
                 }
             }
         } else {
@@ -247,6 +274,12 @@ __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(cons
         if (g.c_full != nullptr) st_stream((u32x4*)(g.c_full + (int64_t)er * g.N + en), pack8(f));
         return;
     }
+    if constexpr (F8) {
+        if (g.out_fp8) {   // (no peers, no bias)
+            store8_e4m3((uint8_t*)g.out + (int64_t)mb * g.N + en, f);
+            return;
+        }
+    }
     // (a bf16 product is rounded before the partial sums are added, as in the other kernels)
     if (!g.out_is_fp32) unpack8(pack8(f), f);
 #pragma unroll
@@ -264,20 +297,20 @@ __global__ __launch_bounds__(waves_of(MB, CB) * 64) void gemm_skinny_kernel(cons
     }
 }
 
-template <bool F32, bool B_NT, int MB, int CB>
+template <int E, bool B_NT, int MB, int CB>
 hipError_t launch_one(const GemmArgs& g, hipStream_t st) {
     constexpr int lds = waves_of(MB, CB) * ring_bytes(MB, CB);
-    auto kfn = gemm_skinny_kernel<F32, B_NT, MB, CB>;
+    auto kfn = gemm_skinny_kernel<E, B_NT, MB, CB>;
     static std::atomic<uint64_t> opted{0};
     if (hipError_t e = lds_opt_in((const void*)kfn, lds, opted); e != hipSuccess) return e;
     hipLaunchKernelGGL(kfn, dim3((unsigned)((g.N + 16 * CB - 1) / (16 * CB)), (unsigned)g.k_splits), dim3(waves_of(MB, CB) * 64), lds, st, g);
     return hipGetLastError();
 }
-template <bool F32, bool B_NT, int CB>
+template <int E, bool B_NT, int CB>
 hipError_t launch_rows(const GemmArgs& g, hipStream_t st) {
-    if (g.M <= 16) return launch_one<F32, B_NT, 1, CB>(g, st);
-    if (g.M <= 32) return launch_one<F32, B_NT, 2, CB>(g, st);
-    return launch_one<F32, B_NT, 4, CB < 4 ? CB : 2>(g, st);   // (64 x 64: more results than threads)
+    if (g.M <= 16) return launch_one<E, B_NT, 1, CB>(g, st);
+    if (g.M <= 32) return launch_one<E, B_NT, 2, CB>(g, st);
+    return launch_one<E, B_NT, 4, CB < 4 ? CB : 2>(g, st);   // (64 x 64: more results than threads)
 }
 
 }  // namespace
@@ -286,16 +319,17 @@ hipError_t launch_rows(const GemmArgs& g, hipStream_t st) {
 // device memory).
 hipError_t load_gemm_skinny() {
     hipFuncAttributes a;
-    return hipFuncGetAttributes(&a, (const void*)gemm_skinny_kernel<false, true, 1, 1>);
+    return hipFuncGetAttributes(&a, (const void*)gemm_skinny_kernel<2, true, 1, 1>);
 }
 
-hipError_t launch_gemm_skinny(const GemmArgs& g, bool b_nt, bool f32, int cb, hipStream_t st) {
-    if (f32) {
-        if (b_nt) return cb == 1 ? launch_rows<true, true, 1>(g, st) : launch_rows<true, true, 2>(g, st);
-        return cb == 1 ? launch_rows<true, false, 1>(g, st) : launch_rows<true, false, 2>(g, st);
+hipError_t launch_gemm_skinny(const GemmArgs& g, bool b_nt, int esize, int cb, hipStream_t st) {
+    if (esize == 1) return cb == 1 ? launch_rows<1, true, 1>(g, st) : cb == 2 ? launch_rows<1, true, 2>(g, st) : launch_rows<1, true, 4>(g, st);
+    if (esize == 4) {
+        if (b_nt) return cb == 1 ? launch_rows<4, true, 1>(g, st) : launch_rows<4, true, 2>(g, st);
+        return cb == 1 ? launch_rows<4, false, 1>(g, st) : launch_rows<4, false, 2>(g, st);
     }
-    if (b_nt) return cb == 1 ? launch_rows<false, true, 1>(g, st) : cb == 2 ? launch_rows<false, true, 2>(g, st) : launch_rows<false, true, 4>(g, st);
-    return cb == 1 ? launch_rows<false, false, 1>(g, st) : cb == 2 ? launch_rows<false, false, 2>(g, st) : launch_rows<false, false, 4>(g, st);
+    if (b_nt) return cb == 1 ? launch_rows<2, true, 1>(g, st) : cb == 2 ? launch_rows<2, true, 2>(g, st) : launch_rows<2, true, 4>(g, st);
+    return cb == 1 ? launch_rows<2, false, 1>(g, st) : cb == 2 ? launch_rows<2, false, 2>(g, st) : launch_rows<2, false, 4>(g, st);
 }
 
 }  // namespace kr

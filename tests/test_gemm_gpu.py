@@ -1938,3 +1938,26 @@ def test_fp32_operands_as_pairs(dev, monkeypatch, M, N, K, W, rank, b_t, parts):
         lo, hi = rank * rows, (rank + 1) * rows
         assert out.dtype == torch.float32 and torch.equal(out.double(), want[lo:hi] + mine.double().sum(0))
         assert torch.equal(c[:lo], want[:lo].to(BF16)) and torch.equal(c[hi:], want[hi:].to(BF16))
+
+
+@pytest.mark.parametrize("form", [None, 101, 201, 401, 102, 203, 404])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (16, 48, 112), (17, 272, 128), (32, 80, 1040), (33, 1040, 144), (64, 304, 2064)])
+def test_fp8_few_rows_kernel(dev, monkeypatch, M, N, K, form):
+    """fp8 operands with at most 64 rows: units of k that are not full, columns past N, one part of K and several.  Operands of -1, 0,
+    1: the sums are whole numbers below 2^24, so the result is their one rounding to fp8; poisoned beyond the sizes."""
+    if form is not None:
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_SKINNY", str(form))
+    fp8 = torch.float8_e4m3fn
+    big = torch.full((M + N + 2, K + 32), float("nan"), device=dev).to(fp8)
+    a, b = _small_integers((M, K), 1, 1.0, dev), _small_integers((N, K), 2, 1.0, dev)
+    big[:M, :K], big[M + 1:-1, :K] = a.to(fp8), b.to(fp8)
+    lib = _lib.load()
+    out = torch.full((M + 1, N), float("nan"), device=dev).to(fp8)
+    ws = torch.full((lib.kr_gemm_fp8_wide_workspace_bytes(M, N, K) + 4 * 4 * M * N,), 255, dtype=torch.uint8, device=dev)
+    rc = lib.kr_gemm_fp8_wide_ws(big.data_ptr(), K + 32, big[M + 1:].data_ptr(), K + 32, M, N, K, out.data_ptr(), 0, ws.data_ptr(), ws.numel(),
+                                 _lib.current_stream(torch.device("cuda", torch.cuda.current_device())))
+    assert rc == 0
+    want = (a.float() @ b.float().T).clamp(-448, 448).to(fp8)
+    assert torch.equal(out[:M].view(torch.uint8), want.view(torch.uint8)) and bool(out[M:].float().isnan().all())
+    whole = fused.all_gather_matmul(a.to(fp8).view(1, M, K), b.to(fp8).T)[1]
+    assert torch.equal(whole.float(), want.float())      # (-0 and 0)
