@@ -599,8 +599,11 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     workgroups) / 224 (240), K = 8192 68.1 / 66.3, 16384 120 / 109.
 //     Left on the forms they had, which tests/test_capi_host.py and tests/test_gemm_gpu.py name: plain products of whole tiles
 //     (256 columns; 224 are level where they divide N, 512 x 5376 x 6400 50.5 / 50.2, 256 x 7168 x 12928 62.9 / 62.3, and
-//     66 / 63 at 512 x 6656 x 8192); a K that is no multiple of 64 (128x128; 2048 x 2056 x 12296 249 / 133); with transposed B
-//     and at most one peer, ragged shapes of 129 to 272 tiles of 128x128 (1000 x 4096 x 8192 72 / 70, 1000 x 4224 x 4096 56 / 48).
+//     66 / 63 at 512 x 6656 x 8192); with transposed B and at most one peer, ragged shapes of 129 to 272 tiles of 128x128
+//     (1000 x 4096 x 8192 72 / 70, 1000 x 4224 x 4096 56 / 48); whole tiles with a K that is no multiple of 64, and a K
+//     that is no multiple of 16.  Other K make no difference to the parts and cost the 128x128 forms more where they are no multiple of 64:
+//     of 64 such shapes 18 go in parts by the same rule, 0.52 to 0.96 of the time (3144 x 1392 x 15472 270 / 141,
+//     3224 x 1248 x 7136 row-major with a band 142 / 75, 736 x 6416 x 5680 105 / 78, 1016 x 3728 x 2512 38.4 / 36.5).
 // Which 128x128 kernel, by the time of gemm_ks_kernel over that of gemm_reduce_kernel (geometric means over 20 000 random
 // shapes, 1 to 8192 rows, operands in no cache):
 //   transposed B, in parts: 1.034 to 1.042 at every K: gemm_reduce_kernel.  In one pass, K a multiple of 64, no peers:
@@ -649,7 +652,7 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, int n_pe
     const EnvSwitches& env = env_switches();
     const int64_t force = env.gemm_tailsplit;   // 0: off, n: n parts (testing)
     const bool whole = M % 256 == 0 && N % 256 == 0;
-    const bool as_before = K % 64 != 0 || K < 2048 || (!whole && b_nt && n_peers < 2 && tiles > 128 && tiles <= 272);   // see above
+    const bool as_before = K < 2048 || (K % 64 != 0 && (K % 16 != 0 || whole)) || (!whole && b_nt && n_peers < 2 && tiles > 128 && tiles <= 272);   // see above
     if (may_big && dtl_ok && force != 0 && (env.gemm_mfma != 32 || (whole && K % 64 == 0)) && (!as_before || force > 0)) {
         // whole tiles, K from 4096 on, as many parts as there are compute units for: no margin
         const int64_t most = std::min<int64_t>({256 / std::max<int64_t>(1, big_tiles_of(M, N, 256)), kMaxTailSplits, steps / kMinSplitSteps});

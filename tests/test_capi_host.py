@@ -782,3 +782,21 @@ def test_fp8_wide_empty_products_check_the_operand_that_has_elements(lib):
     for off, M, N, want in ((8, 0, 64, 0), (8, 16, 0, _lib.KR_ERR_ALIGNMENT), (0, 16, 0, 0), (0, 0, 64, 0)):
         assert f(FAKE + off, 64, FAKE, 64, M, N, 64, FAKE, 0, None, 0, None) == want
         assert f(FAKE, 64, FAKE + off, 64, N, M, 64, FAKE, 0, None, 0, None) == want
+
+
+@pytest.mark.parametrize("M,N,K,b_t,P", [(736, 6416, 5680, True, 7), (3224, 1248, 7136, False, 3), (3144, 1392, 15472, True, 0), (504, 6656, 8208, False, 1)])
+def test_gemm_plan_few_tiles_and_a_ragged_k_in_parts(lib, M, N, K, b_t, P):
+    """256-row tiles in parts whether or not the last k-step is full, and the workspace for them."""
+    need = lib.kr_gemm_workspace_bytes(M, N, K)
+    p = _lib.gemm_plan(M, N, K, b_t, P, M // (P + 1) if P else M, False, P > 0, workspace_bytes=need)
+    assert p["kernel"] == "gemm_dtl_split_kernel" and p["ragged"] and not p["peers_on_mfma"]
+    assert p["tail_tiles"] * p["tail_splits"] * 1024 * p["tile_n"] <= need <= 64 << 20
+
+
+@pytest.mark.parametrize("M,N,K", [(5486, 3456, 9984), (4360, 4096, 8200), (2312, 8000, 4096)])
+def test_gemm_plan_ragged_shapes_share_their_last_round(lib, M, N, K):
+    need, tiles = lib.kr_gemm_workspace_bytes(M, N, K), -(-M // 256) * -(-N // 256)
+    for b_t in (False, True):
+        p = _lib.gemm_plan(M, N, K, b_t, 7, M // 8, False, True, workspace_bytes=need)
+        assert p["tile"] == 256 and p["tail_tiles"] == tiles % 256 and p["tail_splits"] > 1 and 0 < need <= 64 << 20
+        assert _lib.gemm_plan(M, N, K, b_t, 7, M // 8, False, True)["tail_tiles"] == 0       # no workspace
