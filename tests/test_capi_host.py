@@ -784,7 +784,8 @@ def test_fp8_wide_empty_products_check_the_operand_that_has_elements(lib):
         assert f(FAKE, 64, FAKE + off, 64, N, M, 64, FAKE, 0, None, 0, None) == want
 
 
-@pytest.mark.parametrize("M,N,K,b_t,P", [(736, 6416, 5680, True, 7), (3224, 1248, 7136, False, 3), (3144, 1392, 15472, True, 0), (504, 6656, 8208, False, 1)])
+@pytest.mark.parametrize("M,N,K,b_t,P", [(736, 6416, 5680, True, 7), (3224, 1248, 7136, False, 3), (3144, 1392, 15472, True, 0), (504, 6656, 8208, False, 1),
+                                         (944, 4240, 13360, True, 1), (1100, 1856, 13616, True, 0)])
 def test_gemm_plan_few_tiles_and_a_ragged_k_in_parts(lib, M, N, K, b_t, P):
     """256-row tiles in parts whether or not the last k-step is full, and the workspace for them."""
     need = lib.kr_gemm_workspace_bytes(M, N, K)
