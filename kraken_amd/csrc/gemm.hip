@@ -913,7 +913,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool b_nt, int n_peer
 // fp32 operands split in registers (gemm_f32.hip): 128x128 tiles, S workgroups per tile by the same kind of model
 // as plan_small: 7 us to start and finish, 0.9 us per step of 64 k and round of 256 workgroups.  These choose the parts, they
 // do not give the time: 256 workgroups in one pass measure 1.6 us per step and 13.5 us outside the k loop with row-major B, 1.45
-// and 12 with transposed B, three peers 4 to 5 us more (1000 x 4096, K = 512 .. 8192: 26.6, 40.1, 66.4, 118.6, 216 us).
+// and 12 with transposed B, three peers 1 to 2 us more than one (1000 x 4096, K = 512 .. 4096: 26.9, 38.5, 64.2, 118.5 us).
 static int split_f32(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = (K + 63) / 64;
     if (const int v = env_switches().gemm_splitk; v >= 1 && v <= kMaxSplits) return (int)std::min<int64_t>(v, steps);   // testing and tuning
