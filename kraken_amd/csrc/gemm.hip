@@ -449,7 +449,7 @@ constexpr int kMaxSplits = 16;
 constexpr int kMinSplitSteps = 8;
 // ---- 256x256 kernel: split of the last partial round ------------------------------------------
 // 256 tiles run at a time (one per CU).  When the tile count leaves a last round that is at most
-// 3/8 full and K is long enough, its tiles get S = 256 / tail workgroups each (at least kMinSplitSteps k-steps per
+// 3/8 full (half, with a longer K) and K is long enough, its tiles get S = 256 / tail workgroups each (at least kMinSplitSteps k-steps per
 // part, at most kMaxTailSplits parts), which turns that round from a whole one into tail/256
 // of one; the price is tail * S partial tiles of 256 KiB written and read once.
 constexpr int kMaxTailSplits = 8;
@@ -462,10 +462,12 @@ static void tail_split_plan(int64_t tiles, int64_t K, int* tail_out, int* splits
     const int64_t tail = tiles % 256;
     // (measured: 16..64 tail tiles gain 5-25 % from K = 4096 on; 128 tail tiles at K = 2048 lose
     // 12 %: half a round saved does not pay for two more launches and 64 MiB of parts)
+    // 97 to 128 tiles in two parts each from K = 8192 on, us: 5632 x 4224 (374 tiles) row-major x 11264 469 / 428, x 8192 351 / 324, transposed
+    // 447 / 421, 336 / 322; 6080 x 4096 (384) 462 / 439, 344 / 331, 439 / 422, 322 / 320; x 4096 188 / 197.
     // Ragged shapes the same, us, whole rounds / in parts, transposed B unless said: 5486 x 3456 x 9984 397 / 310 (308 tiles),
     // 4900 x 3648 x 4096 172 / 152, row-major 188 / 157, 2312 x 8000 x 6144 271 / 218, 4584 x 7744 x 5376 348 / 324; below K = 4096
     // transposed B gains little and less with a K of 2048: 4600 x 4096 x 3072 131 / 124, x 2048 88 / 95.
-    if (tail == 0 || (tail > 96 && tiles > 128) || (K < 4096 && force <= 0)) return;
+    if (tail == 0 || (tail > (K >= 8192 ? 128 : 96) && tiles > 128) || (K < 4096 && force <= 0)) return;
     int64_t s = std::min<int64_t>(256 / tail, kMaxTailSplits);
     s = std::min<int64_t>(s, (K / 64) / kMinSplitSteps);
     if (force > 0) s = std::min<int64_t>(force, K / 64);
