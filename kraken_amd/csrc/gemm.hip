@@ -467,8 +467,11 @@ static void tail_split_plan(int64_t tiles, int64_t K, int* tail_out, int* splits
     // Ragged shapes the same, us, whole rounds / in parts, transposed B unless said: 5486 x 3456 x 9984 397 / 310 (308 tiles),
     // 4900 x 3648 x 4096 172 / 152, row-major 188 / 157, 2312 x 8000 x 6144 271 / 218, 4584 x 7744 x 5376 348 / 324; below K = 4096
     // transposed B gains little and less with a K of 2048: 4600 x 4096 x 3072 131 / 124, x 2048 88 / 95.
-    if (tail == 0 || (tail > (K >= 8192 ? 128 : 96) && tiles > 128) || (K < 4096 && force <= 0)) return;
-    int64_t s = std::min<int64_t>(256 / tail, kMaxTailSplits);
+    // A K from 3072 on and up to 48 such tiles, four parts: 4104 x 4096 (272 tiles) x 3072 125 / 116, row-major 132 / 118, x 3648 146 / 130,
+    // 169 / 132; 4864 x 4096 (304) x 3072 126 / 124, 129 / 125, x 3648 149 / 139, 163 / 143; 64 tiles x 3072 124 / 128.
+    const bool short_k = K < 4096 && tiles > 128;
+    if (tail == 0 || (tail > (K >= 8192 ? 128 : short_k ? 48 : 96) && tiles > 128) || (K < (short_k ? 3072 : 4096) && force <= 0)) return;
+    int64_t s = std::min<int64_t>(256 / tail, short_k ? 4 : kMaxTailSplits);
     s = std::min<int64_t>(s, (K / 64) / kMinSplitSteps);
     if (force > 0) s = std::min<int64_t>(force, K / 64);
     if (s < 2) return;

@@ -794,7 +794,7 @@ def test_gemm_plan_few_tiles_and_a_ragged_k_in_parts(lib, M, N, K, b_t, P):
     assert p["tail_tiles"] * p["tail_splits"] * 1024 * p["tile_n"] <= need <= 64 << 20
 
 
-@pytest.mark.parametrize("M,N,K", [(5486, 3456, 9984), (4360, 4096, 8200), (2312, 8000, 4096), (6080, 4096, 8192), (5632, 4224, 11264)])
+@pytest.mark.parametrize("M,N,K", [(5486, 3456, 9984), (4360, 4096, 8200), (2312, 8000, 4096), (6080, 4096, 8192), (5632, 4224, 11264), (4104, 4096, 3072), (4864, 4096, 3648)])
 def test_gemm_plan_ragged_shapes_share_their_last_round(lib, M, N, K):
     need, tiles = lib.kr_gemm_workspace_bytes(M, N, K), -(-M // 256) * -(-N // 256)
     for b_t in (False, True):

@@ -1863,11 +1863,13 @@ def _small_integers(shape, seed, density, dev):
     (2312, 4104, 264, 8, 3),       # the band's tiles ahead of the others, both its edges inside a tile
     (2312, 4104, 264, 8, 7),       # ... the last band, which ends with the matrix
     (3000, 3000, 72, 4, 0), (6144, 3072, 128, 2, 1), (2560, 4096, 64, 2, 0),
-    (520, 2056, 4112, 8, 3), (736, 3608, 4144, 8, 7), (504, 6656, 4112, 8, 0), (944, 2960, 6944, 2, 1)])      # few tiles, all in parts, the last k-step not full
+    (520, 2056, 4112, 8, 3), (736, 3608, 4144, 8, 7), (504, 6656, 4112, 8, 0), (944, 2960, 6944, 2, 1),
+    (4104, 4096, 3080, 4, 2), (5632, 4224, 8192, 8, 0)])      # few tiles, all in parts, the last k-step not full
 def test_reduce_scatter_of_many_tiles(dev, M, N, K, W, rank, b_t):
-    """More than 128 tiles of 256 x 256.  Operands of -1, 0, 1 (a quarter of b's are not zero): every sum is an integer far
-    below 256 (six standard deviations at K = 4160: 160, seven peers 7), so product, sum and rounding are exact."""
-    a, b = _small_integers((M, K), 1, 1.0, dev), _small_integers((K, N), 2, 0.25, dev)
+    """More than 128 tiles of 256 x 256.  Operands of -1, 0, 1 (a quarter of b's are not zero, an eighth with a
+    K above 5000): every sum is an integer far below 256 (six standard deviations at K = 4160: 160, at K = 8192: 160; seven peers
+    7), so product, sum and rounding are exact."""
+    a, b = _small_integers((M, K), 1, 1.0, dev), _small_integers((K, N), 2, 0.25 if K <= 5000 else 0.125, dev)
     peers = _small_integers((W - 1, M // W, N), 3, 1.0, dev)
     c = torch.full((M, N), float("nan"), dtype=BF16, device=dev)
     out = fused.gemm_reduce_scatter(a, b.T.contiguous().T if b_t else b, peers=peers, rank=rank, c_scratch=c)
