@@ -1637,8 +1637,8 @@ extern "C" int kr_gemm_reduce_pairs_ws(const void* A, const void* B, int64_t M, 
     g.k_splits = 1;
     g.mi16 = 1;
     // Peers on the matrix cores spread a value that is not finite over 16 columns: only where the bf16 product of three times
-    // the K did so too.  (In the epilogue 4096 x 4096 x 1024 takes 107 us with one peer, so 101.)
-    const bool many = ((M + 127) / 128) * ((N + 127) / 128) > 512;
+    // the K does so too (many_big_tiles: 3 K from 256 on).  (In the epilogue 4096 x 4096 x 1024 takes 107 us with one peer, so 101.)
+    const bool many = ((M + 127) / 128) * ((N + 127) / 128) > 512 && 3 * K >= 256;
     g.peers_on_mfma = K % 64 != 0 ? 0 : env_switches().gemm_peers >= 0 ? env_switches().gemm_peers : many;
     int tail, splits;
     pairs_split_plan(M, N, K, &tail, &splits);

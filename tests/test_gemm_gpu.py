@@ -1943,6 +1943,17 @@ def test_fp32_operands_as_pairs(dev, monkeypatch, M, N, K, W, rank, b_t, parts):
         assert torch.equal(c[:lo], want[:lo].to(BF16)) and torch.equal(c[hi:], want[hi:].to(BF16))
 
 
+def test_fp32_operands_and_a_peer_that_is_not_finite(dev):
+    """More than 512 tiles of 128 x 128 and a K of 64: the infinity of one element of a peer stays in that element."""
+    M, N, K = 2304, 4096, 64
+    a, b = _small_integers((M, K), 1, 1.0, dev).float(), _small_integers((K, N), 2, 1.0, dev).float()
+    peers = _small_integers((1, M, N), 3, 1.0, dev)
+    peers[0, 300, 1029] = float("inf")
+    want = a @ b + peers[0].float()
+    for given in (peers, list(peers)):      # the native form and the general path
+        assert torch.equal(fused.gemm_one_shot_all_reduce_fused(a, b, peers=given), want)
+
+
 @pytest.mark.parametrize("form", [None, 101, 201, 401, 102, 203, 404])
 @pytest.mark.parametrize("M,N,K", [(1, 16, 16), (16, 48, 112), (17, 272, 128), (32, 80, 1040), (33, 1040, 144), (64, 304, 2064)])
 def test_fp8_few_rows_kernel(dev, monkeypatch, M, N, K, form):
