@@ -265,9 +265,11 @@ int kr_gemm_reduce_ptrs_bf16(const void* A, int64_t lda_m, int64_t lda_k,
  * The K loop of those tiles is split over S workgroups per tile.  Two launches (three for the
  * tail form: the full rounds run as usual first): the S partial products go to the workspace in fp32; a
  * second kernel sums them in the order 0..S-1 and applies the epilogue (peers, bias, band, c_full)
- * with the adds in the same order and the same rounding as the one-pass kernel.  Results are
- * reproducible run to run and differ from the unsplit result only by the fp32 rounding of the
- * order in which the k-steps are summed.  `workspace`: device memory, 16-byte aligned, of at
+ * with the adds in the same order as the one-pass kernel.  The tail form rounds as that kernel does:
+ * its results differ from the unsplit ones only by the fp32 rounding of the order in which the k-steps
+ * are summed.  Where all tiles are in parts, of 256 rows, a bf16 result whose tile has all its rows in the band is rounded
+ * once, product, peers and bias summed in fp32 (with peers: K a multiple of 64); other bf16 results, as those of one pass
+ * over 128x128 tiles, also round the product.  Results are reproducible run to run.  `workspace`: device memory, 16-byte aligned, of at
  * least kr_gemm_workspace_bytes(M, N, K) bytes (0: this shape is not split); its contents
  * before the call do not matter and are undefined after it.  Calls that use one workspace must
  * not overlap (same stream, or otherwise ordered).  workspace == NULL, a workspace that is too

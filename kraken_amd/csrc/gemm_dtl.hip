@@ -1143,7 +1143,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_dtl_tail_finish_kernel(const
     // and adds its peers on the matrix cores (or has none) sums product, peers and bias in fp32 and
     // rounds once; every other tile of a bf16 result rounds the product to bf16 first and adds the
     // peers and the bias to that.
-    const bool tile_in_band = tile_m * BM >= g.band_row0 && tile_m * BM + BM <= g.band_row0 + g.band_rows;
+    // (A last panel that is not full: one of a launch of whole rounds rounds the product first, so its tiles in parts do too.
+    // Where every tile is in parts there is no such launch, and the panel rounds once.)
+    const bool all_in_parts = g.tail_tiles == g.tiles_m * g.tiles_n;
+    const bool tile_in_band = tile_m * BM >= g.band_row0 && tile_m * BM + BM <= g.band_row0 + g.band_rows &&
+                              (all_in_parts || (tile_n + 1) * (WN * WTNX) <= g.N);
     const bool peers_exact = g.peers_on_mfma && g.n_peers > 0 && tile_in_band;
     const bool bias_exact = g.bias != nullptr && tile_in_band && (g.n_peers == 0 || peers_exact);
 #pragma unroll

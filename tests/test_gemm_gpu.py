@@ -1880,6 +1880,31 @@ def test_reduce_scatter_of_many_tiles(dev, M, N, K, W, rank, b_t):
     assert bool(c[lo:hi].isnan().all())      # the band's own rows are not the scratch's
 
 
+@pytest.mark.parametrize("P", [0, 1, 7])
+@pytest.mark.parametrize("M,N,K", [(4136, 4104, 4096), (4352, 4096, 4096), (4360, 4096, 3072)])
+def test_rounding_of_tiles_in_parts_behind_whole_rounds(dev, M, N, K, P):
+    """289 and 272 tiles, the last ones in parts: with a workspace the bits are those without.  Integers, so every sum is exact, of
+    nine bits and more, so rounding once and twice differ: tiles that are whole and in the band add peers and bias in fp32, the others
+    round the product first."""
+    g = torch.Generator(device=dev).manual_seed(M + P)
+    rnd = lambda *s: torch.randint(-3, 4, s, generator=g, device=dev).to(BF16)      # noqa: E731
+    a, b, bias, peers = rnd(M, K), rnd(K, N), rnd(N), rnd(max(P, 1), M, N)
+    lib, stream = _lib.load(), _lib.current_stream(dev)
+    need = lib.kr_gemm_workspace_bytes(M, N, K)
+    assert _lib.gemm_plan(M, N, K, False, P, M, workspace_bytes=need)["tail_tiles"] == (33 if N == 4104 else 16 if K == 4096 else 32)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    outs = [torch.empty(M, N, dtype=BF16, device=dev) for _ in range(2)]
+    args = [a.data_ptr(), K, 1, b.data_ptr(), N, 1, M, N, K, peers.data_ptr(), P, M * N, bias.data_ptr(), 0, M, None]
+    assert lib.kr_gemm_reduce_bf16(*args, outs[0].data_ptr(), 0, 0, stream) == 0
+    assert lib.kr_gemm_reduce_ws_bf16(*args, outs[1].data_ptr(), 0, 0, ws.data_ptr(), need, stream) == 0
+    product, added = a.float() @ b.float(), peers[:P].float().sum(0) + bias.float()
+    want = (product.to(BF16).float() + added).to(BF16)
+    m, n = M // 256 * 256, N // 256 * 256
+    want[:m, :n] = (product + added)[:m, :n].to(BF16)
+    assert torch.equal(outs[0], want)
+    assert torch.equal(outs[1], want)
+
+
 @pytest.mark.parametrize("P", [1, 2, 3, 4, 7, 8])
 @pytest.mark.parametrize("M,N,K", [(264, 264, 64), (520, 328, 136), (90, 8, 64), (383, 640, 72)])
 def test_epilogue_at_the_edges(dev, tile, M, N, K, P):
