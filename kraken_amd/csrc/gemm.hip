@@ -604,13 +604,14 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     workgroups) / 224 (240), K = 8192 68.1 / 66.3, 16384 120 / 109.
 //     Left on the forms they had, which tests/test_capi_host.py and tests/test_gemm_gpu.py name: plain products of whole tiles
 //     (256 columns; 224 are level where they divide N, 512 x 5376 x 6400 50.5 / 50.2, 256 x 7168 x 12928 62.9 / 62.3, and
-//     66 / 63 at 512 x 6656 x 8192); with transposed B and at most one peer, 129 to 272 tiles of 128x128 of which few rows
-//     and no columns are missing (N a multiple of 128, at most 32 rows less than one of M: 1000 x 4096 x 8192 72 / 70, 1000 x 4224 x 4096
-//     56 / 48); whole tiles with a K that is no multiple of 64, and a K that is no multiple of 16.  Others, by the same rule:
+//     66 / 63 at 512 x 6656 x 8192); whole tiles with a K that is no multiple of 64, and a K that is no multiple of 16.  Others, by
+//     the same rule:
 //     a K that is no multiple of 64, which makes no difference to the parts and costs the 128x128 forms more: 18 of 64 shapes go in
 //     parts, 0.52 to 0.96 of the time (3144 x 1392 x 15472 270 / 141, 3224 x 1248 x 7136 row-major with a band 142 / 75, 736 x 6416
 //     x 5680 105 / 78, 1016 x 3728 x 2512 38.4 / 36.5); with transposed B and at most one peer 27 of 60 shapes of 129 to 272 tiles,
-//     0.52 to 1.00 (944 x 4240 x 13360 with one peer 247 / 129, 1100 x 1856 x 13616 plain 233 / 122, 1144 x 2320 x 6784 69 / 58).
+//     0.52 to 1.00 (944 x 4240 x 13360 with one peer 247 / 129, 1100 x 1856 x 13616 plain 233 / 122, 1144 x 2320 x 6784 69 / 58); of
+//     54 of those with N a multiple of 128 and at most 32 rows less than one of M 30 go in parts, 0.63 to 0.92 of the time but for one
+//     (1000 x 4096 x 8192 plain 71.3 / 73.0; 992 x 4352 x 13824 with one peer 186 / 117, 1000 x 4224 x 4096 plain 55.1 / 48.1).
 // Which 128x128 kernel, by the time of gemm_ks_kernel over that of gemm_reduce_kernel (geometric means over 20 000 random
 // shapes, 1 to 8192 rows, operands in no cache):
 //   transposed B, in parts: 1.034 to 1.042 at every K: gemm_reduce_kernel.  In one pass, K a multiple of 64, no peers:
@@ -659,7 +660,7 @@ static SmallPlan plan_small(int64_t M, int64_t N, int64_t K, bool b_nt, int n_pe
     const EnvSwitches& env = env_switches();
     const int64_t force = env.gemm_tailsplit;   // 0: off, n: n parts (testing)
     const bool whole = M % 256 == 0 && N % 256 == 0;
-    const bool as_before = K < 2048 || (K % 64 != 0 && (K % 16 != 0 || whole)) || (!whole && b_nt && n_peers < 2 && tiles > 128 && tiles <= 272 && N % 128 == 0 && M % 128 >= 96);   // see above
+    const bool as_before = K < 2048 || (K % 64 != 0 && (K % 16 != 0 || whole));   // see above
     if (may_big && dtl_ok && force != 0 && (env.gemm_mfma != 32 || (whole && K % 64 == 0)) && (!as_before || force > 0)) {
         // whole tiles, K from 4096 on, as many parts as there are compute units for: no margin
         const int64_t most = std::min<int64_t>({256 / std::max<int64_t>(1, big_tiles_of(M, N, 256)), kMaxTailSplits, steps / kMinSplitSteps});
