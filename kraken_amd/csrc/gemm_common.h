@@ -356,13 +356,14 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
     // ---- up to seven peers, and the wave has rows of the band -----------------------------------
     // Straight-line batches of kBatch chunks, peer loads double-buffered one batch ahead across slab boundaries.  A chunk's
     // row goes to `out` or to c_full, lane by lane (edges of the matrix and of the band), and neither loads nor stores are
-    // under a branch, where the waits could not count them: a lane outside the band loads a valid address, a peer past the
-    // last repeats the last one and is masked, and both stores go out, out of range where they are not meant.
+    // under a branch, where the waits could not count them: a lane outside the band loads a valid address, a peer that is not
+    // there is one address of the first one for all lanes and is masked, and both stores go out, out of range where they are not meant.
+    // (Four peers that read the last one four times: 2520 x 7232 x 1024 83.4 us, 700 x 4160 x 1024 with an fp32 result 22.7; so 80.7, 21.7.)
     // Tiles at the edges used to take the loads behind the stores, as below, also for rows outside the band, and held up the
     // others: 7392 x 5056 x 896 with a band and seven peers 128 -> 96 us, 2520 x 7232 x 1024 70.5 -> 51.6, 1448 x 2048 x 832
     // 20.5 -> 16.9, fp32 results 700 x 4160 x 1024 with one peer 20.1 -> 17.8.
     auto with_peers = [&](auto np_c) __attribute__((always_inline)) {
-        constexpr int P = decltype(np_c)::value;
+        constexpr int P = decltype(np_c)::value, kSure = P > 3 ? 4 : 1;   // peers that are there whatever the call
         constexpr int kBatch = (P <= 3 ? 2 : 1) * (BM >= 256 ? 2 : 1), kBatches = EP_ITERS / kBatch;
         static_assert(EP_ITERS % kBatch == 0 && kBatches % 2 == 0, "the two peer buffers alternate with a static parity");
         constexpr uint32_t kOob = 0x80000000u;
@@ -383,7 +384,10 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
                 const int m = row_of(chunk_abs + c);
                 const int64_t off = inside(m) ? (int64_t)(m - band_lo) * g.N + n : safe_off;
 #pragma unroll
-                for (int q = 0; q < P; ++q) pv[buf][c][q] = ld_stream((const u32x4*)((const uint16_t*)g.peer.p[min(q, n_peers - 1)] + off));
+                for (int q = 0; q < P; ++q) {
+                    const bool there = q < kSure || q < n_peers;
+                    pv[buf][c][q] = ld_stream((const u32x4*)((const uint16_t*)g.peer.p[there ? q : 0] + (there ? off : 0)));
+                }
             }
         };
         issue(std::integral_constant<int, 0>{}, 0);
@@ -408,8 +412,12 @@ __device__ __forceinline__ void gemm_epilogue_impl(const GemmArgs& g, const int 
                 for (int c = 0; c < kBatch; ++c) {
 #pragma unroll
                     for (int q = 0; q < P; ++q) {
-                        const uint32_t keep = q < n_peers ? 0xffffffffu : 0u;
                         const u32x4 v = pv[b & 1][c][q];
+                        if (q < kSure) {
+                            add8(v, f[c]);
+                            continue;
+                        }
+                        const uint32_t keep = q < n_peers ? 0xffffffffu : 0u;
                         add8(u32x4{v.x & keep, v.y & keep, v.z & keep, v.w & keep}, f[c]);
                     }
 #pragma unroll

@@ -1927,6 +1927,17 @@ def test_epilogue_at_the_edges(dev, tile, M, N, K, P):
         assert torch.equal(c[:lo].float(), want[:lo]) and torch.equal(c[hi:].float(), want[hi:]) and bool(c[lo:hi].isnan().all())
 
 
+@pytest.mark.parametrize("P", [1, 2, 4, 5, 6])
+@pytest.mark.parametrize("M,N", [(264, 328), (3, 8)])
+def test_epilogue_of_peers_that_are_not_there(dev, tile, M, N, P):
+    """Fewer peers than the epilogue's form has room for: what it reads in their place (values that are not finite here) is not added."""
+    a, b, peers = _small_integers((M, 72), 1, 1.0, dev), _small_integers((72, N), 2, 0.25, dev), _small_integers((P, M, N), 3, 1.0, dev)
+    peers[0, 0, :8] = torch.tensor([float("inf"), float("-inf"), 1, 2, 3, 4, 5, float("inf")])
+    for dtype in (BF16, torch.float32):
+        out = fused.gemm_one_shot_all_reduce_fused(a, b, peers=peers, out_dtype=dtype)
+        assert torch.equal(out.float(), a.float() @ b.float() + peers.float().sum(0))
+
+
 @pytest.mark.parametrize("parts", [0, 3])
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("M,N,K,W,rank", [(65, 8, 8, 1, 0), (128, 264, 40, 2, 1), (256, 256, 64, 2, 0), (260, 520, 72, 4, 2), (520, 328, 1000, 8, 7)])
