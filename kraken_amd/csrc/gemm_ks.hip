@@ -51,7 +51,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_ks_kernel(const GemmArgs g) 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int mh = wave >> 1, kh = wave & 1;   // rows 64 mh .. +63 of the tile, k 32 kh .. +31 of a stage
     int tile_m, tile_n;
-    tile_of(g, blockIdx.x, 0, tile_m, tile_n);
+    // (no band region here, and 0.2 us less than tile_of: 256 x 4096 x 2048 with one peer 23.4 / 23.2 us, 512 x 5120 x 1536 19.0 / 18.8)
+    tile_schedule(g, schedule_position(g, blockIdx.x), tile_m, tile_n);
     const int m0 = tile_m * BT, n0 = tile_n * BT;
     // k-steps of this workgroup: all of them, or the share of split blockIdx.y
     const int kt_all = (g.K + BKS - 1) / BKS;
