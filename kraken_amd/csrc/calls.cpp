@@ -388,13 +388,26 @@ Done product(const at::Tensor& a, const at::Tensor& b, const at::Tensor* peers, 
     if (bias != nullptr && (bias->dim() != 1 || bias->size(0) != N || bias->get_device() != index)) return kNotHere;
     if (c_full != nullptr && (c_full->dim() != 2 || c_full->size(0) != M || c_full->size(1) != N || c_full->get_device() != index)) return kNotHere;
     // (fp32: strides the kernels refuse, and more tiles than the one that splits in registers is for, go the general way)
-    const bool pairs = f32 && gemm_f32_pairs(M, N, K) == 1;
+    bool pairs = f32 && gemm_f32_pairs(M, N, K) == 1;
+    const bool few = ((M + 127) / 128) * ((N + 127) / 128) <= 512;
     if (f32 && (a.stride(0) < K || (b.stride(1) == 1 ? b.stride(0) < N : b.stride(1) < K))) return kNotHere;
-    if (f32 && !pairs && ((M + 127) / 128) * ((N + 127) / 128) > 512) return kNotHere;
+    if (f32 && !pairs && !few) return kNotHere;
+    at::Tensor parts;
+    {
+        const NoGil released;
+        out = at::empty({rows, N}, a.options().dtype(out_fp32 ? at::kFloat : at::kBFloat16));
+        if (pairs) {
+            try {
+                parts = at::empty({M + N, (K + 31) / 32 * 64}, a.options().dtype(at::kBFloat16));
+            } catch (const c10::OutOfMemoryError&) {     // (in registers it needs no memory)
+                if (!few) throw;
+                pairs = false;
+            }
+        }
+    }
     const Scratch ws(index, pairs ? gemm_pairs_workspace_bytes(M, N, K) : f32 ? gemm_f32_workspace_bytes(M, N, K) : gemm_workspace_bytes(M, N, K), stream);
     if (PyErr_Occurred()) return kError;
     const NoGil released;
-    out = at::empty({rows, N}, a.options().dtype(out_fp32 ? at::kFloat : at::kBFloat16));
     const void *ap = a.const_data_ptr(), *bp = b.const_data_ptr();
     const void* pp = peers != nullptr ? peers->const_data_ptr() : nullptr;
     const void* biasp = bias != nullptr ? bias->const_data_ptr() : nullptr;
@@ -407,9 +420,7 @@ Done product(const at::Tensor& a, const at::Tensor& b, const at::Tensor* peers, 
         const void* table[KR_MAX_WORLD];
         for (int q = 0; q < P; ++q) table[q] = (const uint16_t*)pp + q * pstride;
         if (pairs) {
-            const int64_t width = (K + 31) / 32 * 64;
-            const at::Tensor parts = at::empty({M + N, width}, a.options().dtype(at::kBFloat16));
-            uint16_t *apart = (uint16_t*)parts.mutable_data_ptr(), *bpart = apart + M * width;
+            uint16_t *apart = (uint16_t*)parts.mutable_data_ptr(), *bpart = apart + M * parts.size(1);
             rc = split_pairs_fp32(ap, a.stride(0), bp, b.stride(0), b.stride(1), M, N, K, apart, bpart, stream);
             if (rc == KR_OK)
                 rc = gemm_reduce_pairs_ws(apart, bpart, M, N, K, table, P, biasp, row0, rows, cp, op, out_fp32, pivot, ws.p, ws.bytes, stream);

@@ -153,10 +153,15 @@ def launch(name, a, b, M, N, peers, n_peers, peers_stride, bias, band_row0, band
         plist = peers if isinstance(peers, (list, tuple)) else [] if peers is None else list(peers)
         dev = _lib.require_device(a, b, *plist, bias, c_full, out)
         table = (ctypes.c_void_p * max(n_peers, 1))(*[t.data_ptr() for t in plist])
+        width, pairs = -(-K // 32) * 64, None
         if fp32_pairs(a, b):
+            try:
+                pairs = torch.empty((M + N, width), dtype=torch.bfloat16, device=dev)
+            except torch.OutOfMemoryError:      # in registers it needs no memory
+                if not fp32_direct(a, b):
+                    raise
+        if pairs is not None:
             stream = _lib.current_stream(dev)
-            width = -(-K // 32) * 64
-            pairs = torch.empty((M + N, width), dtype=torch.bfloat16, device=dev)
             ap, bp = pairs.data_ptr(), pairs.data_ptr() + M * width * 2
             rc = lib.kr_split_pairs_fp32(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), b.stride(1), M, N, K, ap, bp, stream)
             _lib.check(rc, name)

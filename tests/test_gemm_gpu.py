@@ -1979,6 +1979,34 @@ def test_fp32_operands_as_pairs(dev, monkeypatch, M, N, K, W, rank, b_t, parts):
         assert torch.equal(c[:lo], want[:lo].to(BF16)) and torch.equal(c[hi:], want[hi:].to(BF16))
 
 
+@pytest.mark.parametrize("b_t", [False, True])
+def test_fp32_operands_as_pairs_without_memory_for_them(dev, b_t):
+    """A shape whose parts take 165 MB that are not to be had: it runs in registers.  Integers as above, exact."""
+    from kraken_amd.fused import _gemm
+    M, N, K = 1316, 3136, 9280
+    a, b = _small_integers((M, K), 1, 1.0, dev).float(), _small_integers((K, N), 2, 1.0, dev).float()
+    want = a @ b
+    peers = _small_integers((1, M, N), 3, 1.0, dev)
+    a, b = a.cpu(), (b.T.contiguous().T if b_t else b).cpu()
+    torch.cuda.empty_cache()
+    a, b = a.to(dev), b.to(dev)      # (in memory of their own: no cached rest of it holds the parts)
+    assert _gemm.fp32_pairs(a, b)
+    total = torch.cuda.mem_get_info(dev)[1]
+    try:
+        for given in (peers, list(peers)):      # the native form and the general path
+            _gemm._workspaces.clear()
+            torch.cuda.empty_cache()
+            torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (100 << 20)) / total, dev)
+            with pytest.raises(torch.OutOfMemoryError):
+                torch.empty(4 * (M + N) * K, dtype=torch.uint8, device=dev)
+            out = fused.gemm_one_shot_all_reduce_fused(a, b, peers=given)
+            torch.cuda.set_per_process_memory_fraction(1.0, dev)
+            assert torch.equal(out, want + peers[0].float())
+            del out
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+
+
 def test_fp32_operands_and_a_peer_that_is_not_finite(dev):
     """More than 512 tiles of 128 x 128 and a K of 64: the infinity of one element of a peer stays in that element."""
     M, N, K = 2304, 4096, 64
