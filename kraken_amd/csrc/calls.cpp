@@ -53,7 +53,7 @@ decltype(&kr_gemm_fp8_wide_ws) gemm_fp8_wide_ws;
 PyObject* raw_stream;       // device index -> handle of its current stream
 PyObject* row_exchange;     // (device index, bytes, stream) -> (workspace tensor, status tensor) of the split-row kernel
 PyObject* row_watch;        // (status tensor): look at it once the work enqueued so far is done
-PyObject* gemm_workspace;   // (device index, bytes, stream) -> workspace tensor
+PyObject* gemm_workspace;   // (device index, bytes, stream) -> workspace tensor or None
 PyObject* waits_check;      // (): raises if a bounded wait of an earlier call ran out
 
 struct Ref {                // a reference that is given back
@@ -359,14 +359,14 @@ PyObject* rms_norm(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
 // What a product does where its operands are of a form the kernels read: launched, left to the general path, or a Python error.
 enum Done { kLaunched, kNotHere, kError };
 
-// The stream's scratch, `bytes` of it.
+// The stream's scratch, `bytes` of it; none where none is needed or to be had.
 struct Scratch {
     Ref tensor;
     void* p = nullptr;
     int64_t bytes = 0;
     Scratch(int64_t index, int64_t need, void* stream)
         : tensor(need > 0 ? PyObject_CallFunction(gemm_workspace, "LLK", (long long)index, (long long)need, (unsigned long long)(uintptr_t)stream) : nullptr) {
-        if (tensor.p == nullptr) return;
+        if (tensor.p == nullptr || tensor.p == Py_None) return;
         const at::Tensor& t = THPVariable_Unpack(tensor.p);
         p = t.mutable_data_ptr();
         bytes = t.numel();

@@ -132,12 +132,16 @@ def workspace(dev: torch.device, nbytes: int) -> torch.Tensor | None:
     return stream_workspace(dev.index if dev.index is not None else torch.cuda.current_device(), nbytes, _lib.current_stream(dev))
 
 
-def stream_workspace(index: int, nbytes: int, stream: int) -> torch.Tensor:
-    """``workspace`` for a device index and the handle of its current stream."""
+def stream_workspace(index: int, nbytes: int, stream: int) -> torch.Tensor | None:
+    """``workspace`` for a device index and the handle of its current stream.  Where the memory is not to be had: the
+    smaller buffer that is there, or None; the entry points share fewer K loops then, or none."""
     key = (index, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=torch.device("cuda", index))
+        try:
+            ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=torch.device("cuda", index))
+        except torch.OutOfMemoryError:
+            return ws
         _workspaces[key] = ws
     return ws
 

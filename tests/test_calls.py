@@ -248,6 +248,19 @@ def test_native_calls_run_on_the_current_stream_and_in_a_graph(dev):
         assert torch.equal(out.cpu(), orc.reduce(stack.cpu()))
 
 
+def test_workspace_that_is_not_to_be_had(monkeypatch):
+    from kraken_amd.fused import _gemm
+
+    def full(*args, **kwargs):
+        raise torch.OutOfMemoryError("full")
+
+    small = torch.zeros(8, dtype=torch.uint8)
+    monkeypatch.setattr(_gemm, "_workspaces", {(0, 5): small})
+    monkeypatch.setattr(torch, "empty", full)
+    assert _gemm.stream_workspace(0, 16, 5) is small and _gemm.stream_workspace(0, 16, 7) is None
+    assert _gemm._workspaces == {(0, 5): small}
+
+
 @pytest.mark.parametrize("name,n", [("reduce_scatter_sent", 6), ("gather_matmul", 7)])
 def test_overlap_calls_that_are_not_of_the_common_form(name, n):
     fn = getattr(_lib.calls(), name)

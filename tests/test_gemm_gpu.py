@@ -1979,6 +1979,38 @@ def test_fp32_operands_as_pairs(dev, monkeypatch, M, N, K, W, rank, b_t, parts):
         assert torch.equal(c[:lo], want[:lo].to(BF16)) and torch.equal(c[hi:], want[hi:].to(BF16))
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+def test_products_without_memory_for_their_workspace(dev, fp8):
+    """A last round that runs in parts, and an fp8 product of few tiles in parts: in one pass where the parts have no room."""
+    from kraken_amd.fused import _gemm
+    lib, dt = _lib.load(), torch.float8_e4m3fn if fp8 else BF16
+    M, N, K = (264, 4112, 8192) if fp8 else (4136, 4104, 4096)
+    need = lib.kr_gemm_fp8_wide_workspace_bytes(M, N, K) if fp8 else lib.kr_gemm_workspace_bytes(M, N, K)
+    a, b = _small_integers((M, K), 1, 1.0, dev), _small_integers((N, K), 2, 0.25, dev)
+    want = (a.float() @ b.float().T).to(dt)
+    a, b, out = a.cpu().to(dt), b.cpu().to(dt), M * N * a.element_size()
+    kept = dict(_gemm._workspaces)
+    try:
+        for listed in (False, True):      # the native form and the general path
+            _gemm._workspaces.clear()
+            torch.cuda.empty_cache()
+            ad, bd = a.to(dev), b.to(dev)
+            room = torch.cuda.memory_reserved(dev) + out + need // 2
+            torch.cuda.set_per_process_memory_fraction(room / torch.cuda.mem_get_info(dev)[1], dev)
+            with pytest.raises(torch.OutOfMemoryError):
+                torch.empty(need + out, dtype=torch.uint8, device=dev)
+            if fp8:
+                c = fused.all_gather_matmul(list(ad.view(1, M, K)) if listed else ad.view(1, M, K), bd.T)[1]
+            else:
+                c = fused.gemm_one_shot_all_reduce_fused(ad, bd.T, peers=[] if listed else None, out_dtype=BF16)
+            torch.cuda.set_per_process_memory_fraction(1.0, dev)
+            assert torch.equal(c.float(), want.float())
+            del c, ad, bd
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+        _gemm._workspaces.update(kept)
+
+
 @pytest.mark.parametrize("b_t", [False, True])
 def test_fp32_operands_as_pairs_without_memory_for_them(dev, b_t):
     """A shape whose parts take 165 MB that are not to be had: it runs in registers.  Integers as above, exact."""
