@@ -167,11 +167,14 @@ def _all_gather_matmul_fp8(a_shared, peers: PeerBuffers, b, a_out, progress, **k
     return a_out, c
 
 
-def _common_form(a_shared, b, a_out, progress, rank=0, splits_per_rank=1, gather=None, **kwargs):
+_DEFAULT = object()     # (None that is named means gather=False)
+
+
+def _common_form(a_shared, b, a_out, progress, rank=0, splits_per_rank=1, gather=_DEFAULT, **kwargs):
     """The call in native code where its arguments are of the common form: nothing but sizes named, and no tangents about."""
     if kwargs or forward_ad._current_level >= 0:
         return None
-    if gather is None:
+    if gather is _DEFAULT:
         gather = not isinstance(a_shared, torch.Tensor)     # (a stack that is not contiguous goes the general way in any case)
     if type(gather) is not bool:
         return None

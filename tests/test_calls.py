@@ -261,6 +261,16 @@ def test_workspace_that_is_not_to_be_had(monkeypatch):
     assert _gemm._workspaces == {(0, 5): small}
 
 
+@pytest.mark.parametrize("kw,native", [({}, True), ({"gather": True}, True), ({"gather": False}, False), ({"gather": None}, None), ({"gather": 1}, None)])
+def test_gather_as_it_is_named(monkeypatch, kw, native):
+    """A mode that is named is taken by the native form only as True or False; the default is its own."""
+    from kraken_amd.fused.all_gather_matmul import _common_form
+    seen = []
+    monkeypatch.setattr(_lib, "calls", lambda: type("Calls", (), {"gather_matmul": staticmethod(lambda *args: seen.append(args[6]))}))
+    assert _common_form([torch.zeros(2, 8)], torch.zeros(8, 8), None, None, **kw) is None
+    assert seen == ([] if native is None else [native])
+
+
 @pytest.mark.parametrize("name,n", [("reduce_scatter_sent", 6), ("gather_matmul", 7)])
 def test_overlap_calls_that_are_not_of_the_common_form(name, n):
     fn = getattr(_lib.calls(), name)
@@ -332,7 +342,7 @@ def test_gathered_products_take_both_paths_alike(dev, monkeypatch, m, N, K, W):
         ok = 0
         for (form, shards), (bf, b) in itertools.product(forms.items(), {"columns": rnd(N, K).T, "wide": rnd(N, 2 * K)[:, :K].T, "rows": rnd(K, N)}.items()):
             for kw in ({}, {"gather": True}, {"gather": False}, {"gather": True, "rank": W - 1, "splits_per_rank": 2}, {"gather": True, "splits_per_rank": 3},
-                       {"gather": True, "rank": W}, {"gather": 1}, {"gather": 0}):
+                       {"gather": True, "rank": W}, {"gather": 1}, {"gather": 0}, {"gather": None}):
                 for given in ("both", "neither", "flags", "many flags", "small"):
                     def run():
                         a_out = None if given in ("neither", "flags") else room[:W].reshape(W * m, K) if form == "in the result" else torch.zeros(W * m, K, device=dev).to(dtype)
