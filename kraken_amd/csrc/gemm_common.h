@@ -161,7 +161,6 @@ __device__ __forceinline__ int xcd_position(int wg, int ntiles) {
 __device__ __forceinline__ int schedule_position(const GemmArgs& g, int wg, int first = 0) {
     const int ntiles = g.tiles_m * g.tiles_n;
     if (ntiles % kXcds != 0 && (g.tail_tiles == 0 || g.tail_tiles == ntiles)) return xcd_position(wg, ntiles);
-    if (ntiles % kXcds != 0 && first == 0 && g.tail_tiles % kXcds == ntiles % kXcds) return xcd_position(wg, ntiles - g.tail_tiles);
     if (ntiles % kXcds != 0 && first == 0) return xcd_position(wg, ntiles - g.tail_tiles);
     if (ntiles % kXcds != 0 || first % kXcds != 0) return first + wg;
     return (wg % kXcds) * (ntiles / kXcds) + first / kXcds + wg / kXcds;
