@@ -295,7 +295,8 @@ def test_fp32_products_are_taken(dev, monkeypatch, M, N, K, W):
             assert _same(monkeypatch, lambda: [fused.gemm_one_shot_all_reduce_fused(a, b, bias=bias, out_dtype=dtype)], (b.stride(), dtype))
         assert _same(monkeypatch, lambda: [fused.gemm_reduce_scatter(a, b, peers=peers, rank=W - 1, c_scratch=c), c.clone()], b.stride())
     for odd in (a[:, ::2], rnd(K, M).T, rnd(M * K + 1)[1:].view(M, K), a[:1].expand(M, K), a.double(), a.to(BF16)):
-        _same(monkeypatch, lambda: [fused.gemm_one_shot_all_reduce_fused(odd, rnd(odd.shape[1], N))[:0]], odd.stride())
+        b = rnd(odd.shape[1], N)
+        _same(monkeypatch, lambda: [fused.gemm_one_shot_all_reduce_fused(odd, b)], (odd.dtype, odd.stride()))
 
 
 @pytest.mark.gpu

@@ -1725,19 +1725,22 @@ def test_fp32_operands_split_in_registers(dev, monkeypatch, M, N, K, b_t):
         assert ((out - ar.double() @ br.double()).abs() <= 2.0 ** -15 * (ar.abs().double() @ br.abs().double())).all(), splits
 
 
+@pytest.mark.parametrize("pairs", [None, "0"])
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("M,N,K", [(2304, 4096, 256), (2200, 4104, 72), (256, 4096, 260)])
-def test_fp32_operands_split_in_a_pass(dev, M, N, K, b_t):
-    """More than 512 tiles of 128 x 128, and a K that is no multiple of 8: the operands are split by a pass of their own
-    and multiplied as a bf16 product of 3K.  Integers up to 2^11 (hi and lo parts exact) times integers up to 8, every
-    sum below 2^24: exact."""
+def test_fp32_operands_split_in_a_pass(dev, monkeypatch, M, N, K, b_t, pairs):
+    """More than 512 tiles of 128 x 128: the operands are split by a pass of their own, as pairs, and with KRAKEN_AMD_GEMM_PAIRS=0, and for a K
+    that is no multiple of 8, into three blocks that are multiplied as a bf16 product of 3K.  Integers up to 2^11 (hi and lo
+    parts exact) times integers up to 8, every sum below 2^24: exact."""
     from kraken_amd.fused import _gemm
+    if pairs is not None:
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_PAIRS", pairs)
     g = torch.Generator().manual_seed(K)
     a = torch.randint(-2047, 2048, (M, K), generator=g).float().to(dev)
     b = torch.randint(-8, 9, (K, N), generator=g).float().to(dev)
     assert K * 2047 * 8 < 1 << 24
     bd = b.T.contiguous().T if b_t else b
-    assert not _gemm.fp32_direct(a, bd)
+    assert not _gemm.fp32_direct(a, bd) and _gemm.fp32_pairs(a, bd) == (pairs is None and K % 8 == 0)
     assert torch.equal(fused.gemm_one_shot_all_reduce_fused(a, bd), a @ b)
 
 
@@ -1863,12 +1866,12 @@ def _small_integers(shape, seed, density, dev):
     (2312, 4104, 264, 8, 3),       # the band's tiles ahead of the others, both its edges inside a tile
     (2312, 4104, 264, 8, 7),       # ... the last band, which ends with the matrix
     (3000, 3000, 72, 4, 0), (6144, 3072, 128, 2, 1), (2560, 4096, 64, 2, 0),
-    (520, 2056, 4112, 8, 3), (736, 3608, 4144, 8, 7), (504, 6656, 4112, 8, 0), (944, 2960, 6944, 2, 1),
-    (4104, 4096, 3080, 4, 2), (5632, 4224, 8192, 8, 0)])      # few tiles, all in parts, the last k-step not full
+    (4104, 4096, 3080, 4, 2), (5632, 4224, 8192, 8, 0),      # 272 tiles, 16 in four parts; 374 tiles, 118 in two
+    (520, 2056, 4112, 8, 3), (736, 3608, 4144, 8, 7), (504, 6656, 4112, 8, 0), (944, 2960, 6944, 2, 1)])      # few tiles, all in parts, the last k-step not full
 def test_reduce_scatter_of_many_tiles(dev, M, N, K, W, rank, b_t):
-    """More than 128 tiles of 256 x 256.  Operands of -1, 0, 1 (a quarter of b's are not zero, an eighth with a
-    K above 5000): every sum is an integer far below 256 (six standard deviations at K = 4160: 160, at K = 8192: 160; seven peers
-    7), so product, sum and rounding are exact."""
+    """More than 128 tiles of 256 x 256, and fewer that are all in parts.  Operands of -1, 0, 1 (a sixth of b's are not zero, a twelfth with a
+    K above 5000; two thirds of a's): every sum is an integer far below 256 (six standard deviations at K = 4160: 129, at
+    K = 8192: 128; seven peers 7), so product, sum and rounding are exact."""
     a, b = _small_integers((M, K), 1, 1.0, dev), _small_integers((K, N), 2, 0.25 if K <= 5000 else 0.125, dev)
     peers = _small_integers((W - 1, M // W, N), 3, 1.0, dev)
     c = torch.full((M, N), float("nan"), dtype=BF16, device=dev)
@@ -1977,6 +1980,35 @@ def test_fp32_operands_as_pairs(dev, monkeypatch, M, N, K, W, rank, b_t, parts):
         lo, hi = rank * rows, (rank + 1) * rows
         assert out.dtype == torch.float32 and torch.equal(out.double(), want[lo:hi] + mine.double().sum(0))
         assert torch.equal(c[:lo], want[:lo].to(BF16)) and torch.equal(c[hi:], want[hi:].to(BF16))
+
+
+@pytest.mark.parametrize("where", [None, "mfma", "first", "last", "epilogue"])
+@pytest.mark.parametrize("M,N,K,W,rank", [
+    (2304, 4096, 128, 2, 1),       # 144 whole tiles, the band starts inside a tile
+    (2312, 4104, 192, 8, 3),       # ragged rows and columns
+    (2304, 4096, 72, 3, 0),        # a K that is no multiple of 64: peers in the epilogue whatever is asked for
+    (4136, 4104, 1024, 2, 0),      # 289 tiles, 33 of them in parts behind a whole round
+    (4352, 4096, 1024, 8, 7)])     # 272, 16 in parts
+def test_fp32_operands_as_pairs_in_whole_rounds(dev, monkeypatch, M, N, K, W, rank, where):
+    """More than 512 tiles of 128 x 128, the route of such calls: peers on the matrix cores, ahead of the k loop and behind it, and in the
+    epilogue.  Integers as above, exact."""
+    from kraken_amd.fused import _gemm
+    if where is not None:
+        monkeypatch.setenv("KRAKEN_AMD_GEMM_PEERS", where)
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    rnd = lambda v, *s: torch.randint(-v, v + 1, s, generator=g, device=dev)      # noqa: E731
+    a, b, bias = rnd(2047, M, K).float(), rnd(8, N, K).float(), rnd(8, N).to(BF16)
+    peers = rnd(8, W - 1, M, N).to(BF16)
+    assert K * 2047 * 8 + W * 8 < 1 << 24 and _gemm.fp32_pairs(a, b.T)
+    assert (_lib.load().kr_gemm_pairs_workspace_bytes(M, N, K) > 0) == (K == 1024)
+    want = a.double() @ b.double().T
+    out = fused.gemm_one_shot_all_reduce_fused(a, b.T, peers=peers, bias=bias)
+    assert out.dtype == torch.float32 and torch.equal(out.double(), want + peers.double().sum(0) + bias.double())
+    mine, c = peers[:, :M // W].contiguous(), torch.full((M, N), float("nan"), dtype=BF16, device=dev)
+    out = fused.gemm_reduce_scatter(a, b.T, peers=mine, rank=rank, c_scratch=c)
+    lo, hi = rank * (M // W), (rank + 1) * (M // W)
+    assert torch.equal(out.double(), want[lo:hi] + mine.double().sum(0))
+    assert torch.equal(c[:lo], want[:lo].to(BF16)) and torch.equal(c[hi:], want[hi:].to(BF16)) and bool(c[lo:hi].isnan().all())
 
 
 @pytest.mark.parametrize("fp8", [False, True])
