@@ -609,7 +609,7 @@ static int64_t split_k_workspace_bytes(int64_t M, int64_t N, int S) { return (in
 //     a K that is no multiple of 64, which makes no difference to the parts and costs the 128x128 forms more: 18 of 64 shapes go in
 //     parts, 0.52 to 0.96 of the time (3144 x 1392 x 15472 270 / 141, 3224 x 1248 x 7136 row-major with a band 142 / 75, 736 x 6416
 //     x 5680 105 / 78, 1016 x 3728 x 2512 38.4 / 36.5); with transposed B and at most one peer 27 of 60 shapes of 129 to 272 tiles,
-//     0.52 to 1.00 (944 x 4240 x 13360 with one peer 247 / 129, 1100 x 1856 x 13616 plain 233 / 122, 1144 x 2320 x 6784 69 / 58); of
+//     0.52 to 1.00 (944 x 4240 x 13360 with one peer 247 / 129, 2200 x 1856 x 13616 plain 233 / 122, 1144 x 2320 x 6784 69 / 58); of
 //     54 of those with N a multiple of 128 and at most 32 rows less than one of M 30 go in parts, 0.63 to 0.92 of the time but for one
 //     (1000 x 4096 x 8192 plain 71.3 / 73.0; 992 x 4352 x 13824 with one peer 186 / 117, 1000 x 4224 x 4096 plain 55.1 / 48.1).
 // Which 128x128 kernel, by the time of gemm_ks_kernel over that of gemm_reduce_kernel (geometric means over 20 000 random
@@ -1108,8 +1108,8 @@ static int gemm_reduce(const void* A, int64_t lda_m, int64_t lda_k, const void* 
     g.pivot_tiles = (int)(((pt % g.tiles_m) + g.tiles_m) % g.tiles_m);
     // 256-row tiles with a band: the band's tiles as a region of their own at the head of the order, dealt to all XCDs, the others behind
     // them.  In one order the band lies with one to four of the XCDs, whose compute units are then the last to get to the tiles beyond the
-    // first round: us, one order / two regions, 6144 x 3072 x 2048 (288 tiles, one peer) 102.5 / 86.0, 3000 x 3000 x 600 34.1 / 26.7,
-    // 7392 x 5056 x 896 (580 tiles, seven peers) 96.0 / 78.6, 8192 x 4096 x 1024 72.7 / 63.6.  An XCD then works on two sets of
+    // first round: us, one order / two regions, 6144 x 3072 x 2048 (288 tiles, one peer) 102.5 / 86.0, 3000 x 3000 x 600 37.6 / 34.9,
+    // 7392 x 5056 x 896 (580 tiles, seven peers) 96.0 / 78.6, 8192 x 4096 x 1024 with one peer 72.7 / 63.6.  An XCD then works on two sets of
     // panels at first, which a long K does not win back: 8192 x 8192 x 3584 343 / 352, 5000 x 5000 x 5000 234 / 242, 4600 x 6000 x 4096
     // 192 / 186, 7360 x 3328 x 3072 155 / 134.
     g.band_tile0 = g.band_tile_rows = 0;
